@@ -17,7 +17,7 @@ namespace mi355 {
 
 #pragma clang fp contract(off)
 
-template <int UNROLL, bool ROW_MAJOR_SCALES>
+template <int UNROLL, bool ROW_MAJOR_SCALES, bool F16>
 __global__ __launch_bounds__(256) void group_quant_kernel(const v4i *__restrict__ x, v2i *__restrict__ q,
                                                           float *__restrict__ s, uint32_t total_chunks,
                                                           uint32_t groups_per_row, int64_t s_stride_m,
@@ -33,24 +33,25 @@ __global__ __launch_bounds__(256) void group_quant_kernel(const v4i *__restrict_
     for (int u = 0; u < UNROLL; ++u) {
         uint32_t c = base + u * 256u;
         if (c < total_chunks) {  // total_chunks is a multiple of 16: a DPP row is active or idle as a whole
-            v2i o;
-            float sc;
-            quant_chunk(v[u], o, sc);
-            __builtin_nontemporal_store(o, q + c);
+            const v4i in[1] = {v[u]};
+            v2i o[1];
+            float sc[1];
+            quant_chunks<F16, 1>(in, o, sc);
+            __builtin_nontemporal_store(o[0], q + c);
             if ((threadIdx.x & 15u) == 0) {
                 uint32_t g = c >> 4;
                 if (ROW_MAJOR_SCALES) {
-                    s[g] = sc;
+                    s[g] = sc[0];
                 } else {
                     uint32_t row = g / groups_per_row, col = g - row * groups_per_row;
-                    s[(int64_t)row * s_stride_m + (int64_t)col * s_stride_g] = sc;
+                    s[(int64_t)row * s_stride_m + (int64_t)col * s_stride_g] = sc[0];
                 }
             }
         }
     }
 }
 
-// fp16 and fp32 activations (the reference widens any input dtype to fp32 first,
+// fp32 activations, and 16-bit ones with an eps of their own (the reference widens any input dtype to fp32 first,
 // quantization/fp8act_quant_kernel.py:52): one lane = 8 elements, true divisions.  Not the hot path.
 template <typename T>
 __global__ __launch_bounds__(256) void group_quant_wide_kernel(const T *__restrict__ x, v2i *__restrict__ q,
@@ -69,7 +70,7 @@ __global__ __launch_bounds__(256) void group_quant_wide_kernel(const T *__restri
             f[4 + i] = as_f32((uint32_t)b[i]);
         }
     } else if constexpr (sizeof(T) == 2 && !__is_same(T, _Float16)) {
-        // bf16 bits (T = uint16_t): the path of a non-default eps, whose floor is no bf16 value
+        // bf16 bits (T = uint16_t)
         const v4i a = __builtin_nontemporal_load((const v4i *)x + c);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -77,7 +78,6 @@ __global__ __launch_bounds__(256) void group_quant_wide_kernel(const T *__restri
             f[2 * i + 1] = as_f32((uint32_t)a[i] & 0xffff0000u);
         }
     } else {
-        typedef _Float16 h8 __attribute__((ext_vector_type(8)));
         const h8 h = __builtin_bit_cast(h8, __builtin_nontemporal_load((const v4i *)x + c));
 #pragma unroll
         for (int i = 0; i < 8; ++i) f[i] = (float)h[i];
@@ -128,7 +128,6 @@ __global__ __launch_bounds__(256) void group_quant_any_kernel(const T *__restric
                 f[2 * i + 1] = as_f32((uint32_t)a[i] & 0xffff0000u);
             }
         } else {
-            typedef _Float16 h8 __attribute__((ext_vector_type(8)));
             const h8 h = __builtin_bit_cast(h8, *((const v4i *)xg + c));
 #pragma unroll
             for (int i = 0; i < 8; ++i) f[i] = (float)h[i];
@@ -221,25 +220,33 @@ extern "C" int mi355_group_quant_fp8(const void *x, int32_t x_dtype, void *q, fl
     const bool row_major = (s_stride_g == 1 && s_stride_m == (int64_t)G) || (M == 1 && s_stride_g == 1) ||
                            (G == 1 && s_stride_m == 1);
     const int eps_default = (eps == 1e-10f) ? 1 : 0;
-    constexpr int UNROLL = 4;
-    uint32_t blocks = (uint32_t)((chunks + 256 * UNROLL - 1) / (256 * UNROLL));
     hipStream_t st = (hipStream_t)stream;
     if (x_dtype == MI355_DTYPE_F32)
         return launch(group_quant_wide_kernel<float>, dim3((uint32_t)((chunks + 255) / 256)), dim3(256), 0, st,
                       (const float *)x, (v2i *)q, s, (uint32_t)chunks, G, s_stride_m, s_stride_g, eps);
-    if (x_dtype == MI355_DTYPE_F16)
-        return launch(group_quant_wide_kernel<_Float16>, dim3((uint32_t)((chunks + 255) / 256)), dim3(256), 0, st,
-                      (const _Float16 *)x, (v2i *)q, s, (uint32_t)chunks, G, s_stride_m, s_stride_g, eps);
-    // The two-FMA quotient of the bf16 kernel is proven for scales RN(amax/448) of a bf16 amax and of the default
+    const bool f16 = x_dtype == MI355_DTYPE_F16;
+    // The short quotient of the 16-bit kernels is proven for scales RN(amax/448) of a 16-bit amax and of the default
     // floor 1e-10 only; with any other eps a group below the floor has a scale outside that set, so such calls take
     // the kernel with true divisions (fp8act_quant_kernel.py:63-113 hands eps through to the kernel).
-    if (!eps_default)
+    if (!eps_default) {
+        if (f16)
+            return launch(group_quant_wide_kernel<_Float16>, dim3((uint32_t)((chunks + 255) / 256)), dim3(256), 0, st,
+                          (const _Float16 *)x, (v2i *)q, s, (uint32_t)chunks, G, s_stride_m, s_stride_g, eps);
         return launch(group_quant_wide_kernel<uint16_t>, dim3((uint32_t)((chunks + 255) / 256)), dim3(256), 0, st,
                       (const uint16_t *)x, (v2i *)q, s, (uint32_t)chunks, G, s_stride_m, s_stride_g, eps);
-    if (row_major)
-        return launch((group_quant_kernel<UNROLL, true>), dim3(blocks), dim3(256), 0, st, (const v4i *)x,
-                           (v2i *)q, s, (uint32_t)chunks, G, s_stride_m, s_stride_g);
-    else
-        return launch((group_quant_kernel<UNROLL, false>), dim3(blocks), dim3(256), 0, st, (const v4i *)x,
-                           (v2i *)q, s, (uint32_t)chunks, G, s_stride_m, s_stride_g);
+    }
+    // Four chunks per lane where that still gives every compute unit two workgroups, else one: a small input is bound by
+    // the latency of its one load, and the arithmetic of four chunks in a row behind it only adds to that ([8, 14336]
+    // and [64, 4096]: 2.7 us a launch in a captured graph with four, 1.95 with one, where an empty kernel takes 1.8;
+    // [640, 4096]: 3.3 and 2.6; from [1024, 4096] on the two are level).
+    auto go = [&](auto unroll) {
+        constexpr int U = decltype(unroll)::value;
+        const auto kernel = row_major ? (f16 ? group_quant_kernel<U, true, true> : group_quant_kernel<U, true, false>)
+                                      : (f16 ? group_quant_kernel<U, false, true> : group_quant_kernel<U, false, false>);
+        const uint32_t blocks = (uint32_t)((chunks + 256 * U - 1) / (256 * U));
+        return launch(kernel, dim3(blocks), dim3(256), 0, st, (const v4i *)x, (v2i *)q, s, (uint32_t)chunks, G, s_stride_m,
+                      s_stride_g);
+    };
+    if (chunks >= (int64_t)device_cus() * 2048) return go(std::integral_constant<int, 4>{});
+    return go(std::integral_constant<int, 1>{});
 }

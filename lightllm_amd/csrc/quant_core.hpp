@@ -6,18 +6,21 @@
 //     amax = max(max|x|, eps);  s = amax / 448;  q = e4m3fn_rtne(clamp(x / s, -448, 448))
 // Doing two IEEE divisions per element would make the kernels VALU-bound, so:
 //   * s = amax/448 is formed as q0 = amax*c, s = fma(fma(-q0,448,amax), c, q0) with c = RN(1/448);
-//     this equals RN(amax/448) for every bf16 amax and for the default eps (checked exhaustively on
+//     this equals RN(amax/448) for every bf16 and every fp16 amax and for the default eps (checked exhaustively on
 //     the CPU); calls with any other eps do not come here (they take quant_chunk_f32).
-//   * x/s is formed as y0 = x*r, y = fma(fma(-y0,s,x), r, y0) with r = RN(1/s) (a true division,
-//     once per lane).  For every pair (bf16 amax, bf16 |x| <= amax) this equals RN(x/s) whenever
-//     |x/s| >= 2^-10, and below that both round to the e4m3 zero - also checked exhaustively on the CPU
-//     (oracle_fast_quant_mismatches in the test oracle replays exactly these operations).
+//   * x/s is formed as y = fma(x, r, x*d) from r, a little under 1/s (v_rcp_f32, two ulps taken off), and the rest
+//     d = fma(-s, r, 1) * r >= 0 that r + d misses 1/s by no more than 2^-46 of: two operations per element.  For every
+//     pair (amax, |x| <= amax) of bf16 or of fp16 values the e4m3 byte of y is that of RN(x/s), whatever the last bit of
+//     the reciprocal is - also checked exhaustively on the CPU (oracle_fast_quant_mismatches in the test oracle replays exactly these
+//     operations for a reciprocal off by -1, 0 and +1 ulp).  With r and d positive -0 stays -0, as -0/s is.
 #pragma once
 #include "common.hpp"
 
 namespace mi355 {
 
-#pragma clang fp contract(off)
+// (no contraction of a product and a sum anywhere in this arithmetic; the pragma stands inside each function so that
+// it does not reach the rest of a file that includes this one)
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp_max_u32(uint32_t v) {
@@ -39,17 +42,6 @@ __device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b) {
     return __builtin_bit_cast(uint32_t, r);
 }
 
-// RN(x/s) wherever it matters (see the header), with the sign taken from x: the correction step turns
-// -0 into +0, and the reference's -0/s = -0 keeps its sign bit through the cast (byte 0x80).
-// No clamp is needed: |x| <= amax and s = RN(max(amax,eps)/448) bound |x/s| by 448*(1+2^-23), which the
-// e4m3 cast rounds to 448, exactly what clamp-then-cast gives.
-__device__ __forceinline__ float quot(float x, float s, float r) {
-    float y0 = x * r;
-    float e = __builtin_fmaf(-y0, s, x);
-    float y = __builtin_fmaf(e, r, y0);
-    return as_f32((as_u32(y) & 0x7fffffffu) | (as_u32(x) & 0x80000000u));
-}
-
 // A group that holds a NaN or an infinity (outside the reference's contract: its max and clamp leave NaN
 // unspecified) is poisoned as a whole: scale = NaN, every byte 0x7F with the sign bit of its element.
 __device__ __forceinline__ void nonfinite_chunk(uint32_t s0, uint32_t s1, uint32_t s2, uint32_t s3, uint32_t s4,
@@ -59,9 +51,10 @@ __device__ __forceinline__ void nonfinite_chunk(uint32_t s0, uint32_t s1, uint32
     scale = as_f32(0x7fc00000u);
 }
 
-// Quantize 8 consecutive fp32 values (fp16 / fp32 activations, widened by the caller) with true IEEE divisions:
-// the two-FMA quotient above is only proven for bf16 inputs.
+// Quantize 8 consecutive fp32 values (fp32 activations, or any with another eps, widened by the caller) with true IEEE
+// divisions: the short quotient above is only proven for 16-bit inputs and the default eps.
 __device__ __forceinline__ void quant_chunk_f32(const float (&f)[8], float eps, v2i &out, float &scale) {
+#pragma clang fp contract(off)
     uint32_t mx = 0;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -94,42 +87,82 @@ __device__ __forceinline__ void quant_chunk_f32(const float (&f)[8], float eps, 
     scale = s;
 }
 
-// Quantize one 16-byte chunk of bf16 with the default floor eps = 1e-10; the group amax is shared through the DPP row.
-__device__ __forceinline__ void quant_chunk(const v4i &v, v2i &out, float &scale) {
-    constexpr float eps = 1e-10f;
-    uint32_t d0 = (uint32_t)v[0], d1 = (uint32_t)v[1], d2 = (uint32_t)v[2], d3 = (uint32_t)v[3];
-    // |x| as integers: for non-negative floats the integer order is the float order.
-    uint32_t m = pk_max_u16(pk_max_u16(d0 & 0x7fff7fffu, d1 & 0x7fff7fffu),
-                            pk_max_u16(d2 & 0x7fff7fffu, d3 & 0x7fff7fffu));
-    uint32_t hi = m >> 16, lo = m & 0xffffu;
-    uint32_t mx = (hi > lo ? hi : lo) << 16;
-    mx = row16_max_u32(mx);
-    if (mx > 0x7f7fffffu) {  // the same for all 16 lanes of the group
-        nonfinite_chunk((d0 >> 15) & 1u, d0 >> 31, (d1 >> 15) & 1u, d1 >> 31, (d2 >> 15) & 1u, d2 >> 31,
-                        (d3 >> 15) & 1u, d3 >> 31, out, scale);
-        return;
-    }
-    float amax = as_f32(mx);
-    amax = amax > eps ? amax : eps;
-    const float c = 1.0f / 448.0f;
-    float q0 = amax * c;
-    const float s = __builtin_fmaf(__builtin_fmaf(-q0, 448.0f, amax), c, q0);
-    float r = 1.0f / s;
-    float f[8];
-    f[0] = as_f32(d0 << 16); f[1] = as_f32(d0 & 0xffff0000u);
-    f[2] = as_f32(d1 << 16); f[3] = as_f32(d1 & 0xffff0000u);
-    f[4] = as_f32(d2 << 16); f[5] = as_f32(d2 & 0xffff0000u);
-    f[6] = as_f32(d3 << 16); f[7] = as_f32(d3 & 0xffff0000u);
+// Quantize N 16-byte chunks of bf16 (F16: fp16) with the default floor eps = 1e-10; the group amax is shared through the DPP row.
+// About 50 vector operations per chunk.  (Chunks of one lane are interleaved; non-finite groups are handled behind one
+// test that the whole wave takes or skips.)  No clamp is needed: |x| <= amax and s = RN(max(amax,eps)/448) bound |x/s| by
+// 448*(1+2^-23), which the e4m3 cast rounds to 448, exactly what clamp-then-cast gives.
+template <bool F16, int N>
+__device__ __forceinline__ void quant_chunks(const v4i (&v)[N], v2i (&out)[N], float (&scale)[N]) {
+#pragma clang fp contract(off)
+    constexpr uint32_t kEps = 0x2edbe6ffu;  // 1e-10f
+    uint32_t mx[N];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) f[i] = quot(f[i], s, r);
-    int w0 = 0, w1 = 0;
-    w0 = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], w0, false);
-    w0 = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], w0, true);
-    w1 = __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], w1, false);
-    w1 = __builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], w1, true);
-    out[0] = w0;
-    out[1] = w1;
-    scale = s;
+    for (int k = 0; k < N; ++k) {
+        // |x| as integers: for non-negative floats the integer order is the float order.
+        const uint32_t m = pk_max_u16(pk_max_u16((uint32_t)v[k][0] & 0x7fff7fffu, (uint32_t)v[k][1] & 0x7fff7fffu),
+                                      pk_max_u16((uint32_t)v[k][2] & 0x7fff7fffu, (uint32_t)v[k][3] & 0x7fff7fffu));
+        const uint32_t hi = m >> 16, lo = m & 0xffffu, w = hi > lo ? hi : lo;
+        if constexpr (F16) mx[k] = as_u32((float)__builtin_bit_cast(_Float16, (uint16_t)w));
+        else mx[k] = w << 16;
+    }
+#pragma unroll
+    for (int k = 0; k < N; ++k) mx[k] = row16_max_u32(mx[k]);
+    uint32_t top = mx[0];
+#pragma unroll
+    for (int k = 1; k < N; ++k) top = mx[k] > top ? mx[k] : top;
+    const float c = 1.0f / 448.0f;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const float amax = as_f32(mx[k] > kEps ? mx[k] : kEps);
+        const float q0 = amax * c;
+        const float s = __builtin_fmaf(__builtin_fmaf(-q0, 448.0f, amax), c, q0);
+        const float r = as_f32(as_u32(__builtin_amdgcn_rcpf(s)) - 2u);
+        const float d = __builtin_fmaf(-s, r, 1.0f) * r;
+        float f[8];
+        if constexpr (F16) {
+            const h8 h = __builtin_bit_cast(h8, v[k]);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) f[i] = (float)h[i];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                f[2 * i] = as_f32((uint32_t)v[k][i] << 16);
+                f[2 * i + 1] = as_f32((uint32_t)v[k][i] & 0xffff0000u);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f[i] = __builtin_fmaf(f[i], r, f[i] * d);
+        int w0 = 0, w1 = 0;
+        w0 = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], w0, false);
+        w0 = __builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], w0, true);
+        w1 = __builtin_amdgcn_cvt_pk_fp8_f32(f[4], f[5], w1, false);
+        w1 = __builtin_amdgcn_cvt_pk_fp8_f32(f[6], f[7], w1, true);
+        out[k][0] = w0;
+        out[k][1] = w1;
+        scale[k] = s;
+    }
+    // (no asm in this block to hold its arithmetic behind the branch: even an empty one there cost a weight stream that
+    // quantizes its activations 6 % - N = 28672, K = 4096, one row: 23.4 us against 22.0)
+    if (__builtin_expect(__ballot(top > 0x7f7fffffu) != 0ull, 0)) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            if (mx[k] > 0x7f7fffffu) {  // the same for all 16 lanes of the group
+                const uint32_t d0 = (uint32_t)v[k][0], d1 = (uint32_t)v[k][1], d2 = (uint32_t)v[k][2], d3 = (uint32_t)v[k][3];
+                nonfinite_chunk((d0 >> 15) & 1u, d0 >> 31, (d1 >> 15) & 1u, d1 >> 31, (d2 >> 15) & 1u, d2 >> 31,
+                                (d3 >> 15) & 1u, d3 >> 31, out[k], scale[k]);
+            }
+        }
+    }
+}
+
+// One chunk of bf16.
+__device__ __forceinline__ void quant_chunk(const v4i &v, v2i &out, float &scale) {
+    const v4i a[1] = {v};
+    v2i o[1];
+    float s[1];
+    quant_chunks<false, 1>(a, o, s);
+    out = o[0];
+    scale = s[0];
 }
 
 }  // namespace mi355

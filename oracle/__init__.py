@@ -40,7 +40,7 @@ def lib() -> ctypes.CDLL:
         _lib.oracle_moe_align2_rows.restype = ctypes.c_int64
         _lib.oracle_moe_align2_rows.argtypes = [ctypes.c_int64, ctypes.c_int32, ctypes.c_int32]
         _lib.oracle_fast_quant_mismatches.restype = ctypes.c_int64
-        _lib.oracle_fast_quant_mismatches.argtypes = [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint32]
+        _lib.oracle_fast_quant_mismatches.argtypes = [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint32, ctypes.c_int32]
     return _lib
 
 
@@ -214,9 +214,9 @@ def grouped_block_gemm(Xq, Xs, W, Ws, expert_to_token_index, expert_to_weights, 
     return out
 
 
-def fast_quant_mismatches(amax_lo: int = 0, amax_hi: int = 0x7F80, step: int = 1) -> int:
-    """Pairs (bf16 amax, bf16 x) for which the HIP quantizer's division shortcut would differ from IEEE."""
-    return int(lib().oracle_fast_quant_mismatches(amax_lo, amax_hi, step))
+def fast_quant_mismatches(amax_lo: int = 0, amax_hi: int = 0x7F80, step: int = 1, f16: bool = False) -> int:
+    """Pairs (amax, x) of bf16 (fp16) values for which the HIP quantizer's division shortcut would differ from IEEE."""
+    return int(lib().oracle_fast_quant_mismatches(amax_lo, amax_hi, step, 1 if f16 else 0))
 
 
 def silu_and_mul(x_bf16_bits) -> np.ndarray:

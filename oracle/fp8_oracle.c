@@ -468,47 +468,58 @@ void oracle_block_weight_dequant(const uint8_t *q, const float *s, int64_t N, in
         }
 }
 
+/* fp16 -> fp32, exact (finite values). */
+static float f16_to_f32(uint16_t h) {
+    const uint32_t e = (h >> 10) & 0x1fu, m = h & 0x3ffu;
+    const float v = e == 0 ? ldexpf((float)m, -24) : ldexpf((float)(1024u + m), (int)e - 25);
+    return (h & 0x8000u) ? -v : v;
+}
+
 /*
  * Replays, on the CPU, the exact operation sequence the HIP quantizer uses in place of two IEEE
- * divisions (csrc/quant_core.hpp: quant_chunk/quot), for every bf16 group maximum with bit pattern in
- * [amax_lo, amax_hi) stepping by `step`, against every bf16 element of either sign with |x| <= amax
- * (and every |x| < eps when the eps floor applies).  Returns how many (amax, x) pairs give a byte or a
- * scale different from the IEEE closed form above.  Zero for the whole range means the kernel's
- * shortcut is exact; it must stay in step with the kernel source.
+ * divisions (csrc/quant_core.hpp: quant_chunks), for every 16-bit group maximum (f16 = 0: bf16, 1: fp16) with bit
+ * pattern in [amax_lo, amax_hi) stepping by `step`, against every element of the same type with |x| <= amax
+ * (and every |x| < eps when the eps floor applies).  The hardware reciprocal may be off by one unit in the last place:
+ * every pair is replayed with the correctly rounded one and its two neighbours.  Negative elements mirror the positive
+ * ones operation by operation but for the sign of zero, which is checked by itself.  Returns how many (amax, x,
+ * reciprocal) cases give a byte or a scale different from the IEEE closed form above.  Zero for the whole range means the
+ * kernel's shortcut is exact; it must stay in step with the kernel source.
  */
-int64_t oracle_fast_quant_mismatches(uint32_t amax_lo, uint32_t amax_hi, uint32_t step) {
+int64_t oracle_fast_quant_mismatches(uint32_t amax_lo, uint32_t amax_hi, uint32_t step, int32_t f16) {
     const float eps = 1e-10f, c448 = 1.0f / 448.0f;
+    const uint32_t top = f16 ? 0x7bffu : 0x7f7fu;
     int64_t bad = 0;
-    for (uint32_t ab = amax_lo; ab < amax_hi && ab <= 0x7f7fu; ab += step) {
-        float amax = oracle_bf16_to_f32((uint16_t)ab);
+    for (uint32_t ab = amax_lo; ab < amax_hi && ab <= top; ab += step) {
+        float amax = f16 ? f16_to_f32((uint16_t)ab) : oracle_bf16_to_f32((uint16_t)ab);
         uint32_t xmax = ab;
         if (!(amax > eps)) {
             if (ab != 0) continue;       /* every maximum below eps gives the same scale: test it once, */
             amax = eps;
-            xmax = 0x2edbu;              /* against every bf16 magnitude below 1e-10 */
+            xmax = f16 ? 0u : 0x2edbu;   /* against every bf16 magnitude below 1e-10 (no fp16 one is but zero) */
         }
         volatile float s_ref = amax / 448.0f;
         /* kernel: scale */
         float q0 = amax * c448;
         float s = fmaf(fmaf(-q0, 448.0f, amax), c448, q0);
         if (f32_to_bits(s) != f32_to_bits(s_ref)) { ++bad; continue; }
-        volatile float r = 1.0f / s;
+        volatile float rn = 1.0f / s;
+        float r[3], d[3];
+        for (int i = 0; i < 3; ++i) {
+            r[i] = bits_to_f32(f32_to_bits(rn) + (uint32_t)(i - 1) - 2u);
+            d[i] = fmaf(-s, r[i], 1.0f) * r[i];
+            /* -0 */
+            const float z = -0.0f;
+            if (f32_to_bits(fmaf(z, r[i], z * d[i])) != 0x80000000u) ++bad;
+        }
         for (uint32_t xb = 0; xb <= xmax; ++xb) {
-            for (uint32_t sign = 0; sign <= 0x8000u; sign += 0x8000u) {
-                float x = oracle_bf16_to_f32((uint16_t)(xb | sign));
-                /* reference */
-                volatile float y = x / s_ref;
-                float cl = y;
-                if (cl > 448.0f) cl = 448.0f;
-                if (cl < -448.0f) cl = -448.0f;
-                uint8_t want = oracle_f32_to_e4m3fn(cl);
-                /* kernel */
-                float y0 = x * r;
-                float e = fmaf(-y0, s, x);
-                float y1 = fmaf(e, r, y0);
-                float fixed = bits_to_f32((f32_to_bits(y1) & 0x7fffffffu) | (f32_to_bits(x) & 0x80000000u));
-                uint8_t got = oracle_f32_to_e4m3fn(fixed);
-                if ((got & 0x7f) == 0x7f) got = (uint8_t)((got & 0x80) | 0x7e); /* the hardware cast saturates */
+            const float x = f16 ? f16_to_f32((uint16_t)xb) : oracle_bf16_to_f32((uint16_t)xb);
+            /* reference */
+            volatile float y = x / s_ref;
+            const uint8_t want = oracle_f32_to_e4m3fn(y > 448.0f ? 448.0f : y);
+            /* kernel */
+            for (int i = 0; i < 3; ++i) {
+                uint8_t got = oracle_f32_to_e4m3fn(fmaf(x, r[i], x * d[i]));
+                if (got == 0x7f) got = 0x7e; /* the hardware cast saturates */
                 if (got != want) ++bad;
             }
         }

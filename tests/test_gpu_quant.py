@@ -231,3 +231,23 @@ def test_other_group_sizes(hip, dtype, M, K, group):
     xq2, xs2 = per_token_group_quant_fp8(x.cuda(), group, column_major_scales=True)
     torch.cuda.synchronize()
     assert np.array_equal(tr.bits_of(xs2.contiguous()), s_ref.view(np.uint32)) and np.array_equal(tr.bits_of(xq2), q_ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M", [4095, 4096, 4097])
+def test_one_or_four_chunks_per_lane(hip, dtype, M):
+    """Both sides of the line between one and four chunks per lane (524288 chunks on 256 compute units), a last workgroup
+    that is full and one that is not, fp16 and bf16, row-major and column-major scales."""
+    from lightllm_amd.quantization import per_token_group_quant_fp8
+
+    K = 1024
+    print(f"quant chunks per lane {dtype} M={M}", flush=True)
+    x = torch.randn((M, K), generator=H.gen(M), dtype=torch.float32)
+    x[:, ::61] *= 29.0
+    x[7] = 0.0
+    x = x.to(dtype)
+    q_ref, s_ref = oracle.group_quant_fp8_f32(x.float().numpy())
+    for columns in (False, True):
+        xq, xs = per_token_group_quant_fp8(x.cuda(), 128, column_major_scales=columns, scale_tma_aligned=columns)
+        assert np.array_equal(tr.bits_of(xs.contiguous()), s_ref.view(np.uint32))
+        assert np.array_equal(tr.bits_of(xq), q_ref)

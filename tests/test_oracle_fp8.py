@@ -135,6 +135,16 @@ def test_kernel_division_shortcut_is_exact():
     assert oracle.fast_quant_mismatches(0, 0x7F80, 1) == 0
 
 
+def test_kernel_division_shortcut_is_exact_for_fp16():
+    """The same for every (fp16 group maximum, fp16 element) pair."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    lanes = 16   # interleaved maxima, so that every lane has the same work
+    with ThreadPoolExecutor(8) as pool:
+        bad = pool.map(lambda i: oracle.fast_quant_mismatches(i, 0x7C00, lanes, f16=True), range(lanes))
+        assert sum(bad) == 0
+
+
 # ---- the weight quantizer ------------------------------------------------------------------------------
 @pytest.mark.parametrize("N,K", [(256, 384), (200, 300), (128, 128)])
 def test_weight_quant_equals_torch_closed_form(N, K):
