@@ -181,6 +181,23 @@ int mi355_block_fp8_gemm_dtype(const void *A, const void *B, const float *As, co
                                int32_t c_dtype, void *stream);
 
 /* ---------------------------------------------------------------------------
+ * The quantized linear in one call: quantizer + GEMM, 16-bit activations in, 16-bit outputs out
+ * replaces: FP8w8a8B128QuantizationMethod.apply (lightllm/common/quantization/w8a8.py:433-474)
+ *
+ * x   bf16 / fp16 (fp32 with x_q given) [M,K] contiguous;  W e4m3fn [N,K], row stride ldw;  Ws fp32, element (nb,kb) at
+ *     Ws[nb*ws_n + kb*ws_k];  C [M,N], row stride ldc, c_dtype MI355_DTYPE_BF16 / _F16
+ * x_q, x_s  room for the quantized activations e4m3fn [M,K] and their scales fp32 [M,K/128] (16-byte aligned), or both
+ *     NULL where mi355_block_fp8_linear_fused() returns 1 for (M, N, K, x_dtype): few rows, whose activations are quantized
+ *     inside the weight stream (packed operands only: ldw = K, 16-byte aligned).  Same bytes, same scales either way.
+ * ws  as for mi355_block_fp8_gemm, of mi355_block_fp8_linear_workspace_bytes() bytes (0: none needed).
+ */
+int32_t mi355_block_fp8_linear_fused(int64_t M, int64_t N, int64_t K, int32_t x_dtype);
+size_t mi355_block_fp8_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t x_dtype);
+int mi355_block_fp8_linear(const void *x, int32_t x_dtype, const void *W, const float *Ws, void *C, int64_t M, int64_t N,
+                           int64_t K, int64_t ldw, int64_t ws_n, int64_t ws_k, int64_t ldc, void *x_q, float *x_s,
+                           void *ws, size_t ws_bytes, int32_t c_dtype, void *stream);
+
+/* ---------------------------------------------------------------------------
  * moe_align_fused / moe_align2 : routing tables for the grouped GEMM
  * replaces: moe_align_fused (lightllm/common/basemodel/triton_kernel/fused_moe/grouped_fused_moe.py:388-396)
  *           moe_align2      (same file :399-477)

@@ -44,6 +44,12 @@ SIGNATURES = {
         [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i32, _i32,
          _vp, _sz, _i32, _i32, _vp],
     ),
+    "mi355_block_fp8_linear_fused": (_i32, [_i64, _i64, _i64, _i32]),
+    "mi355_block_fp8_linear_workspace_bytes": (_sz, [_i64, _i64, _i64, _i32]),
+    "mi355_block_fp8_linear": (
+        _c.c_int,
+        [_vp, _i32, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _sz, _i32, _vp],
+    ),
     "mi355_moe_align_fused": (_c.c_int, [_vp, _vp, _i64, _i32, _vp, _vp, _vp, _vp]),
     "mi355_moe_align": (_c.c_int, [_vp, _i64, _i32, _vp, _i64, _vp]),
     "mi355_moe_align1": (_c.c_int, [_vp, _i64, _vp, _i64, _i32, _vp, _i64, _vp, _vp]),

@@ -25,10 +25,36 @@
 // Algorithmic bytes per K step and CTA: 16*TNW*128 weight bytes + 16*MT*128 activation bytes (L2 resident).
 #pragma once
 #include "gemm_tile.hpp"
+#include "quant_core.hpp"
 
 namespace mi355 {
 
 constexpr int kStreamWaves = 4;
+
+// Activations quantized by the wave that multiplies them (at most 8 rows).  A K step is exactly one quantization group
+// per row and a wave owns its K steps alone, so the 1x128 quantizer needs nothing from any other wave: XR 16-byte loads
+// bring 4*XR rows of 128 bf16 / fp16 values (16 lanes of a DPP row = one group), quant_chunks leaves 8 e4m3 bytes per
+// lane, which go to the X block of the wave's LDS area, and the group's scale goes to 16 floats beside it.  The bytes
+// and scales are the stand-alone quantizer's.  Rows from 4*XR on hold whatever was there: they are MFMA columns of
+// their own and are never stored.
+struct XQuant {
+    static __device__ __forceinline__ uint32_t offset(int i, int lane, int M, uint32_t ldx) {
+        return (uint32_t)min(4 * i + (lane >> 4), M - 1) * ldx + (uint32_t)(lane & 15) * 16u;
+    }
+    template <int XR, bool F16>
+    static __device__ __forceinline__ void store(const v4i (&x)[XR], uint8_t *xblock, float *scales, int lane) {
+        const uint32_t ch = (uint32_t)(lane & 15);
+        v2i q[XR];
+        float sc[XR];
+        quant_chunks<F16, XR>(x, q, sc);
+#pragma unroll
+        for (int i = 0; i < XR; ++i) {
+            const uint32_t row = (uint32_t)(4 * i + (lane >> 4));
+            *(v2i *)(xblock + row * 128u + ((ch >> 1) ^ swz(row)) * 16u + (ch & 1u) * 8u) = q[i];
+            if (ch == 0) scales[row] = sc[i];
+        }
+    }
+};
 
 template <int MT, int TNW>
 struct StreamCfg {
@@ -54,10 +80,10 @@ struct StreamCfg {
     static constexpr int scale_lds_bytes(int steps) { return steps * kScaleStride * 4; }
 };
 
-template <int MT, int TNW>
+template <int MT, int TNW, int NX>
 struct StreamRegs {
     v4i w[2 * TNW];  // 16*TNW rows x 128 B of W: instruction i holds rows 8i + lane/8, 16-byte chunk lane%8
-    v4i x[2 * MT];   // 16*MT rows x 128 B of X, same arrangement
+    v4i x[NX];       // 16*MT rows x 128 B of X, same arrangement (XR: 4*XR rows of 16-bit values, see XQuant)
     float xs[MT];    // activation scales of rows 16*mt + lane%16 (unused when they are staged in LDS)
     float ws;        // weight scale of this (n block, K step)
 };
@@ -65,10 +91,14 @@ struct StreamRegs {
 // XSL: the activation scales of the CTA's K range are staged in LDS by one coalesced pass at the start (the host
 // checks that the range fits); otherwise every wave gathers them per step, which costs as many cache-line
 // accesses as the X block itself (16 rows x 4 bytes per request).
-template <int MT, int TNW, bool SPLIT, bool XSL>
+// XR > 0: X is the unquantized activation matrix (XQuant above; XSL is false then).
+template <int MT, int TNW, bool SPLIT, bool XSL, int XR = 0, bool F16 = false>
 __global__ __launch_bounds__(256) void block_fp8_gemm_stream_kernel(const GemmArgs p) {
+    static_assert(XR == 0 || (MT == 1 && !XSL), "unquantized activations: at most 16 rows, no staged scales");
     using Cfg = StreamCfg<MT, TNW>;
-    constexpr int D = Cfg::depth(XSL);
+    constexpr int NX = XR ? XR : 2 * MT;
+    using Regs = StreamRegs<MT, TNW, NX>;
+    constexpr int D = Cfg::depth(XSL || XR);
     constexpr int BN = Cfg::BN;
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
 
@@ -100,9 +130,12 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_stream_kernel(const GemmAr
     uint32_t woff[2 * TNW];
 #pragma unroll
     for (int i = 0; i < 2 * TNW; ++i) woff[i] = (uint32_t)min(n0 + 8 * i + sub, p.N - 1) * (uint32_t)p.ldw + (uint32_t)pch * 16u;
-    uint32_t xoff[2 * MT];
+    uint32_t xoff[NX];
 #pragma unroll
-    for (int i = 0; i < 2 * MT; ++i) xoff[i] = (uint32_t)min(8 * i + sub, p.M - 1) * (uint32_t)p.ldx + (uint32_t)pch * 16u;
+    for (int i = 0; i < NX; ++i) {
+        if constexpr (XR) xoff[i] = XQuant::offset(i, lane, p.M, (uint32_t)p.ldx);
+        else xoff[i] = (uint32_t)min(8 * i + sub, p.M - 1) * (uint32_t)p.ldx + (uint32_t)pch * 16u;
+    }
     uint32_t soff[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) soff[t] = (uint32_t)min(16 * t + r16, p.M - 1) * (uint32_t)p.xs_m;
@@ -111,7 +144,7 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_stream_kernel(const GemmAr
 
     // ---- stage the activation scales: thread (row group tid/32, step tid%32) walks rows +8 and steps +32, so a
     // row-major scale row is read as whole cache lines; indices past the range repeat the last valid element
-    float *xs_lds = (float *)(lds + Cfg::kLds);
+    float *xs_lds = (float *)(lds + Cfg::kLds) + (XR ? wave * 16 : 0);
     constexpr int kSvRows = 2 * MT, kSvSteps = (Cfg::kMaxScaleSteps + 31) / 32;
     float sv[XSL ? kSvRows * kSvSteps : 1];
     const int steps_cta = kb_end - kb_begin;
@@ -126,14 +159,14 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_stream_kernel(const GemmAr
             }
     }
 
-    auto load = [&](StreamRegs<MT, TNW> &r, int kb) {
+    auto load = [&](Regs &r, int kb) {
         const uint8_t *wk = p.W + (int64_t)kb * kBlockK;
-        const uint8_t *xk = p.X + (int64_t)kb * kBlockK;
+        const uint8_t *xk = p.X + (int64_t)kb * (XR ? 2 * kBlockK : kBlockK);
 #pragma unroll
         for (int i = 0; i < 2 * TNW; ++i) r.w[i] = __builtin_nontemporal_load((const v4i *)(wk + woff[i]));
 #pragma unroll
-        for (int i = 0; i < 2 * MT; ++i) r.x[i] = *(const v4i *)(xk + xoff[i]);
-        if constexpr (!XSL) {
+        for (int i = 0; i < NX; ++i) r.x[i] = *(const v4i *)(xk + xoff[i]);
+        if constexpr (!XSL && XR == 0) {
 #pragma unroll
             for (int t = 0; t < MT; ++t) r.xs[t] = p.Xs[soff[t] + (int64_t)kb * p.xs_k];
         }
@@ -168,17 +201,22 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_stream_kernel(const GemmAr
 #pragma unroll
         for (int j = 0; j < TNW; ++j) acc[t][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
-    auto consume = [&](const StreamRegs<MT, TNW> &r, int kb) {
+    auto consume = [&](const Regs &r, int kb) {
         float xsv[MT];
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
             if constexpr (XSL) xsv[t] = xs_lds[(kb - kb_begin) * Cfg::kScaleStride + 16 * t + r16];
-            else xsv[t] = r.xs[t];
+            else if constexpr (XR == 0) xsv[t] = r.xs[t];
         }
 #pragma unroll
         for (int i = 0; i < 2 * TNW; ++i) *(v4i *)(my + wst[i]) = r.w[i];
+        if constexpr (XR) {
+            XQuant::store<XR, F16>(r.x, my + Cfg::kXOff, xs_lds, lane);
+            xsv[0] = xs_lds[r16];
+        } else {
 #pragma unroll
-        for (int i = 0; i < 2 * MT; ++i) *(v4i *)(my + xst[i]) = r.x[i];
+            for (int i = 0; i < 2 * MT; ++i) *(v4i *)(my + xst[i]) = r.x[i];
+        }
         // LDS operations of one wave execute in order: the reads below see the writes above
         v8i wf[TNW];
 #pragma unroll
@@ -202,7 +240,7 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_stream_kernel(const GemmAr
     };
 
     // ---- the stream: DEPTH register sets rotate; the compiler places the vmcnt waits
-    StreamRegs<MT, TNW> regs[D];
+    Regs regs[D];
 #pragma unroll
     for (int d = 0; d < D; ++d)
         if (d < steps) load(regs[d], first + d * kStreamWaves);

@@ -20,18 +20,22 @@
 // Everything else is the streaming kernel's: plain coalesced 16-byte loads (8 lanes per 128-byte row segment), a
 // few K steps in flight in registers, the transposition into MFMA operand order through a wave-private LDS area
 // with no barrier in the loop, the activation scales of the whole K range staged in LDS by one coalesced pass.
+//
+// XR > 0: X is the bf16 or fp16 activation matrix itself and every wave quantizes the rows of its own K steps (see
+// XQuant in gemm_stream.hpp): no quantizer launch, no staged activation scales.
 #pragma once
 #include "gemm_stream.hpp"
 
 namespace mi355 {
 
-template <int MT, int TB>
+template <int MT, int TB, int XR = 0>
 struct CuStreamCfg {
     static_assert(TB >= 1 && TB <= 8, "a tile of up to 128 rows touches at most two 128-row scale blocks");
     static constexpr int kWaves = 8, kThreads = 512;
     static constexpr int KW = kWaves;                    // K phases
     static constexpr int BN = 16 * TB;
-    static constexpr int kSet = 8 * TB + 8 * MT;         // registers of one K step in flight
+    static constexpr int NX = XR ? XR : 2 * MT;          // activation loads of a K step
+    static constexpr int kSet = 8 * TB + 4 * NX;         // registers of one K step in flight
     static constexpr int kDepth = kSet * 6 <= 132 ? 6 : (132 / kSet < 1 ? 1 : 132 / kSet);
     static constexpr int kXOff = 16 * TB * 128;
     static constexpr int kWaveLds = (16 * TB + 16 * MT) * 128;
@@ -41,21 +45,23 @@ struct CuStreamCfg {
     static constexpr int kScaleStride = 16 * MT + 1;  // floats per K step in the staged scales
     static constexpr int kMaxScaleUnits = 5;          // registers a thread stages scales through: K / 128 <= 160 / MT
     static constexpr int max_steps() { return 32 * (kMaxScaleUnits / MT); }
-    // behind the waves' areas: activation scales [KB][16*MT + 1], then weight scales [2][KB]
-    static constexpr int ws_off(int KB) { return kLds + KB * kScaleStride * 4; }
+    // behind the waves' areas: activation scales [KB][16*MT + 1] (XR: 16 floats per wave), then weight scales [2][KB]
+    static constexpr int ws_off(int KB) { return kLds + (XR ? kWaves * 64 : KB * kScaleStride * 4); }
     static constexpr int lds_bytes(int KB) { return ws_off(KB) + 2 * KB * 4; }
 };
 
-template <int MT, int TB>
+template <int MT, int TB, int NX>
 struct CuStreamRegs {
     v4i w[2 * TB];
-    v4i x[2 * MT];
+    v4i x[NX];
 };
 
 // XHI: M > 8, rows 8..15 of the first activation row block exist and are loaded.
-template <int MT, int TB, bool XHI>
+template <int MT, int TB, bool XHI, int XR = 0, bool F16 = false>
 __global__ __launch_bounds__(512) void block_fp8_gemm_streamcu_kernel(const GemmArgs p) {
-    using Cfg = CuStreamCfg<MT, TB>;
+    static_assert(XR == 0 || MT == 1, "unquantized activations: at most 16 rows");
+    using Cfg = CuStreamCfg<MT, TB, XR>;
+    using Regs = CuStreamRegs<MT, TB, Cfg::NX>;
     constexpr int D = Cfg::kDepth, KW = Cfg::KW, nblk = TB;
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
 
@@ -74,9 +80,12 @@ __global__ __launch_bounds__(512) void block_fp8_gemm_streamcu_kernel(const Gemm
     uint32_t woff[2 * TB];
 #pragma unroll
     for (int i = 0; i < 2 * TB; ++i) woff[i] = (uint32_t)min(n0 + 8 * i + sub, p.N - 1) * (uint32_t)p.ldw + (uint32_t)pch * 16u;
-    uint32_t xoff[2 * MT];
+    uint32_t xoff[Cfg::NX];
 #pragma unroll
-    for (int i = 0; i < 2 * MT; ++i) xoff[i] = (uint32_t)min(8 * i + sub, p.M - 1) * (uint32_t)p.ldx + (uint32_t)pch * 16u;
+    for (int i = 0; i < Cfg::NX; ++i) {
+        if constexpr (XR) xoff[i] = XQuant::offset(i, lane, p.M, (uint32_t)p.ldx);
+        else xoff[i] = (uint32_t)min(8 * i + sub, p.M - 1) * (uint32_t)p.ldx + (uint32_t)pch * 16u;
+    }
     // the two 128-row scale blocks the sub-tile can touch, and which of them each of the lane's MFMA blocks reads:
     // block tn of lane group g4 holds output columns n0 + 4*nblk*g4 + 4*tn + [0, 4)
     const int NB = (p.N + kBlockN - 1) / kBlockN;
@@ -91,28 +100,30 @@ __global__ __launch_bounds__(512) void block_fp8_gemm_streamcu_kernel(const Gemm
     // xs_lds[kb * stride + r].  Thread (row group tid / 32, step tid % 32) walks rows + 16 and steps + 32, so a
     // row-major scale row is read as whole cache lines.  The loads are issued here, ahead of the first weight loads,
     // and stored to LDS behind them (memory operations return in order: the store waits for the scales only).
-    float *xs_lds = (float *)(lds + Cfg::kLds);
+    float *xs_lds = (float *)(lds + Cfg::kLds) + (XR ? wave * 16 : 0);
     constexpr int kSv = Cfg::kMaxScaleUnits;
     const int sv_units = ((KB + 31) / 32) * MT;  // (step group, row group) units of 32 steps x 16 rows
     float sv[kSv];
+    if constexpr (XR == 0) {
 #pragma unroll
-    for (int u = 0; u < kSv; ++u) {
-        const int uu = min(u, sv_units - 1);
-        const int row = (uu % MT) * 16 + (tid >> 5), kb = (uu / MT) * 32 + (tid & 31);
-        sv[u] = p.Xs[(int64_t)min(row, p.M - 1) * p.xs_m + (int64_t)min(kb, KB - 1) * p.xs_k];
+        for (int u = 0; u < kSv; ++u) {
+            const int uu = min(u, sv_units - 1);
+            const int row = (uu % MT) * 16 + (tid >> 5), kb = (uu / MT) * 32 + (tid & 31);
+            sv[u] = p.Xs[(int64_t)min(row, p.M - 1) * p.xs_m + (int64_t)min(kb, KB - 1) * p.xs_k];
+        }
     }
     // weight scales: thread t < 256 takes step t of the first scale block, thread 256 + t that of the second
     float *ws_lds = (float *)(lds + Cfg::ws_off(KB));
     const float wsv = wsp[(int64_t)min(tid & 255, KB - 1) * p.ws_k];
 
-    auto load = [&](CuStreamRegs<MT, TB> &r, int kb) {
+    auto load = [&](Regs &r, int kb) {
         const uint8_t *wk = p.W + (int64_t)kb * kBlockK;
-        const uint8_t *xk = p.X + (int64_t)kb * kBlockK;
+        const uint8_t *xk = p.X + (int64_t)kb * (XR ? 2 * kBlockK : kBlockK);
 #pragma unroll
         for (int i = 0; i < 2 * TB; ++i) r.w[i] = __builtin_nontemporal_load((const v4i *)(wk + woff[i]));
 #pragma unroll
-        for (int i = 0; i < 2 * MT; ++i)
-            if (i != 1 || x_hi) r.x[i] = *(const v4i *)(xk + xoff[i]);
+        for (int i = 0; i < Cfg::NX; ++i)
+            if (XR || i != 1 || x_hi) r.x[i] = *(const v4i *)(xk + xoff[i]);
     };
 
     // ---- wave-private LDS: W block rows in MFMA order, then the X block; 128-byte rows, swizzled chunks.
@@ -143,14 +154,21 @@ __global__ __launch_bounds__(512) void block_fp8_gemm_streamcu_kernel(const Gemm
 #pragma unroll
         for (int j = 0; j < TB; ++j) acc[t][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
-    auto consume = [&](const CuStreamRegs<MT, TB> &r, int kb) {
+    auto consume = [&](const Regs &r, int kb) {
         float xsv[MT];
+        if constexpr (XR == 0) {
 #pragma unroll
-        for (int t = 0; t < MT; ++t) xsv[t] = xs_lds[kb * Cfg::kScaleStride + 16 * t + r16];
+            for (int t = 0; t < MT; ++t) xsv[t] = xs_lds[kb * Cfg::kScaleStride + 16 * t + r16];
+        }
 #pragma unroll
         for (int i = 0; i < 2 * TB; ++i) *(v4i *)(my + wst[i]) = r.w[i];
+        if constexpr (XR) {
+            XQuant::store<XR, F16>(r.x, my + Cfg::kXOff, xs_lds, lane);
+            xsv[0] = xs_lds[r16];
+        } else {
 #pragma unroll
-        for (int i = 0; i < 2 * MT; ++i) *(v4i *)(my + xst[i]) = r.x[(i == 1 && !x_hi) ? 0 : i];
+            for (int i = 0; i < 2 * MT; ++i) *(v4i *)(my + xst[i]) = r.x[(i == 1 && !x_hi) ? 0 : i];
+        }
         const float ws0 = ws_lds[kb], ws1 = ws_lds[KB + kb];
         // LDS operations of one wave execute in order: the reads below see the writes above
         v8i xf[MT];
@@ -175,14 +193,16 @@ __global__ __launch_bounds__(512) void block_fp8_gemm_streamcu_kernel(const Gemm
     };
 
     // ---- the stream: D register sets rotate; the compiler places the vmcnt waits
-    CuStreamRegs<MT, TB> regs[D];
+    Regs regs[D];
 #pragma unroll
     for (int d = 0; d < D; ++d)
         if (d < steps) load(regs[d], phase + d * KW);
+    if constexpr (XR == 0) {
 #pragma unroll
-    for (int u = 0; u < kSv; ++u) {
-        const int row = (u % MT) * 16 + (tid >> 5), kb = (u / MT) * 32 + (tid & 31);
-        if (u < sv_units && kb < KB) xs_lds[kb * Cfg::kScaleStride + row] = sv[u];
+        for (int u = 0; u < kSv; ++u) {
+            const int row = (u % MT) * 16 + (tid >> 5), kb = (u / MT) * 32 + (tid & 31);
+            if (u < sv_units && kb < KB) xs_lds[kb * Cfg::kScaleStride + row] = sv[u];
+        }
     }
     if ((tid & 255) < KB) ws_lds[(tid >> 8) * KB + (tid & 255)] = wsv;
     __syncthreads();  // the staged scales are visible

@@ -4,15 +4,25 @@ Mirrors FP8w8a8B128QuantizationMethod / FP8w8a8B128TritonQuantizationMethod of t
 (lightllm/common/quantization/w8a8.py:418-474, 505-533): 128x128 block-quantized e4m3fn weights with
 ``weight_scale_inv`` scales, dynamic per-token-group activation quantization, bf16 output, no bias.
 """
+import functools
 from typing import Callable, List, Optional, Tuple, Union
 
 import torch
 
+from .. import _lib
 from .fp8act_quant_kernel import per_token_group_quant_fp8
 from .fp8w8a8_block_gemm_kernel import w8a8_block_fp8_matmul
 from .fp8w8a8_block_quant_kernel import weight_quant
 from .quantize_method import QuantizationMethod, WeightPack
 from .registry import QUANTMETHODS
+
+
+@functools.lru_cache(maxsize=4096)
+def _linear_plan(rows: int, n: int, k: int, dtype: torch.dtype, device_index: int) -> Tuple[bool, int]:
+    """(quantized inside the GEMM's kernel, workspace bytes) of a linear: what the library says for the device."""
+    lib, code = _lib.lib(), _lib.DTYPE_CODES[dtype]
+    return (bool(lib.mi355_block_fp8_linear_fused(rows, n, k, code)),
+            lib.mi355_block_fp8_linear_workspace_bytes(rows, n, k, code))
 
 
 class FP8w8a8B128QuantizationMethod(QuantizationMethod):
@@ -96,6 +106,9 @@ class FP8w8a8B128Mi355QuantizationMethod(FP8w8a8B128QuantizationMethod):
         bias: Optional[torch.Tensor] = None,
     ) -> torch.Tensor:
         assert bias is None, f"Bias addition is not supported in {self.method_name} for now"
+        result = self._linear(input_tensor, weight_pack, out, use_custom_tensor_mananger)
+        if result is not None:
+            return result
         qinput_tensor, qweight, input_scale, weight_scale, out = self._dynamic_quant_input(
             input_tensor, weight_pack, out, use_custom_tensor_mananger
         )
@@ -103,6 +116,45 @@ class FP8w8a8B128Mi355QuantizationMethod(FP8w8a8B128QuantizationMethod):
             qinput_tensor, qweight, input_scale, weight_scale, out, (self.block_size, self.block_size),
             dtype=input_tensor.dtype,
         )
+        return out
+
+    def _linear(self, x: torch.Tensor, weight_pack: WeightPack, out: Optional[torch.Tensor],
+                use_custom_tensor_mananger: bool) -> Optional[torch.Tensor]:
+        """The linear in one library call: packed 16-bit activations and outputs, a packed weight.  Anything else (and
+        anything that is wrong) returns None and goes step by step, where every operator checks its own operands."""
+        w, ws = weight_pack.weight, weight_pack.weight_scale
+        dtype = x.dtype
+        if (dtype is not torch.bfloat16 and dtype is not torch.float16) or x.ndim != 2 or w.ndim != 2 or ws.ndim != 2:
+            return None
+        (m, k), (n, wk) = x.shape, w.shape
+        if k != wk or m == 0 or n == 0 or k % 128 != 0 or ws.shape != ((n + 127) // 128, k // 128):
+            return None
+        if not (x.is_cuda and w.is_cuda and ws.is_cuda and x.is_contiguous() and w.is_contiguous()
+                and w.dtype is torch.float8_e4m3fn and ws.dtype is torch.float32):
+            return None
+        device = x.device
+        alloc = self._alloc_func(use_custom_tensor_mananger)
+        if out is None:
+            out = alloc((m, n), dtype=dtype, device=device)
+        if out.shape != (m, n) or not out.is_cuda or not out.is_contiguous() or out.dtype not in (torch.bfloat16, torch.float16):
+            return None
+        x_ptr, w_ptr = x.data_ptr(), w.data_ptr()
+        if (x_ptr | w_ptr) & 15:
+            return None
+        fused, ws_need = _linear_plan(m, n, k, dtype, device.index)
+        xq_ptr = xs_ptr = ws_ptr = None
+        if not fused:
+            x_q = alloc((m, k), dtype=torch.float8_e4m3fn, device=device)
+            x_s = alloc((m, k // 128), dtype=torch.float32, device=device)
+            xq_ptr, xs_ptr = x_q.data_ptr(), x_s.data_ptr()
+        stream = _lib.stream_ptr(device)
+        if ws_need:
+            ws_ptr = _lib.workspace(device, ws_need, stream).data_ptr()
+        code = _lib.lib().mi355_block_fp8_linear(
+            x_ptr, _lib.DTYPE_CODES[dtype], w_ptr, ws.data_ptr(), out.data_ptr(), m, n, k, k, ws.stride(0), ws.stride(1), n,
+            xq_ptr, xs_ptr, ws_ptr, ws_need, _lib.DTYPE_CODES[out.dtype], stream,
+        )
+        _lib.check(code, "fp8 linear")
         return out
 
     @property

@@ -1,0 +1,69 @@
+"""GPU parity of the linear in one library call (quantization method `apply`, mi355_block_fp8_linear): bit for bit the
+stand-alone quantizer followed by the GEMM, whichever of the two the shape takes."""
+import pytest
+import torch
+
+from tests import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+
+def _composed(x, wq, ws, out_dtype):
+    from lightllm_amd.quantization import per_token_group_quant_fp8, w8a8_block_fp8_matmul
+
+    xq, xs = per_token_group_quant_fp8(x, 128)
+    out = torch.full((x.shape[0], wq.shape[0]), float("nan"), dtype=out_dtype, device=x.device)
+    return w8a8_block_fp8_matmul(xq, wq.t(), xs, ws.t(), out, [128, 128])
+
+
+# one shape per kernel that quantizes in its stream (256 compute units): per-unit stream of 1..5 row blocks, the last one
+# ragged; 64-row tiles with one K step per wave; 16-row tiles whole and with K shared, a K that the waves do not share
+# evenly, a last tile of 8 rows and an N that is not a multiple of 8
+SHAPES = [(4096, 4096), (4090, 2176), (7168, 2304), (12288, 2048), (16300, 2048), (20480, 2304), (28672, 512),
+          (2112, 7168), (6144, 1024), (1004, 640), (72, 128)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("N,K", SHAPES)
+def test_quantized_in_the_stream(hip, N, K, dtype):
+    from lightllm_amd import _lib
+    from lightllm_amd.quantization import QUANTMETHODS, WeightPack
+
+    wq, ws = H.quantized_weights(N, K, seed=N + K, device="cuda")
+    method, pack = QUANTMETHODS.get("fp8w8a8-b128"), WeightPack(wq, ws)
+    for M in (1, 3, 4, 5, 8, 9):
+        print(f"linear M={M} N={N} K={K} {dtype}", flush=True)
+        fused = hip.mi355_block_fp8_linear_fused(M, N, K, _lib.DTYPE_CODES[dtype])
+        assert fused == (M <= 8), (M, fused)
+        x = H.activations(M, K, seed=M, outliers=True).to(dtype).cuda()
+        x[M // 2, :128] = 0.0                       # a group on the eps floor
+        if M > 1:
+            x[M - 1, K - 3] = float("nan")          # a poisoned group stays in its row
+        out = method.apply(x, pack)
+        want = _composed(x, wq, ws, dtype)
+        assert out.dtype == dtype and out.shape == (M, N)
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16)), (M, N, K)
+        assert not torch.isnan(out[: max(M - 1, 1)]).any()
+
+
+def test_output_argument_and_odd_operands(hip):
+    """A caller's output tensor is filled and returned; activations that are not 16-byte aligned, a strided weight scale
+    and fp32 outputs keep the behaviour of the step-by-step path."""
+    from lightllm_amd.quantization import QUANTMETHODS, WeightPack
+
+    M, N, K = 3, 512, 1024
+    wq, ws = H.quantized_weights(N, K, seed=3, device="cuda")
+    method = QUANTMETHODS.get("fp8w8a8-b128")
+    x = H.activations(M, K, seed=4).cuda()
+    want = _composed(x, wq, ws, torch.bfloat16)
+    out = torch.empty_like(want)
+    assert method.apply(x, WeightPack(wq, ws), out=out) is out and torch.equal(out, want)
+    wide = torch.zeros((ws.shape[0], 2 * ws.shape[1]), dtype=torch.float32, device="cuda")
+    wide[:, ::2] = ws
+    assert torch.equal(method.apply(x, WeightPack(wq, wide[:, ::2])), want)
+    buf = torch.empty(M * K + 1, dtype=torch.bfloat16, device="cuda")
+    shifted = buf[1:].view(M, K).copy_(x)
+    with pytest.raises(ValueError):                 # the quantizer needs 16-byte aligned activations
+        method.apply(shifted, WeightPack(wq, ws))
+    with pytest.raises(AssertionError):
+        method.apply(x.float(), WeightPack(wq, ws))
