@@ -1,6 +1,7 @@
 // Host side of the block-scaled FP8 GEMM entry points: argument checks, kernel choice, launches.
-#include <cstdlib>
+#include <algorithm>
 
+#include "gemm_gstream.hpp"
 #include "gemm_pp.hpp"
 #include "gemm_small.hpp"
 #include "gemm_stream.hpp"
@@ -77,6 +78,29 @@ template <int BM, int BN, int WM, int WN, int NSTAGE>
 static int launch_grouped_tile(GemmArgs &a, int grid, hipStream_t st) {
     if (a.bias) return launch_tile<BM, BN, WM, WN, NSTAGE, kGrouped, true>(a, grid, st);
     return launch_tile<BM, BN, WM, WN, NSTAGE, kGrouped, false>(a, grid, st);
+}
+
+// A grouped launch of weight streams over the entries of a 16- or 32-row schedule.
+template <bool BIAS>
+static int launch_gstream_as(GemmArgs &a, int block_m, int num_experts, hipStream_t st) {
+    const int KB = a.K / kBlockK;
+    const int lds_bytes = GStreamCfg<2>::lds_bytes(KB);
+    if (lds_bytes > kMaxLds) return MI355_EUNSUPPORTED;
+    a.tiles_n = (a.N + GStreamCfg<1>::BN - 1) / GStreamCfg<1>::BN;
+    a.total_tiles = a.tiles_m * a.tiles_n;
+    // an exact schedule has at most E more entries than it would with every block full
+    const int64_t grid = std::max<int64_t>(4096, 2 * (int64_t)num_experts * a.tiles_n);
+    if (a.total_tiles <= grid) {
+        constexpr auto kernel = block_fp8_gemm_gstream_kernel<BIAS, false>;
+        if (!allow_lds<kernel>(kMaxLds)) return MI355_ELAUNCH;
+        return launch(kernel, dim3(a.total_tiles), dim3(256), lds_bytes, st, a, block_m);
+    }
+    constexpr auto kernel = block_fp8_gemm_gstream_kernel<BIAS, true>;
+    if (!allow_lds<kernel>(kMaxLds)) return MI355_ELAUNCH;
+    return launch(kernel, dim3((uint32_t)grid), dim3(256), lds_bytes, st, a, block_m);
+}
+static int launch_gstream(GemmArgs &a, int block_m, int num_experts, hipStream_t st) {
+    return a.bias ? launch_gstream_as<true>(a, block_m, num_experts, st) : launch_gstream_as<false>(a, block_m, num_experts, st);
 }
 
 #ifndef MI355_SK_PANEL
@@ -1143,15 +1167,15 @@ extern "C" int mi355_reset_workspace(void *ws, size_t ws_bytes, void *stream) {
 }
 
 extern "C" int32_t mi355_grouped_block_m(int64_t num_pairs, int32_t num_experts, int64_t N, int64_t K) {
-    (void)K;
     if (num_experts <= 0) return 64;
     const int64_t avg = num_pairs / num_experts;
     // 256-row schedule blocks run as the persistent launch with two queues: blocks of more than 64 rows on the
     // 256x256 ping-pong tile (it skips the empty 64-row halves of ragged blocks), the others on the 64x512
-    // weight-streaming tile.  That launch needs more tiles than compute units; where it has them it is the faster
-    // one from about 12 rows per expert on (256 experts, top-8, N=4096 K=7168: 512 tokens 1275 us against 1291 for
-    // 32-row blocks, 1024 tokens 1314 against 1500, 2048 tokens 1421 against 1885; the same within 1 % at 384
-    // tokens).  With fewer rows the 16-row tiles stream the weights at 6.0 TB/s and nothing beats them.
+    // weight-streaming tile.  That launch needs more tiles than compute units.  With fewer rows the weight streams of
+    // 16- and 32-row schedules (gemm_gstream.hpp) are ahead: they read at 6 to 7 TB/s until many experts have more than
+    // 32 rows and are read twice (256 experts, top-8, N = 4096, K = 7168, 16 / 24 / 32 rows per expert: 1179 / 1327 / 1755
+    // us for the 32-row stream against 1277 / 1302 / 1318; 32 experts, 16 / 22 / 32 rows: 155 / 171 / 225 against 174 / 175 /
+    // 177; N = 7168, K = 2048: 86.5 / 97.6 / 125 against 100 / 102 / 105).
     const int cus = device_cus();
     const int64_t tiles256 = (int64_t)num_experts * ((N + 255) / 256);
     const bool two_queues = tiles256 > cus;
@@ -1170,13 +1194,13 @@ extern "C" int32_t mi355_grouped_block_m(int64_t num_pairs, int32_t num_experts,
         if (tiles256 * 2 <= cus && avg > (large_expert ? 32 : 64) && avg <= (large_expert ? 160 : 256)) return 128;
         if ((int64_t)num_experts * N * K <= 500000000ll && K <= 2048 && avg <= (K <= 1536 ? 224 : 112)) return 128;
     }
-    //  * with 8 experts every block re-reads a large expert, and 64-row blocks beat blocks of the average size
-    //    (Mixtral down, 16 / 32 rows per expert: 84.2 / 86.6 us against 102.5 / 108.9)
-    if (num_experts <= 8 && avg > 8 && avg <= 40) return 64;
-    //  * the two-queue launch takes over from 12 rows per expert where an expert's N is wide, from 25 where it is
-    //    not: the row-sized ring tiles stream small experts better (Qwen3-235B gate_up, N = 3072, 16 rows: 308 us
-    //    against 373; DeepSeek-V2-Lite, 12 / 24 rows: 68.3 / 81.7 against 86.1 / 89.0)
-    if (avg > 64 || (two_queues && avg >= (N >= 4096 ? 12 : 25))) return 256;
+    //  * with 8 experts every block re-reads a large expert, and 64-row blocks beat blocks of the average size from 21
+    //    rows per expert on (Mixtral down, 20 / 24 rows: 84.8 / 86.1 us against 77.8 / 96.3 for the 32-row stream); with K
+    //    under 2048, where 16- and 32-row blocks are ring tiles, from 9
+    if (num_experts <= 8 && avg > (K >= 2048 ? 20 : 8) && avg <= 40) return 64;
+    //  * the two-queue launch takes over from 21 rows per expert where an expert's N is wide (12 with a short K), from 25
+    //    where it is not (Qwen3-30B gate_up, N = 1536, 24 rows: 84.6 us for the 32-row stream against 92.6)
+    if (avg > 64 || (two_queues && avg >= (N >= 4096 ? (K >= 2048 ? 21 : 12) : 25))) return 256;
     if (avg <= 16) return 16;
     if (avg <= 32) return 32;
     return 64;
@@ -1248,10 +1272,20 @@ static int grouped_block_fp8_gemm_impl(const void *Xq, const float *Xs, const vo
         a.blocks_per_xcd = (a.total_tiles + 7) / 8;
         return a.blocks_per_xcd * 8;
     };
-    if ((int64_t)table_rows * ((N + 127) / 128) >= (1ll << 31)) return MI355_EUNSUPPORTED;
+    if ((int64_t)table_rows * ((N + 63) / 64) >= (1ll << 31)) return MI355_EUNSUPPORTED;
     switch (block_m) {
-        case 16: return launch_grouped_tile<16, 128, 1, 4, 4>(a, finish(128), st);
-        case 32: return launch_grouped_tile<32, 128, 1, 4, 4>(a, finish(128), st);
+        case 16:
+        case 32: {
+            // weight streams; the ring tiles keep the short K (fewer than 16 steps), where the streams' waves get too few
+            // steps each (128 experts, N = 2048, K = 768, top-8, 4 / 8 tokens: 14.7 / 22.2 us against 11.5 / 19.3 for the
+            // ring, level from 16 tokens on; K = 1408, 4 tokens: 16.4 against 14.9), and a K whose scales do not fit the LDS
+            if (KB >= 16) {
+                const int r = launch_gstream(a, block_m, num_experts, st);
+                if (r != MI355_EUNSUPPORTED) return r;
+            }
+            if (block_m == 16) return launch_grouped_tile<16, 128, 1, 4, 4>(a, finish(128), st);
+            return launch_grouped_tile<32, 128, 1, 4, 4>(a, finish(128), st);
+        }
         case 64: return launch_grouped_tile<64, 128, 1, 4, 4>(a, finish(128), st);
         case 128: return launch_grouped_tile<128, 128, 2, 2, 2>(a, finish(128), st);
         case 256:
