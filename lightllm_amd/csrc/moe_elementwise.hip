@@ -21,8 +21,11 @@
 // below the bf16 rounding that follows.  The fused kernel runs exactly this code and then exactly the
 // stand-alone quantizer's code, so its bytes and scales equal those of silu_and_mul followed by the group
 // quantizer.
-#include "quant_core.hpp"
+#include <algorithm>
 #include <string.h>
+#include <type_traits>
+
+#include "quant_core.hpp"
 
 namespace mi355 {
 
@@ -78,6 +81,12 @@ __device__ __forceinline__ v4i silu_mul_chunk(const v4i &g, const v4i &u) {
     }
     return o;
 }
+
+// Four chunks per lane where that still gives every compute unit two workgroups, else one: a small launch is bound by the
+// latency of its loads and of the arithmetic behind them, not by the memory (silu_and_mul / with the quantizer, in a
+// captured graph: [4, 28672] 3.7 / 4.5 us with four, 2.3 / 2.5 with one; [512, 4096] 3.9 / 4.8 and 2.8 / 3.1; level from
+// [512, 28672] on).
+static bool unroll_pays(int64_t chunks) { return chunks >= (int64_t)device_cus() * 2048; }
 
 // Row/column of output chunk c (8 elements) when a row holds cpr chunks.
 struct ChunkPos {
@@ -173,27 +182,19 @@ __global__ __launch_bounds__(256) void silu_and_mul_general_kernel(const uint16_
 }
 
 // One lane = one 8-element chunk of the OUTPUT; 16 lanes (a DPP row) = one quantization group.
-// A group never straddles rows (H % 128 == 0), so the masked-row test is uniform inside a DPP row.
-template <int UNROLL, bool MASKED>
+template <int UNROLL>
 __global__ __launch_bounds__(256) void silu_mul_quant_kernel(const uint16_t *__restrict__ in, v2i *__restrict__ q,
                                                              float *__restrict__ s, uint32_t total_chunks,
                                                              uint32_t cpr, uint32_t q256, uint32_t r256,
                                                              int64_t in_stride_m, int64_t s_stride_m,
-                                                             int64_t s_stride_g, const int32_t *__restrict__ masked_m,
-                                                             uint32_t rows_per_expert) {
+                                                             int64_t s_stride_g) {
     const uint32_t base = blockIdx.x * (256u * UNROLL) + threadIdx.x;
     v4i g[UNROLL], u[UNROLL];
     ChunkPos p[UNROLL];
-    bool live[UNROLL];
 #pragma unroll
     for (int k = 0; k < UNROLL; ++k) {
         p[k] = k == 0 ? chunk_pos(base, cpr) : chunk_next(p[k - 1], cpr, q256, r256);
-        live[k] = base + k * 256u < total_chunks;
-        if (MASKED && live[k]) {
-            uint32_t e = p[k].row / rows_per_expert, t = p[k].row - e * rows_per_expert;
-            live[k] = (int32_t)t < masked_m[e];
-        }
-        if (live[k]) {
+        if (base + k * 256u < total_chunks) {
             const uint16_t *row = in + (int64_t)p[k].row * in_stride_m;
             g[k] = __builtin_nontemporal_load((const v4i *)(row + (size_t)p[k].col * 8));
             u[k] = __builtin_nontemporal_load((const v4i *)(row + ((size_t)cpr + p[k].col) * 8));
@@ -201,7 +202,7 @@ __global__ __launch_bounds__(256) void silu_mul_quant_kernel(const uint16_t *__r
     }
 #pragma unroll
     for (int k = 0; k < UNROLL; ++k) {
-        if (live[k]) {
+        if (base + k * 256u < total_chunks) {
             v4i a = silu_mul_chunk(g[k], u[k]);
             v2i o;
             float sc;
@@ -210,6 +211,33 @@ __global__ __launch_bounds__(256) void silu_mul_quant_kernel(const uint16_t *__r
             if ((threadIdx.x & 15u) == 0)
                 s[(int64_t)p[k].row * s_stride_m + (int64_t)(p[k].col >> 4) * s_stride_g] = sc;
         }
+    }
+}
+
+// The same for the first masked_m[e] rows of every expert's rows_per_expert padded ones: the `each` workgroups of an expert
+// walk over its rows in use only.  (With a lane per padded chunk the launch was as long as the padding: 32 experts
+// x 512 rows, 16 of them in use, H = 2048: 15.8 us, 5.1 this way; all 512 in use: 39.9 and 32.2.)  A group never straddles rows (H % 128 == 0), so
+// the loop's end is uniform inside a DPP row.
+__global__ __launch_bounds__(256) void silu_mul_quant_masked_kernel(const uint16_t *__restrict__ in, v2i *__restrict__ q,
+                                                                    float *__restrict__ s, uint32_t cpr,
+                                                                    int64_t in_stride_m, int64_t s_stride_m,
+                                                                    int64_t s_stride_g,
+                                                                    const int32_t *__restrict__ masked_m,
+                                                                    uint32_t rows_per_expert, uint32_t each) {
+    const uint32_t e = blockIdx.x / each, part = blockIdx.x - e * each;
+    const uint32_t rows = min((uint32_t)max(masked_m[e], 0), rows_per_expert), total = rows * cpr;
+    const int64_t row0 = (int64_t)e * rows_per_expert;
+    for (uint32_t c = part * 256u + threadIdx.x; c < total; c += each * 256u) {
+        const ChunkPos p = chunk_pos(c, cpr);
+        const int64_t r = row0 + p.row;
+        const uint16_t *row = in + r * in_stride_m;
+        const v4i g = __builtin_nontemporal_load((const v4i *)(row + (size_t)p.col * 8));
+        const v4i u = __builtin_nontemporal_load((const v4i *)(row + ((size_t)cpr + p.col) * 8));
+        v2i o;
+        float sc;
+        quant_chunk(silu_mul_chunk(g, u), o, sc);
+        __builtin_nontemporal_store(o, q + (r * cpr + p.col));
+        if ((threadIdx.x & 15u) == 0) s[r * s_stride_m + (int64_t)(p.col >> 4) * s_stride_g] = sc;
     }
 }
 
@@ -344,11 +372,14 @@ extern "C" int mi355_silu_and_mul(const void *in, void *out, int64_t M, int64_t 
     if (vec) {
         int64_t chunks = M * (H / 8);
         if (chunks >= (int64_t)1 << 32) return MI355_EUNSUPPORTED;
-        constexpr int UNROLL = 4;
         const uint32_t cpr = (uint32_t)(H / 8);
-        uint32_t blocks = (uint32_t)((chunks + 256 * UNROLL - 1) / (256 * UNROLL));
-        return launch((silu_and_mul_kernel<UNROLL>), dim3(blocks), dim3(256), 0, st, (const uint16_t *)in,
-                           (uint16_t *)out, (uint32_t)chunks, cpr, 256u / cpr, 256u % cpr, in_stride_m, out_stride_m);
+        auto go = [&](auto unroll) {
+            constexpr int U = decltype(unroll)::value;
+            return launch(silu_and_mul_kernel<U>, dim3((uint32_t)((chunks + 256 * U - 1) / (256 * U))), dim3(256), 0, st,
+                          (const uint16_t *)in, (uint16_t *)out, (uint32_t)chunks, cpr, 256u / cpr, 256u % cpr, in_stride_m,
+                          out_stride_m);
+        };
+        return unroll_pays(chunks) ? go(std::integral_constant<int, 4>{}) : go(std::integral_constant<int, 1>{});
     } else {
         int64_t total = M * H;
         if ((total + 255) / 256 >= (int64_t)1 << 31) return MI355_EUNSUPPORTED;
@@ -387,18 +418,23 @@ extern "C" int mi355_silu_and_mul_group_quant_fp8(const void *in, void *q, float
     if (((uintptr_t)in & 15) || (in_stride_m % 8) || ((uintptr_t)q & 7) || ((uintptr_t)s & 3)) return MI355_EALIGN;
     int64_t chunks = M * (H / 8);
     if (chunks >= (int64_t)1 << 32) return MI355_EUNSUPPORTED;
-    constexpr int UNROLL = 4;
     const uint32_t cpr = (uint32_t)(H / 8);
-    uint32_t blocks = (uint32_t)((chunks + 256 * UNROLL - 1) / (256 * UNROLL));
     hipStream_t st = (hipStream_t)stream;
-    if (masked_m)
-        return launch((silu_mul_quant_kernel<UNROLL, true>), dim3(blocks), dim3(256), 0, st,
-                           (const uint16_t *)in, (v2i *)q, s, (uint32_t)chunks, cpr, 256u / cpr, 256u % cpr,
-                           in_stride_m, s_stride_m, s_stride_g, masked_m, (uint32_t)rows_per_expert);
-    else
-        return launch((silu_mul_quant_kernel<UNROLL, false>), dim3(blocks), dim3(256), 0, st,
-                           (const uint16_t *)in, (v2i *)q, s, (uint32_t)chunks, cpr, 256u / cpr, 256u % cpr,
-                           in_stride_m, s_stride_m, s_stride_g, masked_m, 1u);
+    if (masked_m) {
+        // about eight workgroups per compute unit over all experts, never more than an expert has chunks for
+        const int64_t experts = M / rows_per_expert, most = (rows_per_expert * cpr + 255) / 256;
+        const int64_t each = std::max<int64_t>(1, std::min<int64_t>(most, 8 * (int64_t)device_cus() / experts));
+        return launch(silu_mul_quant_masked_kernel, dim3((uint32_t)(experts * each)), dim3(256), 0, st, (const uint16_t *)in,
+                      (v2i *)q, s, cpr, in_stride_m, s_stride_m, s_stride_g, masked_m, (uint32_t)rows_per_expert,
+                      (uint32_t)each);
+    }
+    auto go = [&](auto unroll) {
+        constexpr int U = decltype(unroll)::value;
+        return launch(silu_mul_quant_kernel<U>, dim3((uint32_t)((chunks + 256 * U - 1) / (256 * U))), dim3(256), 0, st,
+                      (const uint16_t *)in, (v2i *)q, s, (uint32_t)chunks, cpr, 256u / cpr, 256u % cpr, in_stride_m,
+                      s_stride_m, s_stride_g);
+    };
+    return unroll_pays(chunks) ? go(std::integral_constant<int, 4>{}) : go(std::integral_constant<int, 1>{});
 }
 
 extern "C" int mi355_moe_sum_reduce(const void *in, void *out, int64_t T, int32_t topk, int64_t H, void *stream) {

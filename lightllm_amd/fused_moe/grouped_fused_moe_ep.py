@@ -50,12 +50,13 @@ def _check_operands(x, xs, w, ws, out, rows):
     return E, N, K
 
 
-def _launch(x, xs, w, ws, out, index, counts, rows, stride, E, N, K, block_m=None):
+def _launch(x, xs, w, ws, out, index, counts, rows, stride, E, N, K, block_m=None, reused=None):
+    """-> (schedule table, block_m); ``reused`` is that pair of an earlier launch over the same counts."""
     lib = _lib.lib()
     if block_m is None:
         block_m = lib.mi355_grouped_block_m(rows, E, N, K)
     assert block_m in _BLOCK_MS
-    table = moe_align2(rows, counts, block_m)
+    table = reused[0] if reused is not None and reused[1] == block_m else moe_align2(rows, counts, block_m)
     wsp = _lib.workspace(out.device, lib.mi355_grouped_workspace_bytes(table.shape[0])) if block_m == 256 else None
     code = lib.mi355_grouped_block_fp8_gemm(
         x.data_ptr(), xs.data_ptr(), w.data_ptr(), ws.data_ptr(), index.data_ptr(), xs.data_ptr(), counts.data_ptr(),
@@ -63,13 +64,10 @@ def _launch(x, xs, w, ws, out, index, counts, rows, stride, E, N, K, block_m=Non
         wsp.data_ptr() if wsp is not None else None, wsp.numel() if wsp is not None else 0, _lib.stream_ptr(out.device),
     )
     _lib.check(code, "grouped fp8 gemm")
+    return table, block_m
 
 
-def _deepgemm_grouped_fp8_nt_masked(input_tuple: Tuple[torch.Tensor, torch.Tensor],
-                                    w_tuple: Tuple[torch.Tensor, torch.Tensor], out: torch.Tensor,
-                                    masked_m: torch.Tensor, expected_m: int):
-    """out[e, :masked_m[e]] = blockscaled(x[e, :masked_m[e]] @ w[e].T).  ``expected_m`` (DeepGEMM's tiling hint) is
-    used the same way: it picks the row block."""
+def _masked(input_tuple, w_tuple, out, masked_m, expected_m, reused=None):
     x, xs = input_tuple
     w, ws = w_tuple
     assert x.ndim == 3 and out.ndim == 3 and masked_m.dtype == torch.int32 and masked_m.is_contiguous()
@@ -79,7 +77,15 @@ def _deepgemm_grouped_fp8_nt_masked(input_tuple: Tuple[torch.Tensor, torch.Tenso
     block_m = None
     if expected_m is not None and expected_m > 0:
         block_m = _lib.lib().mi355_grouped_block_m(int(min(expected_m, T)) * E, E, N, K)
-    _launch(x, xs, w, ws, out, _masked_row_table(E, T, x.device), masked_m, E * T, T, E, N, K, block_m)
+    return _launch(x, xs, w, ws, out, _masked_row_table(E, T, x.device), masked_m, E * T, T, E, N, K, block_m, reused)
+
+
+def _deepgemm_grouped_fp8_nt_masked(input_tuple: Tuple[torch.Tensor, torch.Tensor],
+                                    w_tuple: Tuple[torch.Tensor, torch.Tensor], out: torch.Tensor,
+                                    masked_m: torch.Tensor, expected_m: int):
+    """out[e, :masked_m[e]] = blockscaled(x[e, :masked_m[e]] @ w[e].T).  ``expected_m`` (DeepGEMM's tiling hint) is
+    used the same way: it picks the row block."""
+    _masked(input_tuple, w_tuple, out, masked_m, expected_m)
     return out
 
 
@@ -115,9 +121,9 @@ def masked_group_gemm(recv_x: Tuple[torch.Tensor, torch.Tensor], masked_m: torch
     gemm_out_a = torch.empty((E, padded_m, N), device=x.device, dtype=dtype)
     qsilu_out = torch.empty((E, padded_m, N // 2), dtype=w1.dtype, device=x.device)
     qsilu_out_scale = torch.empty((E, padded_m, N // 2 // 128), device=x.device, dtype=torch.float32)
-    _deepgemm_grouped_fp8_nt_masked(recv_x, (w1, w1_scale), gemm_out_a, masked_m, expected_m)
+    schedule = _masked(recv_x, (w1, w1_scale), gemm_out_a, masked_m, expected_m)
     silu_and_mul_masked_post_quant_fwd(gemm_out_a, qsilu_out, qsilu_out_scale, 128, masked_m)
     del gemm_out_a
     gemm_out_b = torch.empty((E, padded_m, w2.shape[1]), device=x.device, dtype=dtype)
-    _deepgemm_grouped_fp8_nt_masked((qsilu_out, qsilu_out_scale), (w2, w2_scale), gemm_out_b, masked_m, expected_m)
+    _masked((qsilu_out, qsilu_out_scale), (w2, w2_scale), gemm_out_b, masked_m, expected_m, schedule)
     return gemm_out_b

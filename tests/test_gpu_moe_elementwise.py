@@ -273,3 +273,47 @@ def test_weight_dequant_every_byte(hip):
     nan = (want & 0x7FFF) > 0x7F80
     assert np.array_equal(got[~nan], want[~nan])
     assert np.all((got[nan] & 0x7FFF) > 0x7F80)
+
+
+@pytest.mark.parametrize("M", [4095, 4096, 4097])
+def test_one_or_four_chunks_per_lane(hip, M):
+    """Both sides of the line between one and four chunks per lane (524288 chunks on 256 compute units): every row must
+    come out as it does in a small launch."""
+    from lightllm_amd.fused_moe import silu_and_mul_fwd, silu_and_mul_post_quant_fwd
+
+    print(f"silu chunks per lane M={M}", flush=True)
+    H_ = 1024
+    x = torch.randn((M, 2 * H_), generator=H.gen(M)).to(torch.bfloat16).cuda()
+    act = torch.empty((M, H_), dtype=torch.bfloat16, device="cuda")
+    q = torch.empty((M, H_), dtype=torch.float8_e4m3fn, device="cuda")
+    s = torch.empty((M, H_ // 128), dtype=torch.float32, device="cuda")
+    silu_and_mul_fwd(x, act)
+    silu_and_mul_post_quant_fwd(x, q, s)
+    for r in (0, 1500, M - 33):
+        a, b, c = torch.empty_like(act[:33]), torch.empty_like(q[:33]), torch.empty_like(s[:33])
+        silu_and_mul_fwd(x[r:r + 33], a)
+        silu_and_mul_post_quant_fwd(x[r:r + 33], b, c)
+        assert torch.equal(a, act[r:r + 33])
+        assert torch.equal(b.view(torch.uint8), q[r:r + 33].view(torch.uint8)) and torch.equal(c, s[r:r + 33])
+
+
+@pytest.mark.parametrize("E,T,H_,rows", [(5, 40, 256, [0, 1, 40, 7, 39]), (2, 3000, 1536, [2999, 1]),
+                                         (700, 8, 128, [8, 0, 3] * 233 + [5])])
+def test_masked_rows_walk(hip, E, T, H_, rows):
+    """Experts with no, one and all rows in use; more rows than the workgroups of an expert cover at once; more experts
+    than workgroups: rows in use as the flat kernel gives them, all others untouched."""
+    from lightllm_amd.fused_moe import silu_and_mul_masked_post_quant_fwd, silu_and_mul_post_quant_fwd
+
+    print(f"silu masked E={E} T={T} H={H_}", flush=True)
+    x = torch.randn((E, T, 2 * H_), generator=H.gen(T)).to(torch.bfloat16).cuda()
+    q = torch.full((E, T, H_), 0x55, dtype=torch.uint8, device="cuda").view(torch.float8_e4m3fn)
+    s = torch.full((E, T, H_ // 128), -3.0, dtype=torch.float32, device="cuda")
+    m = torch.tensor(rows, dtype=torch.int32, device="cuda")
+    silu_and_mul_masked_post_quant_fwd(x, q, s, 128, m)
+    fq = torch.empty((E * T, H_), dtype=torch.float8_e4m3fn, device="cuda")
+    fs = torch.empty((E * T, H_ // 128), dtype=torch.float32, device="cuda")
+    silu_and_mul_post_quant_fwd(x.view(E * T, 2 * H_), fq, fs)
+    used = torch.arange(T, device="cuda")[None, :] < m[:, None]
+    want_q = torch.where(used[..., None], fq.view(torch.uint8).view(E, T, H_), torch.tensor(0x55, dtype=torch.uint8, device="cuda"))
+    want_s = torch.where(used[..., None], fs.view(E, T, -1), torch.tensor(-3.0, device="cuda"))
+    assert torch.equal(q.view(torch.uint8), want_q) and torch.equal(s, want_s)
