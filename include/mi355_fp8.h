@@ -287,6 +287,24 @@ int mi355_grouped_block_fp8_gemm_bias(const void *Xq, const float *Xs, const voi
                                       void *ws, size_t ws_bytes, int32_t out_dtype, const void *bias,
                                       int32_t bias_dtype, int64_t bias_stride_e, void *stream);
 
+/* ---------------------------------------------------------------------------
+ * The routed-expert FFN in one call (fused_experts_impl, .../fused_moe/grouped_fused_moe.py:992-1115, "blocked" layout without
+ * limit / alpha): moe_align_fused, moe_align2, the activation quantizer, the gate_up GEMM, mi355_silu_and_mul_group_quant_fp8, the
+ * down GEMM with the routed weight and moe_sum_reduce, with the results of those entry points called one by one.
+ *     out[t] = sum_k weight[t, k] * ( silu_mul( x[t] . w1[e]^T ) . w2[e]^T ),  e = topk_ids[t, k]
+ * x bf16 [T, hidden], topk_ids int32 [T, topk], topk_weights fp32 [T, topk], w1 e4m3fn [E, 2*inter, hidden], w2 e4m3fn
+ * [E, hidden, inter] with fp32 128x128-block scales s1, s2, out bf16 [T, hidden] (may be x); all contiguous; hidden and inter
+ * multiples of 128.  b1 [E, 2*inter] / b2 [E, hidden]: optional biases, as for mi355_grouped_block_fp8_gemm_bias.
+ * scratch: mi355_routed_ffn_scratch_bytes() bytes, 16-byte aligned, any contents.  workspace: as for
+ * mi355_grouped_block_fp8_gemm, of mi355_routed_ffn_workspace_bytes() bytes (0: none used). */
+size_t mi355_routed_ffn_scratch_bytes(int64_t T, int32_t topk, int32_t E, int64_t hidden, int64_t inter);
+size_t mi355_routed_ffn_workspace_bytes(int64_t T, int32_t topk, int32_t E, int64_t hidden, int64_t inter);
+int mi355_routed_ffn(const void *x, const int32_t *topk_ids, const float *topk_weights, int64_t T, int32_t topk, int32_t E,
+                     int64_t hidden, int64_t inter, const void *w1, const float *s1, const void *w2, const float *s2,
+                     const void *b1, int32_t b1_dtype, int64_t b1_stride_e, const void *b2, int32_t b2_dtype,
+                     int64_t b2_stride_e, void *out, void *scratch, size_t scratch_bytes, void *ws, size_t ws_bytes,
+                     void *stream);
+
 /* ---- element-wise steps between / after the two expert GEMMs ------------------------------------------------ */
 
 /*

@@ -72,6 +72,13 @@ SIGNATURES = {
         [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i64, _i64, _i32, _i32, _i64, _i64, _i32, _vp, _vp,
          _c.c_size_t, _i32, _vp, _i32, _i64, _vp],
     ),
+    "mi355_routed_ffn_scratch_bytes": (_sz, [_i64, _i32, _i32, _i64, _i64]),
+    "mi355_routed_ffn_workspace_bytes": (_sz, [_i64, _i32, _i32, _i64, _i64]),
+    "mi355_routed_ffn": (
+        _c.c_int,
+        [_vp, _vp, _vp, _i64, _i32, _i32, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _i32, _i64, _vp, _i32, _i64, _vp, _vp, _sz,
+         _vp, _sz, _vp],
+    ),
     "mi355_silu_and_mul": (_c.c_int, [_vp, _vp, _i64, _i64, _i64, _i64, _vp]),
     "mi355_silu_and_mul_ex": (_c.c_int, [_vp, _vp, _i64, _i64, _i64, _i64, _i32, _i32, _f32, _f32, _vp]),
     "mi355_silu_and_mul_group_quant_fp8": (

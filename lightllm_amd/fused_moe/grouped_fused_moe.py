@@ -6,7 +6,8 @@ lightllm/common/basemodel/triton_kernel/fused_moe/grouped_fused_moe.py of the re
 the work is done by ``mi355_moe_align_fused``, ``mi355_moe_align2`` and ``mi355_grouped_block_fp8_gemm``.
 Only the fp8 128x128-block branch exists here (use_fp8_w8a8=True with 3-D weight scales).
 """
-from typing import Optional
+import functools
+from typing import Optional, Tuple
 
 import torch
 
@@ -182,6 +183,68 @@ def grouped_matmul(
     return (table, block_m)
 
 
+@functools.lru_cache(maxsize=4096)
+def _ffn_sizes(tokens: int, topk: int, experts: int, hidden: int, inter: int, device_index: int) -> Tuple[int, int]:
+    """(scratch bytes, workspace bytes) of a routed FFN: what the library says for the device."""
+    lib, shape = _lib.lib(), (tokens, topk, experts, hidden, inter)
+    return lib.mi355_routed_ffn_scratch_bytes(*shape), lib.mi355_routed_ffn_workspace_bytes(*shape)
+
+
+def _routed_ffn(x, w1, w2, topk_weights, topk_ids, w1_scale, w2_scale, w1_bias, w2_bias, inplace,
+                alloc_tensor_func) -> Optional[torch.Tensor]:
+    """The routed FFN in one library call per chunk of tokens.  Operands the call does not take as they are (and anything
+    that is wrong) return None and go step by step, where every operator checks its own."""
+    tokens, hidden = x.shape
+    E, n, k = w1.shape
+    inter, topk = n // 2, topk_ids.shape[1]
+    f32 = torch.float32
+    if tokens == 0 or topk == 0 or topk_ids.shape[0] < tokens or w1_scale is None or w2_scale is None:
+        return None
+    if w2.shape != (E, hidden, inter) or hidden % 128 != 0:
+        return None
+    if w1_scale.shape != (E, n // 128, k // 128) or w2_scale.shape != (E, hidden // 128, inter // 128):
+        return None
+    if not (topk_ids.dtype is torch.int32 and topk_weights.dtype is f32 and w1.dtype is torch.float8_e4m3fn
+            and w2.dtype is torch.float8_e4m3fn and w1_scale.dtype is f32 and w2_scale.dtype is f32):
+        return None
+    for t in (topk_ids, topk_weights, w1_scale, w2_scale):
+        if not t.is_contiguous():
+            return None
+    for t in (x, w1, w2, topk_ids, topk_weights, w1_scale, w2_scale, w1_bias, w2_bias):
+        if t is not None and not t.is_cuda:
+            return None
+    bias = []
+    for b, cols in ((w1_bias, n), (w2_bias, hidden)):
+        if b is None:
+            bias += [None, 0, 0]
+        elif b.shape == (E, cols) and b.stride(1) == 1 and b.dtype in _lib.DTYPE_CODES:
+            bias += [b.data_ptr(), _lib.DTYPE_CODES[b.dtype], b.stride(0)]
+        else:
+            return None
+    device = x.device
+    rows = min(tokens, FFN_MOE_CHUNK_SIZE)
+    scratch_need, ws_need = _ffn_sizes(rows, topk, E, hidden, inter, device.index)
+    last = tokens % FFN_MOE_CHUNK_SIZE
+    if tokens > rows and last:
+        last_need = _ffn_sizes(last, topk, E, hidden, inter, device.index)
+        scratch_need, ws_need = max(scratch_need, last_need[0]), max(ws_need, last_need[1])
+    scratch = alloc_tensor_func((scratch_need,), dtype=torch.uint8, device=device)
+    out = x if inplace else alloc_tensor_func(x.shape, dtype=x.dtype, device=device)
+    stream = _lib.stream_ptr(device)
+    ws = _lib.workspace(device, ws_need, stream) if ws_need else None
+    call = _lib.lib().mi355_routed_ffn
+    for begin in range(0, tokens, FFN_MOE_CHUNK_SIZE):
+        count = min(tokens - begin, FFN_MOE_CHUNK_SIZE)
+        code = call(
+            x.data_ptr() + begin * hidden * 2, topk_ids.data_ptr() + begin * topk * 4, topk_weights.data_ptr() + begin * topk * 4,
+            count, topk, E, hidden, inter, w1.data_ptr(), w1_scale.data_ptr(), w2.data_ptr(), w2_scale.data_ptr(), *bias,
+            out.data_ptr() + begin * hidden * 2, scratch.data_ptr(), scratch_need, ws.data_ptr() if ws is not None else None,
+            ws.numel() if ws is not None else 0, stream,
+        )
+        _lib.check(code, "fused_experts")
+    return out
+
+
 def fused_experts_impl(
     hidden_states: torch.Tensor,
     w1: torch.Tensor,
@@ -224,6 +287,11 @@ def fused_experts_impl(
     E, N, _ = w1.shape
     assert N % 256 == 0 and w2.shape[2] == N // 2, "intermediate size must be a multiple of 128"
     topk_num = topk_ids.shape[1]
+    if fused_act and run_config is None:
+        out = _routed_ffn(hidden_states, w1, w2, topk_weights, topk_ids, w1_scale, w2_scale, w1_bias, w2_bias, inplace,
+                          alloc_tensor_func)
+        if out is not None:
+            return out
     M = min(num_tokens, FFN_MOE_CHUNK_SIZE)
     device, dtype = hidden_states.device, hidden_states.dtype
 

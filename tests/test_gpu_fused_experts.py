@@ -118,3 +118,34 @@ def test_fused_experts_inplace_and_deterministic(hip):
     torch.cuda.synchronize()
     assert torch.equal(a, b)
     assert c.data_ptr() == xin.data_ptr() and torch.equal(c, a)
+
+
+# the first launch's pair limit and one past it, single tokens and experts, more experts than it counts, ids that are not 16-byte
+# aligned, schedules of two block sizes (E = 8, 12 rows per expert, K = 2048 / 768), 256-row blocks
+@pytest.mark.parametrize("T,E,topk,Hd,I", [(1, 1, 1, 128, 128), (3, 1024, 8, 256, 128), (3, 1025, 8, 256, 128),
+                                           (512, 16, 8, 256, 128), (513, 16, 8, 256, 128), (4095, 5, 1, 128, 128),
+                                           (4097, 5, 1, 128, 128), (37, 7, 3, 384, 256), (48, 8, 2, 2048, 768),
+                                           (300, 4, 2, 1024, 1024)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_fused_experts_in_one_call_equals_the_steps(hip, T, E, topk, Hd, I, offset):
+    """An (empty) run_config sends the layer through the operators one by one: the same bits, in place too."""
+    from lightllm_amd.fused_moe import fused_experts_impl
+
+    print(f"fused_experts one call T={T} E={E} topk={topk} H={Hd} I={I} offset={offset}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(T + E)
+    w1 = torch.randint(0, 0x70, (E, 2 * I, Hd), dtype=torch.uint8, device="cuda", generator=g).view(torch.float8_e4m3fn)
+    w2 = torch.randint(0, 0x70, (E, Hd, I), dtype=torch.uint8, device="cuda", generator=g).view(torch.float8_e4m3fn)
+    s1 = torch.rand((E, 2 * I // 128, Hd // 128), device="cuda", generator=g) * 1e-3
+    s2 = torch.rand((E, Hd // 128, I // 128), device="cuda", generator=g) * 1e-3
+    x = H.activations(T, Hd, seed=T).cuda()
+    ids, tw = H.routing(T, E, topk, seed=T + E)
+    ids_buf = torch.empty(offset + T * topk, dtype=torch.int32, device="cuda")
+    ids_dev = ids_buf[offset:].view(T, topk).copy_(ids)
+    kw = dict(use_fp8_w8a8=True, w1_scale=s1, w2_scale=s2)
+    want = fused_experts_impl(x, w1, w2, tw.cuda(), ids_dev, run_config={}, **kw)
+    got = fused_experts_impl(x, w1, w2, tw.cuda(), ids_dev, **kw)
+    inp = x.clone()
+    fused_experts_impl(inp, w1, w2, tw.cuda(), ids_dev, inplace=True, **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    assert torch.equal(inp.view(torch.int16), want.view(torch.int16))

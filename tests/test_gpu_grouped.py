@@ -52,6 +52,13 @@ def test_moe_align_fused_reference_vectors(hip):
     _check_align(ids, torch.arange(ids.numel(), dtype=torch.float32).reshape(5121, 8), 257)
 
 
+@pytest.mark.parametrize("pairs", [1, 3, 1023, 1025, 4095, 4096, 4097, 16383, 16385, 49153])
+def test_moe_align_fused_at_the_ends_of_its_passes(hip, pairs):
+    print(f"moe_align_fused {pairs} pairs", flush=True)
+    ids = torch.randint(0, 9, (pairs, 1), generator=H.gen(pairs), dtype=torch.int32)
+    _check_align(ids, torch.rand((pairs, 1), generator=H.gen(pairs + 1)), 9)
+
+
 def test_moe_align_and_align1_reference_vectors(hip):
     """Golden vectors of the reference's test_moe_align / test_moe_align1 (test_grouped_fused_moe.py:26-77), then
     the two-step form against the oracle at sizes that span several 4096-pair steps and every padding."""
