@@ -142,6 +142,8 @@ class FP8w8a8B128Mi355QuantizationMethod(FP8w8a8B128QuantizationMethod):
         if (x_ptr | w_ptr) & 15:
             return None
         fused, ws_need = _linear_plan(m, n, k, dtype, device.index)
+        if fused and x_ptr < out.data_ptr() + 2 * m * n and out.data_ptr() < x_ptr + 2 * m * k:
+            fused = False  # every workgroup of the stream reads all of x: one that is done must not store over it
         xq_ptr = xs_ptr = ws_ptr = None
         if not fused:
             x_q = alloc((m, k), dtype=torch.float8_e4m3fn, device=device)

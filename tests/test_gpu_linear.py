@@ -67,3 +67,19 @@ def test_output_argument_and_odd_operands(hip):
         method.apply(shifted, WeightPack(wq, ws))
     with pytest.raises(AssertionError):
         method.apply(x.float(), WeightPack(wq, ws))
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 4096, 4096), (4, 4096, 4096), (4, 6144, 4096), (8, 2048, 4096)])
+def test_output_over_the_activations(hip, M, N, K):
+    """An output that shares memory with the activations (whole, or its rows behind a part of them) holds what a separate one does."""
+    from lightllm_amd.quantization import QUANTMETHODS, WeightPack
+
+    wq, ws = H.quantized_weights(N, K, seed=N + K, device="cuda")
+    x = H.activations(M, K, seed=M).cuda()
+    want = _composed(x, wq, ws, torch.bfloat16)
+    for shift in (0, 64):
+        buf = torch.zeros(M * max(N, K) + shift, dtype=torch.bfloat16, device="cuda")
+        mine = buf[: M * K].view(M, K).copy_(x)
+        out = buf[shift: shift + M * N].view(M, N)
+        assert QUANTMETHODS.get("fp8w8a8-b128").apply(mine, WeightPack(wq, ws), out=out) is out
+        assert torch.equal(out, want), shift
