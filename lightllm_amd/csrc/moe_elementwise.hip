@@ -227,7 +227,9 @@ __global__ __launch_bounds__(256) void silu_mul_quant_masked_kernel(const uint16
     const uint32_t e = blockIdx.x / each, part = blockIdx.x - e * each;
     const uint32_t rows = min((uint32_t)max(masked_m[e], 0), rows_per_expert), total = rows * cpr;
     const int64_t row0 = (int64_t)e * rows_per_expert;
-    for (uint32_t c = part * 256u + threadIdx.x; c < total; c += each * 256u) {
+    // 64 bits: up to 2^32 - 1 chunks, and a step past them must not wrap
+    for (uint64_t at = part * 256u + threadIdx.x; at < total; at += each * 256u) {
+        const uint32_t c = (uint32_t)at;
         const ChunkPos p = chunk_pos(c, cpr);
         const int64_t r = row0 + p.row;
         const uint16_t *row = in + r * in_stride_m;
