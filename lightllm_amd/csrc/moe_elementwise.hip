@@ -253,28 +253,32 @@ __global__ __launch_bounds__(256) void moe_sum_reduce_kernel(const v4i *__restri
     float acc[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] = 0.f;
+    auto add = [&](const v4i &v) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t d = (uint32_t)v[i];
+            acc[2 * i] += as_f32(d << 16);
+            acc[2 * i + 1] += as_f32(d & 0xffff0000u);
+        }
+    };
     int k = 0;
     for (; k + UNROLL <= topk; k += UNROLL) {
         v4i v[UNROLL];
 #pragma unroll
         for (int j = 0; j < UNROLL; ++j) v[j] = __builtin_nontemporal_load(src + (size_t)(k + j) * cpr);
 #pragma unroll
-        for (int j = 0; j < UNROLL; ++j)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                uint32_t d = (uint32_t)v[j][i];
-                acc[2 * i] += as_f32(d << 16);
-                acc[2 * i + 1] += as_f32(d & 0xffff0000u);
-            }
+        for (int j = 0; j < UNROLL; ++j) add(v[j]);
     }
-    for (; k < topk; ++k) {
-        v4i v = __builtin_nontemporal_load(src + (size_t)k * cpr);
+    if constexpr (UNROLL > 4) {  // the rest, all requests first
+        v4i v[UNROLL - 1];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            uint32_t d = (uint32_t)v[i];
-            acc[2 * i] += as_f32(d << 16);
-            acc[2 * i + 1] += as_f32(d & 0xffff0000u);
-        }
+        for (int j = 0; j < UNROLL - 1; ++j)
+            if (k + j < topk) v[j] = __builtin_nontemporal_load(src + (size_t)(k + j) * cpr);
+#pragma unroll
+        for (int j = 0; j < UNROLL - 1; ++j)
+            if (k + j < topk) add(v[j]);
+    } else {
+        for (; k < topk; ++k) add(__builtin_nontemporal_load(src + (size_t)k * cpr));
     }
     v4i o;
 #pragma unroll
@@ -447,8 +451,12 @@ extern "C" int mi355_moe_sum_reduce(const void *in, void *out, int64_t T, int32_
     if (H % 8 == 0 && !((uintptr_t)in & 15) && !((uintptr_t)out & 15)) {
         int64_t chunks = T * (H / 8);
         if (chunks >= (int64_t)1 << 32) return MI355_EUNSUPPORTED;
-        return launch((moe_sum_reduce_kernel<4>), dim3((uint32_t)((chunks + 255) / 256)), dim3(256), 0, st,
-                           (const v4i *)in, (v4i *)out, (uint32_t)chunks, (uint32_t)(H / 8), topk);
+        // Eight slots requested at once while the launch is bound by latency ([T, topk, H] in a captured graph, four against
+        // eight: [4, 8, 2048] 2.17 and 1.96 us, [64, 8, 7168] 2.37 and 2.15, [512, 8, 2048] 3.82 and 3.21), four where the
+        // memory bounds it ([4096, 8, 7168] 85.7 and 87.7).
+        const auto kernel = unroll_pays(chunks) ? moe_sum_reduce_kernel<4> : moe_sum_reduce_kernel<8>;
+        return launch(kernel, dim3((uint32_t)((chunks + 255) / 256)), dim3(256), 0, st, (const v4i *)in, (v4i *)out,
+                      (uint32_t)chunks, (uint32_t)(H / 8), topk);
     } else {
         int64_t total = T * H;
         if ((total + 255) / 256 >= (int64_t)1 << 31) return MI355_EUNSUPPORTED;

@@ -248,6 +248,12 @@ def test_moe_sum_reduce_bit_exact(hip, T, topk, Hd):
     assert np.array_equal(tr.bits_of(out), oracle.moe_sum_reduce(tr.bits_of(x)))
 
 
+@pytest.mark.parametrize("T,topk,Hd", [(7, 7, 256), (7, 9, 256), (3, 15, 136), (1025, 2, 4096), (1025, 6, 4096), (1024, 8, 4096)])
+def test_moe_sum_reduce_remainders_and_large_launches(hip, T, topk, Hd):
+    """Remainders of the eight-slot form, and both sides of the line (2048 chunks per compute unit) to the four-slot form."""
+    test_moe_sum_reduce_bit_exact(hip, T, topk, Hd)
+
+
 @pytest.mark.parametrize("N,K", [(128, 128), (256, 512), (200, 304), (130, 100), (576, 7168)])
 def test_weight_dequant_bit_exact(hip, N, K):
     from lightllm_amd.quantization import weight_dequant
