@@ -188,7 +188,8 @@ int mi355_block_fp8_gemm_dtype(const void *A, const void *B, const float *As, co
  *     Ws[nb*ws_n + kb*ws_k];  C [M,N], row stride ldc, c_dtype MI355_DTYPE_BF16 / _F16
  * x_q, x_s  room for the quantized activations e4m3fn [M,K] and their scales fp32 [M,K/128] (16-byte aligned), or both
  *     NULL where mi355_block_fp8_linear_fused() returns 1 for (M, N, K, x_dtype): few rows, whose activations are quantized
- *     inside the weight stream (packed operands only: ldw = K, 16-byte aligned).  Same bytes, same scales either way.
+ *     inside the weight stream (packed operands only: ldw = K, 16-byte aligned; C and x must not overlap, MI355_EINVAL if
+ *     they do - with x_q and x_s given C may lie over x).  Same bytes, same scales either way.
  * ws  as for mi355_block_fp8_gemm, of mi355_block_fp8_linear_workspace_bytes() bytes (0: none needed).
  */
 int32_t mi355_block_fp8_linear_fused(int64_t M, int64_t N, int64_t K, int32_t x_dtype);

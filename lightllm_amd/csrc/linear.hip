@@ -127,6 +127,9 @@ extern "C" int mi355_block_fp8_linear(const void *x, int32_t x_dtype, const void
         const bool ws_ok = ws && ((uintptr_t)ws & 15) == 0 && ws_bytes >= f.ws_bytes;
         if (!f.ok || ldw != K || !fast_layout_ok(x, W, K, K, 1, ldw)) return MI355_EUNSUPPORTED;
         if (f.ws_bytes > 0 && !ws_ok) return MI355_EWORKSPACE;
+        // every workgroup reads all of x: one that is done must not store over what another has yet to read
+        const uintptr_t x0 = (uintptr_t)x, c0 = (uintptr_t)C;
+        if (x0 < c0 + 2 * (uintptr_t)((M - 1) * ldc + N) && c0 < x0 + 2 * (uintptr_t)(M * K)) return MI355_EINVAL;
         GemmArgs a = {};
         a.out_f16 = c_dtype == MI355_DTYPE_F16 ? 1 : 0;
         a.X = (const uint8_t *)x;

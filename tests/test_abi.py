@@ -94,6 +94,27 @@ def test_preconditions_are_checked_before_launch():
     assert lib.mi355_moe_align2(None, 0, 16, 4, None, None) == -1
 
 
+def test_linear_that_quantizes_in_its_stream_refuses_an_output_over_its_activations():
+    """Without room for quantized activations every workgroup reads x while others store C: an overlap of the two is
+    refused before any launch (no memory is touched; the addresses are made up)."""
+    from lightllm_amd import _lib
+
+    lib = _lib.lib()
+    x, w, ws, room = 1 << 40, 1 << 41, 1 << 42, 1 << 43
+
+    def call(c, m, n, k, ldc):
+        return lib.mi355_block_fp8_linear(x, 0, w, ws, c, m, n, k, k, k // 128, 1, ldc, None, None, room, 1 << 30, 0, None)
+
+    for m, n, k, ldc in [(1, 4096, 4096, 4096), (4, 4096, 4096, 4096), (8, 2048, 4096, 2048), (4, 2112, 7168, 4096)]:
+        assert lib.mi355_block_fp8_linear_fused(m, n, k, 0) == 1
+        x_bytes, c_bytes = 2 * m * k, 2 * ((m - 1) * ldc + n)
+        for c in (x, x + 64, x + x_bytes - 16, x - c_bytes + 16):
+            assert call(c, m, n, k, ldc) == -1, (m, n, k, c - x)
+        if not torch.cuda.is_available():   # past the check: the launch itself is what fails here
+            for c in (x + x_bytes, x - c_bytes):
+                assert call(c, m, n, k, ldc) == -5, (m, n, k, c - x)
+
+
 REFERENCE_SIGNATURES = {
     # (module, function): signature string of the reference's function of the same name
     ("lightllm_amd.quantization.fp8act_quant_kernel", "per_token_group_quant_fp8"):
