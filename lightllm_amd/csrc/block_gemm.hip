@@ -1171,14 +1171,13 @@ extern "C" int32_t mi355_grouped_block_m(int64_t num_pairs, int32_t num_experts,
     const int64_t avg = num_pairs / num_experts;
     // 256-row schedule blocks run as the persistent launch with two queues: blocks of more than 64 rows on the
     // 256x256 ping-pong tile (it skips the empty 64-row halves of ragged blocks), the others on the 64x512
-    // weight-streaming tile.  That launch needs more tiles than compute units.  With fewer rows the weight streams of
-    // 16- and 32-row schedules (gemm_gstream.hpp) are ahead: they read at 6 to 7 TB/s until many experts have more than
-    // 32 rows and are read twice (256 experts, top-8, N = 4096, K = 7168, 16 / 24 / 32 rows per expert: 1179 / 1327 / 1755
-    // us for the 32-row stream against 1277 / 1302 / 1318; 32 experts, 16 / 22 / 32 rows: 155 / 171 / 225 against 174 / 175 /
-    // 177; N = 7168, K = 2048: 86.5 / 97.6 / 125 against 100 / 102 / 105).
+    // weight-streaming tile.  That launch needs more tiles than compute units, and its time hardly depends on how the rows
+    // are spread.  With fewer rows the weight streams of 16- and 32-row schedules (gemm_gstream.hpp, K of 16 steps
+    // or more) are ahead: they read at 6 to 7 TB/s, once per 32 rows of an expert, so what they cost follows the second reads
+    // of popular experts.  Every line between the two lies where Zipf(1.1) popularity costs the stream its lead.
     const int cus = device_cus();
     const int64_t tiles256 = (int64_t)num_experts * ((N + 255) / 256);
-    const bool two_queues = tiles256 > cus;
+    const bool two_queues = tiles256 > cus, stream = K >= 16 * kBlockK;
     // Measured over Qwen3-MoE (128 experts), DeepSeek-V2-Lite (64), Mixtral (8), a DeepSeek-V3 expert-parallel slice
     // (32 experts, N = 512) and a 16-expert shape, 8 to 8192 tokens, uniform routing:
     //  * 128-row blocks are ahead of the 256-row launch up to a few hundred rows per expert where the whole launch
@@ -1194,13 +1193,36 @@ extern "C" int32_t mi355_grouped_block_m(int64_t num_pairs, int32_t num_experts,
         if (tiles256 * 2 <= cus && avg > (large_expert ? 32 : 64) && avg <= (large_expert ? 160 : 256)) return 128;
         if ((int64_t)num_experts * N * K <= 500000000ll && K <= 2048 && avg <= (K <= 1536 ? 224 : 112)) return 128;
     }
-    //  * with 8 experts every block re-reads a large expert, and 64-row blocks beat blocks of the average size from 21
-    //    rows per expert on (Mixtral down, 20 / 24 rows: 84.8 / 86.1 us against 77.8 / 96.3 for the 32-row stream); with K
-    //    under 2048, where 16- and 32-row blocks are ring tiles, from 9
-    if (num_experts <= 8 && avg > (K >= 2048 ? 20 : 8) && avg <= 40) return 64;
-    //  * the two-queue launch takes over from 21 rows per expert where an expert's N is wide (12 with a short K), from 25
-    //    where it is not (Qwen3-30B gate_up, N = 1536, 24 rows: 84.6 us for the 32-row stream against 92.6)
-    if (avg > 64 || (two_queues && avg >= (N >= 4096 ? (K >= 2048 ? 21 : 12) : 25))) return 256;
+    //  * with 8 experts every block re-reads a large expert, and 64-row blocks beat ring tiles of the average size from 9
+    //    rows per expert on, the weight streams from 21 (Mixtral gate_up, 20 rows, even / Zipf: 156 / 171 us for the 32-row
+    //    stream against 215 / 214) - from 13 where the experts' 64-column tiles just fill the two workgroups a unit holds
+    //    and the second entry of one expert starts another round (Mixtral down, 512 tiles, 12 rows: 74 / 78 against 82 /
+    //    83; 14 rows, with a second entry: 101 against 83; N = 4096, K = 7168: 53 against 46)
+    if (num_experts <= 8) {
+        const int64_t tiles64 = (int64_t)num_experts * ((N + 63) / 64);
+        const bool fills_one_round = tiles64 <= 2 * cus && tiles64 * 5 > 8 * (int64_t)cus;
+        if (avg > (!stream ? 8 : fills_one_round ? 12 : 20) && avg <= 40) return 64;
+    }
+    //  * where an expert's N is wide the two-queue launch takes over from 12 rows per expert under a short K.  Against the
+    //    streams it does so the earlier the more experts there are to be popular, and the less a step costs beside the
+    //    outputs (us for the stream, even / Zipf routing, against the two-queue launch, which is the same for both within
+    //    5 %.  256 experts, N = 4096, K = 7168, 12 / 14 / 16 / 20 rows: 1124 / 1252, 1144 / 1298, 1166 / 1371, 1230 / 1505
+    //    against 1264 ... 1297; N = 7168, K = 2048, 12 / 16 rows: 615 / 683, 666 / 758 against 674 / 688.  128 experts, 16 /
+    //    18 rows: 577 / 664, 595 / 697 against 641 / 677; 12 / 14 rows: 300 / 345, 312 / 351 against 345 / 348.  64 experts,
+    //    20 rows: 298 / 358 against 331 / 374; 14 / 16 rows: 151 / 168, 158 / 192 against 185 / 185.  32 experts, 20 rows:
+    //    145 / 173 against 176 / 221; 16 / 20 rows: 90 / 95, 93 / 104 against 101 / 103)
+    //  * from 25 where N is not wide (Qwen3-30B gate_up, N = 1536, 24 rows: 88 / 100 us for the 32-row stream against 95)
+    int64_t line = 25;
+    if (N >= 4096) {
+        if (!stream) line = 12;
+        else if (K >= 4096) line = num_experts <= 64 ? 21 : num_experts <= 128 ? 17 : 13;
+        else line = num_experts <= 32 ? 17 : num_experts <= 64 ? 16 : 12;
+    }
+    if (avg > 64 || (two_queues && avg >= line)) return 256;
+    //  * a stream's 16-row entries run in pairs, and the workgroups of the second ones, which have nothing to do, show where
+    //    an entry is short and an expert has few tiles (Qwen3-30B gate_up, 16 rows, even / Zipf: 80 / 86 us for 16-row
+    //    entries, 75 / 82 for 32-row ones, 87 / 84 for the ring tiles; level with a longer K or a wide N)
+    if (stream && K < 4096 && N < 4096 && avg > 8 && avg <= 32) return 32;
     if (avg <= 16) return 16;
     if (avg <= 32) return 32;
     return 64;

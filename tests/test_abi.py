@@ -94,6 +94,24 @@ def test_preconditions_are_checked_before_launch():
     assert lib.mi355_moe_align2(None, 0, 16, 4, None, None) == -1
 
 
+def test_grouped_block_m_holds_under_uneven_routing():
+    """The row blocks around the lines between the weight streams and the launches whose time does not depend on how the
+    rows are spread: rows per expert -> block, per (experts, N, K)."""
+    from lightllm_amd import _lib
+
+    lib = _lib.lib()
+    expect = {
+        (256, 4096, 7168): {8: 16, 12: 16, 13: 256, 16: 256, 20: 256}, (256, 7168, 2048): {11: 16, 12: 256, 16: 256},
+        (128, 4096, 7168): {16: 16, 17: 256}, (128, 7168, 2048): {11: 16, 12: 256},
+        (32, 4096, 7168): {16: 16, 20: 32, 21: 256}, (64, 7168, 2048): {15: 16, 16: 256}, (32, 7168, 2048): {16: 16, 17: 256},
+        (128, 4096, 1536): {11: 16, 12: 256}, (128, 3072, 4096): {16: 16, 24: 32, 25: 256},
+        (8, 28672, 4096): {12: 16, 20: 32, 21: 64}, (8, 4096, 14336): {12: 16, 13: 64, 20: 64}, (8, 2048, 4096): {20: 32, 21: 64},
+        (8, 7168, 1024): {8: 16, 9: 64}, (128, 1536, 2048): {8: 16, 9: 32, 24: 32, 25: 256}, (128, 2048, 768): {9: 16, 16: 16},
+    }
+    got = {s: {a: lib.mi355_grouped_block_m(a * s[0], *s) for a in e} for s, e in expect.items()}
+    assert got == expect, {s: (got[s], expect[s]) for s in expect if got[s] != expect[s]}
+
+
 def test_linear_that_quantizes_in_its_stream_refuses_an_output_over_its_activations():
     """Without room for quantized activations every workgroup reads x while others store C: an overlap of the two is
     refused before any launch (no memory is touched; the addresses are made up)."""
