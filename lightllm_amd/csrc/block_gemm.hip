@@ -1166,18 +1166,42 @@ extern "C" int mi355_reset_workspace(void *ws, size_t ws_bytes, void *stream) {
     return launch(zero_words_kernel, dim3(words / 256), dim3(256), 0, (hipStream_t)stream, (uint32_t *)ws, words);
 }
 
+// Whether the entries of a 16- or 32-row schedule run as weight streams or as ring tiles (16 or 32 x 128, DMA into LDS).
+// The stream has no barrier in its K loop, but its 64-column tiles, two to a compute unit, need enough of them to even out.
+// Over 8 to 256 experts, N = 512 to 7168, K = 2048 to 8192, even and uneven routing, weights from HBM, time of the stream
+// over that of the ring tiles:
+//  * fewer than 16 K steps give a wave too few (128 experts, N = 2048, K = 768, top-8, 4 / 8 tokens: 14.7 / 22.2 us against
+//    11.5 / 19.3, level from 16 tokens on; K = 1408, 4 tokens: 16.4 against 14.9)
+//  * up to 8 rows per expert it is ahead (0.73 - 0.97) except with 1 to 1.6 tiles per unit under a K below 7168 (1.02 - 1.09);
+//    the ring tiles take rows that lie a multiple of 4096 bytes apart badly (0.75 - 0.9 wherever there are tiles enough)
+//  * with 9 to 16 rows second entries come into it: one more round if the tiles fill one (1.04 - 1.24), half a round up to
+//    3.1 tiles per unit under a short K (1.02 - 1.11); else 0.8 - 1.0
+//  * from 17 rows on a stream step costs two row blocks: still ahead under a K of 2048 or 7168 (0.86 - 0.98), not between
+//    (0.97 - 1.05), with a narrow N (N = 512, 1024: 1.04 - 1.09) or from 21 rows on (uneven routing: 1.04 - 1.1)
+// With 8 experts or fewer the alternative to it is blocks of 64 rows, far behind where it is taken (mi355_grouped_block_m).
+static bool grouped_streams(int64_t rows_per_expert, int64_t num_experts, int64_t N, int64_t K, int cus) {
+    if (K < 16 * kBlockK) return false;
+    if (num_experts <= 8) return true;
+    const int64_t tiles = num_experts * ((N + 63) / 64);
+    const bool ring_is_slow = K % 4096 == 0;
+    if (rows_per_expert <= 8) return K >= 7168 || ring_is_slow || tiles <= cus || tiles * 5 > 8 * (int64_t)cus;
+    if (rows_per_expert > 16 && !ring_is_slow && (rows_per_expert > 20 || N < 1536 || (K > 2176 && K < 7168))) return false;
+    if (ring_is_slow || (K >= 4096 && rows_per_expert <= 16)) return tiles * 5 > 8 * (int64_t)cus;
+    return tiles * 10 > 31 * (int64_t)cus;
+}
+
 extern "C" int32_t mi355_grouped_block_m(int64_t num_pairs, int32_t num_experts, int64_t N, int64_t K) {
     if (num_experts <= 0) return 64;
     const int64_t avg = num_pairs / num_experts;
     // 256-row schedule blocks run as the persistent launch with two queues: blocks of more than 64 rows on the
     // 256x256 ping-pong tile (it skips the empty 64-row halves of ragged blocks), the others on the 64x512
     // weight-streaming tile.  That launch needs more tiles than compute units, and its time hardly depends on how the rows
-    // are spread.  With fewer rows the weight streams of 16- and 32-row schedules (gemm_gstream.hpp, K of 16 steps
-    // or more) are ahead: they read at 6 to 7 TB/s, once per 32 rows of an expert, so what they cost follows the second reads
+    // are spread.  With fewer rows the weight streams of 16- and 32-row schedules (gemm_gstream.hpp, where they are
+    // taken) are ahead: they read at 6 to 7 TB/s, once per 32 rows of an expert, so what they cost follows the second reads
     // of popular experts.  Every line between the two lies where Zipf(1.1) popularity costs the stream its lead.
     const int cus = device_cus();
     const int64_t tiles256 = (int64_t)num_experts * ((N + 255) / 256);
-    const bool two_queues = tiles256 > cus, stream = K >= 16 * kBlockK;
+    const bool two_queues = tiles256 > cus, stream = grouped_streams(avg, num_experts, N, K, cus);
     // Measured over Qwen3-MoE (128 experts), DeepSeek-V2-Lite (64), Mixtral (8), a DeepSeek-V3 expert-parallel slice
     // (32 experts, N = 512) and a 16-expert shape, 8 to 8192 tokens, uniform routing:
     //  * 128-row blocks are ahead of the 256-row launch up to a few hundred rows per expert where the whole launch
@@ -1298,12 +1322,11 @@ static int grouped_block_fp8_gemm_impl(const void *Xq, const float *Xs, const vo
     switch (block_m) {
         case 16:
         case 32: {
-            // weight streams; the ring tiles keep the short K (fewer than 16 steps), where the streams' waves get too few
-            // steps each (128 experts, N = 2048, K = 768, top-8, 4 / 8 tokens: 14.7 / 22.2 us against 11.5 / 19.3 for the
-            // ring, level from 16 tokens on; K = 1408, 4 tokens: 16.4 against 14.9), and a K whose scales do not fit the LDS
-            if (KB >= 16) {
+            // (a padded layout's rows per expert are not known here: as many as its block holds)
+            const int64_t rows = num_pairs >= num_tokens ? num_pairs / num_experts : block_m == 16 ? 16 : 20;
+            if (grouped_streams(rows, num_experts, N, K, device_cus())) {
                 const int r = launch_gstream(a, block_m, num_experts, st);
-                if (r != MI355_EUNSUPPORTED) return r;
+                if (r != MI355_EUNSUPPORTED) return r;  // (a K whose scales do not fit the LDS)
             }
             if (block_m == 16) return launch_grouped_tile<16, 128, 1, 4, 4>(a, finish(128), st);
             return launch_grouped_tile<32, 128, 1, 4, 4>(a, finish(128), st);

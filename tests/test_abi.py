@@ -112,6 +112,21 @@ def test_grouped_block_m_holds_under_uneven_routing():
     assert got == expect, {s: (got[s], expect[s]) for s in expect if got[s] != expect[s]}
 
 
+def test_grouped_block_m_of_launches_too_small_for_the_weight_streams():
+    """Where the 64-column tiles of the streams are too few, or a step costs two row blocks and nothing pays for it, the
+    rows go to ring tiles, in blocks of the average size and with the lines those have."""
+    from lightllm_amd import _lib
+
+    lib = _lib.lib()
+    expect = {
+        (16, 1024, 3072): {8: 16, 12: 16, 16: 16, 20: 32}, (32, 1536, 2048): {9: 16, 16: 16, 17: 32},
+        (64, 4096, 5120): {16: 16, 17: 256}, (64, 2048, 2048): {9: 32, 16: 32, 20: 32},
+        (16, 1536, 4096): {16: 16, 24: 32},
+    }
+    got = {s: {a: lib.mi355_grouped_block_m(a * s[0], *s) for a in e} for s, e in expect.items()}
+    assert got == expect, {s: (got[s], expect[s]) for s in expect if got[s] != expect[s]}
+
+
 def test_linear_that_quantizes_in_its_stream_refuses_an_output_over_its_activations():
     """Without room for quantized activations every workgroup reads x while others store C: an overlap of the two is
     refused before any launch (no memory is touched; the addresses are made up)."""

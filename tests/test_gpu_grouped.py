@@ -480,3 +480,47 @@ def test_grouped_weight_stream(hip, block_m, N, K, mul_w, bias_dtype):
     cos, rel = H.gemm_metrics(got.cpu(), ref.cpu())
     assert cos >= H.GEMM_MIN_COS and rel <= H.GEMM_MAX_REL, (cos, rel)
     assert (got - ref).abs().max() <= ref.abs().max() * 2 ** -7
+
+
+def _check_stream(hip, counts, N, K, block_m, mul_w, bias_dtype):
+    """`counts` rows per expert, in a random order over the tokens, through grouped_matmul in blocks of `block_m` rows."""
+    from lightllm_amd.fused_moe import grouped_matmul
+    from lightllm_amd.quantization import per_token_group_quant_fp8
+
+    E, T = len(counts), sum(counts)
+    g = H.gen(N + K + T)
+    ids = torch.repeat_interleave(torch.arange(E, dtype=torch.int32), torch.tensor(counts))[torch.randperm(T, generator=g)]
+    ids, tw = ids.view(T, 1).contiguous(), torch.rand((T, 1), generator=g)
+    idx, w, cnt = _align(ids, tw, E)
+    x = H.activations(T, K, seed=N).cuda()
+    wq = torch.zeros((E, N, K), dtype=torch.float8_e4m3fn, device="cuda")
+    ws = torch.ones((E, -(-N // 128), K // 128), dtype=torch.float32, device="cuda")
+    for e in (e for e in range(E) if counts[e]):
+        wq[e], ws[e] = H.quantized_weights(N, K, seed=100 + e, device="cuda")
+    bias = None if bias_dtype is None else (torch.randn((E, N), generator=g) * 0.5).to(bias_dtype).cuda()
+    out = torch.full((T, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    grouped_matmul(T, x, None, cnt, idx, w, wq, ws, 1, out, mul_routed_weight=mul_w, use_fp8_w8a8=True,
+                   run_config={"BLOCK_SIZE_M": block_m}, bias=bias)
+    torch.cuda.synchronize()
+    xq, xs = per_token_group_quant_fp8(x, 128)
+    flat, routed = ids.view(-1).cuda(), tw.view(-1).cuda()
+    for e in (e for e in range(E) if counts[e]):
+        rows = (flat == e).nonzero().view(-1)
+        r = tr.dequant_matmul(xq[rows], xs[rows], wq[e], ws[e], out_dtype=torch.float32)
+        if bias is not None:
+            r = r + bias[e].float()
+        r = r * (routed[rows, None] if mul_w else 1.0)
+        got = out[rows].float()
+        assert not torch.isnan(got).any(), f"expert {e}: a routed row was not written"
+        cos, rel = H.gemm_metrics(got.cpu(), r.cpu())
+        assert cos >= H.GEMM_MIN_COS and rel <= H.GEMM_MAX_REL, (e, cos, rel)
+
+
+@pytest.mark.parametrize("block_m", [16, 32])
+@pytest.mark.parametrize("N,K,mul_w,bias_dtype", [(192, 2048, False, None), (200, 2176, True, None),
+                                                  (1004, 2304, True, torch.bfloat16), (64, 4096, False, torch.float32)])
+def test_grouped_weight_stream_among_idle_experts(hip, block_m, N, K, mul_w, bias_dtype):
+    """What test_grouped_weight_stream looks at, with so many idle experts that the rows per expert are few on average
+    (up to 8: weight streams; more, with this few tiles: ring tiles)."""
+    print(f"grouped weight stream, idle experts, block_m={block_m} N={N} K={K} mul_w={mul_w} bias={bias_dtype}", flush=True)
+    _check_stream(hip, [0, 1, 15, 16, 17, 31, 32, 33, 49, 64] + [0] * 20, N, K, block_m, mul_w, bias_dtype)
