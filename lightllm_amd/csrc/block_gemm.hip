@@ -87,6 +87,7 @@ static int launch_gstream_as(GemmArgs &a, int block_m, int num_experts, hipStrea
     const int lds_bytes = GStreamCfg<2>::lds_bytes(KB);
     if (lds_bytes > kMaxLds) return MI355_EUNSUPPORTED;
     a.tiles_n = (a.N + GStreamCfg<1>::BN - 1) / GStreamCfg<1>::BN;
+    if ((int64_t)a.tiles_m * a.tiles_n >= (1ll << 31)) return MI355_EUNSUPPORTED;
     a.total_tiles = a.tiles_m * a.tiles_n;
     // an exact schedule has at most E more entries than it would with every block full
     const int64_t grid = std::max<int64_t>(4096, 2 * (int64_t)num_experts * a.tiles_n);
@@ -1318,7 +1319,7 @@ static int grouped_block_fp8_gemm_impl(const void *Xq, const float *Xs, const vo
         a.blocks_per_xcd = (a.total_tiles + 7) / 8;
         return a.blocks_per_xcd * 8;
     };
-    if ((int64_t)table_rows * ((N + 63) / 64) >= (1ll << 31)) return MI355_EUNSUPPORTED;
+    if ((int64_t)table_rows * ((N + 127) / 128) >= (1ll << 31)) return MI355_EUNSUPPORTED;
     switch (block_m) {
         case 16:
         case 32: {
@@ -1326,7 +1327,7 @@ static int grouped_block_fp8_gemm_impl(const void *Xq, const float *Xs, const vo
             const int64_t rows = num_pairs >= num_tokens ? num_pairs / num_experts : block_m == 16 ? 16 : 20;
             if (grouped_streams(rows, num_experts, N, K, device_cus())) {
                 const int r = launch_gstream(a, block_m, num_experts, st);
-                if (r != MI355_EUNSUPPORTED) return r;  // (a K whose scales do not fit the LDS)
+                if (r != MI355_EUNSUPPORTED) return r;  // (a K whose scales do not fit the LDS, or 2^31 tiles and more)
             }
             if (block_m == 16) return launch_grouped_tile<16, 128, 1, 4, 4>(a, finish(128), st);
             return launch_grouped_tile<32, 128, 1, 4, 4>(a, finish(128), st);

@@ -127,6 +127,24 @@ def test_grouped_block_m_of_launches_too_small_for_the_weight_streams():
     assert got == expect, {s: (got[s], expect[s]) for s in expect if got[s] != expect[s]}
 
 
+def test_grouped_gemm_takes_schedules_of_up_to_2_31_tiles():
+    """The limit is the launch's own tile count, in 128-column tiles for every block size: a schedule whose 64-column
+    tiles would pass 2^31 is refused by the weight streams alone, and runs as ring tiles (the addresses are made up)."""
+    from lightllm_amd import _lib
+
+    lib = _lib.lib()
+    a = 1 << 40
+
+    def call(block_m, rows, n, k):
+        return lib.mi355_grouped_block_fp8_gemm(a, a, a, a, a, a, a, a, rows, block_m, 1024, 1024, 8, 1, n, k, 0, a, None, 0, None)
+
+    for block_m in (16, 32, 64, 128, 256):
+        for k in (1024, 2048):
+            assert call(block_m, 1 << 20, 1 << 18, k) == -6, (block_m, k)   # 2^31 tiles of 128 columns
+            if not torch.cuda.is_available():   # past the check: the launch itself is what fails here
+                assert call(block_m, 700000, 1 << 18, k) == -5, (block_m, k)
+
+
 def test_linear_that_quantizes_in_its_stream_refuses_an_output_over_its_activations():
     """Without room for quantized activations every workgroup reads x while others store C: an overlap of the two is
     refused before any launch (no memory is touched; the addresses are made up)."""
