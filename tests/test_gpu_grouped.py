@@ -443,7 +443,8 @@ def test_grouped_fp16_output(hip, block_m):
 def test_grouped_weight_stream(hip, block_m, N, K, mul_w, bias_dtype):
     """The weight stream of 16- and 32-row schedules: experts with 0, 1, 15 .. 17, 31 .. 33, 49 and 64 rows (one or two
     row blocks, second entries of an expert), a last n tile that is full, ragged or no multiple of 8, K steps the four
-    waves do not share evenly."""
+    waves do not share evenly.  (Ten experts of 25 rows on average have too few tiles for the streams by now: here the same
+    schedules run as ring tiles, and as streams in the tests below.)"""
     from lightllm_amd.fused_moe import grouped_matmul
     from lightllm_amd.quantization import per_token_group_quant_fp8
 
@@ -524,3 +525,15 @@ def test_grouped_weight_stream_among_idle_experts(hip, block_m, N, K, mul_w, bia
     (up to 8: weight streams; more, with this few tiles: ring tiles)."""
     print(f"grouped weight stream, idle experts, block_m={block_m} N={N} K={K} mul_w={mul_w} bias={bias_dtype}", flush=True)
     _check_stream(hip, [0, 1, 15, 16, 17, 31, 32, 33, 49, 64] + [0] * 20, N, K, block_m, mul_w, bias_dtype)
+
+
+@pytest.mark.parametrize("block_m", [16, 32])
+@pytest.mark.parametrize("K,bias_dtype", [(2048, torch.bfloat16), (2176, None)])
+def test_grouped_weight_stream_with_more_tiles_than_workgroups(hip, block_m, K, bias_dtype):
+    """More than 4096 tiles of 64 columns (16-row schedule 277 entries x 34, 32-row 143 x 34): every workgroup of the
+    launch runs several, of one row block and of two, and meets the skipped and the padding entries on its way."""
+    print(f"grouped weight stream, several tiles a workgroup, block_m={block_m} K={K} bias={bias_dtype}", flush=True)
+    counts = [1, 16, 2400, 17, 0, 1800, 48, 7]
+    T, E, N = sum(counts), len(counts), 2120
+    assert hip.mi355_moe_align2_rows(T, E, block_m) * 34 > 4096
+    _check_stream(hip, counts, N, K, block_m, True, bias_dtype)

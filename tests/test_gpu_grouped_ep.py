@@ -53,6 +53,34 @@ def test_masked_layout(hip, E, T, N, K, masked):
             _close(got[e, :n], _expert_ref(xq[e * T: e * T + n], xs[e * T: e * T + n], wq[e], ws[e]))
 
 
+@pytest.mark.parametrize("K", [2048, 2176])
+@pytest.mark.parametrize("expected_m,block_m", [(8, 16), (16, 32)])
+def test_masked_layout_as_weight_streams(hip, expected_m, block_m, K):
+    """The padded schedule of the weight streams (8 x 4096 rows x 18 column tiles, many more than the workgroups of the
+    launch): a workgroup runs several tiles, the operands of one row block over the sums of two and the other way round,
+    passes the skipped second 16-row entries and stops at the padding.  N is no multiple of 64."""
+    from lightllm_amd.fused_moe import _deepgemm_grouped_fp8_nt_masked
+
+    masked = [1, 16, 4096, 17, 0, 4000, 48, 7]
+    E, T, N = len(masked), 4096, 1096
+    print(f"masked weight stream E={E} T={T} N={N} K={K} block_m={block_m}", flush=True)
+    assert hip.mi355_grouped_block_m(expected_m * E, E, N, K) == block_m
+    assert hip.mi355_moe_align2_rows(E * T, E, block_m) * 18 > 4096
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x = torch.randint(0, 256, (E, T, K), dtype=torch.uint8, device="cuda", generator=g)
+    x = torch.where((x & 0x7f) == 0x7f, 0, x).to(torch.uint8).view(torch.float8_e4m3fn)   # no NaN bytes
+    xs = torch.rand((E, T, K // 128), device="cuda", generator=g) * 1e-3 + 1e-4
+    pairs = [H.quantized_weights(N, K, seed=K + e, device="cuda") for e in range(E)]
+    wq, ws = (torch.stack(list(t)).contiguous() for t in zip(*pairs))
+    out = torch.full((E, T, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    _deepgemm_grouped_fp8_nt_masked((x, xs), (wq, ws), out, torch.tensor(masked, dtype=torch.int32, device="cuda"), expected_m)
+    torch.cuda.synchronize()
+    for e, n in enumerate(masked):
+        assert torch.isnan(out[e, n:]).all(), "rows past masked_m must stay untouched"
+        if n:
+            _close(out[e, :n].float(), tr.dequant_matmul(x[e, :n], xs[e, :n], wq[e], ws[e], out_dtype=torch.float32))
+
+
 def test_contiguous_layout(hip):
     from lightllm_amd.fused_moe import deepgemm_grouped_fp8_nt_contiguous
 
