@@ -149,3 +149,32 @@ def test_fused_experts_in_one_call_equals_the_steps(hip, T, E, topk, Hd, I, offs
     torch.cuda.synchronize()
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
     assert torch.equal(inp.view(torch.int16), want.view(torch.int16))
+
+
+# full chunks and a shorter last one (of another block size: 20 and 3 pairs per expert; 31 and 8), an odd topk, ids of a
+# chunk that are not 16-byte aligned, biases
+@pytest.mark.parametrize("T,E,topk,Hd,I,chunk", [(101, 7, 3, 256, 384, 47), (107, 12, 8, 1024, 1024, 47), (96, 5, 1, 128, 128, 48)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_fused_experts_in_chunks(hip, monkeypatch, T, E, topk, Hd, I, chunk, bias):
+    """More tokens than one pass takes: the one-call form, pass by pass over one scratch, gives the bits of the steps."""
+    from lightllm_amd.fused_moe import fused_experts_impl, grouped_fused_moe
+
+    print(f"fused_experts in chunks T={T} E={E} topk={topk} H={Hd} I={I} chunk={chunk} bias={bias}", flush=True)
+    monkeypatch.setattr(grouped_fused_moe, "FFN_MOE_CHUNK_SIZE", chunk)
+    x = H.activations(T, Hd, seed=T).cuda()
+    w1q, w1s, w2q, w2s = (t.cuda() for t in _experts(E, I, Hd, seed=E))
+    ids, tw = (t.cuda() for t in H.routing(T, E, topk, seed=T + E))
+    kw = dict(use_fp8_w8a8=True, w1_scale=w1s, w2_scale=w2s)
+    if bias:
+        kw["w1_bias"] = torch.randn((E, 2 * I), generator=H.gen(1)).to(torch.bfloat16).cuda()
+        kw["w2_bias"] = torch.randn((E, Hd), generator=H.gen(2)).cuda()
+    want = fused_experts_impl(x, w1q, w2q, tw, ids, run_config={}, **kw)
+    got = fused_experts_impl(x, w1q, w2q, tw, ids, **kw)
+    inp = x.clone()
+    fused_experts_impl(inp, w1q, w2q, tw, ids, inplace=True, **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    assert torch.equal(inp.view(torch.int16), want.view(torch.int16))
+    monkeypatch.undo()   # and those of a single pass
+    whole = fused_experts_impl(x, w1q, w2q, tw, ids, **kw)
+    assert tr.cosine(got.float().cpu(), whole.float().cpu()) >= 0.9999

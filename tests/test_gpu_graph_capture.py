@@ -185,6 +185,61 @@ def test_capture_after_a_warm_up_on_another_stream_allocates_nothing(hip):
         assert torch.equal(eager.view(torch.int16), expect.view(torch.int16))
 
 
+def _replays_follow_the_inputs(call, inputs, fresh, replays=4):
+    """`call()` is run once, captured on torch's own capture stream, and replayed over inputs that `fresh(r)` draws anew
+    each time, against the eager result; eager work and synchronisations sit between the replays."""
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    for r in range(replays):
+        for dst, src in zip(inputs, fresh(r)):
+            dst.copy_(src)
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        got = out.clone()
+        expect = call()
+        torch.cuda.synchronize()
+        assert not torch.isnan(got).any()
+        assert torch.equal(got.view(torch.int16), expect.view(torch.int16)), f"replay {r}"
+
+
+# a per-unit stream, 16-row tiles that share K through the workspace, and more rows than the streams quantize
+@pytest.mark.parametrize("M,N,K,fused,shares_k", [(4, 4096, 4096, 1, False), (4, 2112, 7168, 1, True), (32, 4096, 14336, 0, True)])
+def test_linear_under_graph_capture(hip, M, N, K, fused, shares_k):
+    from lightllm_amd import _lib
+    from lightllm_amd.quantization import QUANTMETHODS, WeightPack
+
+    print(f"graph capture linear M={M} N={N} K={K}", flush=True)
+    code = _lib.DTYPE_CODES[torch.bfloat16]
+    assert hip.mi355_block_fp8_linear_fused(M, N, K, code) == fused
+    assert (hip.mi355_block_fp8_linear_workspace_bytes(M, N, K, code) > 0) == shares_k
+    method, pack = QUANTMETHODS.get("fp8w8a8-b128"), WeightPack(*H.quantized_weights(N, K, seed=51, device="cuda"))
+    x = H.activations(M, K, seed=52).cuda()
+    _replays_follow_the_inputs(lambda: method.apply(x, pack), [x], lambda r: [H.activations(M, K, seed=60 + r)])
+
+
+# the prologue launch and weight streams; more pairs than the prologue takes and 256-row blocks on the workspace
+@pytest.mark.parametrize("T,E,topk,Hd,I", [(24, 16, 4, 2048, 2048), (1400, 24, 4, 1024, 2048)])
+def test_fused_experts_under_graph_capture(hip, T, E, topk, Hd, I):
+    from lightllm_amd.fused_moe import fused_experts
+
+    print(f"graph capture fused_experts T={T} E={E} topk={topk} H={Hd} I={I}", flush=True)
+    assert (hip.mi355_routed_ffn_workspace_bytes(T, topk, E, Hd, I) > 0) == (T == 1400)
+    w1, w2 = ([H.quantized_weights(n, k, seed=70 + e, device="cuda") for e in range(E)] for n, k in ((2 * I, Hd), (Hd, I)))
+    (w1q, w1s), (w2q, w2s) = ((torch.stack(list(t)).contiguous() for t in zip(*w)) for w in (w1, w2))
+    x = H.activations(T, Hd, seed=71).cuda()
+    ids, tw = (t.cuda() for t in H.routing(T, E, topk, seed=72))
+
+    def call():
+        return fused_experts(x, w1q, w2q, tw, ids, use_fp8_w8a8=True, w1_scale=w1s, w2_scale=w2s)
+
+    _replays_follow_the_inputs(call, [x, ids, tw], lambda r: [H.activations(T, Hd, seed=80 + r), *H.routing(T, E, topk, seed=90 + r)])
+
+
 def test_reset_workspace_recovers_dirty_counters(hip):
     """Counter words left non-zero (as an aborted launch would) make a split-K launch wrong; the reset entry point
     restores the invariant."""
