@@ -217,7 +217,8 @@ int mi355_moe_align_fused(const int32_t *topk_ids, const float *topk_weights, in
  *            topk_ids[j] == e else 0; every element is written (the reference zero-fills first, :86).
  * moe_align1 (grouped_fused_moe.py:101-214): compacts each row of that 0/1 table IN PLACE into the ascending pair
  *            indices of its ones and writes the matching weights and the per-expert counts; entries past an
- *            expert's count keep what they held. */
+ *            expert's count keep what they held.
+ * moe_align1 and moe_align_fused read all num_pairs entries of topk_weights, those of pairs that no expert takes too. */
 int mi355_moe_align(const int32_t *topk_ids, int64_t num_pairs, int32_t num_experts, int32_t *out,
                     int64_t out_stride_m, void *stream);
 int mi355_moe_align1(int32_t *experts_info, int64_t info_stride_m, const float *topk_weights, int64_t num_pairs,
@@ -229,7 +230,8 @@ int64_t mi355_moe_align2_rows(int64_t num_pairs, int32_t num_experts, int32_t bl
 
 /* table int32 [rows,4] = (expert, m_index, token_start, tokens in the block); padding rows get expert = -1
  * (:439-446; the fourth column is derived, min(block_m, count - m_index*block_m), so that a GEMM tile needs one
- * 16-byte load to know its work). */
+ * 16-byte load to know its work).  The GEMMs below take the table as it is written here: an expert's blocks in order
+ * and without gaps, the padding rows behind all others. */
 int mi355_moe_align2(const int32_t *expert_token_num, int32_t num_experts, int32_t block_m, int64_t rows,
                      int32_t *table, void *stream);
 
@@ -243,12 +245,14 @@ int mi355_moe_align2(const int32_t *expert_token_num, int32_t num_experts, int32
  *     out[idx, :] = bf16( blockscaled(Xq[row,:] . W[e]^T) * (mul_routed_weight ? expert_to_weight[e*num_pairs+j] : 1) )
  * Xq e4m3fn [T,K] contiguous, Xs fp32 [T,K/128] contiguous (the activation quantizer's output);
  * W e4m3fn [E,N,K] contiguous; Ws fp32 [E, ceil(N/128), K/128] contiguous; out bf16 [num_pairs, N] contiguous.
- * num_pairs is only used as the row stride of expert_to_token_index / expert_to_weight (the number of (token, slot)
- * pairs in LightLLM's use); the masked expert-parallel layout passes a [E, T_pad] table with num_pairs = T_pad.
+ * num_pairs is the row stride of expert_to_token_index / expert_to_weight (the number of (token, slot) pairs in
+ * LightLLM's use) and, where it is no smaller than num_tokens, tells how many rows an expert has on average, by which a
+ * launch of 16- or 32-row blocks picks its kernel; the masked expert-parallel layout passes a [E, T_pad] table with
+ * num_pairs = T_pad and num_tokens = E*T_pad.
  * block_m must be one the library was built for: 16, 32, 64, 128 or 256; mi355_grouped_block_m() suggests one
- * from the rows per expert, the number of experts and an expert's N and K (256 also for batches of 12 to 64 rows
- * per expert when the launch has more tiles than compute units: that suggestion counts on the workspace of
- * mi355_grouped_workspace_bytes(), see below; 128 for small launches; 64 for models of 8 experts).
+ * from the rows per expert, the number of experts and an expert's N and K (256 also for batches of 12 to 25 rows per
+ * expert and more - where the line lies depends on the shape - when the launch has more tiles than compute units: that
+ * suggestion counts on the workspace of mi355_grouped_workspace_bytes(), see below; 128 for small launches; 64 for models of 8 experts).
  * workspace: optional, used by block_m = 256 only: MI355_WS_COUNTER_BYTES bytes that are zero before the launch
  * (the kernel leaves them zero).  With it the launch is persistent - one workgroup per compute unit takes tiles
  * from per-XCD counters and overlaps the first requests of a tile with the stores of the previous one;

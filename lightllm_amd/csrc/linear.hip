@@ -15,7 +15,8 @@ namespace mi355 {
 // against 6.5 / 6.6 / 7.9; 6144 x 4096: 9.4 / 9.7 / 9.9 against 7.6 / 7.9 / 9.3; 28672 x 4096: 25.6 / 24.9 / 25.1
 // against 22.4 / 22.4 / 23.6; 4096 x 14336: 15.3 / 14.9 / 15.4 against 12.9 / 13.2 / 16.2 (59 MB of activations for 8
 // rows); 36864 x 7168: 46.2 / 44.1 / 45.7 against 44.2 / 43.0 / 50.5 (264 MB).  With 16 rows it loses everywhere (N = K =
-// 4096: 9.5 against 10.5).
+// 4096: 9.5 against 10.5).  kFusedBytes is a total over a whole device of 256 units (every workgroup's requests, to the
+// caches all of them share); 5 to 7 rows count as 8 because the loads of 8 are issued, the missing rows repeating the last.
 constexpr int64_t kFusedRows = 8;
 constexpr int64_t kFusedBytes = 40000000;
 

@@ -9,17 +9,18 @@
 //     this equals RN(amax/448) for every bf16 and every fp16 amax and for the default eps (checked exhaustively on
 //     the CPU); calls with any other eps do not come here (they take quant_chunk_f32).
 //   * x/s is formed as y = fma(x, r, x*d) from r, a little under 1/s (v_rcp_f32, two ulps taken off), and the rest
-//     d = fma(-s, r, 1) * r >= 0 that r + d misses 1/s by no more than 2^-46 of: two operations per element.  For every
+//     d = fma(-s, r, 1) * r >= 0: two operations per element.  r + d falls short of 1/s by e^2 of it, e = 1 - s*r being up
+//     to three ulps: about 2^-42 at most, more where d is subnormal (the largest amax).  That is no proof by itself: for every
 //     pair (amax, |x| <= amax) of bf16 or of fp16 values the e4m3 byte of y is that of RN(x/s), whatever the last bit of
-//     the reciprocal is - also checked exhaustively on the CPU (oracle_fast_quant_mismatches in the test oracle replays exactly these
+//     the reciprocal is, checked exhaustively on the CPU (oracle_fast_quant_mismatches in the test oracle replays exactly these
 //     operations for a reciprocal off by -1, 0 and +1 ulp).  With r and d positive -0 stays -0, as -0/s is.
+// No contraction of a product and a sum anywhere in this arithmetic: the pragma stands inside each function so that it does
+// not reach the rest of a file that includes this one.
 #pragma once
 #include "common.hpp"
 
 namespace mi355 {
 
-// (no contraction of a product and a sum anywhere in this arithmetic; the pragma stands inside each function so that
-// it does not reach the rest of a file that includes this one)
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 
 template <int CTRL>
