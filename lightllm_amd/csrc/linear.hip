@@ -1,8 +1,8 @@
 // The block-FP8 linear as one entry point: 16-bit activations in, 16-bit outputs out (quantizer + GEMM).
 //
-// What a decode step spends on a small linear is not the stream over its weights but what surrounds it: on this part a
-// kernel of a few hundred workgroups costs 4 to 5 us in a stream or a captured graph however little it does, so the
-// quantizer in front of a 7 to 20 us weight stream was a fifth to a third of the linear (N = K = 4096, one row).  Up to
+// What a decode step spends on a small linear is not the stream over its weights but what surrounds it: in a captured graph
+// a launch costs 1.7 to 2.7 us however little it does, and the quantizer in front of a 6 to 20 us weight stream was up to a
+// fifth of the linear (N = K = 4096, one row: 8.2 us, 6.5 without it).  Up to
 // kFusedRows rows the weight streams therefore quantize the activations themselves (XQuant in gemm_stream.hpp): every
 // workgroup repeats that work, but it is small - 16 lanes per row and K step - and sits in the shadow of the stream.
 #include "stream_plan.hpp"
