@@ -261,52 +261,74 @@ static int launch_dense(GemmArgs &a, hipStream_t st) {
 }
 
 // Weight-streaming launches for M <= 64 (stream_plan.hpp has the plan).
-template <int MT, int TNW, bool XSL>
+template <int MT, int TNW, bool XSL, bool TURN, int WV>
 static int launch_stream_as(GemmArgs &a, const SkinnyPlan &pl, void *ws, int lds_bytes, hipStream_t st) {
-    using Cfg = StreamCfg<MT, TNW>;
+    using Cfg = StreamCfg<MT, TNW, WV>;
     constexpr int max_lds = Cfg::kLds + (XSL ? Cfg::scale_lds_bytes(Cfg::kMaxScaleSteps) : 0);
-    constexpr auto whole_k = block_fp8_gemm_stream_kernel<MT, TNW, false, XSL>;
-    constexpr auto split_k = block_fp8_gemm_stream_kernel<MT, TNW, true, XSL>;
+    constexpr auto whole_k = block_fp8_gemm_stream_kernel<MT, TNW, false, XSL, 0, false, WV, TURN>;
+    constexpr auto split_k = block_fp8_gemm_stream_kernel<MT, TNW, true, XSL, 0, false, WV, TURN>;
     if (pl.splits <= 1) {
         if (!allow_lds<whole_k>(max_lds)) return MI355_ELAUNCH;
-        return launch(whole_k, dim3(pl.tiles), dim3(256), lds_bytes, st, a);
+        return launch(whole_k, dim3(pl.tiles), dim3(64 * WV), lds_bytes, st, a);
     }
     if (!allow_lds<split_k>(max_lds)) return MI355_ELAUNCH;
     a.splits = pl.splits;
     a.counters = (uint32_t *)ws;
     a.partials = (float *)((uint8_t *)ws + MI355_WS_COUNTER_BYTES);
-    return launch(split_k, dim3(pl.tiles * pl.splits), dim3(256), lds_bytes, st, a);
+    return launch(split_k, dim3(pl.tiles * pl.splits), dim3(64 * WV), lds_bytes, st, a);
 }
 
-// The activation scales of a CTA's K range are staged in LDS when the range is short enough for the staging area.
-template <int MT, int TNW>
+// The activation scales of a CTA's K range are staged in LDS when the range is short enough for the staging area; from 17
+// rows on the plan only has such ranges.
+template <int MT, int TNW, int WV = kStreamWaves>
 static int launch_stream(GemmArgs &a, const SkinnyPlan &pl, void *ws, hipStream_t st) {
-    using Cfg = StreamCfg<MT, TNW>;
+    using Cfg = StreamCfg<MT, TNW, WV>;
     const int KB = a.K / kBlockK;
     const int steps = (KB + pl.splits - 1) / pl.splits;
-    if (steps <= Cfg::kMaxScaleSteps)
-        return launch_stream_as<MT, TNW, true>(a, pl, ws, Cfg::kLds + Cfg::scale_lds_bytes(steps), st);
-    return launch_stream_as<MT, TNW, false>(a, pl, ws, Cfg::kLds, st);
+    a.turn_mask = stream_turn_mask(a.K, KB / pl.splits);
+    if (steps <= Cfg::kMaxScaleSteps) {
+        const int lds_bytes = Cfg::kLds + Cfg::scale_lds_bytes(steps);
+        return a.turn_mask ? launch_stream_as<MT, TNW, true, true, WV>(a, pl, ws, lds_bytes, st)
+                           : launch_stream_as<MT, TNW, true, false, WV>(a, pl, ws, lds_bytes, st);
+    }
+    if constexpr (MT == 1) return launch_stream_as<MT, TNW, false, false, WV>(a, pl, ws, Cfg::kLds, st);
+    return MI355_EUNSUPPORTED;
 }
 
 template <int MT>
 static int launch_stream_mt(GemmArgs &a, const SkinnyPlan &pl, void *ws, hipStream_t st) {
-    switch (pl.tnw) {
-        case 4: return launch_stream<MT, 4>(a, pl, ws, st);
-        case 2: return launch_stream<MT, 2>(a, pl, ws, st);
-        case 1:
-            if constexpr (MT == 1) return launch_stream<1, 1>(a, pl, ws, st);
-            return MI355_EINVAL;
-        default: return MI355_EINVAL;
+    if constexpr (MT == 1) {
+        switch (pl.tnw) {
+            case 4: return launch_stream<1, 4>(a, pl, ws, st);
+            case 1: return launch_stream<1, 1>(a, pl, ws, st);
+            default: return MI355_EINVAL;
+        }
+    } else {
+        if (pl.waves == 8) {
+            switch (pl.tnw) {
+                case 4:
+                    if constexpr (MT < 4) return launch_stream<MT, 4, 8>(a, pl, ws, st);
+                    return MI355_EINVAL;
+                case 2: return launch_stream<MT, 2, 8>(a, pl, ws, st);
+                case 1: return launch_stream<MT, 1, 8>(a, pl, ws, st);
+                default: return MI355_EINVAL;
+            }
+        }
+        switch (pl.tnw) {
+            case 4: return launch_stream<MT, 4>(a, pl, ws, st);
+            case 2: return launch_stream<MT, 2>(a, pl, ws, st);
+            case 1: return launch_stream<MT, 1>(a, pl, ws, st);
+            default: return MI355_EINVAL;
+        }
     }
 }
 
 // ---- the weight stream cut into one equal share per compute unit (gemm_streamcu.hpp)
-template <int TNW>
-static int launch_streamcu_as(GemmArgs &a, hipStream_t st) {
+template <int TNW, bool TURN>
+static int launch_streamcu_turn(GemmArgs &a, hipStream_t st) {
     using Cfg = CuStreamCfg<1, TNW>;
-    constexpr auto kernel_lo = block_fp8_gemm_streamcu_kernel<1, TNW, false>;
-    constexpr auto kernel_hi = block_fp8_gemm_streamcu_kernel<1, TNW, true>;
+    constexpr auto kernel_lo = block_fp8_gemm_streamcu_kernel<1, TNW, false, 0, false, TURN>;
+    constexpr auto kernel_hi = block_fp8_gemm_streamcu_kernel<1, TNW, true, 0, false, TURN>;
     const int lds_bytes = Cfg::lds_bytes(a.K / kBlockK);
     if (lds_bytes > kMaxLds) return MI355_EUNSUPPORTED;
     const int tiles = (a.N + Cfg::BN - 1) / Cfg::BN;
@@ -316,6 +338,12 @@ static int launch_streamcu_as(GemmArgs &a, hipStream_t st) {
     }
     if (!allow_lds<kernel_hi>(kMaxLds)) return MI355_ELAUNCH;
     return launch(kernel_hi, dim3(tiles), dim3(Cfg::kThreads), lds_bytes, st, a);
+}
+
+template <int TNW>
+static int launch_streamcu_as(GemmArgs &a, hipStream_t st) {
+    a.turn_mask = stream_turn_mask(a.K, a.K / kBlockK);
+    return a.turn_mask ? launch_streamcu_turn<TNW, true>(a, st) : launch_streamcu_turn<TNW, false>(a, st);
 }
 
 static int launch_streamcu(GemmArgs &a, int tnw, hipStream_t st) {
@@ -331,14 +359,15 @@ static int launch_streamcu(GemmArgs &a, int tnw, hipStream_t st) {
 
 // ---- the second streaming kernel (activation block shared by the workgroup).  Measured against the first one on
 // the Llama decode shapes it wins only where the first is shortest of registers and N alone fills the device:
-// M = 33..64 with 128-row workgroup tiles (N=28672, K=4096, M=64: 29.7 us against 34.4); with 64-row tiles, few
+// M = 49..64 with 128-row workgroup tiles (N=28672, K=4096, M=64: 29.7 us against 34.4); with 64-row tiles, few
 // tiles or smaller M its barrier per K step costs more than the shared activation block saves
-// (N=4096, K=14336: 21.5-25.2 us against 13.9-19.8).  Only that configuration is built.
+// (N=4096, K=14336: 21.5-25.2 us against 13.9-19.8; N = 28672, M = 48: 28.7 against 24.9 for three row blocks on the
+// first kernel).  Only that configuration is built.  Turned starts (K whole): N = 128256, K = 4096, M = 64 125 us, 102 turned.
 constexpr int kXshareDepth = 4;
 using XshareCfg = ShareCfg<4, 2, kXshareDepth>;
 
 static bool xshare_pays(int64_t M, int64_t N, int64_t K, int cus) {
-    return M > 32 && M <= 64 && (N + 127) / 128 >= (int64_t)cus * 3 / 4 && K / kBlockK <= XshareCfg::kMaxScaleSteps;
+    return M > 48 && M <= 64 && (N + 127) / 128 >= (int64_t)cus * 3 / 4 && K / kBlockK <= XshareCfg::kMaxScaleSteps;
 }
 
 // 128-row workgroup tiles; the K range is split in two while that leaves fewer than two workgroups per compute unit
@@ -360,6 +389,7 @@ static int launch_xshare(GemmArgs &a, int splits, void *ws, hipStream_t st) {
     constexpr int max_lds = XshareCfg::kLds + XshareCfg::scale_lds_bytes(XshareCfg::kMaxScaleSteps);
     const int lds_bytes = XshareCfg::kLds + XshareCfg::scale_lds_bytes(steps);
     const int tiles = (a.N + XshareCfg::BN - 1) / XshareCfg::BN;
+    a.turn_mask = splits > 1 ? 0 : stream_turn_mask(a.K, KB);
     if (splits <= 1) {
         constexpr auto kernel = block_fp8_gemm_xshare_kernel<4, 2, kXshareDepth, false>;
         if (!allow_lds<kernel>(max_lds)) return MI355_ELAUNCH;
@@ -390,11 +420,13 @@ constexpr int64_t kRows128NarrowMaxM = 208;  // the last row count with narrow w
 // for 144 tiles of 256; q_b, N = 24576, K = 1536: 16.6 against 21.4 with K shared by two).
 struct Rows128Plan {
     int wv, bn, splits, tiles, tn;
+    bool turned;  // tiles may start at different K steps (launch_rows128_as)
 };
 
 static Rows128Plan rows128_plan(int64_t M, int64_t N, int64_t K, int cus) {
     Rows128Plan pl;
     const int64_t KB = K / kBlockK;
+    pl.turned = false;
     pl.wv = 8;
     pl.bn = M <= 128 ? 256 : 128;
     pl.tn = M <= 128 ? 2 : 1;
@@ -448,27 +480,53 @@ static size_t rows128_workspace(int64_t M, int64_t N, int64_t K, int cus) {
 
 // Where the kernel pays (Llama-3-8B and DeepSeek-V3 linears, weights rotated so that none is found in the
 // memory-side cache).  At 65..128 rows it beats the 128x128 tiles by 10 to 30 % (DeepSeek-V3 down, M = 128: 39.5 us
-// against 50.0; Llama-3 down: 27.9 against 30.3) unless K is short (q_b, K = 1536: 21.7 against 17.0).  At 33..64
-// rows it beats the streaming kernels on the large weights (DeepSeek-V3 gate_up, down, o at M = 64: 58.4, 31.7,
-// 31.9 us against 72.3, 42.5, 43.1) and loses on the small ones, where its second launch shows (Llama-3 qkv: 15.0
-// against 13.1); at 32 rows and fewer the streaming kernels are the faster ones but for one case (below).
+// against 50.0; Llama-3 down: 27.9 against 30.3) unless K is short (q_b, K = 1536: 21.7 against 17.0).  At 49..64
+// rows it beats the streaming kernels on the large weights (DeepSeek-V3 gate_up at M = 64: 49.5 us against 71.2, down 31.5
+// against 41.2) and loses on the small ones, where its second launch shows (Llama-3 qkv: 14.7 against 11.6); at 48 rows
+// and fewer the streaming kernels are the faster ones but for a few kinds of large weights (below).
+// 49..64 rows: whether the streaming kernel is ahead of ROWS128.  Its workgroups have to fit one round, to fill four fifths of
+// it where their starts are not turned (M = 64: N = 15360, K = 5120, 240 of them 22.1 us against 23.5; 12288 x 5120, 192 of
+// them 21.4 against 21.0; turned, 12288 x 4096 16.7 against 18.0), and on large weights to take 64 weight rows, so that
+// the activations are not read too often (N = 7168, K = 18432, 32 rows a workgroup: 38.2 against 31.6).
+static bool skinny_ahead_of_rows128(int64_t M, int64_t N, int64_t K, int cus) {
+    const SkinnyPlan sp = skinny_plan(M, N, K, cus);
+    const int64_t wgs = (int64_t)sp.tiles * sp.splits;
+    return wgs <= cus && (K % 4096 == 0 || wgs * 5 >= 4 * (int64_t)cus) && (N * K < 60000000ll || sp.tnw == 4);
+}
+
 static bool rows128_pays(int64_t M, int64_t N, int64_t K, int cus) {
     if (M > 384 || M < 16) return false;
-    if (M <= 32) {
-        // 16..32 rows: only where the streaming kernel's 64-row workgroups (two fit a unit) spill into a second,
-        // mostly empty round and this kernel has a well-filled single launch (N = 36864, K = 7168: 576 workgroups on
-        // 512 slots, M = 24 / 32 51.1 / 52.5 us against 46.6 / 46.8 here; on N = 28672, 448 workgroups, the
-        // streaming kernel keeps its lead, 23.8 against 27.4)
+    if (M == 16) {
+        // large weights whose 64-row workgroups come to just over one per unit (N = 18432, K = 7168: 27.5 us against 30.3
+        // for the streaming kernel), a very long K (N = 8192, K = 28672: 45.3 against 50.7), or workgroups that spill into a
+        // mostly empty third round where this kernel has a well-filled single launch (N = 36864, K = 7168)
         const int64_t t64 = (N + 63) / 64;
         const Rows128Plan pl = rows128_plan(M, N, K, cus);
-        // likewise on large weights whose 64-row workgroups come to just over one per unit (N = 18432, K = 7168,
-        // 288 of them, M = 16 / 32: 27.5 / 28.4 us against 30.3 / 34.4), and under a very long K (N = 8192,
-        // K = 28672: 45.3 / 47.0 against 50.7 / 54.6; N = 7168, K = 18432: 27.2 / 28.5 against 30.9 / 31.4)
-        if (N * K >= 100000000ll && pl.tiles <= cus &&
-            ((t64 > cus && t64 * 4 <= 5 * (int64_t)cus) || K >= 18432))
-            return true;
+        if (N * K >= 100000000ll && pl.tiles <= cus && ((t64 > cus && t64 * 4 <= 5 * (int64_t)cus) || K >= 18432)) return true;
         return t64 > 2 * (int64_t)cus && t64 <= 3 * (int64_t)cus && pl.splits == 1 && pl.tiles <= cus &&
                pl.tiles * 20 >= (int64_t)cus * 11;
+    }
+    if (M <= 48) {
+        // 17..48 rows: the streaming kernel's plan fits its tile to the device (skinny_wide_plan) and is ahead, N = 28672,
+        // K = 4096, M = 48: 24.9 us against 30.1; 40960 x 4096, M = 20: 30.5 against 40.2; 57344 x 8192, M = 48: 86 against
+        // 111; 27648 x 5120, M = 40: 31.8 against 33.9; but for these.  From 33 rows on, large weights whose K it would
+        // share (N = 7168, K = 18432, M = 48: 30.2 here against 31.3) and single launches over a short K (N = 24576,
+        // K = 1536, M = 48: 12.0 against 12.0 - 12.2).
+        const int64_t t64 = (N + 63) / 64;
+        const Rows128Plan pl = rows128_plan(M, N, K, cus);
+        const bool one_launch = pl.splits == 1 && pl.tiles <= cus && pl.tiles * 20 >= (int64_t)cus * 11;
+        if (M > 32 && N * K >= 80000000ll && pl.tiles <= cus && skinny_plan(M, N, K, cus).splits > 1) return true;
+        if (M > 32 && K < 2048 && one_launch) return true;
+        if (K % 4096 == 0) return false;  // its turned starts (stream_turn_mask) decide the following, too
+        // 64-row tiles that spill into a third round where this kernel has a well-filled single launch (N = 36864,
+        // K = 7168, M = 20 / 48: 45.8 / 47.5 against 52.5 / 57.2) ...
+        if (t64 > 2 * (int64_t)cus && t64 <= 3 * (int64_t)cus && one_launch) return true;
+        // ... large weights whose 64-row tiles come to just over one per unit (N = 18432, K = 7168, M = 20 / 48: 28.3 / 29.6
+        // against 34.4 / 36.6), and a very long K (N = 7168, K = 18432: on record here, M = 20 / 32 28.5 / 28.6, the
+        // stream 25.9 / 27.2)
+        const bool over_one = t64 > cus && t64 * 4 <= 5 * (int64_t)cus;
+        if (M > 32 && over_one && N * K >= 60000000ll && pl.tiles <= cus) return true;  // (18944 x 3584, M = 48: 19.6, 20.3)
+        return N * K >= 100000000ll && pl.tiles <= cus && (over_one || K >= 18432);
     }
     if (M > 256) {
         // 257..384 rows (the activation block of a step is 48 KiB): still ahead where the 128-row tiles are few, K is
@@ -513,27 +571,22 @@ static bool rows128_pays(int64_t M, int64_t N, int64_t K, int cus) {
         if (tiles * 2 <= cus) return tiles * rows128_splits(M, N, K, cus) * 2 >= cus;
         return tiles <= cus && (M <= 160 || (M <= kRows128NarrowMaxM && tiles * 8 >= (int64_t)cus * 7));
     }
-    // up to 128 rows: a single well-filled launch always pays (narrow or full-width workgroups on 0.55 cus .. cus
+    // up to 64 rows the streaming kernel first, but for N = 14336, K = 4096 and its neighbours, which are on record here
+    // although it is ahead there, too (17.1 us against 19.5)
+    const bool ahead = M <= 64 && skinny_ahead_of_rows128(M, N, K, cus);
+    const bool kept = M <= 64 && K <= 4096 && N * K >= 55000000ll && (N + 63) / 64 < cus;
+    if (ahead && !kept && N * K < 100000000ll) return false;
+    // otherwise a single well-filled launch always pays up to 128 rows (narrow or full-width workgroups on 0.55 cus .. cus
     // tiles with K unshared: DeepSeek-V3 gate_up at M = 64: 49.7 us against 69.9 - 72.5 for the streaming kernels,
     // q_b 12.5 against 15.0, Llama-3 gate_up 29.5 against 29.8)
     const Rows128Plan pl = rows128_plan(M, N, K, cus);
     if (pl.splits == 1 && pl.tiles <= cus && pl.tiles * 20 >= (int64_t)cus * 11) return true;
     if (M > 64) return K / kBlockK >= 16;
-    // 33..64 rows with K shared or more tiles than units: on the large weights, and not where the
-    // shared-activation streaming kernel runs (lm_head, N = 128256, K = 4096, M = 64: 116 us against 110 - its small
-    // workgroups fill the second round better)
+    // 49..64 rows with K shared or more tiles than units: not where the shared-activation streaming kernel runs (its small
+    // workgroups fill the second round better), else from 60 MB of weights on (M = 64: N = 10240, K = 8192 24.2 us against
+    // 30.7 for the streaming kernel; 16384 x 7168, 256 workgroups there, 29.7 against 26.3)
     if (pl.tiles > cus || xshare_pays(M, N, K, cus)) return false;
-    // ... unless the streaming kernel's workgroups come out as one per unit with K whole (N = 16384, K = 7168,
-    // M = 64: 25.9 us against 29.9) ...
-    const SkinnyPlan sp = skinny_plan(M, N, K, cus);
-    const int64_t wgs = (int64_t)sp.tiles * sp.splits;
-    if (N * K >= 100000000ll) return !(sp.splits == 1 && wgs == cus);
-    // ... and on the mid-size ones (from 35 MB) where they come out as neither one nor two per unit: N = 10240,
-    // K = 8192 (640 of them), M = 64: 24.5 us against 33.6; 14336 x 4096 (896): 19.6 against 24.0; 12288 x 4096 (768):
-    // 18.0 against 22.4; 5120 x 13824 (640): 21.4 against 28.8.  With 512 or 256 of them it keeps its lead (8192 x
-    // 8192: 21.3 against 22.9; 16384 x 4096: 18.7 against 21.3), and on smaller weights the second launch shows
-    // (6144 x 4096: 12.8 against 14.6).
-    return N * K >= 35000000ll && wgs != cus && wgs != 2 * (int64_t)cus;
+    return kept || (N * K >= 60000000ll && !ahead);
 }
 
 static bool rows128_limits_ok(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t as_m, int64_t as_k, int cus) {
@@ -549,12 +602,21 @@ static bool rows128_limits_ok(int64_t M, int64_t N, int64_t K, int64_t lda, int6
 
 template <int MT, int WV, int TN = (MT <= 8 ? 2 : 1)>
 static int launch_rows128_as(GemmArgs &a, const Rows128Plan &pl, void *ws, hipStream_t st) {
+    const bool turned = pl.turned;
     constexpr int NS = MT <= 8 ? 3 : 2;
     using Cfg = Rows128Cfg<MT, NS, TN, WV>;
     const int KB = a.K / kBlockK;
     const int steps = (KB + pl.splits - 1) / pl.splits;
     const int lds_bytes = Cfg::lds_bytes(steps);
     if (lds_bytes > 160 * 1024) return MI355_EUNSUPPORTED;
+    // Turned starts (stream_turn_mask) where a step is mostly weights: up to 96 rows, or weights of 200 MB and more (us, in
+    // step / turned: N = 28672, K = 4096, M = 64 / 80 / 128 29.2 / 30.5 / 36.2 against 26.3 / 28.2 / 37.3; 57344 x 8192,
+    // M = 64 / 128 / 160 115 / 122 / 119 against 85 / 97 / 108; 12288 x 4096, M = 160 31.8 against 33.1).  Tiles over M share
+    // their activation rows in the L2 step by step and lose that (K = 8192: 2 to 6 %).  The two buffers of scale chunks
+    // want a multiple of 16 steps.  From 65 rows on, where the square tiles run as well, a launch asked for by name keeps
+    // K order: its sums are then theirs bit for bit.
+    const bool weights_lead = a.M <= 96 || (int64_t)a.N * a.K >= 200000000ll;
+    a.turn_mask = turned && weights_lead && a.tiles_m <= 1 && KB % (16 * pl.splits) == 0 ? stream_turn_mask(a.K, KB / pl.splits) : 0;
     if (pl.splits <= 1) {
         constexpr auto kernel = block_fp8_gemm_rows128_kernel<MT, NS, TN, WV, false>;
         if (!allow_lds<kernel>(160 * 1024)) return MI355_ELAUNCH;
@@ -680,6 +742,7 @@ static int launch_rowsm(GemmArgs &a, const RowsMPlan &mp, hipStream_t st) {
     a.tiles_n = mp.tiles_n;
     a.total_tiles = mp.tiles_m * mp.tiles_n;
     Rows128Plan pl;
+    pl.turned = false;
     pl.wv = mp.wv;
     pl.bn = 32 * mp.wv;
     pl.splits = 1;
@@ -729,14 +792,20 @@ static int64_t n_split_rows(int64_t M, int64_t N, int64_t K, int cus);
 //   129 <= M <= 208 (192), 0.55 cus .. cus tiles of
 //     160..256 or of 80..112 (64) weight rows         the same, workgroups of that width, K unshared
 //   65 <= M <= 128, K >= 2048                        the same with 256 weight rows per workgroup
-//   33 <= M <= 64, at most cus tiles, N*K >= 1e8 or
-//     (N*K >= 4e7 and the streaming kernel's
-//     workgroups neither cus nor 2 cus)              the same, unless the kernel below would run
-//   33 <= M <= 128, 0.55 cus .. cus tiles of 160,
-//     192 or 256 weight rows with K unshared          the same, workgroups of that width
+//   49 <= M <= 64, at most cus tiles, N*K >= 6e7,
+//     unless the streaming kernel is ahead
+//     (skinny_ahead_of_rows128)                       the same, unless the shared-activation kernel would run
+//   49 <= M <= 128, 0.55 cus .. cus tiles of 160,
+//     192 or 256 weight rows with K unshared          the same, workgroups of that width (up to 64 rows and N*K < 1e8
+//                                                    not where the streaming kernel is ahead)
+//   17 <= M <= 48, K % 4096 != 0 and either 64-row
+//     tiles in a third round, or N*K >= 1e8 and just
+//     over one per unit or K >= 18432; 33 <= M <= 48,
+//     N*K >= 8e7 where the streaming kernel would
+//     share K, or a single launch over K < 2048        the same
 //   M > 384, N <= 5120 (3072), K <= 5120 (7168), one
 //     round of tiles of at most 128 (96) rows         the same kernel tiled over M, K unshared
-//   M <= 64                                          weight streaming (M > 32 and N/128 about the unit count: the
+//   M <= 64                                          weight streaming (M > 48 and N/128 about the unit count: the
 //                                                    kernel that shares the activation block in the workgroup)
 //   few 256x256 tiles, long K                        stream-K (the plain loop would leave most units idle)
 //   128x128 tiles fit one round of two per unit and
@@ -1031,7 +1100,8 @@ static int block_fp8_gemm_impl(const void *A, const void *B, const float *As, co
         }
         case MI355_GEMM_ROWS128: {
             if (!rows128_limits_ok(M, N, K, lda, as_m, as_k, cus)) return MI355_EUNSUPPORTED;
-            const Rows128Plan pl = rows128_plan(M, N, K, cus);
+            Rows128Plan pl = rows128_plan(M, N, K, cus);
+            pl.turned = was_auto || M <= 64;
             if (pl.splits > 1 && (!ws || ws_bytes < rows128_workspace(M, N, K, cus) || ((uintptr_t)ws & 15)))
                 return MI355_EWORKSPACE;
             switch (rows128_mt(M)) {
@@ -1078,6 +1148,7 @@ static int block_fp8_gemm_impl(const void *A, const void *B, const float *As, co
             switch (skinny_mt(M)) {
                 case 1: return launch_stream_mt<1>(a, pl, ws, st);
                 case 2: return launch_stream_mt<2>(a, pl, ws, st);
+                case 3: return launch_stream_mt<3>(a, pl, ws, st);
                 default: return launch_stream_mt<4>(a, pl, ws, st);
             }
         }

@@ -139,15 +139,19 @@ __global__ __launch_bounds__(64 * WV) void block_fp8_gemm_rows128_kernel(const G
     const uint32_t wdst = (uint32_t)Cfg::kXBytes + (uint32_t)wave * (WNS * 128u);
     const uint32_t chunk_off = (uint32_t)Cfg::chunk_off(steps);
 
+    // step `it` in K order, counted from where this tile starts (GemmArgs::turn_mask: 0, or the range is a multiple of 16
+    // steps - the scale chunks alternate between their two buffers across the end of the range, too)
+    const int rot = (int)((5u * tile_n) & (uint32_t)p.turn_mask);
+    auto turn = [&](int it) -> int { return it + rot >= steps ? it + rot - steps : it + rot; };
     auto issue_w = [&](int slot, int it) {
         const uint32_t sb = lds0 + (uint32_t)slot * Cfg::kStage + wdst;
-        const uint8_t *wk = wg + (int64_t)it * kBlockK;
+        const uint8_t *wk = wg + (int64_t)turn(it) * kBlockK;
 #pragma unroll
         for (int i = 0; i < NWW; ++i) dma_g2l_b128(sb + (uint32_t)i * 1024u, wk, woff[i]);
     };
     auto issue_x = [&](int slot, int it) {
         const uint32_t sb = lds0 + (uint32_t)slot * Cfg::kStage;
-        const uint8_t *xk = xg + (int64_t)it * kBlockK;
+        const uint8_t *xk = xg + (int64_t)turn(it) * kBlockK;
 #pragma unroll
         for (int i = 0; i < NXW; ++i) dma_g2l_b128(sb + xdst[i], xk, xoff[i]);
     };
@@ -172,7 +176,7 @@ __global__ __launch_bounds__(64 * WV) void block_fp8_gemm_rows128_kernel(const G
         const int xi = j + NS - 1, wi = j + NS;
         if (xi >= 0 && xi < steps) {
             issue_x(xi % NS, xi);
-            if (xi == 0) issue_scales(0);
+            if (xi == 0 || (turn(xi) & 7) == 0) issue_scales(turn(xi) >> 3);
         }
         if (wi < steps) issue_w(wi % NS, wi);
     }
@@ -209,12 +213,13 @@ __global__ __launch_bounds__(64 * WV) void block_fp8_gemm_rows128_kernel(const G
             const int xi = it + NS - 1;
             if (xi < steps) {
                 issue_x(slot == 0 ? NS - 1 : slot - 1, xi);
-                if ((xi & 7) == 0) issue_scales(xi >> 3);
+                if ((turn(xi) & 7) == 0) issue_scales(turn(xi) >> 3);
             }
         }
         const uint8_t *st = lds + slot * Cfg::kStage;
-        const float ws_cur = wsl[it];
-        const float *sp = (const float *)(lds + sr8 + ((it >> 3) & 1) * Cfg::kChunkBytes + (it & 7) * 4);
+        const int kb = turn(it);
+        const float ws_cur = wsl[kb];
+        const float *sp = (const float *)(lds + sr8 + ((kb >> 3) & 1) * Cfg::kChunkBytes + (kb & 7) * 4);
         v8i wf[TN];
 #pragma unroll
         for (int j = 0; j < TN; ++j) {

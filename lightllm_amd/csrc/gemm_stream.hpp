@@ -56,15 +56,15 @@ struct XQuant {
     }
 };
 
-template <int MT, int TNW>
+template <int MT, int TNW, int WV = kStreamWaves>
 struct StreamCfg {
     static_assert(TNW == 1 || TNW == 2 || TNW == 4 || TNW == 8, "a tile must sit inside one 128-row scale block");
     static constexpr int BN = 16 * TNW;
-    // K steps in flight per wave.  Occupancy counts for more than depth: the deepest pipeline that still leaves a
-    // wave within 256 registers, i.e. two CTAs per CU (measured: M=32 28.9 us at depth 3 -> 25.6 at depth 2,
-    // M=64 36.6 us at depth 2 -> 33.9 at depth 1, M<=16 best at depth 3).
+    // K steps in flight per wave.  Occupancy counts for more than depth: from 17 rows on one step per wave and more
+    // waves is ahead of two or three steps on every shape tried (N = 6144, K = 4096, M = 48, eight waves: 10.3 us at
+    // depth 1, 11.0 at 2, 14.5 at 4; M <= 16 best at depth 3).
     static constexpr int depth(bool xs_in_lds) {
-        if (xs_in_lds) return MT == 1 ? 3 : (MT == 2 ? 2 : 1);
+        if (xs_in_lds) return MT == 1 ? 3 : 1;
         const int set = 8 * TNW + 9 * MT + 1;  // registers of one in-flight K step
         return set * 6 <= 150 ? 6 : (150 / set < 2 ? 2 : 150 / set);
     }
@@ -72,11 +72,12 @@ struct StreamCfg {
     static constexpr int kWaveLds = (16 * TNW + 16 * MT) * 128;
     static constexpr int kAccLds = TNW * MT * 1024;               // one wave's accumulators (fp32)
     static constexpr int kWaveBytes = kWaveLds > kAccLds ? kWaveLds : kAccLds;
-    static constexpr int kLds = kStreamWaves * kWaveBytes + 16;   // + the split-K arrival word
+    static constexpr int kLds = WV * kWaveBytes + 16;   // + the split-K arrival word
     static constexpr int kTileElems = 16 * MT * BN;
     // activation scales of the CTA's K range, staged once: [step][16*MT rows + 1 pad] floats behind kLds
     static constexpr int kScaleStride = 16 * MT + 1;
-    static constexpr int kMaxScaleSteps = 15 * 1024 / (kScaleStride * 4) < 64 ? 15 * 1024 / (kScaleStride * 4) : 64;
+    static constexpr int kScaleRoom = WV == 8 ? 160 * 1024 - kLds : 15 * 1024, kScaleMost = WV == 8 ? 160 : 64;
+    static constexpr int kMaxScaleSteps = kScaleRoom / (kScaleStride * 4) < kScaleMost ? kScaleRoom / (kScaleStride * 4) : kScaleMost;
     static constexpr int scale_lds_bytes(int steps) { return steps * kScaleStride * 4; }
 };
 
@@ -92,10 +93,12 @@ struct StreamRegs {
 // checks that the range fits); otherwise every wave gathers them per step, which costs as many cache-line
 // accesses as the X block itself (16 rows x 4 bytes per request).
 // XR > 0: X is the unquantized activation matrix (XQuant above; XSL is false then).
-template <int MT, int TNW, bool SPLIT, bool XSL, int XR = 0, bool F16 = false>
-__global__ __launch_bounds__(256) void block_fp8_gemm_stream_kernel(const GemmArgs p) {
+// TURN: the tiles start at different K steps (GemmArgs::turn_mask).
+template <int MT, int TNW, bool SPLIT, bool XSL, int XR = 0, bool F16 = false, int WV = kStreamWaves, bool TURN = false>
+__global__ __launch_bounds__(64 * WV) void block_fp8_gemm_stream_kernel(const GemmArgs p) {
     static_assert(XR == 0 || (MT == 1 && !XSL), "unquantized activations: at most 16 rows, no staged scales");
-    using Cfg = StreamCfg<MT, TNW>;
+    static_assert(MT == 1 || XSL, "the plan keeps K ranges within the staged scales from 17 rows on");
+    using Cfg = StreamCfg<MT, TNW, WV>;
     constexpr int NX = XR ? XR : 2 * MT;
     using Regs = StreamRegs<MT, TNW, NX>;
     constexpr int D = Cfg::depth(XSL || XR);
@@ -124,7 +127,7 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_stream_kernel(const GemmAr
     }
     // this wave's K steps: kb_begin + wave, + 4, ...
     const int first = kb_begin + wave;
-    const int steps = first < kb_end ? (kb_end - first + kStreamWaves - 1) / kStreamWaves : 0;
+    const int steps = first < kb_end ? (kb_end - first + WV - 1) / WV : 0;
 
     // ---- per-lane global offsets (rows past the matrix are clamped; their results are never stored)
     uint32_t woff[2 * TNW];
@@ -142,10 +145,11 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_stream_kernel(const GemmAr
     const int NB = (p.N + kBlockN - 1) / kBlockN;
     const float *wsp = p.Ws + (int64_t)min(n0 / kBlockN, NB - 1) * p.ws_n;
 
-    // ---- stage the activation scales: thread (row group tid/32, step tid%32) walks rows +8 and steps +32, so a
+    // ---- stage the activation scales: thread (row group tid/32, step tid%32) walks rows +2*WV and steps +32, so a
     // row-major scale row is read as whole cache lines; indices past the range repeat the last valid element
     float *xs_lds = (float *)(lds + Cfg::kLds) + (XR ? wave * 16 : 0);
-    constexpr int kSvRows = 2 * MT, kSvSteps = (Cfg::kMaxScaleSteps + 31) / 32;
+    constexpr int kSvPass = 2 * WV;  // rows a pass of the workgroup covers
+    constexpr int kSvRows = (16 * MT + kSvPass - 1) / kSvPass, kSvSteps = (Cfg::kMaxScaleSteps + 31) / 32;
     float sv[XSL ? kSvRows * kSvSteps : 1];
     const int steps_cta = kb_end - kb_begin;
     if constexpr (XSL) {
@@ -153,12 +157,16 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_stream_kernel(const GemmAr
         for (int a = 0; a < kSvRows; ++a)
 #pragma unroll
             for (int b = 0; b < kSvSteps; ++b) {
-                const int m = min(8 * a + (tid >> 5), p.M - 1);
+                if (32 * b >= steps_cta && b > 0) continue;
+                const int m = min(kSvPass * a + (tid >> 5), p.M - 1);
                 const int kb = min(kb_begin + min(32 * b + (tid & 31), max(steps_cta - 1, 0)), KB - 1);
                 sv[a * kSvSteps + b] = p.Xs[(int64_t)m * p.xs_m + (int64_t)kb * p.xs_k];
             }
     }
 
+    // K step kb of the range, counted from where this tile starts in it (GemmArgs::turn_mask)
+    const int rot = TURN ? (int)((5u * tile_n) & (uint32_t)p.turn_mask) : 0;
+    auto turn = [&](int kb) -> int { return TURN && kb + rot >= kb_end ? kb + rot - steps_cta : kb + rot; };
     auto load = [&](Regs &r, int kb) {
         const uint8_t *wk = p.W + (int64_t)kb * kBlockK;
         const uint8_t *xk = p.X + (int64_t)kb * (XR ? 2 * kBlockK : kBlockK);
@@ -243,7 +251,7 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_stream_kernel(const GemmAr
     Regs regs[D];
 #pragma unroll
     for (int d = 0; d < D; ++d)
-        if (d < steps) load(regs[d], first + d * kStreamWaves);
+        if (d < steps) load(regs[d], turn(first + d * WV));
     if constexpr (XSL) {
         // the scale loads were issued before the prologue loads, so only they are waited for here
 #pragma unroll
@@ -251,7 +259,7 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_stream_kernel(const GemmAr
 #pragma unroll
             for (int b = 0; b < kSvSteps; ++b) {
                 const int j = 32 * b + (tid & 31);
-                if (j < steps_cta) xs_lds[j * Cfg::kScaleStride + 8 * a + (tid >> 5)] = sv[a * kSvSteps + b];
+                if (j < steps_cta && kSvPass * a + (tid >> 5) < 16 * MT) xs_lds[j * Cfg::kScaleStride + kSvPass * a + (tid >> 5)] = sv[a * kSvSteps + b];
             }
         __syncthreads();
     }
@@ -259,8 +267,8 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_stream_kernel(const GemmAr
 #pragma unroll
         for (int d = 0; d < D; ++d) {
             if (j + d < steps) {
-                consume(regs[d], first + (j + d) * kStreamWaves);
-                if (j + d + D < steps) load(regs[d], first + (j + d + D) * kStreamWaves);
+                consume(regs[d], turn(first + (j + d) * WV));
+                if (j + d + D < steps) load(regs[d], turn(first + (j + d + D) * WV));
             }
         }
     }
@@ -273,15 +281,15 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_stream_kernel(const GemmAr
 #pragma unroll
         for (int j = 0; j < TNW; ++j) *(v4f *)(my + ((t * TNW + j) * 64 + lane) * 16) = acc[t][j];
     __syncthreads();
-    constexpr int FW = (F + kStreamWaves - 1) / kStreamWaves;  // blocks per wave
+    constexpr int FW = (F + WV - 1) / WV;  // blocks per wave
     v4f sum[FW];
 #pragma unroll
     for (int q = 0; q < FW; ++q) {
-        const int f = q * kStreamWaves + wave;
+        const int f = q * WV + wave;
         v4f s = v4f{0.f, 0.f, 0.f, 0.f};
         if (f < F) {
 #pragma unroll
-            for (int w = 0; w < kStreamWaves; ++w) s += *(const v4f *)(lds + w * Cfg::kWaveBytes + (f * 64 + lane) * 16);
+            for (int w = 0; w < WV; ++w) s += *(const v4f *)(lds + w * Cfg::kWaveBytes + (f * 64 + lane) * 16);
         }
         sum[q] = s;
     }
@@ -292,12 +300,12 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_stream_kernel(const GemmAr
         const uint32_t lane_off = (uint32_t)lane * 16u;
 #pragma unroll
         for (int q = 0; q < FW; ++q) {
-            const int f = q * kStreamWaves + wave;
+            const int f = q * WV + wave;
             if (f < F) xch.store(split * (uint32_t)(Cfg::kTileElems * 4) + (uint32_t)f * 1024u + lane_off, sum[q]);
         }
         wait_vmcnt<0>();
         __syncthreads();
-        volatile uint32_t *arrived = (volatile uint32_t *)(lds + kStreamWaves * Cfg::kWaveBytes);
+        volatile uint32_t *arrived = (volatile uint32_t *)(lds + WV * Cfg::kWaveBytes);
         if (tid == 0)
             *arrived = __hip_atomic_fetch_add(p.counters + tile_n, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();
@@ -308,7 +316,7 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_stream_kernel(const GemmAr
             v4f t[FW][kBatch];
 #pragma unroll
             for (int q = 0; q < FW; ++q) {
-                const int f = q * kStreamWaves + wave;
+                const int f = q * WV + wave;
 #pragma unroll
                 for (int d = 0; d < kBatch; ++d)
                     if (f < F && sp0 + d < p.splits)
@@ -316,7 +324,7 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_stream_kernel(const GemmAr
             }
 #pragma unroll
             for (int q = 0; q < FW; ++q) {
-                const int f = q * kStreamWaves + wave;
+                const int f = q * WV + wave;
 #pragma unroll
                 for (int d = 0; d < kBatch; ++d)
                     if (f < F && sp0 + d < p.splits) sum[q] = (sp0 + d == 0) ? t[q][d] : sum[q] + t[q][d];
@@ -328,7 +336,7 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_stream_kernel(const GemmAr
     // ---- store: block f = (mt, tn): lane (r16, g4) holds row m = 16*mt + r16, columns n0 + 4*TNW*g4 + 4*tn + [0,4)
 #pragma unroll
     for (int q = 0; q < FW; ++q) {
-        const int f = q * kStreamWaves + wave;
+        const int f = q * WV + wave;
         if (f >= F) continue;
         const int t = f / TNW, j = f % TNW;
         const int m = 16 * t + r16;

@@ -95,6 +95,7 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_xshare_kernel(const GemmAr
     for (int a = 0; a < kSvRows; ++a)
 #pragma unroll
         for (int b = 0; b < kSvSteps; ++b) {
+            if (b > 0 && 32 * b >= steps) continue;
             const int m = min(8 * a + (tid >> 5), p.M - 1);
             const int kb = kb_begin + min(32 * b + (tid & 31), max(steps - 1, 0));
             sv[a * kSvSteps + b] = p.Xs[(int64_t)m * p.xs_m + (int64_t)kb * p.xs_k];
@@ -105,7 +106,11 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_xshare_kernel(const GemmAr
         v4i x[NX];
         float ws;
     };
-    auto load = [&](Regs &r, int kb) {
+    // step `it` of this workgroup in K order, counted from where its tile starts (GemmArgs::turn_mask)
+    const int rot = (int)((5u * tile_n) & (uint32_t)p.turn_mask);
+    auto turn = [&](int it) -> int { return it + rot >= steps ? it + rot - steps : it + rot; };
+    auto load = [&](Regs &r, int it) {
+        const int kb = kb_begin + turn(it);
         const uint8_t *wk = p.W + (int64_t)kb * kBlockK;
         const uint8_t *xk = p.X + (int64_t)kb * kBlockK;
 #pragma unroll
@@ -162,7 +167,7 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_xshare_kernel(const GemmAr
             const v4i lo = *(const v4i *)(xs_stage + rd0 + t * 2048);
             const v4i hi = *(const v4i *)(xs_stage + rd1 + t * 2048);
             const v8i xf = v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-            const float sc = xs_lds[it * Cfg::kScaleStride + 16 * t + r16] * ws;
+            const float sc = xs_lds[turn(it) * Cfg::kScaleStride + 16 * t + r16] * ws;
 #pragma unroll
             for (int j = 0; j < TNW; ++j) {
                 const v4f part = mfma_16x16x128_fp8(wf[j], xf, v4f{0.f, 0.f, 0.f, 0.f});
@@ -175,7 +180,7 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_xshare_kernel(const GemmAr
     Regs regs[D];
 #pragma unroll
     for (int d = 0; d < D; ++d)
-        if (d < steps) load(regs[d], kb_begin + d);
+        if (d < steps) load(regs[d], d);
 #pragma unroll
     for (int a = 0; a < kSvRows; ++a)
 #pragma unroll
@@ -187,7 +192,7 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_xshare_kernel(const GemmAr
     if (steps > 0) {
         publish(regs[0], 0);
         ws_cur = regs[0].ws;
-        if (D < steps) load(regs[0], kb_begin + D);
+        if (D < steps) load(regs[0], D);
     }
     lds_barrier();  // the staged scales and step 0 are visible
     for (int j = 0; j < steps; j += D) {
@@ -200,7 +205,7 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_xshare_kernel(const GemmAr
                 if (it + 1 < steps) {
                     publish(regs[dn], it + 1);
                     ws_next = regs[dn].ws;
-                    if (it + 1 + D < steps) load(regs[dn], kb_begin + it + 1 + D);
+                    if (it + 1 + D < steps) load(regs[dn], it + 1 + D);
                 }
                 compute(ws_cur, it);
                 ws_cur = ws_next;

@@ -47,27 +47,33 @@ static FusedPlan fused_plan(int64_t M, int64_t N, int64_t K, int32_t x_dtype, in
     return f;
 }
 
-template <int TB, int XR, bool F16>
-static int launch_cu(GemmArgs &a, hipStream_t st) {
+template <int TB, int XR, bool F16, bool TURN>
+static int launch_cu_as(GemmArgs &a, hipStream_t st) {
     using Cfg = CuStreamCfg<1, TB, XR>;
-    constexpr auto kernel = block_fp8_gemm_streamcu_kernel<1, TB, true, XR, F16>;
+    constexpr auto kernel = block_fp8_gemm_streamcu_kernel<1, TB, true, XR, F16, TURN>;
     const int lds_bytes = Cfg::lds_bytes(a.K / kBlockK);
     if (lds_bytes > kMaxLds) return MI355_EUNSUPPORTED;
     if (!allow_lds<kernel>(kMaxLds)) return MI355_ELAUNCH;
     return launch(kernel, dim3((a.N + Cfg::BN - 1) / Cfg::BN), dim3(Cfg::kThreads), lds_bytes, st, a);
 }
 
-template <int TNW, int XR, bool F16>
-static int launch_tiled(GemmArgs &a, const SkinnyPlan &pl, void *ws, hipStream_t st) {
+template <int TB, int XR, bool F16>
+static int launch_cu(GemmArgs &a, hipStream_t st) {
+    a.turn_mask = stream_turn_mask(a.K, a.K / kBlockK);
+    return a.turn_mask ? launch_cu_as<TB, XR, F16, true>(a, st) : launch_cu_as<TB, XR, F16, false>(a, st);
+}
+
+template <int TNW, int XR, bool F16, bool TURN>
+static int launch_tiled_as(GemmArgs &a, const SkinnyPlan &pl, void *ws, hipStream_t st) {
     using Cfg = StreamCfg<1, TNW>;
     constexpr int lds_bytes = Cfg::kLds + kStreamWaves * 64;
     if (pl.splits <= 1) {
-        constexpr auto whole_k = block_fp8_gemm_stream_kernel<1, TNW, false, false, XR, F16>;
+        constexpr auto whole_k = block_fp8_gemm_stream_kernel<1, TNW, false, false, XR, F16, kStreamWaves, TURN>;
         if (!allow_lds<whole_k>(lds_bytes)) return MI355_ELAUNCH;
         return launch(whole_k, dim3(pl.tiles), dim3(256), lds_bytes, st, a);
     }
     if constexpr (TNW == 1) {  // 64-row tiles never share K
-        constexpr auto split_k = block_fp8_gemm_stream_kernel<1, TNW, true, false, XR, F16>;
+        constexpr auto split_k = block_fp8_gemm_stream_kernel<1, TNW, true, false, XR, F16, kStreamWaves, TURN>;
         if (!allow_lds<split_k>(lds_bytes)) return MI355_ELAUNCH;
         a.splits = pl.splits;
         a.counters = (uint32_t *)ws;
@@ -75,6 +81,12 @@ static int launch_tiled(GemmArgs &a, const SkinnyPlan &pl, void *ws, hipStream_t
         return launch(split_k, dim3(pl.tiles * pl.splits), dim3(256), lds_bytes, st, a);
     }
     return MI355_EUNSUPPORTED;
+}
+
+template <int TNW, int XR, bool F16>
+static int launch_tiled(GemmArgs &a, const SkinnyPlan &pl, void *ws, hipStream_t st) {
+    a.turn_mask = stream_turn_mask(a.K, a.K / kBlockK / pl.splits);
+    return a.turn_mask ? launch_tiled_as<TNW, XR, F16, true>(a, pl, ws, st) : launch_tiled_as<TNW, XR, F16, false>(a, pl, ws, st);
 }
 
 template <int XR, bool F16>

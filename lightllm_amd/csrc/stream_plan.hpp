@@ -13,22 +13,93 @@ inline bool fast_layout_ok(const void *A, const void *B, int64_t K, int64_t lda,
            ((uintptr_t)B & 15) == 0;
 }
 
+// Where in its K range (of at least `steps` K steps) a tile starts: GemmArgs::turn_mask.  With rows a multiple of 4 KiB apart the
+// same K step of every row lies in the same few memory channels, and tiles that walk K in step queue there; started at
+// different steps they spread.  (K stands for the distance: a result does not depend on how a weight is padded.)  With any other distance the rows do that by themselves and turning only costs
+// (K = 14336: 0 to 5 % slower), and a range of fewer than 32 steps - 4 KiB of a row - is spread by its neighbours already.
+// us, in step / turned: N = 6144, K = 4096, M = 1 8.1 / 7.4; 28672 x 4096 21.0 / 19.5; 12288 x 4096 13.7 / 11.7; 57344 x 8192
+// 78.5 / 70.8; 8192 x 8192, M = 48, whole K on eight waves 21.8 / 17.3; a shared K of 16 steps is 1 to 3 % slower turned.
+inline int stream_turn_mask(int64_t K, int steps) {
+    if (K % 4096 != 0 || steps < 32) return 0;
+    int m = 0;
+    while (2 * m + 1 < steps) m = 2 * m + 1;
+    return m;
+}
+
 // ---- the stream in tiles of 16, 32 or 64 weight rows, M <= 64
-inline int skinny_mt(int64_t M) { return M <= 16 ? 1 : (M <= 32 ? 2 : 4); }
+inline int skinny_mt(int64_t M) { return M <= 16 ? 1 : (int)((M + 15) / 16); }
 
 struct SkinnyPlan {
     int tnw, splits, tiles;
+    int waves;
 };
 
+// 17..64 rows: four or eight waves a workgroup, tiles of 16, 32 or 64 weight rows, K whole or shared by up to eight
+// workgroups.  A wave has one K step in flight and the waves hide each other's latency, so what a launch takes is what
+// its busiest unit pulls: weights at about 50 GB/s (a unit's misses in flight over the latency of HBM), activations at
+// about 140 (they come from the L2; every workgroup reads all rows of its K range), 97 ns for each K step in a wave's
+// sequence, 280 ns and 625 for each workgroup that shares a tile and 6 us for a further round.  The constants were fitted to
+// 22 (N, K) pairs (N = 1536..36864, K = 1536..18944) at M = 20..64, all candidates timed: the choice is 1.0 % behind
+// the best candidate on average.  Against tiles of 16 / 32 / 64 rows on four waves with K shared until there were two
+// workgroups a unit, us: N = K = 4096, M = 20 / 48 / 64 7.3 / 8.6 / 9.7 (8.9 / 10.0 / 10.1), 6144 x 4096 8.5 / 10.3 /
+// 11.6 (10.2 / 12.3 / 12.8), 4096 x 14336 14.5 / 17.3 / 19.5 (14.9 / 18.8 / 20.1), 28672 x 4096 21.5 / 24.9 (23.8 / 30.1).
+inline int64_t skinny_wide_lds(int waves, int tnw, int mt, int64_t steps) {
+    const int64_t wave = (16 * tnw + 16 * mt) * 128, acc = (int64_t)tnw * mt * 1024;
+    return waves * (wave > acc ? wave : acc) + 16 + steps * (16 * mt + 1) * 4;
+}
+
+// K steps of a workgroup whose activation scales fit: the LDS behind eight waves, 15 KiB behind four (two workgroups a unit).
+inline int64_t skinny_wide_cap(int waves, int tnw, int mt) {
+    const int64_t room = waves == 8 ? kMaxLds - skinny_wide_lds(8, tnw, mt, 0) : 15 * 1024;
+    const int64_t steps = room / ((16 * mt + 1) * 4), most = waves == 8 ? 160 : 64;
+    return steps < most ? steps : most;
+}
+
+inline SkinnyPlan skinny_wide_plan(int64_t M, int64_t N, int64_t K, int cus) {
+    const int mt = skinny_mt(M);
+    const int64_t KB = K / kBlockK;
+    SkinnyPlan best = {0, 1, 0, 8};
+    int64_t best_cost = 0;
+    for (int waves = 4; waves <= 8; waves += 4)
+        for (int tnw = 1; tnw <= 4; tnw *= 2) {
+            if (waves == 8 && tnw == 4 && mt == 4) continue;  // 128 KiB of LDS and half the registers: not built
+            const int64_t tiles = (N + 16 * tnw - 1) / (16 * tnw), cap = skinny_wide_cap(waves, tnw, mt);
+            if (tiles * 4 > MI355_WS_COUNTER_BYTES) continue;  // one arrival counter a tile
+            for (int s = 1; s <= 8; ++s) {
+                const int64_t wgs = tiles * s, steps = (KB + s - 1) / s;
+                if (s > 1 && (KB / s < 2 * waves || 2 * wgs > 5 * (int64_t)cus)) break;
+                if (steps > cap) continue;
+                // workgroups on a unit at a time, by registers (one or two waves a SIMD) and by LDS
+                const bool two = waves == 8 ? tnw > 1 : tnw * mt >= 8;
+                int64_t slots = tnw * mt == 16 ? 1 : (two ? 8 / waves : 4);
+                const int64_t by_lds = kMaxLds / skinny_wide_lds(waves, tnw, mt, steps);
+                if (slots > by_lds) slots = by_lds > 0 ? by_lds : 1;
+                const int64_t per_unit = (wgs + cus - 1) / cus, rounds = (wgs + cus * slots - 1) / (cus * slots);
+                const int64_t cost = per_unit * 2048 * tnw * steps / 50 + per_unit * 2048 * mt * steps / 140 +
+                                     (s > 1 ? 280 + 625 * s : 0) + 6000 * (rounds - 1) + 97 * ((steps + waves - 1) / waves);
+                if (best.tnw == 0 || cost < best_cost) {
+                    best = {tnw, s, (int)tiles, waves};
+                    best_cost = cost;
+                }
+            }
+        }
+    if (best.tnw == 0) {  // a K range too long for eight shares
+        const int64_t cap = skinny_wide_cap(8, 1, mt);
+        best = {1, (int)((KB + cap - 1) / cap), (int)((N + 15) / 16), 8};
+    }
+    return best;
+}
+
 inline SkinnyPlan skinny_plan(int64_t M, int64_t N, int64_t K, int cus) {
+    if (M > 16) return skinny_wide_plan(M, N, K, cus);
     SkinnyPlan pl;
     pl.splits = 1;
+    pl.waves = 4;
     const int64_t t64 = (N + 63) / 64;
     // 64-row tiles that come to just over one per unit leave half the units with twice the work of the others:
     // narrower tiles then (N = 18432, K = 7168, 288 tiles of 64 rows, M = 1 / 16: 22.6 / 26.8 us against 27.9 /
-    // 29.9; N = 18944, K = 3584: 13.2 / 15.2 against 16.4 / 17.3); up to 1.5 per unit for M > 16, where the narrower
-    // tiles have 32 rows (N = 24576, K = 1536, M = 32 / 64: 10.3 / 15.3 against 12.2 / 18.7)
-    bool unbalanced = t64 > cus && t64 * 4 <= (int64_t)cus * (M <= 16 ? 5 : 6);
+    // 29.9; N = 18944, K = 3584: 13.2 / 15.2 against 16.4 / 17.3)
+    bool unbalanced = t64 > cus && t64 * 4 <= (int64_t)cus * 5;
     // up to 8 rows under a long K the 16-row tiles also win wherever the 64-row ones fill less than 84 % of their
     // last round (N = 36864, K = 7168, 2.25 per unit, M = 1 / 8: 39.6 / 41.5 us against 45.4 / 46.2; N = 22016,
     // K = 5120, 1.34 per unit: 19.9 / 21.4 against 22.7 / 23.4); with whole rounds they lose (N = 49152, M = 8: 41.6
@@ -44,23 +115,22 @@ inline SkinnyPlan skinny_plan(int64_t M, int64_t N, int64_t K, int cus) {
         return pl;
     }
     // Otherwise narrow tiles first, then K splits, until there are about two workgroups per compute unit (measured
-    // on N=4096, K=14336: 16-row tiles x 2 splits 13.1 us at M <= 8 against 14.1 for 64-row tiles x 4 splits;
-    // at M > 16, 32-row tiles x 4 splits 16.1 / 20.0 us at M = 32 / 64, 16-row tiles 18.3 / 25.8), never below 16 K
-    // steps per workgroup (4 per wave).
-    pl.tnw = M <= 16 ? 1 : 2;
-    pl.tiles = (int)((N + 16 * pl.tnw - 1) / (16 * pl.tnw));
+    // on N=4096, K=14336: 16-row tiles x 2 splits 13.1 us at M <= 8 against 14.1 for 64-row tiles x 4 splits), never
+    // below 16 K steps per workgroup (4 per wave).
+    pl.tnw = 1;
+    pl.tiles = (int)((N + 15) / 16);
     const int KB = (int)(K / kBlockK);
     pl.splits = (2 * cus + pl.tiles - 1) / pl.tiles;
     // from 1.5 tiles per unit on K stays whole: two splits would make 3 to 4 workgroups per unit and an exchange
-    // (N = 7168, K = 8192, 448 tiles, M = 1 / 16: 12.8 / 13.7 us against 16.7 / 17.9; 14336 x 4096, M = 32: 15.1
-    // against 18.8; 6912 x 6912, M = 1: 10.2 against 12.3)
+    // (N = 7168, K = 8192, 448 tiles, M = 1 / 16: 12.8 / 13.7 us against 16.7 / 17.9; 6912 x 6912, M = 1: 10.2 against
+    // 12.3)
     if (pl.tiles * 2 >= 3 * cus) pl.splits = 1;
     const int max_splits = KB / 16 > 0 ? KB / 16 : 1;
     if (pl.splits > max_splits) pl.splits = max_splits;
     if (pl.splits < 1) pl.splits = 1;
     // a workgroup stages the activation scales of its K range in LDS if the range is short enough; one more split
     // that gets it there pays (N=7168, K=18432, M=16: 72 steps unstaged 37.5 us, 48 steps staged 30.7)
-    const int cap = skinny_mt(M) == 4 ? StreamCfg<4, 2>::kMaxScaleSteps : StreamCfg<1, 1>::kMaxScaleSteps;
+    const int cap = StreamCfg<1, 1>::kMaxScaleSteps;
     const int need = (KB + cap - 1) / cap;
     if (pl.splits < need && need <= max_splits) pl.splits = need;
     return pl;
@@ -98,6 +168,9 @@ inline int streamcu_tnw(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ld
     return (int)tnw;
 }
 
+// (K a multiple of 4096: the streaming kernel gains more from turned starts than this one, whose workgroups have most
+// of the range in flight anyway - N = 12288, K = 4096, M = 1 / 16: 10.4 / 11.3 us against 11.7 / 12.2 here; 20480: 15.2 /
+// 16.7 against 16.5 / 16.8; from four row blocks a unit and 9 rows on this one is level or ahead: 18432: 16.3 / 15.8.)
 // Where it is ahead of the streaming kernel (M = 1 / 8 / 16, weights rotated past the memory-side cache): wherever
 // that kernel has to share K between workgroups (N = 4096, K = 14336: 12.3 - 13.0 / 12.6 - 13.4 / 13.6 - 14.4 us
 // against 13.4 / 13.7 / 14.9; N = 7168, K = 18432: 23.1 / 23.9 / 25.4 against 26.6 / 28.8 / 30.9), and from three
@@ -108,7 +181,8 @@ inline int streamcu_tnw(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ld
 inline bool streamcu_pays(int64_t M, int64_t N, int64_t K, int cus) {
     const int tnw = streamcu_tnw(M, N, K, K, K, K / kBlockK, cus);
     if (tnw == 0) return false;
-    return skinny_plan(M, N, K, cus).splits > 1 || tnw >= 3;
+    if (skinny_plan(M, N, K, cus).splits > 1) return true;
+    return K % 4096 == 0 ? tnw >= 4 && M > 8 : tnw >= 3;
 }
 
 }  // namespace mi355

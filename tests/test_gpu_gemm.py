@@ -321,6 +321,45 @@ def test_per_unit_stream_kernel(hip):
         _run(xq, xs, wq, ws, "streamcu")
 
 
+def _dequant_close(c, xq, xs, wq, ws):
+    """bf16 outputs against the fp32 dequant-matmul: half a bf16 step of the value (2^-9) and the fp32 sums' share, whose
+    order differs (2^-12 of the largest value, K / 128 <= 160 terms)."""
+    ref = tr.dequant_matmul(xq, xs, wq, ws, out_dtype=torch.float32)
+    assert not torch.isnan(c.float()).any()
+    bound = ref.abs() * 2 ** -8 + ref.abs().max() * 2 ** -11
+    assert bool(((c.float() - ref).abs() <= bound).all()), ((c.float() - ref).abs() / bound).max().item()
+
+
+# M at the edges of the 2, 3 and 4 row-block forms; one K step, fewer steps than waves, ragged last shares, turned starts
+# (K a multiple of 4096, K whole over 32 steps), K beyond what one workgroup stages scales for; N of one row, ragged tiles,
+# tiles of 16, 32 and 64 weight rows on four and on eight waves, more than one workgroup a unit
+@pytest.mark.parametrize("M", [17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("N,K", [(1, 128), (40, 896), (4096, 4096), (4090, 1152), (6144, 4096), (5120, 5120), (12289, 4096),
+                                 (2112, 7168), (24576, 384), (20480, 512), (520, 20608), (136, 36864)])
+def test_stream_17_to_64_rows(hip, M, N, K):
+    print(f"gemm stream M={M} N={N} K={K}", flush=True)
+    xq, xs, wq, ws = _prep(M, N, K, seed=N + K + M, device="cuda")
+    c = _run(xq, xs, wq, ws, "skinny")
+    _dequant_close(c, xq, xs, wq, ws)
+    assert torch.equal(c, _run(xq, xs, wq, ws, "skinny"))
+    assert torch.equal(c, _run(xq, xs.t().contiguous().t(), wq, ws, "skinny"))
+
+
+# turned starts of the other streams, N larger than the turn's period of 32 or 64 tiles: per-unit stream with every K step of a
+# wave in flight (16, 32, 40 steps) and in turns, tiled stream, shared activation block, activation block in LDS (by the
+# table only); an N that is not a multiple of the tile
+@pytest.mark.parametrize("M,N,K,variant", [(1, 4096, 4096, "streamcu"), (16, 4090, 4096, "streamcu"), (8, 4096, 8192, "streamcu"),
+                                           (9, 4096, 2048, "streamcu"), (16, 8190, 5120, "streamcu"), (3, 28668, 4096, "skinny"),
+                                           (16, 12288, 8192, "skinny"), (64, 66000, 4096, "xshare"), (64, 28668, 4096, None),
+                                           (80, 28672, 4096, None), (100, 50176, 4096, None), (49, 28672, 8192, None)])
+def test_turned_starts(hip, M, N, K, variant):
+    print(f"gemm turned starts M={M} N={N} K={K} {variant}", flush=True)
+    xq, xs, wq, ws = _prep(M, N, K, seed=N + K + M, device="cuda")
+    c = _run(xq, xs, wq, ws, variant)
+    _dequant_close(c, xq, xs, wq, ws)
+    assert torch.equal(c, _run(xq, xs, wq, ws, variant))
+
+
 def _lib_cus():
     from lightllm_amd import _lib
 
