@@ -602,22 +602,27 @@ static bool rows128_limits_ok(int64_t M, int64_t N, int64_t K, int64_t lda, int6
 
 template <int MT, int WV, int TN = (MT <= 8 ? 2 : 1)>
 static int launch_rows128_as(GemmArgs &a, const Rows128Plan &pl, void *ws, hipStream_t st) {
-    const bool turned = pl.turned;
     constexpr int NS = MT <= 8 ? 3 : 2;
     using Cfg = Rows128Cfg<MT, NS, TN, WV>;
     const int KB = a.K / kBlockK;
     const int steps = (KB + pl.splits - 1) / pl.splits;
     const int lds_bytes = Cfg::lds_bytes(steps);
     if (lds_bytes > 160 * 1024) return MI355_EUNSUPPORTED;
-    // Turned starts (stream_turn_mask) where a step is mostly weights: up to 96 rows, or weights of 200 MB and more (us, in
-    // step / turned: N = 28672, K = 4096, M = 64 / 80 / 128 29.2 / 30.5 / 36.2 against 26.3 / 28.2 / 37.3; 57344 x 8192,
-    // M = 64 / 128 / 160 115 / 122 / 119 against 85 / 97 / 108; 12288 x 4096, M = 160 31.8 against 33.1).  Tiles over M share
-    // their activation rows in the L2 step by step and lose that (K = 8192: 2 to 6 %).  The two buffers of scale chunks
-    // want a multiple of 16 steps.  From 65 rows on, where the square tiles run as well, a launch asked for by name keeps
-    // K order: its sums are then theirs bit for bit.
-    const bool weights_lead = a.M <= 96 || (int64_t)a.N * a.K >= 200000000ll;
-    a.turn_mask = turned && weights_lead && a.tiles_m <= 1 && KB % (16 * pl.splits) == 0 ? stream_turn_mask(a.K, KB / pl.splits) : 0;
     if (pl.splits <= 1) {
+        // Turned starts (stream_turn_mask) where a step is mostly weights: up to 96 rows, or weights of 200 MB and more (us,
+        // in step / turned: N = 28672, K = 4096, M = 64 / 80 / 128 29.2 / 30.5 / 36.2 against 26.3 / 28.2 / 37.3; 57344 x
+        // 8192, M = 64 / 128 / 160 115 / 122 / 119 against 85 / 97 / 108; 12288 x 4096, M = 160 31.8 against 33.1).  Tiles over
+        // M share their activation rows in the L2 step by step and lose that (K = 8192: 2 to 6 %).  The two buffers of scale
+        // chunks want a multiple of 16 steps.  From 65 rows on, where the square tiles run as well, a launch asked for by
+        // name keeps K order: its sums are then theirs bit for bit.
+        if constexpr (MT <= 10 && TN == 2) {
+            const bool weights_lead = a.M <= 96 || (int64_t)a.N * a.K >= 200000000ll;
+            if (pl.turned && weights_lead && a.tiles_m <= 1 && KB % 16 == 0 && (a.turn_mask = stream_turn_mask(a.K, KB)) != 0) {
+                constexpr auto turned = block_fp8_gemm_rows128_kernel<MT, NS, TN, WV, false, true>;
+                if (!allow_lds<turned>(160 * 1024)) return MI355_ELAUNCH;
+                return launch(turned, dim3(pl.tiles), dim3(Cfg::kThreads), lds_bytes, st, a);
+            }
+        }
         constexpr auto kernel = block_fp8_gemm_rows128_kernel<MT, NS, TN, WV, false>;
         if (!allow_lds<kernel>(160 * 1024)) return MI355_ELAUNCH;
         return launch(kernel, dim3(pl.tiles), dim3(Cfg::kThreads), lds_bytes, st, a);

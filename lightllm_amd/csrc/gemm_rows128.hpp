@@ -75,7 +75,8 @@ __device__ __forceinline__ void rows128_store(const GemmArgs &p, int row, int nb
     }
 }
 
-template <int MT, int NS, int TN, int WV, bool SPLIT>
+// TURN: the tiles start at different K steps (GemmArgs::turn_mask).
+template <int MT, int NS, int TN, int WV, bool SPLIT, bool TURN = false>
 __global__ __launch_bounds__(64 * WV) void block_fp8_gemm_rows128_kernel(const GemmArgs p) {
     using Cfg = Rows128Cfg<MT, NS, TN, WV>;
     constexpr int WNS = Cfg::WNS, NXW = Cfg::NXW, XG = Cfg::XG, NWW = Cfg::NWW, XH = Cfg::XH;
@@ -141,8 +142,8 @@ __global__ __launch_bounds__(64 * WV) void block_fp8_gemm_rows128_kernel(const G
 
     // step `it` in K order, counted from where this tile starts (GemmArgs::turn_mask: 0, or the range is a multiple of 16
     // steps - the scale chunks alternate between their two buffers across the end of the range, too)
-    const int rot = (int)((5u * tile_n) & (uint32_t)p.turn_mask);
-    auto turn = [&](int it) -> int { return it + rot >= steps ? it + rot - steps : it + rot; };
+    const int rot = TURN ? (int)((5u * tile_n) & (uint32_t)p.turn_mask) : 0;
+    auto turn = [&](int it) -> int { return TURN && it + rot >= steps ? it + rot - steps : it + rot; };
     auto issue_w = [&](int slot, int it) {
         const uint32_t sb = lds0 + (uint32_t)slot * Cfg::kStage + wdst;
         const uint8_t *wk = wg + (int64_t)turn(it) * kBlockK;
