@@ -423,10 +423,20 @@ struct Rows128Plan {
     bool turned;  // tiles may start at different K steps (launch_rows128_as)
 };
 
+struct RowsMPlan {
+    int mt, wv, tiles_m, tiles_n;
+};
+static RowsMPlan rowsm_plan(int64_t M, int64_t N, int64_t K, int cus);
+static bool rows128_two_tiles(int64_t M, int64_t N, int64_t K, int cus);  // M in two tiles: rowsm_plan's launch
+
 static Rows128Plan rows128_plan(int64_t M, int64_t N, int64_t K, int cus) {
     Rows128Plan pl;
     const int64_t KB = K / kBlockK;
     pl.turned = false;
+    if (rows128_two_tiles(M, N, K, cus)) {
+        const RowsMPlan mp = rowsm_plan(M, N, K, cus);
+        return {mp.wv, 32 * mp.wv, 1, mp.tiles_m * mp.tiles_n, 2, false};
+    }
     pl.wv = 8;
     pl.bn = M <= 128 ? 256 : 128;
     pl.tn = M <= 128 ? 2 : 1;
@@ -496,6 +506,7 @@ static bool skinny_ahead_of_rows128(int64_t M, int64_t N, int64_t K, int cus) {
 
 static bool rows128_pays(int64_t M, int64_t N, int64_t K, int cus) {
     if (M > 384 || M < 16) return false;
+    if (rows128_two_tiles(M, N, K, cus)) return true;
     if (M == 16) {
         // large weights whose 64-row workgroups come to just over one per unit (N = 18432, K = 7168: 27.5 us against 30.3
         // for the streaming kernel), a very long K (N = 8192, K = 28672: 45.3 against 50.7), or workgroups that spill into a
@@ -589,8 +600,10 @@ static bool rows128_pays(int64_t M, int64_t N, int64_t K, int cus) {
     return kept || (N * K >= 60000000ll && !ahead);
 }
 
+static bool rowsm_limits_ok(const RowsMPlan &pl, int64_t M, int64_t K, int64_t lda, int64_t as_m, int64_t as_k);
 static bool rows128_limits_ok(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t as_m, int64_t as_k, int cus) {
     if (M > 384) return false;
+    if (rows128_two_tiles(M, N, K, cus)) return rowsm_limits_ok(rowsm_plan(M, N, K, cus), M, K, lda, as_m, as_k);
     if (M * lda >= (1ll << 32) || M * as_m * 4 >= (1ll << 32) || as_k * 32 >= (1ll << 32)) return false;
     const Rows128Plan pl = rows128_plan(M, N, K, cus);
     const int64_t steps = (K / kBlockK + pl.splits - 1) / pl.splits;
@@ -670,27 +683,32 @@ static int launch_rows128(GemmArgs &a, const Rows128Plan &pl, void *ws, hipStrea
 // columns, 144 tiles at M = 4096, 72 at M = 2048) and its lone round is bound by the latency of its K steps; tiles of
 // 16*mt rows x 32*wv weight rows with mt chosen so that tiles_m * tiles_n just fits the units put a workgroup on
 // (nearly) every unit, each with less to load and to multiply per step.
-struct RowsMPlan {
-    int mt, wv, tiles_m, tiles_n;
-};
-
+// Which of the tiles: up to N = 4608 (5120 from 769 rows on) the fewest row blocks, then the fewest bytes a unit loads per K
+// step.  Beyond, the least of 146 mt + 134 wv + 90 t (mt/2 + wv) / cus (+ 371 on two ring slots) over the fewest row blocks and one more for every
+// width: what a step of one tile takes (its X block is read by every wave, its W rows once) and what all t tiles
+// pull together; fitted to 60 shapes of M = 200..4096 with every candidate timed, 1.6 % behind the best on average.  (N = 6144,
+// K = 4096, M = 450: 5 row blocks x 160 weight rows 28.2 us, 3 x 256 31.8; 8192 x 4096, M = 400: 29.7 / 36.9.)
 static RowsMPlan rowsm_plan(int64_t M, int64_t N, int64_t /*K*/, int cus) {
     RowsMPlan best = {0, 0, 0, 0};
     if (M <= 0 || cus < 8) return best;
     const int64_t blocks = (M + 15) / 16;
-    int64_t best_bytes = 0;
+    const bool wide = N > 5120 || (N > 4608 && M <= 768);
+    int64_t best_cost = 0;
     for (int wv = 8; wv >= 5; --wv) {
         const int64_t tn = (N + 32 * wv - 1) / (32 * wv);
         if (tn > cus) continue;
         const int64_t room = cus / tn;                       // m tiles that fit one round
-        const int64_t mt = (blocks + room - 1) / room;       // row blocks per tile
-        if (mt > 13 || (mt <= 8 && wv == 7)) continue;       // kernels built: 5, 6, 8 waves up to 8 blocks; 5..8 up to 13
-        const int64_t tm = (blocks + mt - 1) / mt;
-        if (tm < 2 || tm * tn * 20 < (int64_t)cus * 11) continue;
-        const int64_t bytes = (16 * mt + 32 * wv) * 128;      // what a unit loads per K step
-        if (best.mt == 0 || mt < best.mt || (mt == best.mt && bytes < best_bytes)) {
-            best = {(int)mt, wv, (int)tm, (int)tn};
-            best_bytes = bytes;
+        const int64_t fewest = (blocks + room - 1) / room;   // row blocks per tile
+        for (int64_t mt = fewest; mt <= fewest + (wide ? 1 : 0); ++mt) {
+            if (mt > 13 || (mt <= 8 && wv == 7)) continue;   // kernels built: 5, 6, 8 waves up to 8 blocks; 5..8 up to 13
+            const int64_t tm = (blocks + mt - 1) / mt;
+            if (tm < 2 || tm * tn * 20 < (int64_t)cus * 11) continue;
+            const int64_t cost = wide ? 146 * mt + 134 * wv + 45 * tm * tn * (mt + 2 * wv) / cus + (mt > 8 ? 371 : 0)
+                                      : mt * 65536 + 16 * mt + 32 * wv;
+            if (best.mt == 0 || cost < best_cost) {
+                best = {(int)mt, wv, (int)tm, (int)tn};
+                best_cost = cost;
+            }
         }
     }
     return best;
@@ -712,14 +730,29 @@ static bool rowsm_limits_ok(const RowsMPlan &pl, int64_t M, int64_t K, int64_t l
 // tiles shares K between idle units and takes most of the gain: 2..6 row blocks on N <= 3072 are still 1.04 to 1.3
 // times ahead (q_a+kv_a, N = 2112, K = 7168, M = 512 / 1024 / 2048: 1.11 / 1.12 / 1.04), a single block or a wider N
 // is behind.  From K = 8192 on the kernels that share K win everywhere.
+// On a wider N, K <= 5120: up to 960 rows and N = 15360 with at most 8 row blocks (us, before / here: N = 6144, K = 4096, M = 450 /
+// 700 / 850 36.4 / 41.4 / 43.0 against 28.2 / 33.9 / 35.6; 8192 x 4096, M = 400 / 640 36.4 / 42.9 against 29.7 / 37.2; 10240
+// x 5120, M = 512 55.4 / 45.3; 12288 x 4096, M = 400 / 640 44.2 / 45.3 against 37.1 / 44.3).
 static bool rowsm_pays(int64_t M, int64_t N, int64_t K, int cus) {
     if (M <= 384) return false;
     const int64_t KB = K / kBlockK;
     if (KB < 12 || KB > 56) return false;
     const RowsMPlan pl = rowsm_plan(M, N, K, cus);
     if (pl.mt == 0 || pl.mt > 8) return false;
-    if (KB <= 40) return N <= 5120;
+    if (KB <= 40) return N <= 5120 || (M <= 960 && N <= 15360 && KB >= 16);
     return pl.mt >= 2 && pl.mt <= 6 && N <= 3072;
+}
+
+// 209..352 rows on a wide N: ROWS128 as two m tiles of up to 11 row blocks in one round instead of two 256-row tiles, a third of
+// them padding, or 128x128 tiles in two rounds (us, before / here: N = 27648, K = 5120, M = 220 / 288 / 333 / 352 59.1 / 68.2 /
+// 73.7 / 69.2 against 53.7 / 58.9 / 67.4 / 66.6, at 384 level; 28672 x 4608, M = 300 63.7 / 56.3; 15360 x 5120, M = 330 54.2 /
+// 45.8; 24576 x 1536, M = 333 27.4 / 22.3; 16384 x 4096, M = 256 40.8 / 36.7).  (K = 4096 beyond N = 16384 is on record with
+// the square tiles, although the gain is the same there: 28672 x 4096, M = 224 / 320 48.5 / 60.7 against 44.3 / 51.9.)
+static bool rows128_two_tiles(int64_t M, int64_t N, int64_t K, int cus) {
+    const int64_t KB = K / kBlockK;
+    if (M <= 208 || M > 352 || N < 12288 || KB < 12 || KB > 44 || (K % 4096 == 0 && N > 16384)) return false;
+    const RowsMPlan pl = rowsm_plan(M, N, K, cus);
+    return pl.mt > 0 && pl.mt <= 11;
 }
 
 template <int MT>
@@ -809,7 +842,9 @@ static int64_t n_split_rows(int64_t M, int64_t N, int64_t K, int cus);
 //     N*K >= 8e7 where the streaming kernel would
 //     share K, or a single launch over K < 2048        the same
 //   M > 384, N <= 5120 (3072), K <= 5120 (7168), one
-//     round of tiles of at most 128 (96) rows         the same kernel tiled over M, K unshared
+//     round of tiles of at most 128 (96) rows; 385..960
+//     rows, N <= 15360, K <= 5120                     the same kernel tiled over M, K unshared
+//   209..352 rows, N >= 12288, 1536 <= K <= 5632      the same, two tiles over M
 //   M <= 64                                          weight streaming (M > 48 and N/128 about the unit count: the
 //                                                    kernel that shares the activation block in the workgroup)
 //   few 256x256 tiles, long K                        stream-K (the plain loop would leave most units idle)
@@ -1105,6 +1140,7 @@ static int block_fp8_gemm_impl(const void *A, const void *B, const float *As, co
         }
         case MI355_GEMM_ROWS128: {
             if (!rows128_limits_ok(M, N, K, lda, as_m, as_k, cus)) return MI355_EUNSUPPORTED;
+            if (rows128_two_tiles(M, N, K, cus)) return launch_rowsm(a, rowsm_plan(M, N, K, cus), st);
             Rows128Plan pl = rows128_plan(M, N, K, cus);
             pl.turned = was_auto || M <= 64;
             if (pl.splits > 1 && (!ws || ws_bytes < rows128_workspace(M, N, K, cus) || ((uintptr_t)ws & 15)))

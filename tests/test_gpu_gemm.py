@@ -525,6 +525,22 @@ def test_rows_tiled_over_m_where_the_table_sends_it(hip, M, N, K):
     assert torch.equal(_run(xq, xs, wq, ws, None).view(torch.int16), _run(xq, xs, wq, ws, "rowsm").view(torch.int16))
 
 
+# 209..352 rows in two tiles of the activation-block stream, 385..960 rows on a wider N: the edges of both ranges, row counts
+# that leave the last tile one row, N that leaves the last column of tiles one weight row, the shortest and longest K
+@pytest.mark.parametrize("M,N,K,variant", [(209, 12288, 2048, "rows128"), (225, 12289, 1536, "rows128"), (352, 27648, 1536, "rows128"),
+                                           (333, 27648, 5120, "rows128"), (337, 20481, 1664, "rows128"), (256, 16384, 4096, "rows128"),
+                                           (385, 5376, 2048, "rowsm"), (401, 15360, 2048, "rowsm"), (960, 6017, 2176, "rowsm"),
+                                           (450, 6144, 4096, "rowsm"), (700, 5120, 5120, "rowsm"), (513, 8193, 2304, "rowsm")])
+def test_rows_tiled_over_m_on_a_wider_n(hip, M, N, K, variant):
+    print(f"gemm rows tiled over M, wider N M={M} N={N} K={K}", flush=True)
+    xq, xs, wq, ws = _prep(M, N, K, seed=M + N)
+    c = _run(xq, xs, wq, ws, None)
+    assert torch.equal(c.view(torch.int16), _run(xq, xs, wq, ws, variant).view(torch.int16))
+    _dequant_close(c, xq, xs, wq, ws)
+    # no share of K: the same sums as the 256-row tiles
+    assert torch.equal(c.view(torch.int16), _run(xq, xs, wq, ws, "tile256").view(torch.int16))
+
+
 def test_unit_scales_is_plain_matmul(hip):
     """All scales 1: the result is the plain product of the fp8 values, exact in fp32 for K=128."""
     print("gemm unit scales", flush=True)
