@@ -1,5 +1,7 @@
 """ctypes binding of libmi355fp8.so (the C ABI declared in include/mi355_fp8.h)."""
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
@@ -7,6 +9,7 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libmi355fp8.so")
+CALL_PATH = os.path.join(_HERE, "lib", "_mi355call.so")
 
 GEMM_AUTO, GEMM_TILE256, GEMM_TILE128, GEMM_SKINNY, GEMM_GENERIC, GEMM_TILE256x128 = 0, 1, 2, 3, 4, 5
 GEMM_TILE256_RING, GEMM_TILE256_ONCE, GEMM_TILE256_STREAMK, GEMM_SKINNY_XSHARE = 6, 7, 8, 9
@@ -115,6 +118,24 @@ def lib() -> ctypes.CDLL:
                     fn.argtypes = args
                 _lib = handle
     return _lib
+
+
+_linear = None
+
+
+def linear_call():
+    """mi355_block_fp8_linear as a CPython function over integers (csrc/pycall.c): a quarter of the cost of the ctypes call."""
+    global _linear
+    if _linear is None:
+        lib()
+        if not os.path.exists(CALL_PATH):
+            raise Mi355Error(f"{CALL_PATH} is missing: build it with `python -m lightllm_amd.build`")
+        loader = importlib.machinery.ExtensionFileLoader("_mi355call", CALL_PATH)
+        spec = importlib.util.spec_from_file_location("_mi355call", CALL_PATH, loader=loader)
+        module = importlib.util.module_from_spec(spec)
+        loader.exec_module(module)
+        _linear = module.linear
+    return _linear
 
 
 def check(code: int, what: str) -> None:

@@ -1,12 +1,14 @@
-"""Compiles the HIP sources under csrc/ into lib/libmi355fp8.so for gfx950 with hipcc."""
+"""Compiles the HIP sources under csrc/ into lib/libmi355fp8.so for gfx950 with hipcc, and its CPython entry beside it."""
 import os
 import subprocess
 import sys
+import sysconfig
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 LIB_DIR = os.path.join(_HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libmi355fp8.so")
+CALL_PATH = os.path.join(LIB_DIR, "_mi355call.so")
 SOURCES = ["capi.hip", "group_quant.hip", "weight_quant.hip", "block_gemm.hip", "linear.hip", "moe_align.hip", "moe_elementwise.hip", "routed_ffn.hip", "probe.hip"]
 # packed-fp32 VALU ops are switched off for every kernel of this library
 FLAGS = [
@@ -47,6 +49,9 @@ def build(verbose: bool = False) -> str:
         raise RuntimeError("hipcc failed")
     cmd = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH] + objs
     subprocess.check_call(cmd)
+    # the CPython entry beside it, bound to the library by its path
+    subprocess.check_call(["gcc", "-O2", "-Wall", "-Wextra", "-shared", "-fPIC", "-I" + sysconfig.get_paths()["include"],
+                           os.path.join(CSRC, "pycall.c"), "-o", CALL_PATH, LIB_PATH, "-Wl,-rpath,$ORIGIN"])
     return LIB_PATH
 
 

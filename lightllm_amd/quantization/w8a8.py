@@ -134,15 +134,20 @@ class FP8w8a8B128Mi355QuantizationMethod(FP8w8a8B128QuantizationMethod):
             return None
         device = x.device
         alloc = self._alloc_func(use_custom_tensor_mananger)
-        if out is None:
-            out = alloc((m, n), dtype=dtype, device=device)
-        if out.shape != (m, n) or not out.is_cuda or not out.is_contiguous() or out.dtype not in (torch.bfloat16, torch.float16):
-            return None
+        if out is None and alloc is torch.empty:
+            out, out_dtype = x.new_empty((m, n)), dtype
+        else:
+            if out is None:
+                out = alloc((m, n), dtype=dtype, device=device)
+            out_dtype = out.dtype
+            if out.shape != (m, n) or not out.is_cuda or not out.is_contiguous() or out_dtype not in (torch.bfloat16, torch.float16):
+                return None
         x_ptr, w_ptr = x.data_ptr(), w.data_ptr()
         if (x_ptr | w_ptr) & 15:
             return None
         fused, ws_need = _linear_plan(m, n, k, dtype, device.index)
-        if fused and x_ptr < out.data_ptr() + 2 * m * n and out.data_ptr() < x_ptr + 2 * m * k:
+        out_ptr = out.data_ptr()
+        if fused and x_ptr < out_ptr + 2 * m * n and out_ptr < x_ptr + 2 * m * k:
             fused = False  # every workgroup of the stream reads all of x: one that is done must not store over it
         xq_ptr = xs_ptr = ws_ptr = None
         if not fused:
@@ -152,11 +157,13 @@ class FP8w8a8B128Mi355QuantizationMethod(FP8w8a8B128QuantizationMethod):
         stream = _lib.stream_ptr(device)
         if ws_need:
             ws_ptr = _lib.workspace(device, ws_need, stream).data_ptr()
-        code = _lib.lib().mi355_block_fp8_linear(
-            x_ptr, _lib.DTYPE_CODES[dtype], w_ptr, ws.data_ptr(), out.data_ptr(), m, n, k, k, ws.stride(0), ws.stride(1), n,
-            xq_ptr, xs_ptr, ws_ptr, ws_need, _lib.DTYPE_CODES[out.dtype], stream,
+        ws_n, ws_k = ws.stride()
+        code = _lib.linear_call()(
+            x_ptr, _lib.DTYPE_CODES[dtype], w_ptr, ws.data_ptr(), out_ptr, m, n, k, k, ws_n, ws_k, n,
+            xq_ptr, xs_ptr, ws_ptr, ws_need, _lib.DTYPE_CODES[out_dtype], stream,
         )
-        _lib.check(code, "fp8 linear")
+        if code:
+            _lib.check(code, "fp8 linear")
         return out
 
     @property

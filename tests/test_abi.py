@@ -372,3 +372,22 @@ def test_shape_table_off_256_compute_units(cus):
     # decode rows stream the weights on every count
     assert lib.mi355_block_fp8_gemm_plan(1, 28672, 4096, 1 << 34, cus) == _SKINNY
     assert lib.mi355_block_fp8_gemm_plan(8, 4096, 14336, 0, cus) in (_SKINNY, _T128, _CU)
+
+
+def test_linear_call_is_the_c_entry():
+    """The CPython entry of the one-call linear passes its integers (None: a null pointer) to the C entry as ctypes does and
+    refuses anything else."""
+    from lightllm_amd import _lib
+
+    lib, call = _lib.lib(), _lib.linear_call()
+    good = [64, 0, 64, 64, 64, 1, 128, 128, 128, 1, 1, 128, None, None, None, 0, 0, None]
+    for place, value in [(0, None), (2, None), (4, 0), (5, -1), (6, -5), (7, 100), (8, 64), (11, 127), (16, 1), (16, 7), (5, 0), (6, 0)]:
+        args = list(good)
+        args[place] = value
+        assert call(*args) == lib.mi355_block_fp8_linear(*args), (place, value)
+    assert call((1 << 64) - 64, 0, None, 64, 64, 1, 128, 128, 128, 1, 1, 128, None, None, None, 0, 0, None) == -1
+    for bad in (good[:-1], good + [0], [1.5] + good[1:], ["x"] + good[1:]):
+        with pytest.raises(TypeError):
+            call(*bad)
+    with pytest.raises(OverflowError):
+        call(1 << 64, *good[1:])
