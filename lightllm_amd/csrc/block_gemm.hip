@@ -323,6 +323,15 @@ static int launch_stream_mt(GemmArgs &a, const SkinnyPlan &pl, void *ws, hipStre
     }
 }
 
+// 65..128 rows (skinny_many_rows_plan)
+template <int MT>
+static int launch_stream_many_rows(GemmArgs &a, const SkinnyPlan &pl, void *ws, hipStream_t st) {
+    if constexpr (MT < 8) {
+        if (pl.tnw == 2) return launch_stream<MT, 2, 8>(a, pl, ws, st);
+    }
+    return launch_stream<MT, 1, 8>(a, pl, ws, st);
+}
+
 // ---- the weight stream cut into one equal share per compute unit (gemm_streamcu.hpp)
 template <int TNW, bool TURN>
 static int launch_streamcu_turn(GemmArgs &a, hipStream_t st) {
@@ -829,7 +838,9 @@ static int64_t n_split_rows(int64_t M, int64_t N, int64_t K, int cus);
 //     split of stream-K instead)                     the weight stream with the activation block in LDS
 //   129 <= M <= 208 (192), 0.55 cus .. cus tiles of
 //     160..256 or of 80..112 (64) weight rows         the same, workgroups of that width, K unshared
-//   65 <= M <= 128, K >= 2048                        the same with 256 weight rows per workgroup
+//   65 <= M <= 128, K >= 2048                        the same with 256 weight rows per workgroup; under the same name the
+//                                                    weight streaming kernel where one round of its tiles is ahead
+//                                                    (skinny_many_rows_plan)
 //   49 <= M <= 64, at most cus tiles, N*K >= 6e7,
 //     unless the streaming kernel is ahead
 //     (skinny_ahead_of_rows128)                       the same, unless the shared-activation kernel would run
@@ -930,6 +941,12 @@ static size_t workspace_bytes_for(int64_t M, int64_t N, int64_t K, int32_t varia
         if (n1 > 0) {
             const size_t rest = workspace_bytes_for(M, N - n1, K, MI355_GEMM_AUTO, cus);
             return rest > (size_t)MI355_WS_COUNTER_BYTES ? rest : (size_t)MI355_WS_COUNTER_BYTES;
+        }
+        if (variant == MI355_GEMM_ROWS128) {
+            // 65..128 rows may run as the weight stream, and where a limit of that is not met as the kernel of the name
+            const SkinnyPlan sp = skinny_many_rows_plan(M, N, K, cus);
+            const size_t stream = sp.tnw > 0 && sp.splits > 1 ? skinny_workspace(M, sp) : 0;
+            return std::max(stream, workspace_bytes_for(M, N, K, variant, cus));
         }
     }
     if (variant == MI355_GEMM_TILE256_STREAMK) {
@@ -1141,6 +1158,20 @@ static int block_fp8_gemm_impl(const void *A, const void *B, const float *As, co
         case MI355_GEMM_ROWS128: {
             if (!rows128_limits_ok(M, N, K, lda, as_m, as_k, cus)) return MI355_EUNSUPPORTED;
             if (rows128_two_tiles(M, N, K, cus)) return launch_rowsm(a, rowsm_plan(M, N, K, cus), st);
+            if (was_auto) {
+                // the shape table's choice only: a caller that asks for this kernel gets it
+                const SkinnyPlan sp = skinny_many_rows_plan(M, N, K, cus);
+                const bool fits = N * ldb_n < (1ll << 32) && M * as_m < (1ll << 32) &&
+                                  (sp.splits == 1 || (ws && ((uintptr_t)ws & 15) == 0 && ws_bytes >= skinny_workspace(M, sp)));
+                if (sp.tnw > 0 && fits) {
+                    switch (skinny_mt(M)) {
+                        case 5: return launch_stream_many_rows<5>(a, sp, ws, st);
+                        case 6: return launch_stream_many_rows<6>(a, sp, ws, st);
+                        case 7: return launch_stream_many_rows<7>(a, sp, ws, st);
+                        default: return launch_stream_many_rows<8>(a, sp, ws, st);
+                    }
+                }
+            }
             Rows128Plan pl = rows128_plan(M, N, K, cus);
             pl.turned = was_auto || M <= 64;
             if (pl.splits > 1 && (!ws || ws_bytes < rows128_workspace(M, N, K, cus) || ((uintptr_t)ws & 15)))

@@ -1,20 +1,20 @@
-// Block-scaled FP8 GEMM for decode-size M (<= 64) on gfx950: a weight-streaming kernel.
+// Block-scaled FP8 GEMM for decode-size M (<= 128) on gfx950: a weight-streaming kernel.
 //
 // At these sizes the GEMM is a single pass over the N x K weight bytes, so the kernel is built around the
 // memory system, not the MFMA: every wave issues plain 16-byte-per-lane global loads in which 8 consecutive
-// lanes cover one 128-byte row segment (fully coalesced), keeps 1-3 K-steps of them in flight in registers,
+// lanes cover one 128-byte row segment (fully coalesced), keeps one (from 17 rows on) to three K steps of them in flight in registers,
 // and only then rearranges the bytes into MFMA operand order through a small wave-private LDS area
 // (ds_write_b128 / ds_read_b128, no workgroup barrier in the loop).  Loads that target LDS directly
 // (global_load_lds) sustain visibly less HBM bandwidth than plain loads on this part, which is why the
 // streaming path does not use them.
 //
 // Work decomposition
-//   CTA = 4 waves, owns 16*TNW weight rows (n) and a contiguous range of K steps (cross-CTA split-K only when N
-//   alone gives too few CTAs; TNW is picked so that N / (16*TNW) is about the number of CUs).  Inside the CTA
+//   CTA = 4 or 8 waves (WV), owns 16*TNW weight rows (n) and a contiguous range of K steps (cross-CTA split-K only
+//   when N alone gives too few CTAs; stream_plan.hpp picks TNW, WV and the split).  Inside the CTA
 //   the waves take the K steps round-robin, so the four waves together read 512 consecutive bytes of every
 //   row; each wave multiplies all its rows (TNW MFMA row blocks) by all 16*MT token rows for its own K steps
 //   and folds the scales exactly like the tiled kernel
-//   (acc += partial * (Xs[m,kb] * Ws[nb,kb])).  After the loop the four partial accumulators are added
+//   (acc += partial * (Xs[m,kb] * Ws[nb,kb])).  After the loop the partial accumulators of the waves are added
 //   through LDS; with cross-CTA splits the sum goes to the workspace and the last CTA to arrive adds the
 //   splits in order (deterministic) before the bf16 store.
 //
@@ -59,6 +59,7 @@ struct XQuant {
 template <int MT, int TNW, int WV = kStreamWaves>
 struct StreamCfg {
     static_assert(TNW == 1 || TNW == 2 || TNW == 4 || TNW == 8, "a tile must sit inside one 128-row scale block");
+    static_assert(MT <= 8, "");
     static constexpr int BN = 16 * TNW;
     // K steps in flight per wave.  Occupancy counts for more than depth: from 17 rows on one step per wave and more
     // waves is ahead of two or three steps on every shape tried (N = 6144, K = 4096, M = 48, eight waves: 10.3 us at
@@ -69,7 +70,10 @@ struct StreamCfg {
         return set * 6 <= 150 ? 6 : (150 / set < 2 ? 2 : 150 / set);
     }
     static constexpr int kXOff = 16 * TNW * 128;                  // X block follows the W block
-    static constexpr int kWaveLds = (16 * TNW + 16 * MT) * 128;
+    // rows beyond 64 pass through the X block's place in a second turn, so that eight waves and the scales of up to 160
+    // steps fit beside it
+    static constexpr int XB = MT < 4 ? MT : 4;
+    static constexpr int kWaveLds = (16 * TNW + 16 * XB) * 128;
     static constexpr int kAccLds = TNW * MT * 1024;               // one wave's accumulators (fp32)
     static constexpr int kWaveBytes = kWaveLds > kAccLds ? kWaveLds : kAccLds;
     static constexpr int kLds = WV * kWaveBytes + 16;   // + the split-K arrival word
@@ -125,7 +129,7 @@ __global__ __launch_bounds__(64 * WV) void block_fp8_gemm_stream_kernel(const Ge
         kb_begin = (int)split * per + min((int)split, rem);
         kb_end = kb_begin + per + ((int)split < rem ? 1 : 0);
     }
-    // this wave's K steps: kb_begin + wave, + 4, ...
+    // this wave's K steps: kb_begin + wave, + WV, ...
     const int first = kb_begin + wave;
     const int steps = first < kb_end ? (kb_end - first + WV - 1) / WV : 0;
 
@@ -193,9 +197,10 @@ __global__ __launch_bounds__(64 * WV) void block_fp8_gemm_stream_kernel(const Ge
         const int rho = 16 * (rem >> 2) + 4 * a + (rem & 3);
         wst[i] = (uint32_t)rho * 128u + (((uint32_t)pch ^ swz((uint32_t)rho)) * 16u);
     }
-    uint32_t xst[2 * MT];
+    constexpr int XB = Cfg::XB;
+    uint32_t xst[2 * XB];
 #pragma unroll
-    for (int i = 0; i < 2 * MT; ++i) {
+    for (int i = 0; i < 2 * XB; ++i) {
         const int row = 8 * i + sub;
         xst[i] = (uint32_t)Cfg::kXOff + (uint32_t)row * 128u + (((uint32_t)pch ^ swz((uint32_t)row)) * 16u);
     }
@@ -223,9 +228,10 @@ __global__ __launch_bounds__(64 * WV) void block_fp8_gemm_stream_kernel(const Ge
             xsv[0] = xs_lds[r16];
         } else {
 #pragma unroll
-            for (int i = 0; i < 2 * MT; ++i) *(v4i *)(my + xst[i]) = r.x[i];
+            for (int i = 0; i < 2 * XB; ++i) *(v4i *)(my + xst[i]) = r.x[i];
         }
-        // LDS operations of one wave execute in order: the reads below see the writes above
+        // LDS operations of one wave execute in order: the reads below see the writes above, and the second turn's writes
+        // follow the first one's reads
         v8i wf[TNW];
 #pragma unroll
         for (int j = 0; j < TNW; ++j) {
@@ -235,8 +241,14 @@ __global__ __launch_bounds__(64 * WV) void block_fp8_gemm_stream_kernel(const Ge
         }
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
-            const v4i lo = *(const v4i *)(my + Cfg::kXOff + rd0 + t * 2048);
-            const v4i hi = *(const v4i *)(my + Cfg::kXOff + rd1 + t * 2048);
+            if constexpr (MT > XB) {
+                if (t == XB) {
+#pragma unroll
+                    for (int i = 0; i < 2 * (MT - XB); ++i) *(v4i *)(my + xst[i]) = r.x[2 * XB + i];
+                }
+            }
+            const v4i lo = *(const v4i *)(my + Cfg::kXOff + rd0 + (t % XB) * 2048);
+            const v4i hi = *(const v4i *)(my + Cfg::kXOff + rd1 + (t % XB) * 2048);
             const v8i xf = v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
             const float sc = xsv[t] * r.ws;
 #pragma unroll
@@ -273,7 +285,7 @@ __global__ __launch_bounds__(64 * WV) void block_fp8_gemm_stream_kernel(const Ge
         }
     }
 
-    // ---- add the four waves' accumulators; wave w ends up owning the MFMA blocks f = mt*TNW + tn with f % 4 == w
+    // ---- add the waves' accumulators; wave w ends up owning the MFMA blocks f = mt*TNW + tn with f % WV == w
     // (each wave first overwrites its own transposition area: LDS operations of a wave execute in order)
     constexpr int F = MT * TNW;
 #pragma unroll

@@ -44,7 +44,7 @@ struct SkinnyPlan {
 // workgroups a unit, us: N = K = 4096, M = 20 / 48 / 64 7.3 / 8.6 / 9.7 (8.9 / 10.0 / 10.1), 6144 x 4096 8.5 / 10.3 /
 // 11.6 (10.2 / 12.3 / 12.8), 4096 x 14336 14.5 / 17.3 / 19.5 (14.9 / 18.8 / 20.1), 28672 x 4096 21.5 / 24.9 (23.8 / 30.1).
 inline int64_t skinny_wide_lds(int waves, int tnw, int mt, int64_t steps) {
-    const int64_t wave = (16 * tnw + 16 * mt) * 128, acc = (int64_t)tnw * mt * 1024;
+    const int64_t wave = (16 * tnw + 16 * (mt < 4 ? mt : 4)) * 128, acc = (int64_t)tnw * mt * 1024;
     return waves * (wave > acc ? wave : acc) + 16 + steps * (16 * mt + 1) * 4;
 }
 
@@ -134,6 +134,38 @@ inline SkinnyPlan skinny_plan(int64_t M, int64_t N, int64_t K, int cus) {
     const int need = (KB + cap - 1) / cap;
     if (pl.splits < need && need <= max_splits) pl.splits = need;
     return pl;
+}
+
+// 65..128 rows: the same kernel on eight waves, one workgroup a unit in one round, against the weight stream with the
+// activation block in LDS, whose tiles are wide and share K over a second launch where N is narrow.  Both times are models in
+// ns, fitted to 38 (N, K) pairs (N = 512..28672, K = 1536..18432) at M = 65..128: this kernel's by what a workgroup does
+// (234 points, 4 % rms), the other's by its rows and the weights' size (158 points, 6 % rms).  What is taken is 0.4 % behind
+// the better of all candidates on average.  us, M = 72 / 96 / 128, before in brackets: N = K = 4096 11.3 / 12.4 / 14.6 (15.6
+// / 17.0 / 18.7), 6144 x 4096 13.0 / 14.6 (16.0 / 17.1), 7168 x 2048 9.0 / 10.1 (15.2 / 16.6), 2112 x 7168 12.0 / 13.5 (16.0 /
+// 17.2), M = 128 there stays.  32 weight rows stop at 112: with eight row blocks the accumulators spill (6144 x 4096, M =
+// 128: 25.9 against 18.4).  tnw 0: not here.
+inline SkinnyPlan skinny_many_rows_plan(int64_t M, int64_t N, int64_t K, int cus) {
+    SkinnyPlan best = {0, 1, 0, 8};
+    if (M <= 64 || M > 128 || K % kBlockK != 0 || K / kBlockK < 16) return best;
+    const int64_t mt = (M + 15) / 16, KB = K / kBlockK;
+    const int64_t weights = (N * K + 999999) / 1000000;  // MB
+    const int64_t alternative = 8228 + 713 * mt + weights * (902 + 109 * mt) / 10 + 19 * KB;
+    int64_t best_cost = alternative - alternative / 33;
+    for (int tnw = 1; tnw <= (mt < 8 ? 2 : 1); ++tnw) {
+        const int64_t tiles = (N + 16 * tnw - 1) / (16 * tnw), cap = skinny_wide_cap(8, tnw, (int)mt);
+        for (int s = 1; s <= 8; ++s) {
+            const int64_t steps = (KB + s - 1) / s;
+            if (tiles * s > cus || KB / s < 8) break;
+            if (steps > cap) continue;
+            const int64_t cost = 3433 + 264 * mt + steps * (145 * tnw + 220 * mt + 68 * mt * tnw) / 10 +
+                                 124 * ((steps + 7) / 8) + (s > 1 ? 1764 + 169 * s : 0) + weights * 56;
+            if (cost < best_cost) {
+                best = {tnw, s, (int)tiles, 8};
+                best_cost = cost;
+            }
+        }
+    }
+    return best;
 }
 
 inline size_t skinny_workspace(int64_t M, const SkinnyPlan &pl) {
