@@ -118,17 +118,21 @@ int mi355_block_weight_quant_fp8(const void *w, int32_t w_dtype, void *q, float 
                                         compute units (partial tiles added up through the workspace, in K order:
                                         deterministic); falls back to MI355_GEMM_TILE256 where sharing gains nothing */
 
-#define MI355_GEMM_SKINNY_XSHARE 9 /* weight streaming, M <= 64, the activation block of a K step shared by the workgroup */
+#define MI355_GEMM_SKINNY_XSHARE 9 /* weight streaming, 33 <= M <= 64, the activation block of a K step shared by the
+                                     workgroup; the shape table takes it from 49 rows on */
 #define MI355_GEMM_ROWS128 10 /* weight streaming, M <= 384, the activation block of a K step in LDS: 256 weight rows per
-                                 workgroup up to 128 rows, 128 beyond; a second launch adds the partial sums when K is shared */
+                                 workgroup up to 128 rows, 128 beyond; a second launch adds the partial sums when K is shared;
+                                 209..352 rows on a wide N run as two tiles over M.  Where the shape table picks it for
+                                 65..128 rows it runs the kernel of MI355_GEMM_SKINNY if one round of that is ahead */
 
 #define MI355_GEMM_SKINNY_CU 11 /* weight streaming, M <= 16: the weight rows cut into one equal share per compute unit,
                                   one workgroup of 8 waves per share and the whole K (no partial sums between
-                                  workgroups); where N / 16 gives the units 1..8 row blocks each */
+                                  workgroups); where N / 16 gives the units 1..5 row blocks each */
 
 #define MI355_GEMM_ROWS_MTILED 12 /* the kernel of MI355_GEMM_ROWS128 tiled over M as well: one round of tiles of
                                      16..128 rows x 160..256 weight rows, K unshared, no workspace; for more than 384
-                                     rows on a narrow N (at most 5120 weight rows, K <= 7168) */
+                                     rows on a narrow N (at most 5120 weight rows, K <= 7168; 385..960 rows: at most 15360,
+                                     K <= 5120) */
 
 #define MI355_WS_COUNTER_BYTES 65536
 
