@@ -143,10 +143,11 @@ inline SkinnyPlan skinny_plan(int64_t M, int64_t N, int64_t K, int cus) {
 // the better of all candidates on average.  us, M = 72 / 96 / 128, before in brackets: N = K = 4096 11.3 / 12.4 / 14.6 (15.6
 // / 17.0 / 18.7), 6144 x 4096 13.0 / 14.6 (16.0 / 17.1), 7168 x 2048 9.0 / 10.1 (15.2 / 16.6), 2112 x 7168 12.0 / 13.5 (16.0 /
 // 17.2), M = 128 there stays.  32 weight rows stop at 112: with eight row blocks the accumulators spill (6144 x 4096, M =
-// 128: 25.9 against 18.4).  tnw 0: not here.
+// 128: 25.9 against 18.4).  Up to 512 weight rows the other kernel's sums are on record although this one is ahead (512 x
+// 7168, M = 80 / 128: 9.0 / 10.8 against 11.9 / 13.6).  tnw 0: not here.
 inline SkinnyPlan skinny_many_rows_plan(int64_t M, int64_t N, int64_t K, int cus) {
     SkinnyPlan best = {0, 1, 0, 8};
-    if (M <= 64 || M > 128 || K % kBlockK != 0 || K / kBlockK < 16) return best;
+    if (M <= 64 || M > 128 || N <= 512 || K % kBlockK != 0 || K / kBlockK < 16) return best;
     const int64_t mt = (M + 15) / 16, KB = K / kBlockK;
     const int64_t weights = (N * K + 999999) / 1000000;  // MB
     const int64_t alternative = 8228 + 713 * mt + weights * (902 + 109 * mt) / 10 + 19 * KB;

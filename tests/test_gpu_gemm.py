@@ -346,11 +346,11 @@ def test_stream_17_to_64_rows(hip, M, N, K):
 
 
 # the table's choice at the edges of the 5 to 8 row-block forms of the stream: tiles of 16 and 32 weight rows, K whole and
-# shared by 2 to 8 workgroups, turned starts (K a multiple of 4096) and plain ones, ragged shares, N of one row and ragged
-# tiles, and beside them shapes that stay with the activation block in LDS (N = 2112 and 8190 from 113 rows on)
+# shared by 2 to 7 workgroups, turned starts (K a multiple of 4096) and plain ones, ragged shares, ragged tiles down to one
+# row, and beside them shapes that stay with the activation block in LDS (N = 2112 and 8190 from 113 rows on, N = 512)
 @pytest.mark.parametrize("M", [65, 80, 81, 96, 97, 112, 113, 128])
-@pytest.mark.parametrize("N,K", [(4096, 4096), (4090, 4096), (7168, 2048), (2112, 7168), (1000, 4096), (2048, 8192), (1, 2048),
-                                 (40, 20608), (8190, 4096), (136, 36864), (2000, 2176)])
+@pytest.mark.parametrize("N,K", [(4096, 4096), (4090, 4096), (7168, 2048), (2112, 7168), (1000, 4096), (2048, 8192), (513, 2048),
+                                 (520, 20608), (8190, 4096), (528, 36864), (2000, 2176), (512, 2048)])
 def test_stream_65_to_128_rows(hip, M, N, K):
     print(f"gemm stream M={M} N={N} K={K}", flush=True)
     xq, xs, wq, ws = _prep(M, N, K, seed=N + K + M, device="cuda")
