@@ -9,7 +9,8 @@ import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libmi355fp8.so")
-CALL_PATH = os.path.join(_HERE, "lib", "_mi355call.so")
+# one file per CPython version: the entry is built against the interpreter's own headers
+CALL_PATH = os.path.join(_HERE, "lib", "_mi355call" + importlib.machinery.EXTENSION_SUFFIXES[0])
 
 GEMM_AUTO, GEMM_TILE256, GEMM_TILE128, GEMM_SKINNY, GEMM_GENERIC, GEMM_TILE256x128 = 0, 1, 2, 3, 4, 5
 GEMM_TILE256_RING, GEMM_TILE256_ONCE, GEMM_TILE256_STREAMK, GEMM_SKINNY_XSHARE = 6, 7, 8, 9
@@ -124,17 +125,19 @@ _linear = None
 
 
 def linear_call():
-    """mi355_block_fp8_linear as a CPython function over integers (csrc/pycall.c): a quarter of the cost of the ctypes call."""
+    """mi355_block_fp8_linear over integers: as a CPython function (csrc/pycall.c, a quarter of the cost of the ctypes call), or
+    as the ctypes function where that entry was not built for this interpreter.  Either way the entry of the library above."""
     global _linear
     if _linear is None:
-        lib()
+        entry = lib().mi355_block_fp8_linear
         if not os.path.exists(CALL_PATH):
-            raise Mi355Error(f"{CALL_PATH} is missing: build it with `python -m lightllm_amd.build`")
-        loader = importlib.machinery.ExtensionFileLoader("_mi355call", CALL_PATH)
-        spec = importlib.util.spec_from_file_location("_mi355call", CALL_PATH, loader=loader)
-        module = importlib.util.module_from_spec(spec)
-        loader.exec_module(module)
-        _linear = module.linear
+            _linear = entry
+        else:
+            loader = importlib.machinery.ExtensionFileLoader("_mi355call", CALL_PATH)
+            spec = importlib.util.spec_from_file_location("_mi355call", CALL_PATH, loader=loader)
+            module = importlib.util.module_from_spec(spec)
+            loader.exec_module(module)
+            _linear = module.linear_at(ctypes.cast(entry, _vp).value)
     return _linear
 
 

@@ -1,5 +1,7 @@
 """Compiles the HIP sources under csrc/ into lib/libmi355fp8.so for gfx950 with hipcc, and its CPython entry beside it."""
+import importlib.machinery
 import os
+import shutil
 import subprocess
 import sys
 import sysconfig
@@ -8,7 +10,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 LIB_DIR = os.path.join(_HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libmi355fp8.so")
-CALL_PATH = os.path.join(LIB_DIR, "_mi355call.so")
+CALL_PATH = os.path.join(LIB_DIR, "_mi355call" + importlib.machinery.EXTENSION_SUFFIXES[0])
 SOURCES = ["capi.hip", "group_quant.hip", "weight_quant.hip", "block_gemm.hip", "linear.hip", "moe_align.hip", "moe_elementwise.hip", "routed_ffn.hip", "probe.hip"]
 # packed-fp32 VALU ops are switched off for every kernel of this library
 FLAGS = [
@@ -49,10 +51,24 @@ def build(verbose: bool = False) -> str:
         raise RuntimeError("hipcc failed")
     cmd = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH] + objs
     subprocess.check_call(cmd)
-    # the CPython entry beside it, bound to the library by its path
-    subprocess.check_call(["gcc", "-O2", "-Wall", "-Wextra", "-shared", "-fPIC", "-I" + sysconfig.get_paths()["include"],
-                           os.path.join(CSRC, "pycall.c"), "-o", CALL_PATH, LIB_PATH, "-Wl,-rpath,$ORIGIN"])
+    _build_call(verbose)
     return LIB_PATH
+
+
+def _build_call(verbose: bool) -> None:
+    """The CPython entry.  It is linked against nothing (it gets the address of the C entry), and where the interpreter's headers or
+    a C compiler are missing it is left out: the package calls through ctypes then."""
+    if os.path.exists(CALL_PATH):
+        os.remove(CALL_PATH)
+    include = sysconfig.get_paths()["include"]
+    cc = next((c for c in (os.environ.get("CC"), "gcc", "cc", "clang") if c and shutil.which(c.split()[0])), None)
+    if cc is None or not os.path.exists(os.path.join(include, "Python.h")):
+        print(f"[build] no {'C compiler' if cc is None else 'Python.h'}: the one-call linear goes through ctypes", file=sys.stderr)
+        return
+    cmd = cc.split() + ["-O2", "-Wall", "-Wextra", "-shared", "-fPIC", "-I" + include, os.path.join(CSRC, "pycall.c"), "-o", CALL_PATH]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    subprocess.check_call(cmd)
 
 
 if __name__ == "__main__":

@@ -391,3 +391,33 @@ def test_linear_call_is_the_c_entry():
             call(*bad)
     with pytest.raises(OverflowError):
         call(1 << 64, *good[1:])
+
+
+@pytest.mark.parametrize("with_entry", [True, False])
+def test_linear_call_of_a_copied_package(tmp_path, with_entry):
+    """A built package that was copied elsewhere calls the linear of its own library, the only one that is mapped; without
+    the CPython entry beside it (not built for this interpreter) it does so through ctypes."""
+    import shutil
+    import subprocess
+    import sys
+
+    from lightllm_amd import _lib
+
+    if with_entry and not os.path.exists(_lib.CALL_PATH):
+        pytest.skip("the CPython entry is not built for this interpreter")
+    skip = shutil.ignore_patterns("obj", "csrc", "__pycache__", *([] if with_entry else ["_mi355call*"]))
+    shutil.copytree(os.path.join(ROOT, "lightllm_amd"), tmp_path / "lightllm_amd", ignore=skip)
+    code = """
+from lightllm_amd import _lib
+call = _lib.linear_call()
+args = [64, 0, 64, 64, 64, 1, 128, 128, 64, 1, 1, 128, None, None, None, 0, 0, None]
+print(call(*args) == _lib.lib().mi355_block_fp8_linear(*args) == -2)
+for name in sorted({line.split()[-1] for line in open("/proc/self/maps") if "mi355" in line}):
+    print(name)
+"""
+    run = subprocess.run([sys.executable, "-c", code], cwd=tmp_path, capture_output=True, text=True, timeout=300,
+                         env={**os.environ, "PYTHONPATH": str(tmp_path)})
+    assert run.returncode == 0, run.stderr[-2000:]
+    lib_dir = str(tmp_path / "lightllm_amd" / "lib")
+    want = [os.path.join(lib_dir, os.path.basename(p)) for p in ([_lib.CALL_PATH] if with_entry else []) + [_lib.LIB_PATH]]
+    assert run.stdout.split("\n")[:-1] == ["True"] + want
