@@ -291,7 +291,11 @@ static int launch_stream(GemmArgs &a, const SkinnyPlan &pl, void *ws, hipStream_
         return a.turn_mask ? launch_stream_as<MT, TNW, true, true, WV>(a, pl, ws, lds_bytes, st)
                            : launch_stream_as<MT, TNW, true, false, WV>(a, pl, ws, lds_bytes, st);
     }
-    if constexpr (MT == 1) return launch_stream_as<MT, TNW, false, false, WV>(a, pl, ws, Cfg::kLds, st);
+    if constexpr (MT == 1) {
+        // (up to 8 rows the quantizing stream runs the same K order, linear.hip: the linear has the bits of quantizer + GEMM)
+        return a.turn_mask ? launch_stream_as<MT, TNW, false, true, WV>(a, pl, ws, Cfg::kLds, st)
+                           : launch_stream_as<MT, TNW, false, false, WV>(a, pl, ws, Cfg::kLds, st);
+    }
     return MI355_EUNSUPPORTED;
 }
 

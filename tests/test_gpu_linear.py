@@ -46,6 +46,27 @@ def test_quantized_in_the_stream(hip, N, K, dtype):
         assert not torch.isnan(out[: max(M - 1, 1)]).any()
 
 
+# 64-row tiles with K whole over more steps than the stream stages activation scales for, K a multiple of 4096: the starts of
+# the tiles are turned, in the quantizing stream and behind the quantizer alike
+@pytest.mark.parametrize("M,N,K", [(1, 16384, 12288), (4, 16384, 12288), (3, 16380, 16384)])
+def test_quantized_in_the_stream_on_a_long_k(hip, M, N, K):
+    from lightllm_amd import _lib
+    from lightllm_amd.quantization import QUANTMETHODS, WeightPack
+
+    print(f"linear M={M} N={N} K={K}", flush=True)
+    assert hip.mi355_block_fp8_linear_fused(M, N, K, _lib.DTYPE_CODES[torch.bfloat16]) == 1
+    assert hip.mi355_block_fp8_gemm_variant(M, N, K) == _lib.GEMM_SKINNY
+    wq, ws = H.quantized_weights(N, K, seed=N + K, device="cuda")
+    x = H.activations(M, K, seed=M, outliers=True).cuda()
+    method, want = QUANTMETHODS.get("fp8w8a8-b128"), _composed(x, wq, ws, torch.bfloat16)
+    assert torch.equal(method.apply(x, WeightPack(wq, ws)), want)
+    # an output over the activations takes the two launches
+    buf = torch.zeros(M * max(N, K), dtype=torch.bfloat16, device="cuda")
+    mine = buf[: M * K].view(M, K).copy_(x)
+    out = buf[: M * N].view(M, N)
+    assert torch.equal(method.apply(mine, WeightPack(wq, ws), out=out), want)
+
+
 def test_output_argument_and_odd_operands(hip):
     """A caller's output tensor is filled and returned; activations that are not 16-byte aligned, a strided weight scale
     and fp32 outputs keep the behaviour of the step-by-step path."""
