@@ -161,7 +161,7 @@ __global__ __launch_bounds__(64 * WV) void block_fp8_gemm_stream_kernel(const Ge
         for (int a = 0; a < kSvRows; ++a)
 #pragma unroll
             for (int b = 0; b < kSvSteps; ++b) {
-                if (32 * b >= steps_cta && b > 0) continue;
+                if (kSvSteps > 2 && b > 0 && 32 * b >= steps_cta) continue;  // (eight waves: up to 160 steps)
                 const int m = min(kSvPass * a + (tid >> 5), p.M - 1);
                 const int kb = min(kb_begin + min(32 * b + (tid & 31), max(steps_cta - 1, 0)), KB - 1);
                 sv[a * kSvSteps + b] = p.Xs[(int64_t)m * p.xs_m + (int64_t)kb * p.xs_k];
