@@ -403,6 +403,11 @@ static int launch_xshare(GemmArgs &a, int splits, void *ws, hipStream_t st) {
     const int lds_bytes = XshareCfg::kLds + XshareCfg::scale_lds_bytes(steps);
     const int tiles = (a.N + XshareCfg::BN - 1) / XshareCfg::BN;
     a.turn_mask = splits > 1 ? 0 : stream_turn_mask(a.K, KB);
+    if (a.turn_mask) {
+        constexpr auto kernel = block_fp8_gemm_xshare_kernel<4, 2, kXshareDepth, false, true>;
+        if (!allow_lds<kernel>(max_lds)) return MI355_ELAUNCH;
+        return launch(kernel, dim3(tiles), dim3(256), lds_bytes, st, a);
+    }
     if (splits <= 1) {
         constexpr auto kernel = block_fp8_gemm_xshare_kernel<4, 2, kXshareDepth, false>;
         if (!allow_lds<kernel>(max_lds)) return MI355_ELAUNCH;

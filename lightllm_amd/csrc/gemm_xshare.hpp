@@ -41,7 +41,8 @@ struct ShareCfg {
     static constexpr int scale_lds_bytes(int steps) { return steps * kScaleStride * 4; }
 };
 
-template <int MT, int TNW, int DEPTH, bool SPLIT>
+// TURN: the tiles start at different K steps (GemmArgs::turn_mask).
+template <int MT, int TNW, int DEPTH, bool SPLIT, bool TURN = false>
 __global__ __launch_bounds__(256) void block_fp8_gemm_xshare_kernel(const GemmArgs p) {
     using Cfg = ShareCfg<MT, TNW, DEPTH>;
     constexpr int D = DEPTH, NX = Cfg::NX, BN = Cfg::BN;
@@ -95,7 +96,6 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_xshare_kernel(const GemmAr
     for (int a = 0; a < kSvRows; ++a)
 #pragma unroll
         for (int b = 0; b < kSvSteps; ++b) {
-            if (b > 0 && 32 * b >= steps) continue;
             const int m = min(8 * a + (tid >> 5), p.M - 1);
             const int kb = kb_begin + min(32 * b + (tid & 31), max(steps - 1, 0));
             sv[a * kSvSteps + b] = p.Xs[(int64_t)m * p.xs_m + (int64_t)kb * p.xs_k];
@@ -107,8 +107,8 @@ __global__ __launch_bounds__(256) void block_fp8_gemm_xshare_kernel(const GemmAr
         float ws;
     };
     // step `it` of this workgroup in K order, counted from where its tile starts (GemmArgs::turn_mask)
-    const int rot = (int)((5u * tile_n) & (uint32_t)p.turn_mask);
-    auto turn = [&](int it) -> int { return it + rot >= steps ? it + rot - steps : it + rot; };
+    const int rot = TURN ? (int)((5u * tile_n) & (uint32_t)p.turn_mask) : 0;
+    auto turn = [&](int it) -> int { return TURN && it + rot >= steps ? it + rot - steps : it + rot; };
     auto load = [&](Regs &r, int it) {
         const int kb = kb_begin + turn(it);
         const uint8_t *wk = p.W + (int64_t)kb * kBlockK;
