@@ -640,15 +640,20 @@ static int launch_rows128_as(GemmArgs &a, const Rows128Plan &pl, void *ws, hipSt
     const int lds_bytes = Cfg::lds_bytes(steps);
     if (lds_bytes > 160 * 1024) return MI355_EUNSUPPORTED;
     if (pl.splits <= 1) {
-        // Turned starts (stream_turn_mask) where a step is mostly weights: up to 96 rows, or weights of 200 MB and more (us,
-        // in step / turned: N = 28672, K = 4096, M = 64 / 80 / 128 29.2 / 30.5 / 36.2 against 26.3 / 28.2 / 37.3; 57344 x
-        // 8192, M = 64 / 128 / 160 115 / 122 / 119 against 85 / 97 / 108; 12288 x 4096, M = 160 31.8 against 33.1).  Tiles over
-        // M share their activation rows in the L2 step by step and lose that (K = 8192: 2 to 6 %).  The two buffers of scale
-        // chunks want a multiple of 16 steps.  From 65 rows on, where the square tiles run as well, a launch asked for by
-        // name keeps K order: its sums are then theirs bit for bit.
+        // Turned starts (stream_turn_mask) where a step is mostly weights: up to 96 rows (80 beyond K = 16384), or weights of
+        // 200 MB and more (450 at K = 16384) (us, in step / turned: N = 28672, K = 4096, M = 64 / 80 / 128 29.2 / 30.5 / 36.2
+        // against 26.3 / 28.2 / 37.3; 57344 x 8192, M = 64 / 128 / 160 115 / 122 / 119 against 85 / 97 / 108; 36864 x 20480, M =
+        // 128 172 / 180; 22656 x 16384, M = 128 124 / 128; 12288 x 4096, M = 160 31.8 / 33.1).  Not with narrow workgroups on K =
+        // 8192: tile t's rows then start 5 t or 6 t times 2^18 bytes on, its steps 5 t times 128, and the two meet again on the
+        // same channels (32768 x 8192, M = 64 63.3 / 82.1; 24576: 50.6 / 60.6; with 256 weight rows 45056: 1.18 times ahead).
+        // Tiles over M share their activation rows in the L2 step by step and lose that (K = 8192: 2 to 6 %).  The two buffers
+        // of scale chunks want a multiple of 16 steps.  From 65 rows on, where the square tiles run as well, a launch asked for
+        // by name keeps K order: its sums are then theirs bit for bit.
         if constexpr (MT <= 10 && TN == 2) {
-            const bool weights_lead = a.M <= 96 || (int64_t)a.N * a.K >= 200000000ll;
-            if (pl.turned && weights_lead && a.tiles_m <= 1 && KB % 16 == 0 && (a.turn_mask = stream_turn_mask(a.K, KB)) != 0) {
+            const int64_t weights = (int64_t)a.N * a.K;
+            const bool weights_lead = a.M <= (a.K <= 16384 ? 96 : 80) || (a.K <= 16384 && weights >= (a.K < 16384 ? 200000000ll : 450000000ll));
+            const bool meets = WV < 8 && a.K == 8192;
+            if (pl.turned && weights_lead && !meets && a.tiles_m <= 1 && KB % 16 == 0 && (a.turn_mask = stream_turn_mask(a.K, KB)) != 0) {
                 constexpr auto turned = block_fp8_gemm_rows128_kernel<MT, NS, TN, WV, false, true>;
                 if (!allow_lds<turned>(160 * 1024)) return MI355_ELAUNCH;
                 return launch(turned, dim3(pl.tiles), dim3(Cfg::kThreads), lds_bytes, st, a);
