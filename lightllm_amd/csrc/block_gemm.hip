@@ -265,37 +265,42 @@ template <int MT, int TNW, bool XSL, bool TURN, int WV>
 static int launch_stream_as(GemmArgs &a, const SkinnyPlan &pl, void *ws, int lds_bytes, hipStream_t st) {
     using Cfg = StreamCfg<MT, TNW, WV>;
     constexpr int max_lds = Cfg::kLds + (XSL ? Cfg::scale_lds_bytes(Cfg::kMaxScaleSteps) : 0);
-    constexpr auto whole_k = block_fp8_gemm_stream_kernel<MT, TNW, false, XSL, 0, false, WV, TURN>;
-    constexpr auto split_k = block_fp8_gemm_stream_kernel<MT, TNW, true, XSL, 0, false, WV, TURN>;
     if (pl.splits <= 1) {
+        constexpr auto whole_k = block_fp8_gemm_stream_kernel<MT, TNW, false, XSL, 0, false, WV, TURN>;
         if (!allow_lds<whole_k>(max_lds)) return MI355_ELAUNCH;
         return launch(whole_k, dim3(pl.tiles), dim3(64 * WV), lds_bytes, st, a);
     }
-    if (!allow_lds<split_k>(max_lds)) return MI355_ELAUNCH;
-    a.splits = pl.splits;
-    a.counters = (uint32_t *)ws;
-    a.partials = (float *)((uint8_t *)ws + MI355_WS_COUNTER_BYTES);
-    return launch(split_k, dim3(pl.tiles * pl.splits), dim3(64 * WV), lds_bytes, st, a);
+    if constexpr (MT == 1 || XSL) {
+        constexpr auto split_k = block_fp8_gemm_stream_kernel<MT, TNW, true, XSL, 0, false, WV, TURN>;
+        if (!allow_lds<split_k>(max_lds)) return MI355_ELAUNCH;
+        a.splits = pl.splits;
+        a.counters = (uint32_t *)ws;
+        a.partials = (float *)((uint8_t *)ws + MI355_WS_COUNTER_BYTES);
+        return launch(split_k, dim3(pl.tiles * pl.splits), dim3(64 * WV), lds_bytes, st, a);
+    }
+    return MI355_EUNSUPPORTED;
+}
+
+template <int MT, int TNW, bool XSL, int WV>
+static int launch_stream_form(GemmArgs &a, const SkinnyPlan &pl, void *ws, int lds_bytes, hipStream_t st) {
+    return a.turn_mask ? launch_stream_as<MT, TNW, XSL, true, WV>(a, pl, ws, lds_bytes, st)
+                       : launch_stream_as<MT, TNW, XSL, false, WV>(a, pl, ws, lds_bytes, st);
 }
 
 // The activation scales of a CTA's K range are staged in LDS when the range is short enough for the staging area; from 17
-// rows on the plan only has such ranges.
+// rows on the plan says so, and only 64-row tiles on four waves run without.  Up to 8 rows the quantizing stream (linear.hip)
+// runs the same K order, so that the linear has the bits of quantizer + GEMM.
 template <int MT, int TNW, int WV = kStreamWaves>
 static int launch_stream(GemmArgs &a, const SkinnyPlan &pl, void *ws, hipStream_t st) {
     using Cfg = StreamCfg<MT, TNW, WV>;
     const int KB = a.K / kBlockK;
     const int steps = (KB + pl.splits - 1) / pl.splits;
     a.turn_mask = stream_turn_mask(a.K, KB / pl.splits);
-    if (steps <= Cfg::kMaxScaleSteps) {
+    if (pl.staged && steps <= Cfg::kMaxScaleSteps) {
         const int lds_bytes = Cfg::kLds + Cfg::scale_lds_bytes(steps);
-        return a.turn_mask ? launch_stream_as<MT, TNW, true, true, WV>(a, pl, ws, lds_bytes, st)
-                           : launch_stream_as<MT, TNW, true, false, WV>(a, pl, ws, lds_bytes, st);
+        return launch_stream_form<MT, TNW, true, WV>(a, pl, ws, lds_bytes, st);
     }
-    if constexpr (MT == 1) {
-        // (up to 8 rows the quantizing stream runs the same K order, linear.hip: the linear has the bits of quantizer + GEMM)
-        return a.turn_mask ? launch_stream_as<MT, TNW, false, true, WV>(a, pl, ws, Cfg::kLds, st)
-                           : launch_stream_as<MT, TNW, false, false, WV>(a, pl, ws, Cfg::kLds, st);
-    }
+    if constexpr (MT == 1 || (MT <= 4 && TNW == 4 && WV == 4)) return launch_stream_form<MT, TNW, false, WV>(a, pl, ws, Cfg::kLds, st);
     return MI355_EUNSUPPORTED;
 }
 
@@ -1229,8 +1234,9 @@ static int block_fp8_gemm_impl(const void *A, const void *B, const float *As, co
         }
         case MI355_GEMM_SKINNY: {
             const int ok = skinny_check(M, N, K, lda, ldb_n, as_m, cus, ws && ((uintptr_t)ws & 15) == 0, ws_bytes);
-            if (ok != MI355_OK) return ok;
-            const SkinnyPlan pl = skinny_plan(M, N, K, cus);
+            const bool whole = ok == MI355_EWORKSPACE && skinny_runs_whole(M, N, K, cus);  // (AUTO does not come here then)
+            if (ok != MI355_OK && !whole) return ok;
+            const SkinnyPlan pl = whole ? skinny_whole_plan(N) : skinny_plan(M, N, K, cus);
             switch (skinny_mt(M)) {
                 case 1: return launch_stream_mt<1>(a, pl, ws, st);
                 case 2: return launch_stream_mt<2>(a, pl, ws, st);
@@ -1301,7 +1307,9 @@ extern "C" int mi355_block_fp8_gemm_noalloc(const void *A, const void *B, const 
     const size_t need = mi355_block_fp8_gemm_workspace_bytes(M, N, K, variant);
     // a forced kernel that needs more than the array holds is an error; the shape table (MI355_GEMM_AUTO) gets
     // the whole array and takes the next best plan that fits into it
-    if (need > kScratchBytes && variant != MI355_GEMM_AUTO) return MI355_ESCRATCH;
+    if (need > kScratchBytes && variant != MI355_GEMM_AUTO &&
+        !(variant == MI355_GEMM_SKINNY && skinny_runs_whole(M, N, K, device_cus())))
+        return MI355_ESCRATCH;
     void *ws = nullptr;
     if (need > 0) {
         ws = scratch_ptr();

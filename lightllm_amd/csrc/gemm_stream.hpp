@@ -65,7 +65,7 @@ struct StreamCfg {
     // waves is ahead of two or three steps on every shape tried (N = 6144, K = 4096, M = 48, eight waves: 10.3 us at
     // depth 1, 11.0 at 2, 14.5 at 4; M <= 16 best at depth 3).
     static constexpr int depth(bool xs_in_lds) {
-        if (xs_in_lds) return MT == 1 ? 3 : 1;
+        if (xs_in_lds || MT > 1) return MT == 1 ? 3 : 1;
         const int set = 8 * TNW + 9 * MT + 1;  // registers of one in-flight K step
         return set * 6 <= 150 ? 6 : (150 / set < 2 ? 2 : 150 / set);
     }
@@ -101,7 +101,6 @@ struct StreamRegs {
 template <int MT, int TNW, bool SPLIT, bool XSL, int XR = 0, bool F16 = false, int WV = kStreamWaves, bool TURN = false>
 __global__ __launch_bounds__(64 * WV) void block_fp8_gemm_stream_kernel(const GemmArgs p) {
     static_assert(XR == 0 || (MT == 1 && !XSL), "unquantized activations: at most 16 rows, no staged scales");
-    static_assert(MT == 1 || XSL, "the plan keeps K ranges within the staged scales from 17 rows on");
     using Cfg = StreamCfg<MT, TNW, WV>;
     constexpr int NX = XR ? XR : 2 * MT;
     using Regs = StreamRegs<MT, TNW, NX>;

@@ -32,7 +32,17 @@ inline int skinny_mt(int64_t M) { return M <= 16 ? 1 : (int)((M + 15) / 16); }
 struct SkinnyPlan {
     int tnw, splits, tiles;
     int waves;
+    bool staged = true;  // from 17 rows on: the activation scales of a workgroup's K range are staged in LDS
 };
+
+// K whole without a workspace and for any K: 64-row tiles on four waves, the scales gathered step by step.
+inline SkinnyPlan skinny_whole_plan(int64_t N) { return {4, 1, (int)((N + 63) / 64), 4, false}; }
+
+// Where a caller's own choice of the streaming kernel runs so if the workspace of its plan is missing: N alone gives the units
+// work, or K is too short to gain from being shared.
+inline bool skinny_runs_whole(int64_t M, int64_t N, int64_t K, int cus) {
+    return M > 16 && M <= 64 && ((N + 31) / 32 * 2 >= 3 * (int64_t)cus || K / kBlockK < 32);
+}
 
 // 17..64 rows: four or eight waves a workgroup, tiles of 16, 32 or 64 weight rows, K whole or shared by up to eight
 // workgroups.  A wave has one K step in flight and the waves hide each other's latency, so what a launch takes is what
@@ -83,10 +93,9 @@ inline SkinnyPlan skinny_wide_plan(int64_t M, int64_t N, int64_t K, int cus) {
                 }
             }
         }
-    if (best.tnw == 0) {  // a K range too long for eight shares
-        const int64_t cap = skinny_wide_cap(8, 1, mt);
-        best = {1, (int)((KB + cap - 1) / cap), (int)((N + 15) / 16), 8};
-    }
+    // a K range too long for the staged forms, on more tiles than share it: N = 72704, K = 21376, M = 39 335 us (366 with a second
+    // K step in flight, 551 with K shared by two)
+    if (best.tnw == 0) return skinny_whole_plan(N);
     return best;
 }
 

@@ -374,6 +374,28 @@ def test_shape_table_off_256_compute_units(cus):
     assert lib.mi355_block_fp8_gemm_plan(8, 4096, 14336, 0, cus) in (_SKINNY, _T128, _CU)
 
 
+def test_streaming_kernel_by_name_without_a_workspace():
+    """The weight stream asked for by name at 17..64 rows runs K whole where its plan would share K and the workspace is missing
+    (refused only where the launch would gain by sharing: a narrow N under a long K), and takes every N a plan of 64-row tiles has
+    counters for (no memory is touched; the addresses are made up)."""
+    from lightllm_amd import _lib
+
+    if torch.cuda.is_available():
+        pytest.skip("made-up addresses: only where a launch fails for want of a device")
+    lib = _lib.lib()
+
+    def call(m, n, k, ws_bytes):
+        return lib.mi355_block_fp8_gemm(1 << 40, 2 << 40, 3 << 40, 4 << 40, 5 << 40, m, n, k, k, 1, k, n, k // 128, 1, 1, k // 128,
+                                        128, 128, (6 << 40) if ws_bytes else None, ws_bytes, 3, None)
+
+    for m, n, k in [(36, 25337, 22656), (49, 26940, 29824), (27, 31681, 35200), (36, 9509, 3840), (64, 530000, 7808),
+                    (17, 12288, 20608), (40, 20000, 38400)]:
+        for ws_bytes in (0, 1 << 34):
+            assert call(m, n, k, ws_bytes) == -5, (m, n, k, ws_bytes)   # past every check: the launch itself fails here
+    for m, n, k in [(32, 4096, 14336), (64, 2112, 7168)]:
+        assert call(m, n, k, 0) == -4 and call(m, n, k, 1 << 34) == -5
+
+
 def test_linear_call_is_the_c_entry():
     """The CPython entry of the one-call linear passes its integers (None: a null pointer) to the C entry as ctypes does and
     refuses anything else."""

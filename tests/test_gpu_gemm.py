@@ -345,6 +345,26 @@ def test_stream_17_to_64_rows(hip, M, N, K):
     assert torch.equal(c, _run(xq, xs.t().contiguous().t(), wq, ws, "skinny"))
 
 
+# two, three and four row blocks whose scales are gathered step by step: a K beyond what is staged, with and without turned
+# starts, where the plan would share K and (64 rows) where it has no tiles that do, a ragged last tile
+@pytest.mark.parametrize("M,N,K,shares", [(17, 12290, 20608, True), (33, 12288, 28672, True), (48, 12345, 24576, True), (64, 16380, 20608, False)])
+def test_stream_whole_k_without_a_workspace(hip, M, N, K, shares):
+    print(f"gemm stream, no workspace M={M} N={N} K={K}", flush=True)
+    xq, xs, wq, ws = _prep(M, N, K, seed=N + K + M, device="cuda")
+    assert (hip.mi355_block_fp8_gemm_workspace_bytes(M, N, K, 3) > 0) == shares
+    outs = []
+    for xs_any in (xs, xs.t().contiguous().t()):
+        c = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        rc = hip.mi355_block_fp8_gemm(xq.data_ptr(), wq.data_ptr(), xs_any.data_ptr(), ws.data_ptr(), c.data_ptr(), M, N, K, K, 1, K, N,
+                                      xs_any.stride(0), xs_any.stride(1), 1, ws.stride(0), 128, 128, None, 0, 3,
+                                      torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert rc == 0, hip.mi355_error_string(rc)
+        outs.append(c)
+    _dequant_close(outs[0], xq, xs, wq, ws)
+    assert torch.equal(outs[0], outs[1])
+
+
 # the table's choice at the edges of the 5 to 8 row-block forms of the stream: tiles of 16 and 32 weight rows, K whole and
 # shared by 2 to 7 workgroups, turned starts (K a multiple of 4096) and plain ones, ragged shares, ragged tiles down to one
 # row, and beside them shapes that stay with the activation block in LDS (N = 2112 and 8190 from 113 rows on, N = 512)
