@@ -261,16 +261,16 @@ static int launch_dense(GemmArgs &a, hipStream_t st) {
 }
 
 // Weight-streaming launches for M <= 64 (stream_plan.hpp has the plan).
-template <int MT, int TNW, bool XSL, bool TURN, int WV>
+template <int MT, int TNW, bool XSL, bool TURN, int WV, int DEEP = 0>
 static int launch_stream_as(GemmArgs &a, const SkinnyPlan &pl, void *ws, int lds_bytes, hipStream_t st) {
     using Cfg = StreamCfg<MT, TNW, WV>;
     constexpr int max_lds = Cfg::kLds + (XSL ? Cfg::scale_lds_bytes(Cfg::kMaxScaleSteps) : 0);
     if (pl.splits <= 1) {
-        constexpr auto whole_k = block_fp8_gemm_stream_kernel<MT, TNW, false, XSL, 0, false, WV, TURN>;
+        constexpr auto whole_k = block_fp8_gemm_stream_kernel<MT, TNW, false, XSL, 0, false, WV, TURN, DEEP>;
         if (!allow_lds<whole_k>(max_lds)) return MI355_ELAUNCH;
         return launch(whole_k, dim3(pl.tiles), dim3(64 * WV), lds_bytes, st, a);
     }
-    if constexpr (MT == 1 || XSL) {
+    if constexpr (DEEP == 0 && (MT == 1 || XSL)) {
         constexpr auto split_k = block_fp8_gemm_stream_kernel<MT, TNW, true, XSL, 0, false, WV, TURN>;
         if (!allow_lds<split_k>(max_lds)) return MI355_ELAUNCH;
         a.splits = pl.splits;
@@ -281,10 +281,10 @@ static int launch_stream_as(GemmArgs &a, const SkinnyPlan &pl, void *ws, int lds
     return MI355_EUNSUPPORTED;
 }
 
-template <int MT, int TNW, bool XSL, int WV>
+template <int MT, int TNW, bool XSL, int WV, int DEEP = 0>
 static int launch_stream_form(GemmArgs &a, const SkinnyPlan &pl, void *ws, int lds_bytes, hipStream_t st) {
-    return a.turn_mask ? launch_stream_as<MT, TNW, XSL, true, WV>(a, pl, ws, lds_bytes, st)
-                       : launch_stream_as<MT, TNW, XSL, false, WV>(a, pl, ws, lds_bytes, st);
+    return a.turn_mask ? launch_stream_as<MT, TNW, XSL, true, WV, DEEP>(a, pl, ws, lds_bytes, st)
+                       : launch_stream_as<MT, TNW, XSL, false, WV, DEEP>(a, pl, ws, lds_bytes, st);
 }
 
 // The activation scales of a CTA's K range are staged in LDS when the range is short enough for the staging area; from 17
@@ -298,6 +298,9 @@ static int launch_stream(GemmArgs &a, const SkinnyPlan &pl, void *ws, hipStream_
     a.turn_mask = stream_turn_mask(a.K, KB / pl.splits);
     if (pl.staged && steps <= Cfg::kMaxScaleSteps) {
         const int lds_bytes = Cfg::kLds + Cfg::scale_lds_bytes(steps);
+        if constexpr (MT == 2 && TNW == 4 && WV == 4) {
+            if (pl.deep) return launch_stream_form<MT, TNW, true, WV, 2>(a, pl, ws, lds_bytes, st);
+        }
         return launch_stream_form<MT, TNW, true, WV>(a, pl, ws, lds_bytes, st);
     }
     if constexpr (MT == 1 || (MT <= 4 && TNW == 4 && WV == 4)) return launch_stream_form<MT, TNW, false, WV>(a, pl, ws, Cfg::kLds, st);

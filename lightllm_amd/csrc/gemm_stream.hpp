@@ -97,14 +97,14 @@ struct StreamRegs {
 // checks that the range fits); otherwise every wave gathers them per step, which costs as many cache-line
 // accesses as the X block itself (16 rows x 4 bytes per request).
 // XR > 0: X is the unquantized activation matrix (XQuant above; XSL is false then).
-// TURN: the tiles start at different K steps (GemmArgs::turn_mask).
-template <int MT, int TNW, bool SPLIT, bool XSL, int XR = 0, bool F16 = false, int WV = kStreamWaves, bool TURN = false>
+// TURN: the tiles start at different K steps (GemmArgs::turn_mask).  DEEP: K steps in flight per wave, 0 for StreamCfg's.
+template <int MT, int TNW, bool SPLIT, bool XSL, int XR = 0, bool F16 = false, int WV = kStreamWaves, bool TURN = false, int DEEP = 0>
 __global__ __launch_bounds__(64 * WV) void block_fp8_gemm_stream_kernel(const GemmArgs p) {
     static_assert(XR == 0 || (MT == 1 && !XSL), "unquantized activations: at most 16 rows, no staged scales");
     using Cfg = StreamCfg<MT, TNW, WV>;
     constexpr int NX = XR ? XR : 2 * MT;
     using Regs = StreamRegs<MT, TNW, NX>;
-    constexpr int D = Cfg::depth(XSL || XR);
+    constexpr int D = DEEP > 0 ? DEEP : Cfg::depth(XSL || XR);
     constexpr int BN = Cfg::BN;
     extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
 

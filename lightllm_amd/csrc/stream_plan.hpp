@@ -33,6 +33,7 @@ struct SkinnyPlan {
     int tnw, splits, tiles;
     int waves;
     bool staged = true;  // from 17 rows on: the activation scales of a workgroup's K range are staged in LDS
+    bool deep = false;   // two K steps in flight per wave instead of one
 };
 
 // K whole without a workspace and for any K: 64-row tiles on four waves, the scales gathered step by step.
@@ -105,6 +106,9 @@ inline SkinnyPlan skinny_plan(int64_t M, int64_t N, int64_t K, int cus) {
     pl.splits = 1;
     pl.waves = 4;
     const int64_t t64 = (N + 63) / 64;
+    // 32 rows: 64-row tiles in four rounds and more take a second K step in flight (N = 73856, K = 4864, M = 22 64.1 us against
+    // 67.9 with one, 79744 x 2688, M = 24 40.6 / 43.2; level from 2 to 4 rounds; three row blocks lose a third by it)
+    best.deep = mt == 2 && best.waves == 4 && best.tnw == 4 && best.splits == 1 && best.tiles >= 4 * (int64_t)cus;
     // 64-row tiles that come to just over one per unit leave half the units with twice the work of the others:
     // narrower tiles then (N = 18432, K = 7168, 288 tiles of 64 rows, M = 1 / 16: 22.6 / 26.8 us against 27.9 /
     // 29.9; N = 18944, K = 3584: 13.2 / 15.2 against 16.4 / 17.3)
