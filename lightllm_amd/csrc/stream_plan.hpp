@@ -97,6 +97,9 @@ inline SkinnyPlan skinny_wide_plan(int64_t M, int64_t N, int64_t K, int cus) {
     // a K range too long for the staged forms, on more tiles than share it: N = 72704, K = 21376, M = 39 335 us (366 with a second
     // K step in flight, 551 with K shared by two)
     if (best.tnw == 0) return skinny_whole_plan(N);
+    // 32 rows: 64-row tiles in four rounds and more take a second K step in flight (N = 73856, K = 4864, M = 22 64.1 us against
+    // 67.9 with one, 79744 x 2688, M = 24 40.6 / 43.2; level from 2 to 4 rounds; three row blocks lose a third by it)
+    best.deep = mt == 2 && best.waves == 4 && best.tnw == 4 && best.splits == 1 && best.tiles >= 4 * (int64_t)cus;
     return best;
 }
 
@@ -106,9 +109,6 @@ inline SkinnyPlan skinny_plan(int64_t M, int64_t N, int64_t K, int cus) {
     pl.splits = 1;
     pl.waves = 4;
     const int64_t t64 = (N + 63) / 64;
-    // 32 rows: 64-row tiles in four rounds and more take a second K step in flight (N = 73856, K = 4864, M = 22 64.1 us against
-    // 67.9 with one, 79744 x 2688, M = 24 40.6 / 43.2; level from 2 to 4 rounds; three row blocks lose a third by it)
-    best.deep = mt == 2 && best.waves == 4 && best.tnw == 4 && best.splits == 1 && best.tiles >= 4 * (int64_t)cus;
     // 64-row tiles that come to just over one per unit leave half the units with twice the work of the others:
     // narrower tiles then (N = 18432, K = 7168, 288 tiles of 64 rows, M = 1 / 16: 22.6 / 26.8 us against 27.9 /
     // 29.9; N = 18944, K = 3584: 13.2 / 15.2 against 16.4 / 17.3)
