@@ -387,8 +387,13 @@ static int launch_streamcu(GemmArgs &a, int tnw, hipStream_t st) {
 constexpr int kXshareDepth = 4;
 using XshareCfg = ShareCfg<4, 2, kXshareDepth>;
 
+// 33..48 rows: three row blocks on the first kernel are ahead where they run turned or in up to five rounds of 64-row tiles (N =
+// 66176, K = 7424, M = 38 98.0 us against 119 here), this one beyond (86144 x 12672, M = 46 227 against 210; 116480 x 1280, M =
+// 40 38.9 / 35.2).
 static bool xshare_pays(int64_t M, int64_t N, int64_t K, int cus) {
-    return M > 48 && M <= 64 && (N + 127) / 128 >= (int64_t)cus * 3 / 4 && K / kBlockK <= XshareCfg::kMaxScaleSteps;
+    if (M <= 32 || M > 64 || K / kBlockK > XshareCfg::kMaxScaleSteps) return false;
+    if (M <= 48) return K % 4096 != 0 && (N + 63) / 64 >= 5 * (int64_t)cus;
+    return (N + 127) / 128 >= (int64_t)cus * 3 / 4;
 }
 
 // 128-row workgroup tiles; the K range is split in two while that leaves fewer than two workgroups per compute unit
@@ -514,22 +519,59 @@ static size_t rows128_workspace(int64_t M, int64_t N, int64_t K, int cus) {
     return (size_t)MI355_WS_COUNTER_BYTES + (size_t)pl.tiles * pl.splits * 16 * rows128_mt(M) * pl.bn * 4;
 }
 
-// Where the kernel pays (Llama-3-8B and DeepSeek-V3 linears, weights rotated so that none is found in the
-// memory-side cache).  At 65..128 rows it beats the 128x128 tiles by 10 to 30 % (DeepSeek-V3 down, M = 128: 39.5 us
-// against 50.0; Llama-3 down: 27.9 against 30.3) unless K is short (q_b, K = 1536: 21.7 against 17.0).  At 49..64
-// rows it beats the streaming kernels on the large weights (DeepSeek-V3 gate_up at M = 64: 49.5 us against 71.2, down 31.5
-// against 41.2) and loses on the small ones, where its second launch shows (Llama-3 qkv: 14.7 against 11.6); at 48 rows
-// and fewer the streaming kernels are the faster ones but for a few kinds of large weights (below).
-// 49..64 rows: whether the streaming kernel is ahead of ROWS128.  Its workgroups have to fit one round, to fill four fifths of
-// it where their starts are not turned (M = 64: N = 15360, K = 5120, 240 of them 22.1 us against 23.5; 12288 x 5120, 192 of
-// them 21.4 against 21.0; turned, 12288 x 4096 16.7 against 18.0), and on large weights to take 64 weight rows, so that
-// the activations are not read too often (N = 7168, K = 18432, 32 rows a workgroup: 38.2 against 31.6).
-static bool skinny_ahead_of_rows128(int64_t M, int64_t N, int64_t K, int cus) {
-    const SkinnyPlan sp = skinny_plan(M, N, K, cus);
-    const int64_t wgs = (int64_t)sp.tiles * sp.splits;
-    return wgs <= cus && (K % 4096 == 0 || wgs * 5 >= 4 * (int64_t)cus) && (N * K < 60000000ll || sp.tnw == 4);
+// What the two weight streams take at 17..64 rows, in ns, where K is not a multiple of 4096 (turned starts make their own rules
+// below).  Fitted to 1066 shapes of 20 MB and more (N = 900..139000, K = 1024..21500, weights from HBM; 5.0 and 5.6 % rms):
+// taking the smaller is 0.2 % behind the faster one on average.  (Rules drawn from 22 model linears took the streaming kernel
+// where it is up to 29 % behind, us, this one / that: N = 20992, K = 8576, M = 46 40.6 / 52.3; 55680 x 10240, M = 47 103 / 126;
+// 50069 x 2688, M = 46 31.4 / 39.1.)
+static int64_t rows128_ns(int64_t M, int64_t N, int64_t K, const Rows128Plan &pl, int cus) {
+    const int64_t mt = rows128_mt(M), steps = (K / kBlockK + pl.splits - 1) / pl.splits, wgs = (int64_t)pl.tiles * pl.splits;
+    const int64_t rounds = (wgs + cus - 1) / cus;
+    return 4314 + rounds * steps * (584 * mt + 4863 * pl.wv + 615 * mt * pl.wv) / 100 + N * K / 10060 + 3219 * (rounds - 1) +
+           (pl.splits > 1 ? 2079 + 65 * pl.splits + 3429 * wgs * mt / 1000 : 65);
 }
 
+static int64_t skinny_wide_ns(int64_t M, int64_t N, int64_t K, const SkinnyPlan &pl, int cus) {
+    const int64_t mt = skinny_mt(M), steps = (K / kBlockK + pl.splits - 1) / pl.splits, wgs = (int64_t)pl.tiles * pl.splits;
+    const int64_t slots = skinny_wide_slots(pl.waves, pl.tnw, (int)mt, steps);
+    return 1226 + N * K / 17450 + (wgs + cus - 1) / cus * steps * (320 * pl.tnw + 284 * mt) / 10 +
+           150 * ((steps + pl.waves - 1) / pl.waves) + (3231 + 134 * pl.waves) * pl.tnw * mt / 10 +
+           (pl.splits > 1 ? 1479 + 213 * pl.splits : 0) + 3320 * ((wgs + cus * slots - 1) / (cus * slots) - 1);
+}
+
+// 17..64 rows: whether ROWS128 is ahead of the streaming kernel.
+static bool rows128_ahead_of_stream(int64_t M, int64_t N, int64_t K, int cus) {
+    const Rows128Plan pl = rows128_plan(M, N, K, cus);
+    const SkinnyPlan sp = skinny_plan(M, N, K, cus);
+    const int64_t t64 = (N + 63) / 64, wgs = (int64_t)sp.tiles * sp.splits;
+    if (pl.tiles > cus || N * K < 20000000ll) return false;
+    // a single well-filled launch: narrow or full-width workgroups on 0.55 cus .. cus tiles with K unshared
+    const bool one_launch = pl.splits == 1 && pl.tiles * 20 >= (int64_t)cus * 11;
+    const bool over_one = t64 > cus && t64 * 4 <= 5 * (int64_t)cus;  // 64-row tiles that come to just over one per unit
+    // where a caller relies on this kernel's sums (they are those of the square tiles) although the streaming kernel is level or
+    // ahead: a short K (N = 24576, K = 1536, M = 48: 12.4 us here, 11.6), a very long one (7168 x 18432, M = 20 / 32: 28.5 /
+    // 28.6, the stream 25.9 / 27.2) and N = 14336, K = 4096 and its neighbours from 49 rows on (19.5, 17.1)
+    if (M > 32 && M <= 48 && K < 2048 && one_launch) return true;
+    if (M <= 48 && K >= 18432 && N * K >= 100000000ll) return true;
+    if (M > 48 && K <= 4096 && N * K >= 55000000ll && t64 < cus) return true;
+    if (K % 4096 != 0) {
+        if (M > 48 && !one_launch && xshare_pays(M, N, K, cus)) return false;
+        if (pl.splits == 1 && !one_launch) return false;  // K too short to share: 22037 x 1024, M = 61 15.1 us, 13.5 there
+        return rows128_ns(M, N, K, pl, cus) < skinny_wide_ns(M, N, K, sp, cus);
+    }
+    // K a multiple of 4096.  From 49 rows on the streaming kernel where its workgroups fit one round (M = 64, us here / there: N =
+    // 12288, K = 4096 18.0 / 16.7, 8192 x 8192 23.5 / 21.3; 10240 x 8192, two a unit, 24.2 / 30.7; 28672 x 4096, where this one
+    // is turned, 26.3 / 33); below, where it does not share K on 80 MB and more (48 rows, 10240 x 8192: 24.7 / 22.9, on record
+    // here) and its tiles do not come to just over one per unit (18096 x 8192, M = 39: 1.12 times behind)
+    if (M > 48) return wgs > cus && N * K >= 55000000ll && (one_launch || !xshare_pays(M, N, K, cus));
+    if (M > 32) return over_one || (sp.splits > 1 && N * K >= 80000000ll);
+    return false;  // (turned, 17..32 rows: 40960 x 4096, M = 20 40.2 here, 30.5 there; 57344 x 8192, M = 48 111, 86)
+}
+
+// Where the kernel pays (Llama-3-8B and DeepSeek-V3 linears, weights rotated so that none is found in the
+// memory-side cache).  At 65..128 rows it beats the 128x128 tiles by 10 to 30 % (DeepSeek-V3 down, M = 128: 39.5 us
+// against 50.0; Llama-3 down: 27.9 against 30.3) unless K is short (q_b, K = 1536: 21.7 against 17.0).  At 17..64 rows it is
+// the faster one on the larger weights (rows128_ahead_of_stream), at 16 rows on a few kinds of them (below).
 static bool rows128_pays(int64_t M, int64_t N, int64_t K, int cus) {
     if (M > 384 || M < 16) return false;
     if (rows128_two_tiles(M, N, K, cus)) return true;
@@ -543,28 +585,7 @@ static bool rows128_pays(int64_t M, int64_t N, int64_t K, int cus) {
         return t64 > 2 * (int64_t)cus && t64 <= 3 * (int64_t)cus && pl.splits == 1 && pl.tiles <= cus &&
                pl.tiles * 20 >= (int64_t)cus * 11;
     }
-    if (M <= 48) {
-        // 17..48 rows: the streaming kernel's plan fits its tile to the device (skinny_wide_plan) and is ahead, N = 28672,
-        // K = 4096, M = 48: 24.9 us against 30.1; 40960 x 4096, M = 20: 30.5 against 40.2; 57344 x 8192, M = 48: 86 against
-        // 111; 27648 x 5120, M = 40: 31.8 against 33.9; but for these.  From 33 rows on, large weights whose K it would
-        // share (N = 7168, K = 18432, M = 48: 30.2 here against 31.3) and single launches over a short K (N = 24576,
-        // K = 1536, M = 48: 12.0 against 12.0 - 12.2).
-        const int64_t t64 = (N + 63) / 64;
-        const Rows128Plan pl = rows128_plan(M, N, K, cus);
-        const bool one_launch = pl.splits == 1 && pl.tiles <= cus && pl.tiles * 20 >= (int64_t)cus * 11;
-        if (M > 32 && N * K >= 80000000ll && pl.tiles <= cus && skinny_plan(M, N, K, cus).splits > 1) return true;
-        if (M > 32 && K < 2048 && one_launch) return true;
-        if (K % 4096 == 0) return false;  // its turned starts (stream_turn_mask) decide the following, too
-        // 64-row tiles that spill into a third round where this kernel has a well-filled single launch (N = 36864,
-        // K = 7168, M = 20 / 48: 45.8 / 47.5 against 52.5 / 57.2) ...
-        if (t64 > 2 * (int64_t)cus && t64 <= 3 * (int64_t)cus && one_launch) return true;
-        // ... large weights whose 64-row tiles come to just over one per unit (N = 18432, K = 7168, M = 20 / 48: 28.3 / 29.6
-        // against 34.4 / 36.6), and a very long K (N = 7168, K = 18432: on record here, M = 20 / 32 28.5 / 28.6, the
-        // stream 25.9 / 27.2)
-        const bool over_one = t64 > cus && t64 * 4 <= 5 * (int64_t)cus;
-        if (M > 32 && over_one && N * K >= 60000000ll && pl.tiles <= cus) return true;  // (18944 x 3584, M = 48: 19.6, 20.3)
-        return N * K >= 100000000ll && pl.tiles <= cus && (over_one || K >= 18432);
-    }
+    if (M <= 64) return rows128_ahead_of_stream(M, N, K, cus);
     if (M > 256) {
         // 257..384 rows (the activation block of a step is 48 KiB): still ahead where the 128-row tiles are few, K is
         // long and the weights are not small (Llama-3 down at M = 257 / 384: 38.0 / 46.8 us against 66.3 / 66.5;
@@ -608,22 +629,11 @@ static bool rows128_pays(int64_t M, int64_t N, int64_t K, int cus) {
         if (tiles * 2 <= cus) return tiles * rows128_splits(M, N, K, cus) * 2 >= cus;
         return tiles <= cus && (M <= 160 || (M <= kRows128NarrowMaxM && tiles * 8 >= (int64_t)cus * 7));
     }
-    // up to 64 rows the streaming kernel first, but for N = 14336, K = 4096 and its neighbours, which are on record here
-    // although it is ahead there, too (17.1 us against 19.5)
-    const bool ahead = M <= 64 && skinny_ahead_of_rows128(M, N, K, cus);
-    const bool kept = M <= 64 && K <= 4096 && N * K >= 55000000ll && (N + 63) / 64 < cus;
-    if (ahead && !kept && N * K < 100000000ll) return false;
-    // otherwise a single well-filled launch always pays up to 128 rows (narrow or full-width workgroups on 0.55 cus .. cus
-    // tiles with K unshared: DeepSeek-V3 gate_up at M = 64: 49.7 us against 69.9 - 72.5 for the streaming kernels,
-    // q_b 12.5 against 15.0, Llama-3 gate_up 29.5 against 29.8)
+    // 65..128 rows: a single well-filled launch always pays (narrow or full-width workgroups on 0.55 cus .. cus tiles with K
+    // unshared: q_b, M = 65: 12.5 us against 15.0), otherwise from 16 K steps on
     const Rows128Plan pl = rows128_plan(M, N, K, cus);
     if (pl.splits == 1 && pl.tiles <= cus && pl.tiles * 20 >= (int64_t)cus * 11) return true;
-    if (M > 64) return K / kBlockK >= 16;
-    // 49..64 rows with K shared or more tiles than units: not where the shared-activation streaming kernel runs (its small
-    // workgroups fill the second round better), else from 60 MB of weights on (M = 64: N = 10240, K = 8192 24.2 us against
-    // 30.7 for the streaming kernel; 16384 x 7168, 256 workgroups there, 29.7 against 26.3)
-    if (pl.tiles > cus || xshare_pays(M, N, K, cus)) return false;
-    return kept || (N * K >= 60000000ll && !ahead);
+    return K / kBlockK >= 16;
 }
 
 static bool rowsm_limits_ok(const RowsMPlan &pl, int64_t M, int64_t K, int64_t lda, int64_t as_m, int64_t as_k);

@@ -66,6 +66,14 @@ inline int64_t skinny_wide_cap(int waves, int tnw, int mt) {
     return steps < most ? steps : most;
 }
 
+// Workgroups on a unit at a time, by registers (one or two waves a SIMD) and by LDS.
+inline int64_t skinny_wide_slots(int waves, int tnw, int mt, int64_t steps) {
+    const bool two = waves == 8 ? tnw > 1 : tnw * mt >= 8;
+    const int64_t slots = tnw * mt == 16 ? 1 : (two ? 8 / waves : 4);
+    const int64_t by_lds = kMaxLds / skinny_wide_lds(waves, tnw, mt, steps);
+    return slots < by_lds ? slots : (by_lds > 0 ? by_lds : 1);
+}
+
 inline SkinnyPlan skinny_wide_plan(int64_t M, int64_t N, int64_t K, int cus) {
     const int mt = skinny_mt(M);
     const int64_t KB = K / kBlockK;
@@ -80,11 +88,7 @@ inline SkinnyPlan skinny_wide_plan(int64_t M, int64_t N, int64_t K, int cus) {
                 const int64_t wgs = tiles * s, steps = (KB + s - 1) / s;
                 if (s > 1 && (KB / s < 2 * waves || 2 * wgs > 5 * (int64_t)cus)) break;
                 if (steps > cap) continue;
-                // workgroups on a unit at a time, by registers (one or two waves a SIMD) and by LDS
-                const bool two = waves == 8 ? tnw > 1 : tnw * mt >= 8;
-                int64_t slots = tnw * mt == 16 ? 1 : (two ? 8 / waves : 4);
-                const int64_t by_lds = kMaxLds / skinny_wide_lds(waves, tnw, mt, steps);
-                if (slots > by_lds) slots = by_lds > 0 ? by_lds : 1;
+                const int64_t slots = skinny_wide_slots(waves, tnw, mt, steps);
                 const int64_t per_unit = (wgs + cus - 1) / cus, rounds = (wgs + cus * slots - 1) / (cus * slots);
                 const int64_t cost = per_unit * 2048 * tnw * steps / 50 + per_unit * 2048 * mt * steps / 140 +
                                      (s > 1 ? 280 + 625 * s : 0) + 6000 * (rounds - 1) + 97 * ((steps + waves - 1) / waves);

@@ -296,6 +296,26 @@ def test_shape_table_choices_on_256_compute_units():
     assert got == expect, {k: (got[k], expect[k]) for k in expect if got[k] != expect[k]}
 
 
+def test_shape_table_at_17_to_64_rows():
+    """Large weights on either side of the lines between the three weight streams (planned for 256 compute units): each shape
+    was timed on both kernels and runs on the one that is ahead."""
+    from lightllm_amd import _lib
+
+    lib = _lib.lib()
+    SKINNY, XSHARE, ROWS = 3, 9, 10
+    expect = {
+        # one round of wide tiles against a third or a second, nearly empty one of 64-row tiles
+        (46, 20992, 8576): ROWS, (47, 55680, 10240): ROWS, (46, 50069, 2688): ROWS, (51, 18816, 2688): ROWS, (33, 21312, 11264): ROWS,
+        (39, 18096, 8192): ROWS, (22, 51200, 20480): ROWS, (30, 36864, 7168): ROWS,
+        (40, 15360, 5120): SKINNY, (41, 19168, 2176): SKINNY, (33, 8192, 8192): SKINNY, (56, 12288, 4096): SKINNY, (24, 45504, 4096): SKINNY,
+        (60, 16000, 4992): SKINNY, (48, 28672, 4096): SKINNY, (20, 40960, 4096): SKINNY,
+        # more than five rounds of 64-row tiles; turned starts
+        (40, 116480, 1280): XSHARE, (46, 86144, 12672): XSHARE, (38, 66176, 7424): SKINNY, (43, 105664, 4096): SKINNY,
+    }
+    got = {shape: lib.mi355_block_fp8_gemm_plan(*shape, 1 << 32, 256) for shape in expect}
+    assert got == expect, {k: (got[k], expect[k]) for k in expect if got[k] != expect[k]}
+
+
 _T256, _T128, _SKINNY, _GENERIC, _T256x128, _STREAMK, _XSHARE, _ROWS, _CU, _ROWSM = 1, 2, 3, 4, 5, 8, 9, 10, 11, 12
 
 
