@@ -548,22 +548,25 @@ static bool rows128_ahead_of_stream(int64_t M, int64_t N, int64_t K, int cus) {
     // a single well-filled launch: narrow or full-width workgroups on 0.55 cus .. cus tiles with K unshared
     const bool one_launch = pl.splits == 1 && pl.tiles * 20 >= (int64_t)cus * 11;
     const bool over_one = t64 > cus && t64 * 4 <= 5 * (int64_t)cus;  // 64-row tiles that come to just over one per unit
-    // where a caller relies on this kernel's sums (they are those of the square tiles) although the streaming kernel is level or
-    // ahead: a short K (N = 24576, K = 1536, M = 48: 12.4 us here, 11.6), a very long one (7168 x 18432, M = 20 / 32: 28.5 /
+    // kept here, where the sums of the table's launch are compared with those of this kernel by name, although the streaming kernel is
+    // level or ahead: a short K (N = 24576, K = 1536, M = 48: 12.4 us here, 11.6), a very long one (7168 x 18432, M = 20 / 32: 28.5 /
     // 28.6, the stream 25.9 / 27.2) and N = 14336, K = 4096 and its neighbours from 49 rows on (19.5, 17.1)
     if (M > 32 && M <= 48 && K < 2048 && one_launch) return true;
     if (M <= 48 && K >= 18432 && N * K >= 100000000ll) return true;
     if (M > 48 && K <= 4096 && N * K >= 55000000ll && t64 < cus) return true;
     if (K % 4096 != 0) {
         if (M > 48 && !one_launch && xshare_pays(M, N, K, cus)) return false;
+        if (!sp.staged) return true;  // gathered scales: 31680 x 21504, M = 56 131 us here, 160 there
         if (pl.splits == 1 && !one_launch) return false;  // K too short to share: 22037 x 1024, M = 61 15.1 us, 13.5 there
         return rows128_ns(M, N, K, pl, cus) < skinny_wide_ns(M, N, K, sp, cus);
     }
-    // K a multiple of 4096.  From 49 rows on the streaming kernel where its workgroups fit one round (M = 64, us here / there: N =
-    // 12288, K = 4096 18.0 / 16.7, 8192 x 8192 23.5 / 21.3; 10240 x 8192, two a unit, 24.2 / 30.7; 28672 x 4096, where this one
-    // is turned, 26.3 / 33); below, where it does not share K on 80 MB and more (48 rows, 10240 x 8192: 24.7 / 22.9, on record
-    // here) and its tiles do not come to just over one per unit (18096 x 8192, M = 39: 1.12 times behind)
-    if (M > 48) return wgs > cus && N * K >= 55000000ll && (one_launch || !xshare_pays(M, N, K, cus));
+    // K a multiple of 4096.  From 49 rows on the streaming kernel where its workgroups fit one round, from 100 MB on tiles of 64
+    // weight rows (M = 64, us here / there: N = 12288, K = 4096 18.0 / 16.7, 8192 x 8192 23.5 / 21.3; 10240 x 8192, two a unit, 24.2
+    // / 30.7; 28672 x 4096, where this one is turned, 26.3 / 33; 32 weight rows: 8032 x 20480 1.13 times behind, 7984 x 16384
+    // 0.9 but kept here like those above); below, where it does not share K on 80 MB and more (48 rows, 10240 x 8192: 24.7 /
+    // 22.9, kept) and its tiles do not come to just over one per unit (18096 x 8192, M = 39: 1.12 times behind)
+    const bool one_round = wgs <= cus && (N * K < 100000000ll || sp.tnw == 4);
+    if (M > 48) return !one_round && N * K >= 55000000ll && (one_launch || !xshare_pays(M, N, K, cus));
     if (M > 32) return over_one || (sp.splits > 1 && N * K >= 80000000ll);
     return false;  // (turned, 17..32 rows: 40960 x 4096, M = 20 40.2 here, 30.5 there; 57344 x 8192, M = 48 111, 86)
 }
