@@ -46,14 +46,18 @@ inline bool skinny_runs_whole(int64_t M, int64_t N, int64_t K, int cus) {
 }
 
 // 17..64 rows: four or eight waves a workgroup, tiles of 16, 32 or 64 weight rows, K whole or shared by up to eight
-// workgroups.  A wave has one K step in flight and the waves hide each other's latency, so what a launch takes is what
-// its busiest unit pulls: weights at about 50 GB/s (a unit's misses in flight over the latency of HBM), activations at
-// about 140 (they come from the L2; every workgroup reads all rows of its K range), 97 ns for each K step in a wave's
-// sequence, 280 ns and 625 for each workgroup that shares a tile and 6 us for a further round.  The constants were fitted to
-// 22 (N, K) pairs (N = 1536..36864, K = 1536..18944) at M = 20..64, all candidates timed: the choice is 1.0 % behind
-// the best candidate on average.  Against tiles of 16 / 32 / 64 rows on four waves with K shared until there were two
-// workgroups a unit, us: N = K = 4096, M = 20 / 48 / 64 7.3 / 8.6 / 9.7 (8.9 / 10.0 / 10.1), 6144 x 4096 8.5 / 10.3 /
-// 11.6 (10.2 / 12.3 / 12.8), 4096 x 14336 14.5 / 17.3 / 19.5 (14.9 / 18.8 / 20.1), 28672 x 4096 21.5 / 24.9 (23.8 / 30.1).
+// workgroups.  What a launch takes, in ns and beside what all of them have in common: for each of the busiest unit's workgroups
+// 288, and for each of its K steps 14 for 16 weight rows and 16 for 16 rows of activations (they come from the L2; every
+// workgroup reads all rows of its K range); 109 for each K step in a wave's sequence, 162 + 6.5 a wave for each accumulator (they
+// are added up through LDS), 483 and 230 for each workgroup that shares a tile and 3.8 us for a further round.  Tiles of 64
+// weight rows, one or none a unit, want 32 steps: under fewer, two of half the width are ahead (15616 x 2432, M = 23 9.6 us against
+// 11.0).  Fitted to every candidate timed on 1179 shapes (M = 17..64, N = 100..139000, K = 1024..21500, weights from HBM): the
+// choice is 0.9 % behind the best candidate on average and on 8 shapes more than 4 % behind the plan of before the eight-wave
+// forms, which ran 32- or 64-row tiles on four waves with K shared until there were two workgroups a unit.  (A fit to 22 shapes
+// of model linears, part of whose weights came from the memory-side cache, charged the weights at 41 and nothing for the
+// accumulators and was behind that plan on 70: 15722 x 1152, M = 62 12.1 us against 9.9; 8581 x 1280, M = 19 7.4 / 6.6.)  us,
+// that plan in brackets: N = K = 4096, M = 20 / 48 / 64 7.3 / 8.6 / 9.7 (8.9 / 10.0 / 10.1), 6144 x 4096 8.5 / 10.3 / 11.6
+// (10.2 / 12.3 / 12.8), 4096 x 14336 14.5 / 17.3 / 19.5 (14.9 / 18.8 / 20.1), 28672 x 4096 21.5 / 24.9 (23.8 / 30.1).
 inline int64_t skinny_wide_lds(int waves, int tnw, int mt, int64_t steps) {
     const int64_t wave = (16 * tnw + 16 * (mt < 4 ? mt : 4)) * 128, acc = (int64_t)tnw * mt * 1024;
     return waves * (wave > acc ? wave : acc) + 16 + steps * (16 * mt + 1) * 4;
@@ -79,10 +83,14 @@ inline SkinnyPlan skinny_wide_plan(int64_t M, int64_t N, int64_t K, int cus) {
     const int64_t KB = K / kBlockK;
     SkinnyPlan best = {0, 1, 0, 8};
     int64_t best_cost = 0;
+    // four row blocks in four rounds of 64-row tiles, K beyond what four waves stage: 76224 x 17152, M = 64 324 us, 362 for the
+    // best staged form
+    if (mt == 4 && KB > skinny_wide_cap(4, 4, mt) && (N + 63) / 64 >= 4 * (int64_t)cus) return skinny_whole_plan(N);
     for (int waves = 4; waves <= 8; waves += 4)
         for (int tnw = 1; tnw <= 4; tnw *= 2) {
             if (waves == 8 && tnw == 4 && mt == 4) continue;  // 128 KiB of LDS and half the registers: not built
             const int64_t tiles = (N + 16 * tnw - 1) / (16 * tnw), cap = skinny_wide_cap(waves, tnw, mt);
+            if (tnw == 4 && KB < 32 && tiles <= cus) continue;
             if (tiles * 4 > MI355_WS_COUNTER_BYTES) continue;  // one arrival counter a tile
             for (int s = 1; s <= 8; ++s) {
                 const int64_t wgs = tiles * s, steps = (KB + s - 1) / s;
@@ -90,8 +98,8 @@ inline SkinnyPlan skinny_wide_plan(int64_t M, int64_t N, int64_t K, int cus) {
                 if (steps > cap) continue;
                 const int64_t slots = skinny_wide_slots(waves, tnw, mt, steps);
                 const int64_t per_unit = (wgs + cus - 1) / cus, rounds = (wgs + cus * slots - 1) / (cus * slots);
-                const int64_t cost = per_unit * 2048 * tnw * steps / 50 + per_unit * 2048 * mt * steps / 140 +
-                                     (s > 1 ? 280 + 625 * s : 0) + 6000 * (rounds - 1) + 97 * ((steps + waves - 1) / waves);
+                const int64_t cost = per_unit * (steps * (14 * tnw + 16 * mt) + 288) + 109 * ((steps + waves - 1) / waves) +
+                                     (324 + 13 * waves) * tnw * mt / 2 + (s > 1 ? 483 + 230 * s : 0) + 3775 * (rounds - 1);
                 if (best.tnw == 0 || cost < best_cost) {
                     best = {tnw, s, (int)tiles, waves};
                     best_cost = cost;
