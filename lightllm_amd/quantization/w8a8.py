@@ -134,7 +134,7 @@ class FP8w8a8B128Mi355QuantizationMethod(FP8w8a8B128QuantizationMethod):
             return None
         device = x.device
         alloc = self._alloc_func(use_custom_tensor_mananger)
-        if out is None and alloc is torch.empty:
+        if out is None and alloc is torch.empty and type(x) is torch.Tensor:  # (a subclass would hand its type on)
             out, out_dtype = x.new_empty((m, n)), dtype
         else:
             if out is None:

@@ -104,3 +104,19 @@ def test_output_over_the_activations(hip, M, N, K):
         out = buf[shift: shift + M * N].view(M, N)
         assert QUANTMETHODS.get("fp8w8a8-b128").apply(mine, WeightPack(wq, ws), out=out) is out
         assert torch.equal(out, want), shift
+
+
+@pytest.mark.parametrize("M", [2, 40])
+def test_output_of_a_tensor_subclass(hip, M):
+    """Activations of a tensor subclass give a plain tensor, as an output allocated by torch.empty is."""
+    from lightllm_amd.quantization import QUANTMETHODS, WeightPack
+
+    class Tagged(torch.Tensor):
+        pass
+
+    wq, ws = H.quantized_weights(512, 1024, seed=3, device="cuda")
+    x = H.activations(M, 1024, seed=4).cuda()
+    method, pack = QUANTMETHODS.get("fp8w8a8-b128"), WeightPack(wq, ws)
+    for mine in (x.as_subclass(Tagged), torch.nn.Parameter(x, requires_grad=False)):
+        out = method.apply(mine, pack)
+        assert type(out) is torch.Tensor and torch.equal(out, method.apply(x, pack))
