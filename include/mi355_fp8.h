@@ -123,8 +123,10 @@ int mi355_block_weight_quant_fp8(const void *w, int32_t w_dtype, void *q, float 
                                      workgroup; the shape table takes it from 49 rows on */
 #define MI355_GEMM_ROWS128 10 /* weight streaming, M <= 384, the activation block of a K step in LDS: 256 weight rows per
                                  workgroup up to 128 rows, 128 beyond; a second launch adds the partial sums when K is shared;
-                                 209..352 rows on a wide N run as two tiles over M.  Where the shape table picks it for
-                                 65..128 rows it runs the kernel of MI355_GEMM_SKINNY if one round of that is ahead */
+                                 209..352 rows on a wide N run as MI355_GEMM_ROWS_MTILED.  Where the shape table picks it
+                                 for 65..128 rows AUTO may launch MI355_GEMM_SKINNY_ROWS, and under K a multiple of 4096 its
+                                 tiles start at different K steps; by name, from 65 rows on, they add in K order, with the
+                                 sums of the square tiles */
 
 #define MI355_GEMM_SKINNY_CU 11 /* weight streaming, M <= 16: the weight rows cut into one equal share per compute unit,
                                   one workgroup of 8 waves per share and the whole K (no partial sums between
@@ -134,6 +136,9 @@ int mi355_block_weight_quant_fp8(const void *w, int32_t w_dtype, void *q, float 
                                      16..128 rows x 160..256 weight rows, K unshared, no workspace; for more than 384
                                      rows on a narrow N (at most 5120 weight rows, K <= 7168; 385..960 rows: at most 15360,
                                      K <= 5120) */
+
+#define MI355_GEMM_SKINNY_ROWS 13 /* the kernel of MI355_GEMM_SKINNY at 65..128 rows, one round of eight-wave tiles; where the
+                                     shape table would launch it (mi355_block_fp8_gemm_launched) */
 
 #define MI355_WS_COUNTER_BYTES 65536
 
@@ -148,6 +153,12 @@ int32_t mi355_block_fp8_gemm_variant(int64_t M, int64_t N, int64_t K);
  * a kernel that runs without one, so AUTO never returns MI355_EWORKSPACE.  Launches nothing.  No counterpart in the
  * reference; for tests of the table off the device it was measured on, and for callers that size workspaces. */
 int32_t mi355_block_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, size_t ws_bytes, int32_t cus);
+
+/* The code of the kernel that the call of mi355_block_fp8_gemm_plan launches.  It differs from the plan's where the table's
+ * MI355_GEMM_ROWS128 covers more than one kernel: MI355_GEMM_SKINNY_ROWS at 65..128 rows, MI355_GEMM_ROWS_MTILED at 209..352.
+ * Asked for by this code a launch is AUTO's, bit for bit, but for MI355_GEMM_ROWS128 at 65..128 rows (see there) and the
+ * second launch that MI355_GEMM_TILE256 may be followed by.  Launches nothing; no counterpart in the reference. */
+int32_t mi355_block_fp8_gemm_launched(int64_t M, int64_t N, int64_t K, size_t ws_bytes, int32_t cus);
 
 /* Bytes of workspace the launch plan of the CURRENT device needs for this shape and variant (0 = none). */
 size_t mi355_block_fp8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t variant);

@@ -17,6 +17,7 @@ GEMM_TILE256_RING, GEMM_TILE256_ONCE, GEMM_TILE256_STREAMK, GEMM_SKINNY_XSHARE =
 GEMM_ROWS128 = 10
 GEMM_SKINNY_CU = 11
 GEMM_ROWS_MTILED = 12
+GEMM_SKINNY_ROWS = 13
 WS_COUNTER_BYTES = 65536
 DTYPE_CODES = {torch.bfloat16: 0, torch.float32: 1, torch.float16: 2}
 
@@ -31,6 +32,7 @@ SIGNATURES = {
     "mi355_block_weight_quant_fp8": (_c.c_int, [_vp, _i32, _vp, _vp, _i64, _i64, _i32, _vp]),
     "mi355_block_fp8_gemm_variant": (_i32, [_i64, _i64, _i64]),
     "mi355_block_fp8_gemm_plan": (_i32, [_i64, _i64, _i64, _sz, _i32]),
+    "mi355_block_fp8_gemm_launched": (_i32, [_i64, _i64, _i64, _sz, _i32]),
     "mi355_block_fp8_gemm_workspace_bytes": (_sz, [_i64, _i64, _i64, _i32]),
     "mi355_block_fp8_gemm_noalloc": (
         _c.c_int,

@@ -977,12 +977,9 @@ static size_t workspace_bytes_for(int64_t M, int64_t N, int64_t K, int32_t varia
             const size_t rest = workspace_bytes_for(M, N - n1, K, MI355_GEMM_AUTO, cus);
             return rest > (size_t)MI355_WS_COUNTER_BYTES ? rest : (size_t)MI355_WS_COUNTER_BYTES;
         }
-        if (variant == MI355_GEMM_ROWS128) {
-            // 65..128 rows may run as the weight stream, and where a limit of that is not met as the kernel of the name
-            const SkinnyPlan sp = skinny_many_rows_plan(M, N, K, cus);
-            const size_t stream = sp.tnw > 0 && sp.splits > 1 ? skinny_workspace(M, sp) : 0;
-            return std::max(stream, workspace_bytes_for(M, N, K, variant, cus));
-        }
+        // 65..128 rows may run as the streaming kernel, and where a limit of that is not met as the kernel of the name
+        if (variant == MI355_GEMM_ROWS128)
+            return std::max(workspace_bytes_for(M, N, K, MI355_GEMM_SKINNY_ROWS, cus), workspace_bytes_for(M, N, K, variant, cus));
     }
     if (variant == MI355_GEMM_TILE256_STREAMK) {
         const int groups = stream_k_groups(((M + 255) / 256) * ((N + 255) / 256), K / kBlockK, cus, (M + 255) / 256);
@@ -1000,6 +997,10 @@ static size_t workspace_bytes_for(int64_t M, int64_t N, int64_t K, int32_t varia
     if (variant == MI355_GEMM_SKINNY_XSHARE) {
         const int splits = xshare_splits(N, K, cus);
         return splits > 1 ? xshare_workspace(N, splits) : 0;
+    }
+    if (variant == MI355_GEMM_SKINNY_ROWS) {
+        const SkinnyPlan sp = skinny_many_rows_plan(M, N, K, cus);
+        return sp.tnw > 0 && sp.splits > 1 ? skinny_workspace(M, sp) : 0;
     }
     if (variant == MI355_GEMM_ROWS128) {
         if (M > 384) return 0;
@@ -1040,6 +1041,24 @@ static int resolve_auto(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ld
     return variant;
 }
 
+// 65..128 rows on the streaming kernel: its plan, the 32-bit offsets and the workspace of a shared K.
+static int skinny_rows_check(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int64_t as_m, int cus, bool ws_usable,
+                             size_t ws_bytes) {
+    const SkinnyPlan sp = skinny_many_rows_plan(M, N, K, cus);
+    if (sp.tnw == 0 || N * ldw >= (1ll << 32) || M * lda >= (1ll << 32) || M * as_m >= (1ll << 32)) return MI355_EUNSUPPORTED;
+    if (sp.splits > 1 && (!ws_usable || ws_bytes < skinny_workspace(M, sp))) return MI355_EWORKSPACE;
+    return MI355_OK;
+}
+
+// What AUTO launches where the table says ROWS128: 65..128 rows as the streaming kernel where one round of that is ahead, 209..352
+// rows tiled over M.
+static int launched_for(int variant, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int64_t as_m, bool ws_usable,
+                        size_t ws_bytes, int cus) {
+    if (variant != MI355_GEMM_ROWS128) return variant;
+    if (rows128_two_tiles(M, N, K, cus)) return MI355_GEMM_ROWS_MTILED;
+    return skinny_rows_check(M, N, K, lda, ldw, as_m, cus, ws_usable, ws_bytes) == MI355_OK ? MI355_GEMM_SKINNY_ROWS : variant;
+}
+
 }  // namespace mi355
 
 using namespace mi355;
@@ -1053,6 +1072,12 @@ extern "C" int32_t mi355_block_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, si
     if (M <= 0 || N <= 0 || K <= 0 || K % kBlockK != 0) return MI355_GEMM_GENERIC;
     if (cus <= 0) cus = device_cus();
     return resolve_auto(M, N, K, K, K, K / kBlockK, 1, ws_bytes > 0, ws_bytes, cus);
+}
+
+extern "C" int32_t mi355_block_fp8_gemm_launched(int64_t M, int64_t N, int64_t K, size_t ws_bytes, int32_t cus) {
+    if (cus <= 0) cus = device_cus();
+    const int variant = mi355_block_fp8_gemm_plan(M, N, K, ws_bytes, cus);
+    return launched_for(variant, M, N, K, K, K, K / kBlockK, ws_bytes > 0, ws_bytes, cus);
 }
 
 /* The kernel the shape table picks for a packed, aligned problem on the current device (256 compute units when no
@@ -1092,6 +1117,7 @@ static int block_fp8_gemm_impl(const void *A, const void *B, const float *As, co
         const bool ws_usable = ws && ((uintptr_t)ws & 15) == 0;
         variant = fast && blocks128 ? resolve_auto(M, N, K, lda, ldb_n, as_m, as_k, ws_usable, ws_bytes, cus)
                                     : MI355_GEMM_GENERIC;
+        variant = launched_for(variant, M, N, K, lda, ldb_n, as_m, ws_usable, ws_bytes, cus);
     }
     if (was_auto && variant == MI355_GEMM_TILE256) {
         const int64_t n1 = n_split_rows(M, N, K, cus);
@@ -1193,20 +1219,6 @@ static int block_fp8_gemm_impl(const void *A, const void *B, const float *As, co
         case MI355_GEMM_ROWS128: {
             if (!rows128_limits_ok(M, N, K, lda, as_m, as_k, cus)) return MI355_EUNSUPPORTED;
             if (rows128_two_tiles(M, N, K, cus)) return launch_rowsm(a, rowsm_plan(M, N, K, cus), st);
-            if (was_auto) {
-                // the shape table's choice only: a caller that asks for this kernel gets it
-                const SkinnyPlan sp = skinny_many_rows_plan(M, N, K, cus);
-                const bool fits = N * ldb_n < (1ll << 32) && M * as_m < (1ll << 32) &&
-                                  (sp.splits == 1 || (ws && ((uintptr_t)ws & 15) == 0 && ws_bytes >= skinny_workspace(M, sp)));
-                if (sp.tnw > 0 && fits) {
-                    switch (skinny_mt(M)) {
-                        case 5: return launch_stream_many_rows<5>(a, sp, ws, st);
-                        case 6: return launch_stream_many_rows<6>(a, sp, ws, st);
-                        case 7: return launch_stream_many_rows<7>(a, sp, ws, st);
-                        default: return launch_stream_many_rows<8>(a, sp, ws, st);
-                    }
-                }
-            }
             Rows128Plan pl = rows128_plan(M, N, K, cus);
             pl.turned = was_auto || M <= 64;
             if (pl.splits > 1 && (!ws || ws_bytes < rows128_workspace(M, N, K, cus) || ((uintptr_t)ws & 15)))
@@ -1236,6 +1248,17 @@ static int block_fp8_gemm_impl(const void *A, const void *B, const float *As, co
                 case 22: return launch_rows128<22>(a, pl, ws, st);
                 case 23: return launch_rows128<23>(a, pl, ws, st);
                 default: return launch_rows128<24>(a, pl, ws, st);
+            }
+        }
+        case MI355_GEMM_SKINNY_ROWS: {
+            const int ok = skinny_rows_check(M, N, K, lda, ldb_n, as_m, cus, ws && ((uintptr_t)ws & 15) == 0, ws_bytes);
+            if (ok != MI355_OK) return ok;
+            const SkinnyPlan sp = skinny_many_rows_plan(M, N, K, cus);
+            switch (skinny_mt(M)) {
+                case 5: return launch_stream_many_rows<5>(a, sp, ws, st);
+                case 6: return launch_stream_many_rows<6>(a, sp, ws, st);
+                case 7: return launch_stream_many_rows<7>(a, sp, ws, st);
+                default: return launch_stream_many_rows<8>(a, sp, ws, st);
             }
         }
         case MI355_GEMM_ROWS_MTILED: {

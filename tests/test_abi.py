@@ -316,6 +316,27 @@ def test_shape_table_at_17_to_64_rows():
     assert got == expect, {k: (got[k], expect[k]) for k in expect if got[k] != expect[k]}
 
 
+def test_launched_kernel_query():
+    """What AUTO launches where the table's activation-block stream covers more than one kernel: the streaming kernel at 65..128
+    rows (not without its workspace where it shares K), tiles over M at 209..352; the plan's code everywhere else."""
+    from lightllm_amd import _lib
+
+    lib = _lib.lib()
+    ROWS, ROWSM, STREAM = 10, 12, 13
+    for shape, ws_bytes, want in [((72, 4096, 4096), 1 << 30, STREAM), ((96, 7168, 2048), 1 << 30, STREAM), ((96, 2112, 7168), 1 << 30, STREAM),
+                                  ((128, 2112, 7168), 1 << 30, ROWS), ((128, 36864, 7168), 1 << 30, ROWS), ((64, 14336, 4096), 1 << 30, ROWS),
+                                  ((333, 27648, 5120), 0, ROWSM), ((209, 12288, 2048), 0, ROWSM), ((300, 4096, 14336), 1 << 30, ROWS)]:
+        assert lib.mi355_block_fp8_gemm_launched(*shape, ws_bytes, 256) == want, shape
+    seen = set()
+    for m, n, k in _sweep_shapes(5, 3000):
+        for ws_bytes in (0, 65536 + (8 << 20), 1 << 34):
+            plan, v = (f(m, n, k, ws_bytes, 0) for f in (lib.mi355_block_fp8_gemm_plan, lib.mi355_block_fp8_gemm_launched))
+            assert v == plan or (plan == ROWS and (v == STREAM and 65 <= m <= 128 or v == ROWSM and 209 <= m <= 352)), (m, n, k, plan, v)
+            assert v != STREAM or lib.mi355_block_fp8_gemm_workspace_bytes(m, n, k, v) <= min(ws_bytes, 65536 + (8 << 20)), (m, n, k)
+            seen.add(v)
+    assert {ROWS, ROWSM, STREAM} <= seen
+
+
 _T256, _T128, _SKINNY, _GENERIC, _T256x128, _STREAMK, _XSHARE, _ROWS, _CU, _ROWSM = 1, 2, 3, 4, 5, 8, 9, 10, 11, 12
 
 
