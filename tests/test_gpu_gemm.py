@@ -322,8 +322,9 @@ def test_per_unit_stream_kernel(hip):
 
 
 def _dequant_close(c, xq, xs, wq, ws):
-    """bf16 outputs against the fp32 dequant-matmul: half a bf16 step of the value (2^-9) and the fp32 sums' share, whose
-    order differs (2^-12 of the largest value, K / 128 <= 160 terms)."""
+    """bf16 outputs against the fp32 dequant-matmul: half a bf16 step is at most 2^-8 of the value; the fp32 sums, of K / 128 <= 288
+    partial products in another order, differ by at most 288 * 2^-24 of the sum of their magnitudes, which is up to some 30 times
+    the largest output for K = 36864: 2^-11 of it."""
     ref = tr.dequant_matmul(xq, xs, wq, ws, out_dtype=torch.float32)
     assert not torch.isnan(c.float()).any()
     bound = ref.abs() * 2 ** -8 + ref.abs().max() * 2 ** -11
@@ -367,17 +368,27 @@ def test_stream_whole_k_without_a_workspace(hip, M, N, K, shares):
 
 # the table's choice at the edges of the 5 to 8 row-block forms of the stream: tiles of 16 and 32 weight rows, K whole and
 # shared by 2 to 7 workgroups, turned starts (K a multiple of 4096) and plain ones, ragged shares, ragged tiles down to one
-# row, and beside them shapes that stay with the activation block in LDS (N = 2112 and 8190 from 113 rows on, N = 512)
+# row, and beside them shapes that stay with the activation block in LDS (N = 2112, 7168 and 8190 from 113 rows on, N = 512)
 @pytest.mark.parametrize("M", [65, 80, 81, 96, 97, 112, 113, 128])
 @pytest.mark.parametrize("N,K", [(4096, 4096), (4090, 4096), (7168, 2048), (2112, 7168), (1000, 4096), (2048, 8192), (513, 2048),
                                  (520, 20608), (8190, 4096), (528, 36864), (2000, 2176), (512, 2048)])
 def test_stream_65_to_128_rows(hip, M, N, K):
+    from lightllm_amd import _lib
+
     print(f"gemm stream M={M} N={N} K={K}", flush=True)
+    streams = N != 512 and (M <= 112 or N not in (2112, 7168, 8190))
+    if _lib_cus() == 256:
+        assert hip.mi355_block_fp8_gemm_launched(M, N, K, 1 << 34, 0) == (_lib.GEMM_SKINNY_ROWS if streams else _lib.GEMM_ROWS128)
     xq, xs, wq, ws = _prep(M, N, K, seed=N + K + M, device="cuda")
     c = _run(xq, xs, wq, ws)
     _dequant_close(c, xq, xs, wq, ws)
     assert torch.equal(c, _run(xq, xs, wq, ws))
     assert torch.equal(c, _run(xq, xs.t().contiguous().t(), wq, ws))
+    if streams:
+        assert torch.equal(c, _run(xq, xs, wq, ws, "skinny128"))   # what was asserted above to be launched is what ran
+    else:
+        with pytest.raises(ValueError):
+            _run(xq, xs, wq, ws, "skinny128")
 
 
 # turned starts of the other streams, N larger than the turn's period of 32 or 64 tiles: per-unit stream with every K step of a
@@ -560,7 +571,7 @@ def test_rows_tiled_over_m_where_the_table_sends_it(hip, M, N, K):
     assert torch.equal(_run(xq, xs, wq, ws, None).view(torch.int16), _run(xq, xs, wq, ws, "rowsm").view(torch.int16))
 
 
-# 209..352 rows in two tiles of the activation-block stream, 385..960 rows on a wider N: the edges of both ranges, row counts
+# 209..352 rows in two or three tiles of the activation-block stream, 385..960 rows on a wider N: the edges of both ranges, row counts
 # that leave the last tile one row, N that leaves the last column of tiles one weight row, the shortest and longest K
 @pytest.mark.parametrize("M,N,K,variant", [(209, 12288, 2048, "rows128"), (225, 12289, 1536, "rows128"), (352, 27648, 1536, "rows128"),
                                            (333, 27648, 5120, "rows128"), (337, 20481, 1664, "rows128"), (256, 16384, 4096, "rows128"),
@@ -569,6 +580,9 @@ def test_rows_tiled_over_m_where_the_table_sends_it(hip, M, N, K):
 def test_rows_tiled_over_m_on_a_wider_n(hip, M, N, K, variant):
     print(f"gemm rows tiled over M, wider N M={M} N={N} K={K}", flush=True)
     xq, xs, wq, ws = _prep(M, N, K, seed=M + N)
+    if _lib_cus() == 256:
+        from lightllm_amd import _lib
+        assert hip.mi355_block_fp8_gemm_launched(M, N, K, 1 << 34, 0) == _lib.GEMM_ROWS_MTILED
     c = _run(xq, xs, wq, ws, None)
     assert torch.equal(c.view(torch.int16), _run(xq, xs, wq, ws, variant).view(torch.int16))
     _dequant_close(c, xq, xs, wq, ws)
@@ -810,7 +824,11 @@ def test_generic_strides(hip):
 @pytest.mark.parametrize("variant,M,N,K", [("rows128", 100, 1000, 2048), ("rows128", 300, 640, 4096), ("rows128", 64, 160 * 150, 256),
                                            ("tile128", 200, 520, 4096), ("tile256", 300, 520, 1024), ("tile256x128", 768, 520, 4096),
                                            ("skinny", 20, 1000, 4096), ("streamcu", 12, 4096, 4096), ("xshare", 40, 4096, 1024), ("tile256streamk", 600, 1024, 8192),
-                                           ("rowsm", 700, 1000, 2048), ("rowsm", 3000, 2112, 512), (None, 512, 36864, 256)])
+                                           ("rowsm", 700, 1000, 2048), ("rowsm", 3000, 2112, 512), (None, 512, 36864, 256),
+                                           # 65..128 rows, K whole and shared, 209..352 rows in tiles over M, K shared on eight waves
+                                           ("skinny128", 72, 4090, 4096), ("skinny128", 100, 1000, 4096), ("skinny128", 128, 520, 20608),
+                                           (None, 333, 12300, 1536), (None, 250, 16400, 1664), ("skinny", 48, 2112, 7168),
+                                           ("skinny", 64, 1000, 8192)])
 def test_padded_rows_through_the_c_abi(hip, variant, M, N, K):
     """Operands whose rows are longer than they need be (lda > K, ldb_n > K, ldc > N, padded scale rows), as a
     caller that slices larger buffers passes them: every fast kernel against its own result on packed operands
@@ -891,6 +909,8 @@ def test_quant_method_apply(hip):
                                            ("xshare", 50, 4096, 1024), ("tile256streamk", 1000, 2048, 16384),
                                            ("rows128", 100, 1000, 512), ("rows128", 128, 4104, 14336), ("rows128", 250, 1004, 4096),
                                            ("rowsm", 900, 1004, 1024), ("rowsm", 3000, 2112, 512),
+                                           ("skinny128", 72, 4090, 4096), ("skinny128", 100, 1000, 4096), (None, 333, 12300, 1536),
+                                           ("skinny", 48, 2112, 7168), ("skinny", 64, 1000, 8192), ("skinny", 24, 66000, 512),
                                            ("generic", 7, 130, 256), (None, 64, 28672, 4096), (None, 1024, 2112, 7168)])
 def test_fp16_output(hip, variant, M, N, K):
     """C in fp16: the fp32 accumulator is cast to the dtype of C (fp8w8a8_block_gemm_kernel.py:78; LightLLM allocates C
