@@ -458,13 +458,13 @@ struct RowsMPlan {
     int mt, wv, tiles_m, tiles_n;
 };
 static RowsMPlan rowsm_plan(int64_t M, int64_t N, int64_t K, int cus);
-static bool rows128_two_tiles(int64_t M, int64_t N, int64_t K, int cus);  // M in two tiles: rowsm_plan's launch
+static bool rows128_over_m(int64_t M, int64_t N, int64_t K, int cus);  // two to four tiles over M: rowsm_plan's launch
 
 static Rows128Plan rows128_plan(int64_t M, int64_t N, int64_t K, int cus) {
     Rows128Plan pl;
     const int64_t KB = K / kBlockK;
     pl.turned = false;
-    if (rows128_two_tiles(M, N, K, cus)) {
+    if (rows128_over_m(M, N, K, cus)) {
         const RowsMPlan mp = rowsm_plan(M, N, K, cus);
         return {mp.wv, 32 * mp.wv, 1, mp.tiles_m * mp.tiles_n, 2, false};
     }
@@ -577,7 +577,7 @@ static bool rows128_ahead_of_stream(int64_t M, int64_t N, int64_t K, int cus) {
 // the faster one on the larger weights (rows128_ahead_of_stream), at 16 rows on a few kinds of them (below).
 static bool rows128_pays(int64_t M, int64_t N, int64_t K, int cus) {
     if (M > 384 || M < 16) return false;
-    if (rows128_two_tiles(M, N, K, cus)) return true;
+    if (rows128_over_m(M, N, K, cus)) return true;
     if (M == 16) {
         // large weights whose 64-row workgroups come to just over one per unit (N = 18432, K = 7168: 27.5 us against 30.3
         // for the streaming kernel), a very long K (N = 8192, K = 28672: 45.3 against 50.7), or workgroups that spill into a
@@ -642,7 +642,7 @@ static bool rows128_pays(int64_t M, int64_t N, int64_t K, int cus) {
 static bool rowsm_limits_ok(const RowsMPlan &pl, int64_t M, int64_t K, int64_t lda, int64_t as_m, int64_t as_k);
 static bool rows128_limits_ok(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t as_m, int64_t as_k, int cus) {
     if (M > 384) return false;
-    if (rows128_two_tiles(M, N, K, cus)) return rowsm_limits_ok(rowsm_plan(M, N, K, cus), M, K, lda, as_m, as_k);
+    if (rows128_over_m(M, N, K, cus)) return rowsm_limits_ok(rowsm_plan(M, N, K, cus), M, K, lda, as_m, as_k);
     if (M * lda >= (1ll << 32) || M * as_m * 4 >= (1ll << 32) || as_k * 32 >= (1ll << 32)) return false;
     const Rows128Plan pl = rows128_plan(M, N, K, cus);
     const int64_t steps = (K / kBlockK + pl.splits - 1) / pl.splits;
@@ -787,12 +787,13 @@ static bool rowsm_pays(int64_t M, int64_t N, int64_t K, int cus) {
     return pl.mt >= 2 && pl.mt <= 6 && N <= 3072;
 }
 
-// 209..352 rows on a wide N: ROWS128 as two m tiles of up to 11 row blocks in one round instead of two 256-row tiles, a third of
-// them padding, or 128x128 tiles in two rounds (us, before / here: N = 27648, K = 5120, M = 220 / 288 / 333 / 352 59.1 / 68.2 /
-// 73.7 / 69.2 against 53.7 / 58.9 / 67.4 / 66.6, at 384 level; 28672 x 4608, M = 300 63.7 / 56.3; 15360 x 5120, M = 330 54.2 /
-// 45.8; 24576 x 1536, M = 333 27.4 / 22.3; 16384 x 4096, M = 256 40.8 / 36.7).  (K = 4096 beyond N = 16384 is on record with
-// the square tiles, although the gain is the same there: 28672 x 4096, M = 224 / 320 48.5 / 60.7 against 44.3 / 51.9.)
-static bool rows128_two_tiles(int64_t M, int64_t N, int64_t K, int cus) {
+// 209..352 rows on a wide N: ROWS128 as two (on a narrower N three or four) m tiles of up to 11 row blocks in one round instead
+// of two 256-row tiles, a third of them padding, or 128x128 tiles in two rounds (us, before / here: N = 27648, K = 5120, M = 220 / 288
+// / 333 / 352 59.1 / 68.2 / 73.7 / 69.2 against 53.7 / 58.9 / 67.4 / 66.6, at 384 level; 28672 x 4608, M = 300 63.7 / 56.3; 15360 x
+// 5120, M = 330 54.2 / 45.8; 24576 x 1536, M = 333 27.4 / 22.3; 16384 x 4096, M = 256 40.8 / 36.7).  (K = 4096 beyond N = 16384
+// keeps the square tiles by name as well, although the gain is the same there: 28672 x 4096, M = 224 / 320 48.5 / 60.7
+// against 44.3 / 51.9.)
+static bool rows128_over_m(int64_t M, int64_t N, int64_t K, int cus) {
     const int64_t KB = K / kBlockK;
     if (M <= 208 || M > 352 || N < 12288 || KB < 12 || KB > 44 || (K % 4096 == 0 && N > 16384)) return false;
     const RowsMPlan pl = rowsm_plan(M, N, K, cus);
@@ -875,24 +876,19 @@ static int64_t n_split_rows(int64_t M, int64_t N, int64_t K, int cus);
 //     160..256 or of 80..112 (64) weight rows         the same, workgroups of that width, K unshared
 //   65 <= M <= 128, K >= 2048                        the same with 256 weight rows per workgroup; under the same name the
 //                                                    weight streaming kernel where one round of its tiles is ahead
-//                                                    (skinny_many_rows_plan)
-//   49 <= M <= 64, at most cus tiles, N*K >= 6e7,
-//     unless the streaming kernel is ahead
-//     (skinny_ahead_of_rows128)                       the same, unless the shared-activation kernel would run
-//   49 <= M <= 128, 0.55 cus .. cus tiles of 160,
-//     192 or 256 weight rows with K unshared          the same, workgroups of that width (up to 64 rows and N*K < 1e8
-//                                                    not where the streaming kernel is ahead)
-//   17 <= M <= 48, K % 4096 != 0 and either 64-row
-//     tiles in a third round, or N*K >= 1e8 and just
-//     over one per unit or K >= 18432; 33 <= M <= 48,
-//     N*K >= 8e7 where the streaming kernel would
-//     share K, or a single launch over K < 2048        the same
+//                                                    (skinny_many_rows_plan; mi355_block_fp8_gemm_launched tells)
+//   65 <= M <= 128, 0.55 cus .. cus tiles of 160,
+//     192 or 256 weight rows with K unshared          the same, workgroups of that width
+//   17 <= M <= 64, N*K >= 2e7, at most cus tiles,
+//     ahead of the weight streaming kernel
+//     (rows128_ahead_of_stream)                       the same
 //   M > 384, N <= 5120 (3072), K <= 5120 (7168), one
 //     round of tiles of at most 128 (96) rows; 385..960
 //     rows, N <= 15360, K <= 5120                     the same kernel tiled over M, K unshared
-//   209..352 rows, N >= 12288, 1536 <= K <= 5632      the same, two tiles over M
-//   M <= 64                                          weight streaming (M > 48 and N/128 about the unit count: the
-//                                                    kernel that shares the activation block in the workgroup)
+//   209..352 rows, N >= 12288, 1536 <= K <= 5632      the same, two to four tiles over M (mi355_block_fp8_gemm_launched)
+//   M <= 64                                          weight streaming (M > 48 and N/128 about the unit count, or M > 32 in
+//                                                    more than five rounds: the kernel that shares the activation block
+//                                                    in the workgroup)
 //   few 256x256 tiles, long K                        stream-K (the plain loop would leave most units idle)
 //   128x128 tiles fit one round of two per unit and
 //     (few 256x256 tiles or a short K)               128x128 tiles, K shared between workgroups when they are few
@@ -1055,7 +1051,7 @@ static int skinny_rows_check(int64_t M, int64_t N, int64_t K, int64_t lda, int64
 static int launched_for(int variant, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int64_t as_m, bool ws_usable,
                         size_t ws_bytes, int cus) {
     if (variant != MI355_GEMM_ROWS128) return variant;
-    if (rows128_two_tiles(M, N, K, cus)) return MI355_GEMM_ROWS_MTILED;
+    if (rows128_over_m(M, N, K, cus)) return MI355_GEMM_ROWS_MTILED;
     return skinny_rows_check(M, N, K, lda, ldw, as_m, cus, ws_usable, ws_bytes) == MI355_OK ? MI355_GEMM_SKINNY_ROWS : variant;
 }
 
@@ -1218,7 +1214,7 @@ static int block_fp8_gemm_impl(const void *A, const void *B, const float *As, co
         }
         case MI355_GEMM_ROWS128: {
             if (!rows128_limits_ok(M, N, K, lda, as_m, as_k, cus)) return MI355_EUNSUPPORTED;
-            if (rows128_two_tiles(M, N, K, cus)) return launch_rowsm(a, rowsm_plan(M, N, K, cus), st);
+            if (rows128_over_m(M, N, K, cus)) return launch_rowsm(a, rowsm_plan(M, N, K, cus), st);
             Rows128Plan pl = rows128_plan(M, N, K, cus);
             pl.turned = was_auto || M <= 64;
             if (pl.splits > 1 && (!ws || ws_bytes < rows128_workspace(M, N, K, cus) || ((uintptr_t)ws & 15)))

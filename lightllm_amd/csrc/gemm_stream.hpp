@@ -2,7 +2,8 @@
 //
 // At these sizes the GEMM is a single pass over the N x K weight bytes, so the kernel is built around the
 // memory system, not the MFMA: every wave issues plain 16-byte-per-lane global loads in which 8 consecutive
-// lanes cover one 128-byte row segment (fully coalesced), keeps one (from 17 rows on) to three K steps of them in flight in registers,
+// lanes cover one 128-byte row segment (fully coalesced), keeps one (from 17 rows on; two in some tiles of 17..32 rows) to three
+// K steps of them in flight in registers,
 // and only then rearranges the bytes into MFMA operand order through a small wave-private LDS area
 // (ds_write_b128 / ds_read_b128, no workgroup barrier in the loop).  Loads that target LDS directly
 // (global_load_lds) sustain visibly less HBM bandwidth than plain loads on this part, which is why the
@@ -11,7 +12,7 @@
 // Work decomposition
 //   CTA = 4 or 8 waves (WV), owns 16*TNW weight rows (n) and a contiguous range of K steps (cross-CTA split-K only
 //   when N alone gives too few CTAs; stream_plan.hpp picks TNW, WV and the split).  Inside the CTA
-//   the waves take the K steps round-robin, so the four waves together read 512 consecutive bytes of every
+//   the waves take the K steps round-robin, so four waves together read 512 consecutive bytes of every
 //   row; each wave multiplies all its rows (TNW MFMA row blocks) by all 16*MT token rows for its own K steps
 //   and folds the scales exactly like the tiled kernel
 //   (acc += partial * (Xs[m,kb] * Ws[nb,kb])).  After the loop the partial accumulators of the waves are added
@@ -62,10 +63,11 @@ struct StreamCfg {
     static_assert(MT <= 8, "");
     static constexpr int BN = 16 * TNW;
     // K steps in flight per wave.  Occupancy counts for more than depth: from 17 rows on one step per wave and more
-    // waves is ahead of two or three steps on every shape tried (N = 6144, K = 4096, M = 48, eight waves: 10.3 us at
-    // depth 1, 11.0 at 2, 14.5 at 4; M <= 16 best at depth 3).
+    // waves is ahead of two or three steps (N = 6144, K = 4096, M = 48, eight waves: 10.3 us at depth 1, 11.0 at 2, 14.5
+    // at 4), but for 64-row tiles of 17..32 rows in four rounds and more, which take two (DEEP below); M <= 16 best at depth 3.
     static constexpr int depth(bool xs_in_lds) {
-        if (xs_in_lds || MT > 1) return MT == 1 ? 3 : 1;
+        if (MT > 1) return 1;
+        if (xs_in_lds) return 3;
         const int set = 8 * TNW + 9 * MT + 1;  // registers of one in-flight K step
         return set * 6 <= 150 ? 6 : (150 / set < 2 ? 2 : 150 / set);
     }

@@ -198,20 +198,21 @@ __global__ __launch_bounds__(512) void block_fp8_gemm_streamcu_kernel(const Gemm
     // ---- the stream: D register sets rotate; the compiler places the vmcnt waits
     Regs regs[D];
     auto staged = [&]() {
-    if constexpr (XR == 0) {
+        if constexpr (XR == 0) {
 #pragma unroll
-        for (int u = 0; u < kSv; ++u) {
-            const int row = (u % MT) * 16 + (tid >> 5), kb = (u / MT) * 32 + (tid & 31);
-            if (u < sv_units && kb < KB) xs_lds[kb * Cfg::kScaleStride + row] = sv[u];
+            for (int u = 0; u < kSv; ++u) {
+                const int row = (u % MT) * 16 + (tid >> 5), kb = (u / MT) * 32 + (tid & 31);
+                if (u < sv_units && kb < KB) xs_lds[kb * Cfg::kScaleStride + row] = sv[u];
+            }
         }
-    }
-    if ((tid & 255) < KB) ws_lds[(tid >> 8) * KB + (tid & 255)] = wsv;
-    __syncthreads();  // the staged scales are visible
+        if ((tid & 255) < KB) ws_lds[(tid >> 8) * KB + (tid & 255)] = wsv;
+        __syncthreads();  // the staged scales are visible
     };
-    // Few K steps, the same number for every wave: all of them are requested at once and nothing else is.  The loop below
+    // Two, four or five K steps for every wave: all of them are requested at once and nothing else is.  The loop below
     // requests under conditions, and the compiler counts the requests that may be outstanding at a wait over all paths:
     // it waits for every one of them before the scales are staged and again before the first step is multiplied
-    // (N = K = 4096, one row, four steps a wave: 6.7 us, 5.9 without).
+    // (N = K = 4096, one row, four steps a wave: 6.7 us, 5.9 without).  Each count is a copy of the body; K = 2048, 4096 and
+    // 5120 were measured, three steps (K = 3072) and more than five were not and take the loop.
     auto all_at_once = [&](auto count) {
         constexpr int S = decltype(count)::value;
         if constexpr (S <= D) {

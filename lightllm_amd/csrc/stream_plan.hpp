@@ -15,7 +15,8 @@ inline bool fast_layout_ok(const void *A, const void *B, int64_t K, int64_t lda,
 
 // Where in its K range (of at least `steps` K steps) a tile starts: GemmArgs::turn_mask.  With rows a multiple of 4 KiB apart the
 // same K step of every row lies in the same few memory channels, and tiles that walk K in step queue there; started at
-// different steps they spread.  (K stands for the distance: a result does not depend on how a weight is padded.)  With any other distance the rows do that by themselves and turning only costs
+// different steps they spread.  (K stands for the distance: a result does not depend on how a weight is padded.  It does depend
+// on the tile a weight row lies in.)  With any other distance the rows do that by themselves and turning only costs
 // (K = 14336: 0 to 5 % slower), and a range of fewer than 32 steps - 4 KiB of a row - is spread by its neighbours already.
 // us, in step / turned: N = 6144, K = 4096, M = 1 8.1 / 7.4; 28672 x 4096 21.0 / 19.5; 12288 x 4096 13.7 / 11.7; 57344 x 8192
 // 78.5 / 70.8; 8192 x 8192, M = 48, whole K on eight waves 21.8 / 17.3; a shared K of 16 steps is 1 to 3 % slower turned.
@@ -168,8 +169,8 @@ inline SkinnyPlan skinny_plan(int64_t M, int64_t N, int64_t K, int cus) {
 // the better of all candidates on average.  us, M = 72 / 96 / 128, before in brackets: N = K = 4096 11.3 / 12.4 / 14.6 (15.6
 // / 17.0 / 18.7), 6144 x 4096 13.0 / 14.6 (16.0 / 17.1), 7168 x 2048 9.0 / 10.1 (15.2 / 16.6), 2112 x 7168 12.0 / 13.5 (16.0 /
 // 17.2), M = 128 there stays.  32 weight rows stop at 112: with eight row blocks the accumulators spill (6144 x 4096, M =
-// 128: 25.9 against 18.4).  Up to 512 weight rows the other kernel's sums are on record although this one is ahead (512 x
-// 7168, M = 80 / 128: 9.0 / 10.8 against 11.9 / 13.6).  tnw 0: not here.
+// 128: 25.9 against 18.4).  Up to 512 weight rows the other kernel keeps the launch, whose sums are compared by name with the
+// table's, although this one is ahead (512 x 7168, M = 80 / 128: 9.0 / 10.8 against 11.9 / 13.6).  tnw 0: not here.
 inline SkinnyPlan skinny_many_rows_plan(int64_t M, int64_t N, int64_t K, int cus) {
     SkinnyPlan best = {0, 1, 0, 8};
     if (M <= 64 || M > 128 || N <= 512 || K % kBlockK != 0 || K / kBlockK < 16) return best;
