@@ -363,7 +363,7 @@ static int launch_streamcu_turn(GemmArgs &a, hipStream_t st) {
 
 template <int TNW>
 static int launch_streamcu_as(GemmArgs &a, hipStream_t st) {
-    a.turn_mask = stream_turn_mask(a.K, a.K / kBlockK);
+    a.turn_mask = streamcu_turn_mask(a.K, TNW);
     return a.turn_mask ? launch_streamcu_turn<TNW, true>(a, st) : launch_streamcu_turn<TNW, false>(a, st);
 }
 

@@ -59,7 +59,7 @@ static int launch_cu_as(GemmArgs &a, hipStream_t st) {
 
 template <int TB, int XR, bool F16>
 static int launch_cu(GemmArgs &a, hipStream_t st) {
-    a.turn_mask = stream_turn_mask(a.K, a.K / kBlockK);
+    a.turn_mask = streamcu_turn_mask(a.K, TB);
     return a.turn_mask ? launch_cu_as<TB, XR, F16, true>(a, st) : launch_cu_as<TB, XR, F16, false>(a, st);
 }
 

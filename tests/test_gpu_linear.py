@@ -47,15 +47,16 @@ def test_quantized_in_the_stream(hip, N, K, dtype):
 
 
 # 64-row tiles with K whole over more steps than the stream stages activation scales for, K a multiple of 4096: the starts of
-# the tiles are turned, in the quantizing stream and behind the quantizer alike
-@pytest.mark.parametrize("M,N,K", [(1, 16384, 12288), (4, 16384, 12288), (3, 16380, 16384)])
-def test_quantized_in_the_stream_on_a_long_k(hip, M, N, K):
+# the tiles are turned, in the quantizing stream and behind the quantizer alike; the per-unit stream of five row blocks, where
+# they are not
+@pytest.mark.parametrize("M,N,K,variant", [(1, 16384, 12288, 3), (4, 16384, 12288, 3), (3, 16380, 16384, 3), (4, 19200, 16384, 11)])
+def test_quantized_in_the_stream_on_a_long_k(hip, M, N, K, variant):
     from lightllm_amd import _lib
     from lightllm_amd.quantization import QUANTMETHODS, WeightPack
 
     print(f"linear M={M} N={N} K={K}", flush=True)
     assert hip.mi355_block_fp8_linear_fused(M, N, K, _lib.DTYPE_CODES[torch.bfloat16]) == 1
-    assert hip.mi355_block_fp8_gemm_variant(M, N, K) == _lib.GEMM_SKINNY
+    assert hip.mi355_block_fp8_gemm_variant(M, N, K) == variant
     wq, ws = H.quantized_weights(N, K, seed=N + K, device="cuda")
     x = H.activations(M, K, seed=M, outliers=True).cuda()
     method, want = QUANTMETHODS.get("fp8w8a8-b128"), _composed(x, wq, ws, torch.bfloat16)
