@@ -156,8 +156,9 @@ int32_t mi355_block_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, size_t ws_byt
 
 /* The code of the kernel that the call of mi355_block_fp8_gemm_plan launches.  It differs from the plan's where the table's
  * MI355_GEMM_ROWS128 covers more than one kernel: MI355_GEMM_SKINNY_ROWS at 65..128 rows, MI355_GEMM_ROWS_MTILED at 209..352.
- * Asked for by this code a launch is AUTO's, bit for bit, but for MI355_GEMM_ROWS128 at 65..128 rows (see there) and the
- * second launch that MI355_GEMM_TILE256 may be followed by.  Launches nothing; no counterpart in the reference. */
+ * Asked for by this code a launch is AUTO's, bit for bit, but for MI355_GEMM_ROWS128 from 65 rows on under K a multiple of 4096
+ * (see there) and the second launch that MI355_GEMM_TILE256 may be followed by.  Launches nothing; no counterpart in the
+ * reference. */
 int32_t mi355_block_fp8_gemm_launched(int64_t M, int64_t N, int64_t K, size_t ws_bytes, int32_t cus);
 
 /* Bytes of workspace the launch plan of the CURRENT device needs for this shape and variant (0 = none). */
