@@ -387,13 +387,12 @@ static int launch_streamcu(GemmArgs &a, int tnw, hipStream_t st) {
 constexpr int kXshareDepth = 4;
 using XshareCfg = ShareCfg<4, 2, kXshareDepth>;
 
-// 33..48 rows: three row blocks on the first kernel are ahead where they run turned or in up to five rounds of 64-row tiles (N =
-// 66176, K = 7424, M = 38 98.0 us against 119 here), this one beyond (86144 x 12672, M = 46 227 against 210; 116480 x 1280, M =
-// 40 38.9 / 35.2).
+// 33..48 rows: three row blocks on the first kernel are ahead where they run turned or in up to five rounds of 64-row tiles over 8
+// K steps and more (N = 66176, K = 7424, M = 38 98.0 us against 119 here), this one beyond (86144 x 12672, M = 46 227 against 210;
+// 116480 x 1280, M = 40 38.9 / 35.2; 79616 x 256, M = 34 12.9 / 10.3).
 static bool xshare_pays(int64_t M, int64_t N, int64_t K, int cus) {
-    if (M <= 32 || M > 64 || K / kBlockK > XshareCfg::kMaxScaleSteps) return false;
-    if (M <= 48) return K % 4096 != 0 && (N + 63) / 64 >= 5 * (int64_t)cus;
-    return (N + 127) / 128 >= (int64_t)cus * 3 / 4;
+    if (M <= 32 || M > 64 || K / kBlockK > XshareCfg::kMaxScaleSteps || (N + 127) / 128 < (int64_t)cus * 3 / 4) return false;
+    return M > 48 || (K % 4096 != 0 && (K < 1024 || (N + 63) / 64 >= 5 * (int64_t)cus));
 }
 
 // 128-row workgroup tiles; the K range is split in two while that leaves fewer than two workgroups per compute unit
@@ -544,9 +543,9 @@ static bool rows128_ahead_of_stream(int64_t M, int64_t N, int64_t K, int cus) {
     const Rows128Plan pl = rows128_plan(M, N, K, cus);
     const SkinnyPlan sp = skinny_plan(M, N, K, cus);
     const int64_t t64 = (N + 63) / 64, wgs = (int64_t)sp.tiles * sp.splits;
-    if (pl.tiles > cus || N * K < 20000000ll) return false;
     // a single well-filled launch: narrow or full-width workgroups on 0.55 cus .. cus tiles with K unshared
     const bool one_launch = pl.splits == 1 && pl.tiles * 20 >= (int64_t)cus * 11;
+    if (pl.tiles > cus || (N * K < 20000000ll && !one_launch)) return false;
     const bool over_one = t64 > cus && t64 * 4 <= 5 * (int64_t)cus;  // 64-row tiles that come to just over one per unit
     // kept here, where the sums of the table's launch are compared with those of this kernel by name, although the streaming kernel is
     // level or ahead: a short K (N = 24576, K = 1536, M = 48: 12.4 us here, 11.6), a very long one (7168 x 18432, M = 20 / 32: 28.5 /

@@ -309,6 +309,8 @@ def test_shape_table_at_17_to_64_rows():
         (39, 18096, 8192): ROWS, (22, 51200, 20480): ROWS, (30, 36864, 7168): ROWS,
         (40, 15360, 5120): SKINNY, (41, 19168, 2176): SKINNY, (33, 8192, 8192): SKINNY, (56, 12288, 4096): SKINNY, (24, 45504, 4096): SKINNY,
         (60, 16000, 4992): SKINNY, (48, 28672, 4096): SKINNY, (20, 40960, 4096): SKINNY,
+        # the same under few K steps, whatever the weights' size
+        (40, 30208, 512): ROWS, (19, 48128, 256): ROWS, (62, 36583, 384): ROWS, (46, 26624, 128): ROWS, (34, 79616, 256): XSHARE, (30, 12000, 512): SKINNY,
         # more than five rounds of 64-row tiles; turned starts
         (40, 116480, 1280): XSHARE, (46, 86144, 12672): XSHARE, (38, 66176, 7424): SKINNY, (43, 105664, 4096): SKINNY,
     }
