@@ -110,7 +110,7 @@ int mi355_block_weight_quant_fp8(const void *w, int32_t w_dtype, void *q, float 
 #define MI355_GEMM_TILE256 1     /* 256x256x128 CTA tile, 8 waves, LDS double buffer: compute-bound M */
 #define MI355_GEMM_TILE128 2     /* 128x128x128 CTA tile, 4 waves: mid M or few tiles */
 #define MI355_GEMM_SKINNY 3      /* weight-streaming split-K, M <= 64; from 17 rows on without a workspace it runs K whole
-                                    where N alone gives the units work (N above 12256 on 256) or K is below 4096 */
+                                    where N alone gives the units work (N above 12256 on 256); K is shared from 4096 on */
 #define MI355_GEMM_GENERIC 4     /* any strides, no MFMA; correctness fallback */
 #define MI355_GEMM_TILE256x128 5 /* 256x128x128 CTA tile, 8 waves */
 #define MI355_GEMM_TILE256_RING 6 /* the 256x256 tile on the plain ring pipeline (comparison / any scale layout) */

@@ -1268,7 +1268,7 @@ static int block_fp8_gemm_impl(const void *A, const void *B, const float *As, co
         }
         case MI355_GEMM_SKINNY: {
             const int ok = skinny_check(M, N, K, lda, ldb_n, as_m, cus, ws && ((uintptr_t)ws & 15) == 0, ws_bytes);
-            const bool whole = ok == MI355_EWORKSPACE && skinny_runs_whole(M, N, K, cus);  // (AUTO does not come here then)
+            const bool whole = ok == MI355_EWORKSPACE && skinny_runs_whole(M, N, cus);  // (AUTO does not come here then)
             if (ok != MI355_OK && !whole) return ok;
             const SkinnyPlan pl = whole ? skinny_whole_plan(N) : skinny_plan(M, N, K, cus);
             switch (skinny_mt(M)) {
@@ -1342,7 +1342,7 @@ extern "C" int mi355_block_fp8_gemm_noalloc(const void *A, const void *B, const 
     // a forced kernel that needs more than the array holds is an error; the shape table (MI355_GEMM_AUTO) gets
     // the whole array and takes the next best plan that fits into it
     if (need > kScratchBytes && variant != MI355_GEMM_AUTO &&
-        !(variant == MI355_GEMM_SKINNY && skinny_runs_whole(M, N, K, device_cus())))
+        !(variant == MI355_GEMM_SKINNY && skinny_runs_whole(M, N, device_cus())))
         return MI355_ESCRATCH;
     void *ws = nullptr;
     if (need > 0) {

@@ -47,10 +47,8 @@ struct SkinnyPlan {
 inline SkinnyPlan skinny_whole_plan(int64_t N) { return {4, 1, (int)((N + 63) / 64), 4, false}; }
 
 // Where a caller's own choice of the streaming kernel runs so if the workspace of its plan is missing: N alone gives the units
-// work, or K is too short to gain from being shared.
-inline bool skinny_runs_whole(int64_t M, int64_t N, int64_t K, int cus) {
-    return M > 16 && M <= 64 && ((N + 31) / 32 * 2 >= 3 * (int64_t)cus || K / kBlockK < 32);
-}
+// work.
+inline bool skinny_runs_whole(int64_t M, int64_t N, int cus) { return M > 16 && M <= 64 && (N + 31) / 32 * 2 >= 3 * (int64_t)cus; }
 
 // 17..64 rows: four or eight waves a workgroup, tiles of 16, 32 or 64 weight rows, K whole or shared by up to eight
 // workgroups.  What a launch takes, in ns and beside what all of them have in common: for each of the busiest unit's workgroups
@@ -58,8 +56,10 @@ inline bool skinny_runs_whole(int64_t M, int64_t N, int64_t K, int cus) {
 // workgroup reads all rows of its K range); 109 for each K step in a wave's sequence, 162 + 6.5 a wave for each accumulator (they
 // are added up through LDS), 483 and 230 for each workgroup that shares a tile and 3.8 us for a further round.  Tiles of 64
 // weight rows, one or none a unit, want 32 steps: under fewer, two of half the width are ahead (15616 x 2432, M = 23 9.6 us against
-// 11.0).  Fitted to every candidate timed on 1179 shapes (M = 17..64, N = 100..139000, K = 1024..21500, weights from HBM): the
-// choice is 0.9 % behind the best candidate on average and on 8 shapes more than 4 % behind the plan of before the eight-wave
+// 11.0).  K is shared from 32 steps on, so that a caller without a workspace keeps this kernel below (404 x 3456, M = 48, whole / in
+// three 7.7 / 7.3 us), and the partial sums stay within what the entry point without a workspace holds.
+// Fitted to every candidate timed on 1179 shapes (M = 17..64, N = 100..139000, K = 1024..21500, weights from HBM): the choice is
+// 0.9 % behind the best candidate on average and on 8 shapes more than 4 % behind the plan of before the eight-wave
 // forms, which ran 32- or 64-row tiles on four waves with K shared until there were two workgroups a unit.  (A fit to 22 shapes
 // of model linears, part of whose weights came from the memory-side cache, charged the weights at 41 and nothing for the
 // accumulators and was behind that plan on 70: 15722 x 1152, M = 62 12.1 us against 9.9; 8581 x 1280, M = 19 7.4 / 6.6.)  us,
@@ -101,7 +101,7 @@ inline SkinnyPlan skinny_wide_plan(int64_t M, int64_t N, int64_t K, int cus) {
             if (tiles * 4 > MI355_WS_COUNTER_BYTES) continue;  // one arrival counter a tile
             for (int s = 1; s <= 8; ++s) {
                 const int64_t wgs = tiles * s, steps = (KB + s - 1) / s;
-                if (s > 1 && (KB / s < 2 * waves || 2 * wgs > 5 * (int64_t)cus)) break;
+                if (s > 1 && (KB < 32 || KB / s < 2 * waves || 2 * wgs > 5 * (int64_t)cus || wgs * mt * tnw > MI355_NOALLOC_PARTIAL_MIB * 1024)) break;
                 if (steps > cap) continue;
                 const int64_t slots = skinny_wide_slots(waves, tnw, mt, steps);
                 const int64_t per_unit = (wgs + cus - 1) / cus, rounds = (wgs + cus * slots - 1) / (cus * slots);
