@@ -107,13 +107,21 @@ static int launch_gstream(GemmArgs &a, int block_m, int num_experts, hipStream_t
 #ifndef MI355_SK_PANEL
 #define MI355_SK_PANEL 1
 #endif
-// Runs per tile of the panel split (0 = none): the most that keep tiles * runs within the compute units, with
-// (m tiles * runs) a multiple of the 8 XCDs and at least 12 K steps in a run.
+// Runs per tile of the panel split (0 = none; otherwise tiles * runs is within the compute units).  A K step takes a
+// workgroup 1.3 us and the partial tiles, written once and read once, 0.1 us each, so there are as many runs as make
+// 1.3 steps + 0.1 tiles * runs least (us, runs: M = 256, N = 7168, K = 14336 54.3 / 51.7 / 48.6 / 49.5 / 50.2 with 5 .. 9, 7
+// here; M = 512, N = 2560, K = 20480 46.1 / 44.5 / 46.0 with 9 .. 11, 10 here; M = 640, N = 7168, K = 18432 177.9 /
+// 106.4 / 98.5 with 1 .. 3, which is what the units allow).
 static int sk_panel_splits(int tiles_m, int tiles_n, int KB, int cus) {
+    const int64_t tiles = (int64_t)tiles_m * tiles_n;
     int best = 0;
-    for (int s = 2; s <= 32; ++s) {
-        if ((int64_t)tiles_m * tiles_n * s > cus || KB / s < 12) break;
-        if ((tiles_m * s) % 8 == 0) best = s;
+    int64_t best_cost = 0;
+    for (int s = 2; s <= 32 && tiles * s <= cus && KB / s >= 8; ++s) {
+        const int64_t cost = 13 * ((KB + s - 1) / s) + tiles * s;
+        if (best == 0 || cost < best_cost) {
+            best = s;
+            best_cost = cost;
+        }
     }
     return best;
 }
@@ -139,11 +147,18 @@ static int stream_k_groups(int64_t tiles, int64_t KB, int cus, int64_t tiles_m =
 // about 2.5 times as long: sharing pays only where the plain loop leaves most of the device idle.
 static bool stream_k_pays(int64_t tiles, int64_t KB, int cus, int64_t tiles_m) {
     // a panel split that fills three eighths of the device with runs of a long K: measured ahead of every other
-    // kernel from 385 rows on (DeepSeek-V3 down, M = 1024: 128 us against 164 for one workgroup per tile; q_a+kv_a,
-    // M = 2048: 49.6 against 67.9; Llama-3 down, M = 512: 48.8 against 67.8; N = 4096, K = 7168, M = 512, 128
-    // workgroups: 34.5 against 39.8; N = 5120, K = 5120, M = 1024: 47.0 against 53.8), behind them with K = 4096
+    // kernel from 385 rows on, behind them with K = 4096 (us, before / here, 5 % slower to 64 % faster over 260 shapes of 385..4096 rows:
+    // 640 x 7168 x 18432 123 / 104, 640 x 4096 x 7168 57 / 40, 700 x 5120 x 13824 93 / 67, 1280 x 5120 x 8192 96 / 69,
+    // 1772 x 3760 x 27392 281 / 177; 1024 x 7168 x 18432, one workgroup per tile, 164 / 135)
     const int panel = tiles % tiles_m == 0 ? sk_panel_splits((int)tiles_m, (int)(tiles / tiles_m), (int)KB, cus) : 0;
-    if (MI355_SK_PANEL && panel > 0 && KB >= 40 && tiles * panel * 8 >= (int64_t)cus * 3) return true;
+    // (one to three m tiles on a narrow N: the 128-row tiles are ahead, 462 x 1840 x 9344 28.7 us against 32.4, 443 x 2608
+    // x 10240 36.9 / 38.4, 266 x 1232 x 12928 25.5 / 30.2, 597 x 1296 x 11136 30.8 / 34.7; 684 x 1696 x 10112 36.1 / 33.7)
+    const bool few = tiles_m <= 2 ? tiles * 64 < 3 * (int64_t)cus || (tiles * 32 < 3 * (int64_t)cus && KB < 96)
+                                  : tiles_m == 3 && tiles * 64 < 5 * (int64_t)cus && KB < 96;
+    // three m tiles under a short K or on a narrow N keep the 256x128 tiles, which share K the same way, whatever it costs
+    // (600 x 5120 x 6144 52 us against 42, 768 x 2112 x 8192 36.5 / 34.0)
+    const bool kept = tiles_m == 3 && (KB <= 48 || (tiles <= 27 && KB <= 64));
+    if (MI355_SK_PANEL && panel > 0 && KB >= 40 && tiles * panel * 8 >= (int64_t)cus * 3 && !few && !kept) return true;
     const int groups = stream_k_groups(tiles, KB, cus);
     if (groups == 0) return false;
     const int64_t plain = (tiles + groups - 1) / groups * KB, shared = (tiles * KB + groups - 1) / groups;
@@ -186,10 +201,10 @@ static int launch_pp(GemmArgs &a, void *ws, size_t ws_bytes, int cus, int sk_gro
             if (!ws_ok || ws_bytes < stream_k_workspace(sk_groups)) return MI355_EWORKSPACE;
             a.counters = (uint32_t *)ws;
             a.partials = (float *)((uint8_t *)ws + MI355_WS_COUNTER_BYTES);
-            // panel split where the shape allows it: every tile's K range in the same few runs, an XCD working on
-            // one (m tile, run) pair across all n tiles, so that its L2 holds the X rows its workgroups share
+            // panel split where the shape allows it: every tile's K range in the same few runs (the grid is rounded up to the
+            // 8 XCDs)
             a.splits = MI355_SK_PANEL ? sk_panel_splits(a.tiles_m, a.tiles_n, a.K / kBlockK, cus) : 0;
-            if (a.splits > 0) sk_groups = a.total_tiles * a.splits;
+            if (a.splits > 0) sk_groups = (a.total_tiles * a.splits + 7) / 8 * 8;
             const int r = sc4 ? launch_pp_as<false, true, true>(a, sk_groups, lds_bytes, st)
                               : launch_pp_as<false, true, false>(a, sk_groups, lds_bytes, st);
             if (r != MI355_OK) return r;

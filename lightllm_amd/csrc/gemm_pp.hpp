@@ -39,10 +39,12 @@
 //     fp32 accumulators to its own slot of the workspace (two slots per workgroup: a run starts and ends inside at
 //     most one tile each); a second launch (streamk_reduce_kernel) adds the parts of every shared tile in K order
 //     and stores it.  (Adding them in the last workgroup to arrive at a tile was 3 to 8 % slower: one compute unit
-//     reads the parts of a tile at a fraction of the rate the whole device does.)  Where the shape allows it the
-//     host asks for a panel split instead (p.splits > 0): every tile's K range in the same p.splits runs and one
-//     (m tile, run) pair per XCD across all n tiles, so that the workgroups of an XCD share their X rows in its L2
-//     - cut as one sequence, neighbouring runs share nothing and the launch is bound by what they all pull.
+//     reads the parts of a tile at a fraction of the rate the whole device does.)  Where the tiles fill at
+//     most half the device the host asks for a panel split instead (p.splits > 0): every tile's K range in the same
+//     p.splits runs, all m tiles (up to 8) of a few n tiles in one run per XCD, so that the workgroups of an XCD walk
+//     the same K steps of shared X and W rows - cut as one sequence, neighbouring runs share nothing and the launch is
+//     bound by what they all pull (M = 640, N = 7168, K = 18432, 84 tiles: 123 us as one sequence over 256
+//     workgroups, 104 as three runs over 252).
 //   * ROLES (grouped launch with a workspace): schedule blocks with at most 64 rows are weight streams, and this
 //     tile streams badly (32 KiB of W in flight per step, three quarters of the X area and half of the waves
 //     idle).  They go to the 64 x 512 tile of gemm_small.hpp instead, in the same launch: a split kernel has
@@ -144,17 +146,15 @@ __global__ __launch_bounds__(512) void block_fp8_gemm_pp_kernel(const GemmArgs p
     uint32_t u_first = SK ? (uint32_t)((uint64_t)rank * units / gridDim.x) : 0u;
     if constexpr (SK) {
         if (p.splits > 0) {
-            // panel split: every tile's K range is cut into p.splits runs; XCD x takes the (m tile, run) pairs
-            // 8*q + x and, of each, all n tiles - so the workgroups of an XCD read the same X rows and K steps at the
-            // same time and its L2 serves all but the first of them.  rank becomes tile * splits + run.
-            const uint32_t q = in_xcd / (uint32_t)p.tiles_n, tn = in_xcd - q * (uint32_t)p.tiles_n;
-            const uint32_t pr = q * 8u + xcd, tm = pr / (uint32_t)p.splits, run = pr - tm * (uint32_t)p.splits;
-            constexpr uint32_t GM = 8;
-            const uint32_t g = tm / GM, first_m = g * GM, gsz = min((uint32_t)p.tiles_m - first_m, GM);
-            const uint32_t id = g * GM * (uint32_t)p.tiles_n + tn * gsz + (tm - first_m);
+            // panel split: every tile's K range is cut into p.splits runs.  The workgroups in XCD order are numbered
+            // (run, tile in the dense order) and cut into eight equal parts, so that an XCD works on all m tiles (up to
+            // 8) of a few n tiles in one run: its workgroups read the same X and W rows at the same K steps and its L2
+            // serves all but the first of them.  rank becomes tile * splits + run.
+            const uint32_t run = rank / (uint32_t)p.total_tiles, id = rank - run * (uint32_t)p.total_tiles;
             const uint32_t per = (uint32_t)KB / (uint32_t)p.splits, rem = (uint32_t)KB % (uint32_t)p.splits;
             u_first = id * (uint32_t)KB + run * per + min(run, rem);
             u_end = u_first + per + (run < rem ? 1u : 0u);
+            if (run >= (uint32_t)p.splits) u_end = u_first;  // the grid is rounded up to the 8 XCDs: nothing to do
             rank = id * (uint32_t)p.splits + run;
         }
     }
@@ -557,8 +557,9 @@ __global__ __launch_bounds__(512) void block_fp8_gemm_pp_kernel(const GemmArgs p
                 const uint32_t mine = (p.splits > 0 ? rank : 2u * rank + (done.k0 == 0 ? 1u : 0u)) * (uint32_t)Cfg::kPartialBytes + lane_off;
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
+                    if (wave_m * WMS + 16 * i < done.rows)  // (rows past the matrix are not read either)
 #pragma unroll
-                    for (int j = 0; j < TN; ++j) xch.store(mine + (uint32_t)(i * TN + j) * kBlockStride, acc[i][j]);
+                        for (int j = 0; j < TN; ++j) xch.store(mine + (uint32_t)(i * TN + j) * kBlockStride, acc[i][j]);
                 store_tile = false;  // the second launch (streamk_reduce_kernel) adds the parts and stores the tile
             }
         }
@@ -660,6 +661,12 @@ __global__ __launch_bounds__(512) void streamk_reduce_kernel(const GemmArgs p, u
         first_slot = 2u * r_lo + 1u;
         step = 2u;
     }
+    constexpr uint32_t GM = 8;
+    const uint32_t width = GM * (uint32_t)p.tiles_n, g = id / width, first_m = g * GM;
+    const uint32_t gsz = min((uint32_t)p.tiles_m - first_m, GM), in_grp = id - g * width;
+    const int m0 = (int)(first_m + in_grp % gsz) * Cfg::BM, n0 = (int)(in_grp / gsz) * Cfg::BN;
+    const int rl = wave_m * WMS + 16 * (int)i + r16;
+    if (m0 + wave_m * WMS + 16 * (int)i >= p.M) return;  // (the first launch leaves no part of these rows)
     const uint8_t *base = (const uint8_t *)p.partials + (uint32_t)tid * 16u + i * TN * kBlockStride;
     v4f acc[TN];
 #pragma unroll
@@ -672,11 +679,6 @@ __global__ __launch_bounds__(512) void streamk_reduce_kernel(const GemmArgs p, u
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[j] += part[j];
     }
-    constexpr uint32_t GM = 8;
-    const uint32_t width = GM * (uint32_t)p.tiles_n, g = id / width, first_m = g * GM;
-    const uint32_t gsz = min((uint32_t)p.tiles_m - first_m, GM), in_grp = id - g * width;
-    const int m0 = (int)(first_m + in_grp % gsz) * Cfg::BM, n0 = (int)(in_grp / gsz) * Cfg::BN;
-    const int rl = wave_m * WMS + 16 * (int)i + r16;
     if (m0 + rl >= p.M) return;
     const int nbase = n0 + wave_n * WNS;
     uint16_t *cp = p.C + (int64_t)(m0 + rl) * p.ldc + nbase;

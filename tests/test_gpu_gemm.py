@@ -205,6 +205,30 @@ def test_stream_k_launch(hip, M, N, K):
     assert np.abs(got - ref64).max() <= H.GEMM_MAX_REL * np.abs(ref64).max()
 
 
+@pytest.mark.parametrize("M,N,K", [(513, 1024, 2048), (640, 1300, 4992), (700, 260, 16384), (1100, 700, 3200), (1500, 130, 7168),
+                                   (257, 256, 2176)])
+def test_panel_split_of_any_m_tiles(hip, M, N, K):
+    """The panel split where (tiles x runs) is no multiple of the 8 XCDs: the grid is rounded up and its last workgroups
+    have nothing to do; rows past M of the last m tile are neither written to the workspace nor read from it (it holds NaN
+    there).  Same products as the plain tile loop, K summed in runs: one bf16 step of the largest output at most."""
+    from lightllm_amd import _lib
+
+    print(f"gemm panel split M={M} N={N} K={K}", flush=True)
+    xq, xs, wq, ws = _prep(M, N, K, seed=M + N)
+    plain = _run(xq, xs, wq, ws, "tile256").clone()
+    need = hip.mi355_block_fp8_gemm_workspace_bytes(M, N, K, _lib.GEMM_TILE256_STREAMK)
+    assert need > _lib.WS_COUNTER_BYTES
+    _lib.workspace(xq.device, need)[_lib.WS_COUNTER_BYTES:].fill_(0xFF)
+    first = _run(xq, xs, wq, ws, "tile256streamk").clone()
+    assert torch.equal(_run(xq, xs, wq, ws, "tile256streamk").view(torch.int16), first.view(torch.int16))
+    assert (first.float() - plain.float()).abs().max() <= 2 ** -7 * plain.float().abs().max()
+    rows, cols = np.unique(np.r_[0:M:97, M - 1]), np.unique(np.r_[0:N:61, N - 1])
+    ref64 = oracle.dequant_matmul_sampled(tr.bits_of(xq[rows].contiguous()), xs[rows].cpu().numpy(), tr.bits_of(wq),
+                                          ws.cpu().numpy(), np.arange(len(rows)), cols)
+    got = first[rows][:, cols].float().cpu().double().numpy()
+    assert np.abs(got - ref64).max() <= H.GEMM_MAX_REL * np.abs(ref64).max()
+
+
 @pytest.mark.parametrize("M,N,K", [(4096, 16384, 1024), (4000, 16400, 1024), (1100, 16385, 1024)])
 def test_persistent_launch_matches_one_workgroup_per_tile(hip, M, N, K):
     """With the workspace counters the ping-pong kernel is persistent (one workgroup per CU; from the third tile
