@@ -92,13 +92,16 @@ __global__ __launch_bounds__(64 * WV) void block_fp8_gemm_rows128_kernel(const G
         tile_n = blockIdx.x / (uint32_t)p.splits;
         split = blockIdx.x - tile_n * (uint32_t)p.splits;
     } else if (p.tiles_m > 1) {
-        // more rows than one block holds: tiles_m x tiles_n tiles, n fastest, one contiguous run per XCD (workgroup
-        // ids go round-robin over the 8 XCDs), so the workgroups that share an L2 share their activation rows
+        // more rows than one block holds: tiles_m x tiles_n tiles, one contiguous run per XCD (workgroup ids go round-robin
+        // over the 8 XCDs), m fastest inside groups of group_m m tiles: a run is a compact block of tiles, and the L2 fetches
+        // the fewest distinct rows of X and W for it (rowsm_group)
         const uint32_t per_xcd = gridDim.x >> 3;  // the grid is a multiple of 8
         const uint32_t logical = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
         if (logical >= (uint32_t)p.total_tiles) return;
-        tile_m = logical / (uint32_t)p.tiles_n;
-        tile_n = logical - tile_m * (uint32_t)p.tiles_n;
+        const uint32_t width = (uint32_t)(p.group_m * p.tiles_n), first = logical / width * (uint32_t)p.group_m;
+        const uint32_t in_group = logical % width, group = min((uint32_t)p.tiles_m - first, (uint32_t)p.group_m);
+        tile_n = in_group / group;
+        tile_m = first + in_group - tile_n * group;
     } else {
         tile_n = blockIdx.x;
     }

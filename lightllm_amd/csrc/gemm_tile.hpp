@@ -53,6 +53,7 @@ struct GemmArgs {
     int64_t xs_m, xs_k, ws_n, ws_k;
     int32_t vec_store;   // 1: C rows are 16-byte aligned and N % 8 == 0
     int32_t out_f16;     // 0: C is bf16, 1: C is fp16
+    int32_t group_m;     // weight streams over several m tiles: tiles are numbered m first inside groups of so many m tiles
     int32_t turn_mask;   // weight streams: tile t starts (5 t & turn_mask) K steps into its K range (stream_turn_mask)
     // split-K launch only
     int32_t splits;
