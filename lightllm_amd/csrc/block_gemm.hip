@@ -666,14 +666,31 @@ static bool rows128_limits_ok(int64_t M, int64_t N, int64_t K, int64_t lda, int6
     return ((ring + nblk * steps * 4 + 127) & ~127ll) + 2 * 16 * mt * 32 <= 160 * 1024;
 }
 
-template <int MT, int WV, int TN = (MT <= 8 ? 2 : 1)>
+template <int MT, int WV, int TN = (MT <= 8 ? 2 : 1), int XS = 0>
 static int launch_rows128_as(GemmArgs &a, const Rows128Plan &pl, void *ws, hipStream_t st) {
-    constexpr int NS = MT <= 8 ? 3 : 2;
-    using Cfg = Rows128Cfg<MT, NS, TN, WV>;
+    using Cfg = Rows128Cfg<MT, TN, WV, XS>;
     const int KB = a.K / kBlockK;
     const int steps = (KB + pl.splits - 1) / pl.splits;
     const int lds_bytes = Cfg::lds_bytes(steps);
-    if (lds_bytes > 160 * 1024) return MI355_EUNSUPPORTED;
+    if (lds_bytes > 160 * 1024) {
+        // the weight scales of a very long K leave no room for a third slot of X: eight waves of 16 weight rows on two
+        if constexpr (Cfg::NSX == 3 && MT > 8) {
+            Rows128Plan two = pl;
+            two.wv = 8;
+            two.tn = 1;
+            two.bn = 128;
+            const int tiles_n = (a.N + 127) / 128;
+            if (a.tiles_m > 1) {
+                a.tiles_n = tiles_n;
+                a.total_tiles = a.tiles_m * tiles_n;
+                two.tiles = (a.total_tiles + 7) / 8 * 8;
+            } else {
+                two.tiles = tiles_n;
+            }
+            return launch_rows128_as<MT, 8, 1, 2>(a, two, ws, st);
+        }
+        return MI355_EUNSUPPORTED;
+    }
     if (pl.splits <= 1) {
         // Turned starts (stream_turn_mask) where a step is mostly weights: up to 96 rows (80 beyond K = 16384), or weights of
         // 200 MB and more (450 at K = 16384) (us, in step / turned: N = 28672, K = 4096, M = 64 / 80 / 128 29.2 / 30.5 / 36.2
@@ -689,17 +706,17 @@ static int launch_rows128_as(GemmArgs &a, const Rows128Plan &pl, void *ws, hipSt
             const bool weights_lead = a.M <= (a.K <= 16384 ? 96 : 80) || (a.K <= 16384 && weights >= (a.K < 16384 ? 200000000ll : 450000000ll));
             const bool meets = WV < 8 && a.K == 8192;
             if (pl.turned && weights_lead && !meets && a.tiles_m <= 1 && KB % 16 == 0 && (a.turn_mask = stream_turn_mask(a.K, KB)) != 0) {
-                constexpr auto turned = block_fp8_gemm_rows128_kernel<MT, NS, TN, WV, false, true>;
+                constexpr auto turned = block_fp8_gemm_rows128_kernel<MT, TN, WV, false, true, XS>;
                 if (!allow_lds<turned>(160 * 1024)) return MI355_ELAUNCH;
                 return launch(turned, dim3(pl.tiles), dim3(Cfg::kThreads), lds_bytes, st, a);
             }
         }
-        constexpr auto kernel = block_fp8_gemm_rows128_kernel<MT, NS, TN, WV, false>;
+        constexpr auto kernel = block_fp8_gemm_rows128_kernel<MT, TN, WV, false, false, XS>;
         if (!allow_lds<kernel>(160 * 1024)) return MI355_ELAUNCH;
         return launch(kernel, dim3(pl.tiles), dim3(Cfg::kThreads), lds_bytes, st, a);
     }
     if constexpr (WV == 8 && TN == (MT <= 8 ? 2 : 1)) {
-        constexpr auto kernel = block_fp8_gemm_rows128_kernel<MT, NS, TN, 8, true>;
+        constexpr auto kernel = block_fp8_gemm_rows128_kernel<MT, TN, 8, true, false, XS>;
         if (!allow_lds<kernel>(160 * 1024)) return MI355_ELAUNCH;
         a.splits = pl.splits;
         a.partials = (float *)((uint8_t *)ws + MI355_WS_COUNTER_BYTES);  // the counter words stay untouched
@@ -857,8 +874,8 @@ static int rowsm_group(const RowsMPlan &pl) {
 static int launch_rowsm(GemmArgs &a, const RowsMPlan &mp, hipStream_t st) {
     a.tiles_m = mp.tiles_m;
     a.tiles_n = mp.tiles_n;
-    a.total_tiles = mp.tiles_m * mp.tiles_n;
     a.group_m = rowsm_group(mp);
+    a.total_tiles = mp.tiles_m * mp.tiles_n;
     Rows128Plan pl;
     pl.turned = false;
     pl.wv = mp.wv;

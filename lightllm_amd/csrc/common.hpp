@@ -108,11 +108,20 @@ __device__ __forceinline__ void wait_vmcnt() {
     __builtin_amdgcn_s_waitcnt((N & 0xf) | ((N >> 4) << 14) | (0x7 << 4) | (0xf << 8));
 }
 
-// Workgroup barrier that waits for this wave's LDS traffic only (lgkmcnt 0; vmcnt untouched).
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_s_waitcnt(0xf | (0x3 << 14) | (0x7 << 4) | (0 << 8));
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);  // compiler only: no LDS access may move across the barrier
+// Waits until at most N of this wave's LDS operations are outstanding (they complete in order; vmcnt untouched).
+template <int N>
+__device__ __forceinline__ void wait_lgkm() {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);  // compiler only: no LDS access may move across the wait
     __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xf | (0x3 << 14) | (0x7 << 4) | (N << 8));
+    __builtin_amdgcn_sched_barrier(0);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+
+// Workgroup barrier that waits for this wave's LDS traffic only, all of it or all but the last OUTSTANDING operations.
+template <int OUTSTANDING = 0>
+__device__ __forceinline__ void lds_barrier() {
+    wait_lgkm<OUTSTANDING>();
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     __atomic_signal_fence(__ATOMIC_SEQ_CST);

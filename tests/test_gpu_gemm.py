@@ -595,6 +595,47 @@ def test_rows_tiled_over_m_where_the_table_sends_it(hip, M, N, K):
     assert torch.equal(_run(xq, xs, wq, ws, None).view(torch.int16), _run(xq, xs, wq, ws, "rowsm").view(torch.int16))
 
 
+# every count of K steps up to the pipeline's depth and beyond, over the row blocks where the ring slots, the groups of row blocks
+# or the workgroup change; ragged M and N
+@pytest.mark.parametrize("M", [1, 17, 33, 64, 80, 97, 128, 129, 160, 177, 208, 241, 272, 273, 289, 320, 384])
+def test_rows128_k_loop(hip, M):
+    """Fewer than 12 K steps are never shared, so the products are those of the 128x128 tile in the same order: bit-equal."""
+    for steps in range(1, 12):
+        N, K = (300, 128 * steps)
+        print(f"gemm rows128 K loop M={M} steps={steps}", flush=True)
+        xq, xs, wq, ws = _prep(M, N, K, seed=M + steps)
+        c = _run(xq, xs, wq, ws, "rows128").clone()
+        assert torch.equal(c.view(torch.int16), _run(xq, xs, wq, ws, "tile128").view(torch.int16)), steps
+        assert torch.equal(c, _run(xq, xs.t().contiguous().t(), wq, ws, "rows128")), steps
+        wide = torch.zeros((ws.shape[0], 7 * steps), device="cuda")[:, ::7].copy_(ws)  # weight scales with a stride along K
+        assert torch.equal(c, _run(xq, xs, wq, wide, "rows128")), steps
+
+
+@pytest.mark.parametrize("M,N,K", [(20, 512, 12288), (48, 300, 2560), (64, 700, 18432), (128, 512, 7168), (200, 260, 9216)])
+def test_rows128_shared_k_loop(hip, M, N, K):
+    """K shared between workgroups: fp32 sums of a few runs, one bf16 step of the largest output from the whole-K sum at most."""
+    print(f"gemm rows128 shared K M={M} N={N} K={K}", flush=True)
+    xq, xs, wq, ws = _prep(M, N, K, seed=M + N)
+    c = _run(xq, xs, wq, ws, "rows128").clone()
+    assert torch.equal(c, _run(xq, xs, wq, ws, "rows128"))
+    t = _run(xq, xs, wq, ws, "generic").float()
+    assert (c.float() - t).abs().max() <= 2 ** -7 * t.abs().max()
+
+
+def test_rows_tiled_over_m_very_long_k(hip):
+    """13 row blocks on eight waves: from K = 54656 on the weight scales leave no room for a third slot of X, and the launch takes
+    eight waves of 16 weight rows on two slots."""
+    M, N, K = 53248, 250, 55040
+    print(f"gemm rows tiled over M, very long K M={M} N={N} K={K}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    xq = torch.randint(0, 0x78, (M, K), generator=g, device="cuda", dtype=torch.uint8).view(torch.float8_e4m3fn)
+    wq = torch.randint(0, 0x78, (N, K), generator=g, device="cuda", dtype=torch.uint8).view(torch.float8_e4m3fn)
+    xs = torch.rand((M, K // 128), generator=g, device="cuda") + 0.5
+    ws = torch.rand((2, K // 128), generator=g, device="cuda") - 0.5
+    c = _run(xq, xs, wq, ws, "rowsm").clone()
+    assert torch.equal(c.view(torch.int16), _run(xq, xs, wq, ws, "tile128").view(torch.int16))
+
+
 # 209..352 rows in two or three tiles of the activation-block stream, 385..960 rows on a wider N: the edges of both ranges, row counts
 # that leave the last tile one row, N that leaves the last column of tiles one weight row, the shortest and longest K
 @pytest.mark.parametrize("M,N,K,variant", [(209, 12288, 2048, "rows128"), (225, 12289, 1536, "rows128"), (352, 27648, 1536, "rows128"),
