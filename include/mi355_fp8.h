@@ -132,10 +132,10 @@ int mi355_block_weight_quant_fp8(const void *w, int32_t w_dtype, void *q, float 
                                   one workgroup of 8 waves per share and the whole K (no partial sums between
                                   workgroups); where N / 16 gives the units 1..5 row blocks each */
 
-#define MI355_GEMM_ROWS_MTILED 12 /* the kernel of MI355_GEMM_ROWS128 tiled over M as well: one round of tiles of
-                                     16..128 rows x 160..256 weight rows, K unshared, no workspace; for more than 384
-                                     rows on a narrow N (at most 5120 weight rows, K <= 7168; 385..960 rows: at most 15360,
-                                     K <= 5120) */
+#define MI355_GEMM_ROWS_MTILED 12 /* the kernel of MI355_GEMM_ROWS128 tiled over M as well: tiles of 16..208 rows x
+                                     160..256 weight rows, K unshared, no workspace; by this name where one round of them
+                                     exists (the table's name for more than 384 rows on a narrow N: at most 5120 weight
+                                     rows, K <= 7168; 385..960 rows: at most 15360, K <= 5120) */
 
 #define MI355_GEMM_SKINNY_ROWS 13 /* the kernel of MI355_GEMM_SKINNY at 65..128 rows, one round of eight-wave tiles; where the
                                      shape table would launch it (mi355_block_fp8_gemm_launched) */
@@ -157,9 +157,15 @@ int32_t mi355_block_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, size_t ws_byt
 /* The code of the kernel that the call of mi355_block_fp8_gemm_plan launches.  It differs from the plan's where the table's
  * MI355_GEMM_ROWS128 covers more than one kernel: MI355_GEMM_SKINNY_ROWS at 65..128 rows, MI355_GEMM_ROWS_MTILED at 209..352.
  * Asked for by this code a launch is AUTO's, bit for bit, but for MI355_GEMM_ROWS128 from 65 rows on under K a multiple of 4096
- * (see there) and the second launch that MI355_GEMM_TILE256 may be followed by.  Launches nothing; no counterpart in the
- * reference. */
+ * (see there), the second launch that MI355_GEMM_TILE256 may be followed by and calls that run as tiles over M
+ * (mi355_block_fp8_gemm_over_m).  Launches nothing; no counterpart in the reference. */
 int32_t mi355_block_fp8_gemm_launched(int64_t M, int64_t N, int64_t K, size_t ws_bytes, int32_t cus);
+
+/* 1 where that AUTO call runs as tiles over M (the kernel of MI355_GEMM_ROWS_MTILED, in up to four rounds) instead of the kernel
+ * above, 0 where not: at 209..4096 rows, N >= 640 and 1024 <= K <= 20480 it does wherever the tiles are estimated to be 3 % ahead.
+ * K is never shared in them, so the result has the bits of MI355_GEMM_TILE256, and of the kernel above unless that shares K.
+ * Launches nothing; no counterpart in the reference. */
+int32_t mi355_block_fp8_gemm_over_m(int64_t M, int64_t N, int64_t K, size_t ws_bytes, int32_t cus);
 
 /* Bytes of workspace the launch plan of the CURRENT device needs for this shape and variant (0 = none). */
 size_t mi355_block_fp8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t variant);

@@ -33,6 +33,7 @@ SIGNATURES = {
     "mi355_block_fp8_gemm_variant": (_i32, [_i64, _i64, _i64]),
     "mi355_block_fp8_gemm_plan": (_i32, [_i64, _i64, _i64, _sz, _i32]),
     "mi355_block_fp8_gemm_launched": (_i32, [_i64, _i64, _i64, _sz, _i32]),
+    "mi355_block_fp8_gemm_over_m": (_i32, [_i64, _i64, _i64, _sz, _i32]),
     "mi355_block_fp8_gemm_workspace_bytes": (_sz, [_i64, _i64, _i64, _i32]),
     "mi355_block_fp8_gemm_noalloc": (
         _c.c_int,

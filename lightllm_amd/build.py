@@ -11,7 +11,7 @@ CSRC = os.path.join(_HERE, "csrc")
 LIB_DIR = os.path.join(_HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libmi355fp8.so")
 CALL_PATH = os.path.join(LIB_DIR, "_mi355call" + importlib.machinery.EXTENSION_SUFFIXES[0])
-SOURCES = ["capi.hip", "group_quant.hip", "weight_quant.hip", "block_gemm.hip", "linear.hip", "moe_align.hip", "moe_elementwise.hip", "routed_ffn.hip", "probe.hip"]
+SOURCES = ["capi.hip", "group_quant.hip", "weight_quant.hip", "block_gemm.hip", "rows128_few.hip", "rows128_some.hip", "rows128_many.hip", "linear.hip", "moe_align.hip", "moe_elementwise.hip", "routed_ffn.hip", "probe.hip"]
 # packed-fp32 VALU ops are switched off for every kernel of this library
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",

@@ -7,7 +7,7 @@
 #include "gemm_stream.hpp"
 #include "gemm_streamcu.hpp"
 #include "gemm_xshare.hpp"
-#include "gemm_rows128.hpp"
+#include "rows128_launch.hpp"
 #include "gemm_tile.hpp"
 #include "stream_plan.hpp"
 
@@ -454,7 +454,6 @@ static int launch_xshare(GemmArgs &a, int splits, void *ws, hipStream_t st) {
 constexpr int kRows128MinSteps = 6;
 
 static int rows128_mt(int64_t M) { return (int)((M + 15) / 16); }
-constexpr int64_t kRows128NarrowMaxM = 208;  // the last row count with narrow workgroups above 128 rows
 
 // Workgroup width, K sharing and tile count of a launch.  Up to 128 rows a workgroup is 8 waves x 32 weight rows;
 // beyond, 8 waves x 16.  While the tiles leave compute units idle the K range is shared, never below
@@ -463,11 +462,6 @@ constexpr int64_t kRows128NarrowMaxM = 208;  // the last row count with narrow w
 // more, narrower workgroups mean fewer bytes per unit.  It is taken when such a width gives between 0.55 cus and cus
 // tiles (DeepSeek-V3 gate_up, N = 36864: 231 tiles of 160 rows, M = 64 / 128: 50.3 / 62.8 us against 59.4 / 68.8
 // for 144 tiles of 256; q_b, N = 24576, K = 1536: 16.6 against 21.4 with K shared by two).
-struct Rows128Plan {
-    int wv, bn, splits, tiles, tn;
-    bool turned;  // tiles may start at different K steps (launch_rows128_as)
-};
-
 struct RowsMPlan {
     int mt, wv, tiles_m, tiles_n;
 };
@@ -666,104 +660,15 @@ static bool rows128_limits_ok(int64_t M, int64_t N, int64_t K, int64_t lda, int6
     return ((ring + nblk * steps * 4 + 127) & ~127ll) + 2 * 16 * mt * 32 <= 160 * 1024;
 }
 
-template <int MT, int WV, int TN = (MT <= 8 ? 2 : 1), int XS = 0>
-static int launch_rows128_as(GemmArgs &a, const Rows128Plan &pl, void *ws, hipStream_t st) {
-    using Cfg = Rows128Cfg<MT, TN, WV, XS>;
-    const int KB = a.K / kBlockK;
-    const int steps = (KB + pl.splits - 1) / pl.splits;
-    const int lds_bytes = Cfg::lds_bytes(steps);
-    if (lds_bytes > 160 * 1024) {
-        // the weight scales of a very long K leave no room for a third slot of X: eight waves of 16 weight rows on two
-        if constexpr (Cfg::NSX == 3 && MT > 8) {
-            Rows128Plan two = pl;
-            two.wv = 8;
-            two.tn = 1;
-            two.bn = 128;
-            const int tiles_n = (a.N + 127) / 128;
-            if (a.tiles_m > 1) {
-                a.tiles_n = tiles_n;
-                a.total_tiles = a.tiles_m * tiles_n;
-                two.tiles = (a.total_tiles + 7) / 8 * 8;
-            } else {
-                two.tiles = tiles_n;
-            }
-            return launch_rows128_as<MT, 8, 1, 2>(a, two, ws, st);
-        }
-        return MI355_EUNSUPPORTED;
-    }
-    if (pl.splits <= 1) {
-        // Turned starts (stream_turn_mask) where a step is mostly weights: up to 96 rows (80 beyond K = 16384), or weights of
-        // 200 MB and more (450 at K = 16384) (us, in step / turned: N = 28672, K = 4096, M = 64 / 80 / 128 29.2 / 30.5 / 36.2
-        // against 26.3 / 28.2 / 37.3; 57344 x 8192, M = 64 / 128 / 160 115 / 122 / 119 against 85 / 97 / 108; 36864 x 20480, M =
-        // 128 172 / 180; 22656 x 16384, M = 128 124 / 128; 12288 x 4096, M = 160 31.8 / 33.1).  Not with narrow workgroups on K =
-        // 8192: tile t's rows then start 5 t or 6 t times 2^18 bytes on, its steps 5 t times 128, and the two meet again on the
-        // same channels (32768 x 8192, M = 64 63.3 / 82.1; 24576: 50.6 / 60.6; with 256 weight rows 45056: 1.18 times ahead).
-        // Tiles over M share their activation rows in the L2 step by step and lose that (K = 8192: 2 to 6 %).  The two buffers
-        // of scale chunks want a multiple of 16 steps.  From 65 rows on, where the square tiles run as well, a launch asked for
-        // by name keeps K order: its sums are then theirs bit for bit.
-        if constexpr (MT <= 10 && TN == 2) {
-            const int64_t weights = (int64_t)a.N * a.K;
-            const bool weights_lead = a.M <= (a.K <= 16384 ? 96 : 80) || (a.K <= 16384 && weights >= (a.K < 16384 ? 200000000ll : 450000000ll));
-            const bool meets = WV < 8 && a.K == 8192;
-            if (pl.turned && weights_lead && !meets && a.tiles_m <= 1 && KB % 16 == 0 && (a.turn_mask = stream_turn_mask(a.K, KB)) != 0) {
-                constexpr auto turned = block_fp8_gemm_rows128_kernel<MT, TN, WV, false, true, XS>;
-                if (!allow_lds<turned>(160 * 1024)) return MI355_ELAUNCH;
-                return launch(turned, dim3(pl.tiles), dim3(Cfg::kThreads), lds_bytes, st, a);
-            }
-        }
-        constexpr auto kernel = block_fp8_gemm_rows128_kernel<MT, TN, WV, false, false, XS>;
-        if (!allow_lds<kernel>(160 * 1024)) return MI355_ELAUNCH;
-        return launch(kernel, dim3(pl.tiles), dim3(Cfg::kThreads), lds_bytes, st, a);
-    }
-    if constexpr (WV == 8 && TN == (MT <= 8 ? 2 : 1)) {
-        constexpr auto kernel = block_fp8_gemm_rows128_kernel<MT, TN, 8, true, false, XS>;
-        if (!allow_lds<kernel>(160 * 1024)) return MI355_ELAUNCH;
-        a.splits = pl.splits;
-        a.partials = (float *)((uint8_t *)ws + MI355_WS_COUNTER_BYTES);  // the counter words stay untouched
-        const int r = launch(kernel, dim3(pl.tiles * pl.splits), dim3(Cfg::kThreads), lds_bytes, st, a);
-        if (r != MI355_OK) return r;
-        return launch(rows128_reduce_kernel<MT, TN>, dim3((pl.tiles * Cfg::kWaves * MT + 3) / 4), dim3(256), 0, st, a);
-    }
-    return MI355_EINVAL;  // narrow workgroups never share K
-}
-
-template <int MT>
-static int launch_rows128(GemmArgs &a, const Rows128Plan &pl, void *ws, hipStream_t st) {
-    if constexpr (MT <= 8) {
-        if (pl.wv == 5) return launch_rows128_as<MT, 5>(a, pl, ws, st);
-        if (pl.wv == 6) return launch_rows128_as<MT, 6>(a, pl, ws, st);
-    } else if constexpr (MT <= (kRows128NarrowMaxM + 15) / 16) {
-        if (pl.tn == 2) {
-            switch (pl.wv) {
-            case 5: return launch_rows128_as<MT, 5, 2>(a, pl, ws, st);
-            case 6: return launch_rows128_as<MT, 6, 2>(a, pl, ws, st);
-            case 7: return launch_rows128_as<MT, 7, 2>(a, pl, ws, st);
-            case 8: return launch_rows128_as<MT, 8, 2>(a, pl, ws, st);
-            default: return MI355_EINVAL;
-            }
-        }
-        switch (pl.wv) {
-        case 4: return launch_rows128_as<MT, 4>(a, pl, ws, st);
-        case 5: return launch_rows128_as<MT, 5>(a, pl, ws, st);
-        case 6: return launch_rows128_as<MT, 6>(a, pl, ws, st);
-        case 7: return launch_rows128_as<MT, 7>(a, pl, ws, st);
-        default: break;
-        }
-    }
-    return launch_rows128_as<MT, 8>(a, pl, ws, st);
-}
-
 // ---- more rows than that on a narrow N: the same kernel tiled over M as well (tiles_m x tiles_n workgroups in one
 // round, K unshared).  Where N gives few 256-wide tiles the 256x256 launch leaves most units idle (N = 2112: 9 tile
 // columns, 144 tiles at M = 4096, 72 at M = 2048) and its lone round is bound by the latency of its K steps; tiles of
 // 16*mt rows x 32*wv weight rows with mt chosen so that tiles_m * tiles_n just fits the units put a workgroup on
 // (nearly) every unit, each with less to load and to multiply per step.
-// Which of the tiles: up to N = 4608 (5120 from 769 rows on) the fewest row blocks, then the fewest bytes a unit loads per K
-// step.  Beyond, the least of 146 mt + 134 wv + 90 t (mt/2 + wv) / cus (+ 371 on two ring slots) over the fewest row blocks and one more for every
-// width: what a step of one tile takes (its X block is read by every wave, its W rows once) and what all t tiles
-// pull together; fitted to 60 shapes of M = 200..4096 with every candidate timed, 1.6 % behind the best on average.  (N = 6144,
-// K = 4096, M = 450: 5 row blocks x 160 weight rows 28.2 us, 3 x 256 31.8; 8192 x 4096, M = 400: 29.7 / 36.9.)
-static RowsMPlan rowsm_plan(int64_t M, int64_t N, int64_t /*K*/, int cus) {
+// rowsm_round_plan is the tile of a single round: up to N = 4608 (5120 from 769 rows on) the fewest row blocks, then the fewest
+// bytes a unit loads per K step; beyond, by what a step loads and multiplies.  rowsm_plan is what is launched: the tile of the
+// least rowsm_ns over up to four rounds, where that is 4 % less than the round plan's.
+static RowsMPlan rowsm_round_plan(int64_t M, int64_t N, int cus) {
     RowsMPlan best = {0, 0, 0, 0};
     if (M <= 0 || cus < 8) return best;
     const int64_t blocks = (M + 15) / 16;
@@ -789,12 +694,47 @@ static RowsMPlan rowsm_plan(int64_t M, int64_t N, int64_t /*K*/, int cus) {
     return best;
 }
 
+static bool rowsm_lds_ok(int64_t mt, int64_t wv, int64_t K) {
+    const int64_t steps = K / kBlockK, ns = mt <= 8 ? 3 : 2, bn = 32 * wv, nblk = (bn + 2 * kBlockN - 2) / kBlockN;
+    const int64_t ring = ns * (16 * mt * 128 + bn * 128);
+    return ((ring + nblk * steps * 4 + 127) & ~127ll) + 2 * 16 * mt * 32 <= 160 * 1024;
+}
+
+// What the launch takes, in ns: a least-squares fit to 82000 timed launches (9676 shapes of 209..4096 rows, N = 640..36864, K =
+// 1024..18432, the nine most likely tiles of each; weights from HBM; 6 % rms).  A K step of a tile (its products; the X block,
+// which every wave reads; its W rows; two slots of W instead of three; more than six waves), what all tiles pull together, the
+// output and the weights; 2.9 us a round.  The tile of the least estimate is 0.8 % behind the fastest one on average.
+static double rowsm_ns(int64_t M, int64_t N, int64_t K, int64_t mt, int64_t wv, int cus) {
+    const int64_t tm = ((M + 15) / 16 + mt - 1) / mt, tn = (N + 32 * wv - 1) / (32 * wv), t = tm * tn;
+    const double kb = (double)(K / kBlockK), rounds = (double)((t + cus - 1) / cus);
+    const double step = 83.0 + 0.457 * mt * wv + 49.95 * mt + 18.96 * wv + (mt > 8 ? 59.7 : 0.0) + (wv > 6 ? 9.9 : 0.0) + (wv == 8 ? 23.6 : 0.0);
+    return 792.0 + rounds * (2939.0 + kb * step) + 6.0 * kb * t / cus * (mt + 2 * wv) + M * N * 4.91e-4 + N * K * 7.95e-5;
+}
+
+static RowsMPlan rowsm_plan(int64_t M, int64_t N, int64_t K, int cus) {
+    RowsMPlan best = rowsm_round_plan(M, N, cus);
+    if (M <= 208 || M > 4096 || N < 640 || cus < 8) return best;
+    double best_ns = best.mt ? 0.96 * rowsm_ns(M, N, K, best.mt, best.wv, cus) : 0.0;
+    const int64_t blocks = (M + 15) / 16;
+    for (int wv = 5; wv <= 8; ++wv) {
+        const int64_t tn = (N + 32 * wv - 1) / (32 * wv);
+        for (int64_t mt = wv == 7 ? 9 : 1; mt <= 13; ++mt) {
+            const int64_t tm = (blocks + mt - 1) / mt;
+            if (tm * tn > 4 * (int64_t)cus || !rowsm_lds_ok(mt, wv, K)) continue;
+            const double ns = rowsm_ns(M, N, K, mt, wv, cus);
+            if (best.mt == 0 || ns < best_ns) {
+                best = {(int)mt, wv, (int)tm, (int)tn};
+                best_ns = ns;
+            }
+        }
+    }
+    return best;
+}
+
 static bool rowsm_limits_ok(const RowsMPlan &pl, int64_t M, int64_t K, int64_t lda, int64_t as_m, int64_t as_k) {
     if (pl.mt == 0) return false;
     if (M * lda >= (1ll << 32) || M * as_m * 4 >= (1ll << 32) || as_k * 32 >= (1ll << 32)) return false;
-    const int64_t steps = K / kBlockK, ns = pl.mt <= 8 ? 3 : 2, bn = 32 * pl.wv, nblk = (bn + 2 * kBlockN - 2) / kBlockN;
-    const int64_t ring = ns * (16 * pl.mt * 128 + bn * 128);
-    return ((ring + nblk * steps * 4 + 127) & ~127ll) + 2 * 16 * pl.mt * 32 <= 160 * 1024;
+    return rowsm_lds_ok(pl.mt, pl.wv, K);
 }
 
 // Where it pays (forced against the table's previous choice over N = 1024..8192, K = 1536..14336, M = 400..4096,
@@ -812,7 +752,7 @@ static bool rowsm_pays(int64_t M, int64_t N, int64_t K, int cus) {
     if (M <= 384) return false;
     const int64_t KB = K / kBlockK;
     if (KB < 12 || KB > 56) return false;
-    const RowsMPlan pl = rowsm_plan(M, N, K, cus);
+    const RowsMPlan pl = rowsm_round_plan(M, N, cus);
     if (pl.mt == 0 || pl.mt > 8) return false;
     if (KB <= 40) return N <= 5120 || (M <= 960 && N <= 15360 && KB >= 16);
     return pl.mt >= 2 && pl.mt <= 6 && N <= 3072;
@@ -827,28 +767,8 @@ static bool rowsm_pays(int64_t M, int64_t N, int64_t K, int cus) {
 static bool rows128_over_m(int64_t M, int64_t N, int64_t K, int cus) {
     const int64_t KB = K / kBlockK;
     if (M <= 208 || M > 352 || N < 12288 || KB < 12 || KB > 44 || (K % 4096 == 0 && N > 16384)) return false;
-    const RowsMPlan pl = rowsm_plan(M, N, K, cus);
+    const RowsMPlan pl = rowsm_round_plan(M, N, cus);
     return pl.mt > 0 && pl.mt <= 11;
-}
-
-template <int MT>
-static int launch_rowsm_mt(GemmArgs &a, const Rows128Plan &pl, hipStream_t st) {
-    if constexpr (MT <= 8) {
-        switch (pl.wv) {
-            case 5: return launch_rows128_as<MT, 5>(a, pl, nullptr, st);
-            case 6: return launch_rows128_as<MT, 6>(a, pl, nullptr, st);
-            case 8: return launch_rows128_as<MT, 8>(a, pl, nullptr, st);
-            default: return MI355_EINVAL;
-        }
-    } else {
-        switch (pl.wv) {
-            case 5: return launch_rows128_as<MT, 5, 2>(a, pl, nullptr, st);
-            case 6: return launch_rows128_as<MT, 6, 2>(a, pl, nullptr, st);
-            case 7: return launch_rows128_as<MT, 7, 2>(a, pl, nullptr, st);
-            case 8: return launch_rows128_as<MT, 8, 2>(a, pl, nullptr, st);
-            default: return MI355_EINVAL;
-        }
-    }
 }
 
 // m tiles in a group of the launch's tile order (gemm_rows128.hpp): the least sum over the 8 XCDs of the distinct rows of X and W
@@ -883,22 +803,7 @@ static int launch_rowsm(GemmArgs &a, const RowsMPlan &mp, hipStream_t st) {
     pl.splits = 1;
     pl.tiles = (a.total_tiles + 7) / 8 * 8;  // the kernel numbers its tiles per XCD
     pl.tn = 2;
-    switch (mp.mt) {
-        case 1: return launch_rowsm_mt<1>(a, pl, st);
-        case 2: return launch_rowsm_mt<2>(a, pl, st);
-        case 3: return launch_rowsm_mt<3>(a, pl, st);
-        case 4: return launch_rowsm_mt<4>(a, pl, st);
-        case 5: return launch_rowsm_mt<5>(a, pl, st);
-        case 6: return launch_rowsm_mt<6>(a, pl, st);
-        case 7: return launch_rowsm_mt<7>(a, pl, st);
-        case 8: return launch_rowsm_mt<8>(a, pl, st);
-        case 9: return launch_rowsm_mt<9>(a, pl, st);
-        case 10: return launch_rowsm_mt<10>(a, pl, st);
-        case 11: return launch_rowsm_mt<11>(a, pl, st);
-        case 12: return launch_rowsm_mt<12>(a, pl, st);
-        case 13: return launch_rowsm_mt<13>(a, pl, st);
-        default: return MI355_EINVAL;
-    }
+    return launch_rows128(a, pl, mp.mt, true, nullptr, st);
 }
 
 // 256x128 tiles that are too few to occupy the device share the K range the same way.
@@ -1014,6 +919,52 @@ static int64_t n_split_rows(int64_t M, int64_t N, int64_t K, int cus) {
     return n1 > 0 && n1 < N ? n1 : 0;
 }
 
+// What the table's other choices take above 208 rows, in ns: fits to the same shapes (256x256 tiles 2.8 % rms, 128x128 tiles 3.4,
+// panel split of K 5.0, weight stream of one m tile 4.7), 0 for what was not fitted.
+static double other_ns(int64_t M, int64_t N, int64_t K, int variant, int cus) {
+    const double kb = (double)(K / kBlockK), weights = 1e-6 * N * K, out = 1e-6 * M * N, c = cus;
+    const int64_t KB = K / kBlockK, tm = (M + 255) / 256, tn = (N + 255) / 256, t = tm * tn;
+    if (variant == MI355_GEMM_TILE256) {
+        const double in_first = (double)std::min<int64_t>(t, cus) / c;
+        const double common = 1964.0 + kb * (566.0 * t / c - 76.0 * in_first) + 212.6 * out + 30.6 * weights;
+        const int64_t full = (t + cus - 1) / cus;
+        if (n_split_rows(M, N, K, cus) > 0) return common - 670.0 + 8233.0 * full + kb * (1170.0 * (t / cus) + 1076.0 * (t % cus) / c);
+        return common + full * (8233.0 + 1012.0 * kb);
+    }
+    if (variant == MI355_GEMM_TILE128) {
+        const int64_t splits = tile128_splits(M, N, K, cus), w = ((M + 127) / 128) * ((N + 127) / 128) * splits;
+        const double steps = (double)((KB + splits - 1) / splits), two = (double)((w + 2 * cus - 1) / (2 * cus));
+        return 2938.0 + steps * (743.0 * two + 100.9 * ((w + cus - 1) / cus) + 164.9 * w / c) + 2938.0 * two + 81.0 * out + 32.5 * weights +
+               (splits > 1 ? 2069.0 + 11.6 * w : 0.0);
+    }
+    if (variant == MI355_GEMM_TILE256_STREAMK) {
+        const int64_t runs = sk_panel_splits((int)tm, (int)tn, (int)KB, cus);
+        if (runs == 0) return 0.0;
+        return 17671.0 + ((KB + runs - 1) / runs) * (400.0 + 893.0 * t * runs / c) + 20.45 * t * runs + 1141.0 * out + 88.6 * weights;
+    }
+    if (variant == MI355_GEMM_ROWS128) {
+        const int64_t mt = (M + 15) / 16, splits = rows128_splits(M, N, K, cus), w = (N + 127) / 128 * splits;
+        const double steps = (double)((KB + splits - 1) / splits), rounds = (double)((w + cus - 1) / cus);
+        return 1303.0 + rounds * steps * (8.86 * mt - 220.7) + 378.7 * weights + 34.0 * out + 284.8 * mt + (splits > 1 ? 1303.0 + 2.347 * w * mt : 0.0);
+    }
+    return 0.0;
+}
+
+// Tiles over M instead of what the table names: above 208 rows where the estimates say 3 % less (the weight stream's K loop
+// multiplies two thirds as fast as the 256x256 tile's, on tiles that leave little of the device idle and nothing to padding or
+// partial sums).  4400 of 7500 shapes, 1.13 times as fast over all of them, 30 more than 2 % slower (8 % at most); us, before / here:
+// 300 x 4096 x 4096 26.3 / 19.4, 340 x 6144 x 4096 32.0 / 21.4, 300 x 28672 x 4096 68.3 / 51.0, 380 x 27648 x 5120 85.9 / 68.7,
+// 1200 x 6144 x 4096 50.7 / 38.3, 1700 x 5120 x 13824 156 / 122, 1200 x 7168 x 18432 207 / 167, 2500 x 4096 x 4096 55.4 / 46.7.
+// The plan keeps the table's name, by which the kernels' sums are compared; from K = 8192 on the 256x128 tiles with K shared do run
+// under theirs (1.17 times behind there, 1.3 to 1.8 times on a shorter K).
+static bool rowsm_ahead(int64_t M, int64_t N, int64_t K, int variant, int cus) {
+    if (M <= 208 || M > 4096 || N < 640 || K < 1024 || K > 20480 || cus < 192) return false;
+    const RowsMPlan pl = rowsm_plan(M, N, K, cus);
+    if (pl.mt == 0) return false;
+    if (variant == MI355_GEMM_TILE256x128) return K < 8192;
+    return rowsm_ns(M, N, K, pl.mt, pl.wv, cus) < 0.97 * other_ns(M, N, K, variant, cus);
+}
+
 // Workspace of a launch plan on a device with `cus` compute units.
 static size_t workspace_bytes_for(int64_t M, int64_t N, int64_t K, int32_t variant, int cus) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
@@ -1122,6 +1073,13 @@ extern "C" int32_t mi355_block_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, si
     return resolve_auto(M, N, K, K, K, K / kBlockK, 1, ws_bytes > 0, ws_bytes, cus);
 }
 
+extern "C" int32_t mi355_block_fp8_gemm_over_m(int64_t M, int64_t N, int64_t K, size_t ws_bytes, int32_t cus) {
+    if (cus <= 0) cus = device_cus();
+    const int variant = mi355_block_fp8_gemm_launched(M, N, K, ws_bytes, cus);
+    if (variant == MI355_GEMM_ROWS_MTILED) return 1;
+    return rowsm_ahead(M, N, K, variant, cus) && rowsm_limits_ok(rowsm_plan(M, N, K, cus), M, K, K, K / kBlockK, 1) ? 1 : 0;
+}
+
 extern "C" int32_t mi355_block_fp8_gemm_launched(int64_t M, int64_t N, int64_t K, size_t ws_bytes, int32_t cus) {
     if (cus <= 0) cus = device_cus();
     const int variant = mi355_block_fp8_gemm_plan(M, N, K, ws_bytes, cus);
@@ -1166,6 +1124,8 @@ static int block_fp8_gemm_impl(const void *A, const void *B, const float *As, co
         variant = fast && blocks128 ? resolve_auto(M, N, K, lda, ldb_n, as_m, as_k, ws_usable, ws_bytes, cus)
                                     : MI355_GEMM_GENERIC;
         variant = launched_for(variant, M, N, K, lda, ldb_n, as_m, ws_usable, ws_bytes, cus);
+        if (rowsm_ahead(M, N, K, variant, cus) && rowsm_limits_ok(rowsm_plan(M, N, K, cus), M, K, lda, as_m, as_k))
+            variant = MI355_GEMM_ROWS_MTILED;
     }
     if (was_auto && variant == MI355_GEMM_TILE256) {
         const int64_t n1 = n_split_rows(M, N, K, cus);
@@ -1271,32 +1231,7 @@ static int block_fp8_gemm_impl(const void *A, const void *B, const float *As, co
             pl.turned = was_auto || M <= 64;
             if (pl.splits > 1 && (!ws || ws_bytes < rows128_workspace(M, N, K, cus) || ((uintptr_t)ws & 15)))
                 return MI355_EWORKSPACE;
-            switch (rows128_mt(M)) {
-                case 1: return launch_rows128<1>(a, pl, ws, st);
-                case 2: return launch_rows128<2>(a, pl, ws, st);
-                case 3: return launch_rows128<3>(a, pl, ws, st);
-                case 4: return launch_rows128<4>(a, pl, ws, st);
-                case 5: return launch_rows128<5>(a, pl, ws, st);
-                case 6: return launch_rows128<6>(a, pl, ws, st);
-                case 7: return launch_rows128<7>(a, pl, ws, st);
-                case 8: return launch_rows128<8>(a, pl, ws, st);
-                case 9: return launch_rows128<9>(a, pl, ws, st);
-                case 10: return launch_rows128<10>(a, pl, ws, st);
-                case 11: return launch_rows128<11>(a, pl, ws, st);
-                case 12: return launch_rows128<12>(a, pl, ws, st);
-                case 13: return launch_rows128<13>(a, pl, ws, st);
-                case 14: return launch_rows128<14>(a, pl, ws, st);
-                case 15: return launch_rows128<15>(a, pl, ws, st);
-                case 16: return launch_rows128<16>(a, pl, ws, st);
-                case 17: return launch_rows128<17>(a, pl, ws, st);
-                case 18: return launch_rows128<18>(a, pl, ws, st);
-                case 19: return launch_rows128<19>(a, pl, ws, st);
-                case 20: return launch_rows128<20>(a, pl, ws, st);
-                case 21: return launch_rows128<21>(a, pl, ws, st);
-                case 22: return launch_rows128<22>(a, pl, ws, st);
-                case 23: return launch_rows128<23>(a, pl, ws, st);
-                default: return launch_rows128<24>(a, pl, ws, st);
-            }
+            return launch_rows128(a, pl, rows128_mt(M), false, ws, st);
         }
         case MI355_GEMM_SKINNY_ROWS: {
             const int ok = skinny_rows_check(M, N, K, lda, ldb_n, as_m, cus, ws && ((uintptr_t)ws & 15) == 0, ws_bytes);
@@ -1311,6 +1246,7 @@ static int block_fp8_gemm_impl(const void *A, const void *B, const float *As, co
         }
         case MI355_GEMM_ROWS_MTILED: {
             const RowsMPlan mp = rowsm_plan(M, N, K, cus);
+            if (!was_auto && rowsm_round_plan(M, N, cus).mt == 0) return MI355_EUNSUPPORTED;  // by name: a single round
             if (!rowsm_limits_ok(mp, M, K, lda, as_m, as_k)) return MI355_EUNSUPPORTED;
             return launch_rowsm(a, mp, st);
         }

@@ -636,6 +636,21 @@ def test_rows_tiled_over_m_very_long_k(hip):
     assert torch.equal(c.view(torch.int16), _run(xq, xs, wq, ws, "tile128").view(torch.int16))
 
 
+# one to four rounds of tiles, every width of workgroup, one row or one weight row past a tile, the edges of the rule's ranges
+@pytest.mark.parametrize("M,N,K", [(209, 6144, 4096), (300, 4096, 4096), (340, 6145, 4096), (380, 24576, 1536), (1200, 6144, 4096),
+                                   (2500, 4096, 4096), (4096, 640, 1024), (1700, 5120, 13824), (1300, 7169, 20480), (3209, 2112, 7168),
+                                   (1400, 9001, 2048), (300, 28672, 4096), (756, 5056, 6016)])
+def test_tiles_over_m_instead_of_the_tables_kernel(hip, M, N, K):
+    """What AUTO runs there has the bits of the 256x256 tiles (K whole, in order), with row- and column-major activation scales."""
+    print(f"gemm over M M={M} N={N} K={K}", flush=True)
+    if _lib_cus() == 256:
+        assert hip.mi355_block_fp8_gemm_over_m(M, N, K, 1 << 34, 0) == 1
+    xq, xs, wq, ws = _prep(M, N, K, seed=M + N)
+    c = _run(xq, xs, wq, ws, None).clone()
+    assert torch.equal(c.view(torch.int16), _run(xq, xs, wq, ws, "tile256").view(torch.int16))
+    assert torch.equal(c, _run(xq, xs.t().contiguous().t(), wq, ws, None))
+
+
 # 209..352 rows in two or three tiles of the activation-block stream, 385..960 rows on a wider N: the edges of both ranges, row counts
 # that leave the last tile one row, N that leaves the last column of tiles one weight row, the shortest and longest K
 @pytest.mark.parametrize("M,N,K,variant", [(209, 12288, 2048, "rows128"), (225, 12289, 1536, "rows128"), (352, 27648, 1536, "rows128"),
