@@ -25,16 +25,48 @@ using PrologueScan = PairScan<kPrologueThreads, 4>;
 constexpr int64_t kProloguePairs = PrologueScan::kPass;  // one pass: an expert's workgroup holds every pair's expert in registers
 constexpr int32_t kPrologueExperts = 1024;               // counters in LDS
 
+constexpr int64_t kFewPairs = 64;  // one pair per lane of a wave
+
+// The same for at most 64 pairs by one wave, a pair per lane, without LDS and barriers: which pairs precede one, which are of its
+// expert and which are the first of a block are ballots.  Bound by the latency of its one load (four layers of 128 experts, 4
+// tokens: 164.2 us with the counting form, 153.3).
+__device__ __forceinline__ void few_pairs(const int32_t *topk_ids, const float *topk_weights, int32_t num_pairs, int32_t num_experts,
+                                          int32_t *e2t_index, float *e2t_weight, int32_t *e_num, const ScheduleOut &first,
+                                          const ScheduleOut &second, int expert, int lane) {
+    const bool in = lane < num_pairs;
+    const uint32_t id = in ? (uint32_t)topk_ids[lane] : ~0u;
+    const float w = in ? topk_weights[lane] : 0.f;
+    const bool valid = id < (uint32_t)num_experts, before = valid && id < (uint32_t)expert;
+    const uint64_t lt = (1ull << lane) - 1ull, mine = __ballot(id == (uint32_t)expert);
+    const int cnt = __popcll(mine);
+    if (id == (uint32_t)expert) {
+        const int64_t at = (int64_t)expert * num_pairs + __popcll(mine & lt);
+        e2t_index[at] = lane;
+        e2t_weight[at] = w;
+    }
+    if (lane == 0) e_num[expert] = cnt;
+    // the pairs of this lane's expert, by the ten bits of its number
+    uint64_t same = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < 10; ++b) {
+        const uint64_t set = __ballot((id >> b) & 1u);
+        same &= (id >> b) & 1u ? set : ~set;
+    }
+    const uint32_t rank = (uint32_t)__popcll(same & lt);
+    const int tokens = __popcll(__ballot(before));
+    auto blocks = [&](int32_t m) { return __popcll(__ballot(before && rank % (uint32_t)m == 0)); };
+    if (first.block_m) schedule_rows<64>(expert, num_experts, cnt, tokens, blocks(first.block_m), first.block_m, first.rows, first.table, lane);
+    if (second.block_m) schedule_rows<64>(expert, num_experts, cnt, tokens, blocks(second.block_m), second.block_m, second.rows, second.table, lane);
+}
+
 // Workgroups 0 .. E-1: the pair list, the count and the schedule rows of one expert.  The others: 256 chunks each of the
 // activation quantizer (16 lanes of a DPP row = one group; scales [T, K/128] row-major).
+template <bool FEW>
 __global__ __launch_bounds__(kPrologueThreads) void moe_prologue_kernel(
     const int32_t *__restrict__ topk_ids, const float *__restrict__ topk_weights, int32_t num_pairs, int32_t num_experts,
     int32_t *__restrict__ e2t_index, float *__restrict__ e2t_weight, int32_t *__restrict__ e_num, ScheduleOut first,
     ScheduleOut second, const v4i *__restrict__ x, v2i *__restrict__ q, float *__restrict__ s, uint32_t total_chunks) {
     constexpr int T = kPrologueThreads, kW = T / 64;
-    __shared__ int hist[kPrologueExperts];
-    __shared__ int wave_cnt[4 * kW];
-    __shared__ int red[3][kW];
     const int tid = threadIdx.x;
     if (blockIdx.x >= (uint32_t)num_experts) {
         const uint32_t c = (blockIdx.x - (uint32_t)num_experts) * T + tid;
@@ -47,44 +79,52 @@ __global__ __launch_bounds__(kPrologueThreads) void moe_prologue_kernel(
         return;
     }
     const int expert = blockIdx.x;
-    v4i k[4], w[4];
-    PrologueScan::load(topk_ids, (uint32_t)num_pairs, 0, tid, k);
-    PrologueScan::load(topk_weights, (uint32_t)num_pairs, 0, tid, w);
-    for (int e = tid; e < num_experts; e += T) hist[e] = 0;
-    __syncthreads();
+    if constexpr (FEW) {
+        if (tid < 64)
+            few_pairs(topk_ids, topk_weights, num_pairs, num_experts, e2t_index, e2t_weight, e_num, first, second, expert, tid);
+    } else {
+        __shared__ int hist[kPrologueExperts];
+        __shared__ int wave_cnt[4 * kW];
+        __shared__ int red[3][kW];
+        v4i k[4], w[4];
+        PrologueScan::load(topk_ids, (uint32_t)num_pairs, 0, tid, k);
+        PrologueScan::load(topk_weights, (uint32_t)num_pairs, 0, tid, w);
+        for (int e = tid; e < num_experts; e += T) hist[e] = 0;
+        __syncthreads();
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+        for (int c = 0; c < 4; ++c)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if ((uint32_t)k[c][j] < (uint32_t)num_experts) atomicAdd(&hist[k[c][j]], 1);  // others belong to no expert
-    const int cnt = PrologueScan::append(k, w, expert, 0, tid, 0, e2t_index + (int64_t)expert * num_pairs,
-                                         e2t_weight + (int64_t)expert * num_pairs, wave_cnt);
-    if (tid == 0) e_num[expert] = cnt;
-    // tokens and blocks of the experts before this one (the barriers of append() close the histogram)
-    int before[3] = {0, 0, 0};
-    for (int e = tid; e < expert; e += T) {
-        const int n = hist[e];
-        before[0] += n;
-        if (first.block_m) before[1] += (n + first.block_m - 1) / first.block_m;
-        if (second.block_m) before[2] += (n + second.block_m - 1) / second.block_m;
+            for (int j = 0; j < 4; ++j)
+                if ((uint32_t)k[c][j] < (uint32_t)num_experts) atomicAdd(&hist[k[c][j]], 1);  // others belong to no expert
+        const int cnt = PrologueScan::append(k, w, expert, 0, tid, 0, e2t_index + (int64_t)expert * num_pairs,
+                                             e2t_weight + (int64_t)expert * num_pairs, wave_cnt);
+        if (tid == 0) e_num[expert] = cnt;
+        // tokens and blocks of the experts before this one (the barriers of append() close the histogram)
+        int before[3] = {0, 0, 0};
+        for (int e = tid; e < expert; e += T) {
+            const int n = hist[e];
+            before[0] += n;
+            if (first.block_m) before[1] += (n + first.block_m - 1) / first.block_m;
+            if (second.block_m) before[2] += (n + second.block_m - 1) / second.block_m;
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) before[i] += __shfl_xor(before[i], off);
+            if ((tid & 63) == 0) red[i][tid >> 6] = before[i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            before[i] = 0;
+#pragma unroll
+            for (int w = 0; w < kW; ++w) before[i] += red[i][w];
+        }
+        if (first.block_m)
+            schedule_rows<T>(expert, num_experts, cnt, before[0], before[1], first.block_m, first.rows, first.table, tid);
+        if (second.block_m)
+            schedule_rows<T>(expert, num_experts, cnt, before[0], before[2], second.block_m, second.rows, second.table, tid);
     }
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) before[i] += __shfl_xor(before[i], off);
-        if ((tid & 63) == 0) red[i][tid >> 6] = before[i];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        before[i] = 0;
-#pragma unroll
-        for (int w = 0; w < kW; ++w) before[i] += red[i][w];
-    }
-    if (first.block_m)
-        schedule_rows<T>(expert, num_experts, cnt, before[0], before[1], first.block_m, first.rows, first.table, tid);
-    if (second.block_m)
-        schedule_rows<T>(expert, num_experts, cnt, before[0], before[2], second.block_m, second.rows, second.table, tid);
 }
 
 // Where everything between the input and the output lies in the caller's scratch.
@@ -168,7 +208,7 @@ extern "C" int mi355_routed_ffn(const void *x, const int32_t *topk_ids, const fl
     if (pairs <= kProloguePairs && E <= kPrologueExperts && chunks < (1ll << 30)) {
         const ScheduleOut first = {table1, f.rows1, f.block_m1};
         const ScheduleOut second = {table2, f.rows2, f.rows2 ? f.block_m2 : 0};
-        r = launch(moe_prologue_kernel, dim3((uint32_t)(E + (chunks + kPrologueThreads - 1) / kPrologueThreads)),
+        r = launch(pairs <= kFewPairs ? moe_prologue_kernel<true> : moe_prologue_kernel<false>, dim3((uint32_t)(E + (chunks + kPrologueThreads - 1) / kPrologueThreads)),
                    dim3(kPrologueThreads), 0, st, topk_ids, topk_weights, (int32_t)pairs, E, index, weight, count, first, second,
                    (const v4i *)x, (v2i *)(base + f.x_q), x_s, (uint32_t)chunks);
         if (r != MI355_OK) return r;

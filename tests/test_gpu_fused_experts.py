@@ -151,6 +151,13 @@ def test_fused_experts_in_one_call_equals_the_steps(hip, T, E, topk, Hd, I, offs
     assert torch.equal(inp.view(torch.int16), want.view(torch.int16))
 
 
+# up to 64 pairs the tables come from ballots: both sides of that, experts with more than one block, one pair, experts without any
+@pytest.mark.parametrize("T,E,topk,Hd,I", [(64, 1, 1, 256, 128), (32, 2, 2, 2048, 768), (63, 3, 1, 256, 2048), (13, 5, 5, 256, 128),
+                                           (16, 1024, 4, 256, 128), (8, 600, 8, 2048, 128)])
+def test_fused_experts_with_few_pairs(hip, T, E, topk, Hd, I):
+    test_fused_experts_in_one_call_equals_the_steps(hip, T, E, topk, Hd, I, 1)
+
+
 # full chunks and a shorter last one (of another block size: 20 and 3 pairs per expert; 31 and 8), an odd topk, ids of a
 # chunk that are not 16-byte aligned, biases
 @pytest.mark.parametrize("T,E,topk,Hd,I,chunk", [(101, 7, 3, 256, 384, 47), (107, 12, 8, 1024, 1024, 47), (96, 5, 1, 128, 128, 48)])
