@@ -235,10 +235,12 @@ extern "C" int mi355_group_quant_fp8(const void *x, int32_t x_dtype, void *q, fl
         return launch(group_quant_wide_kernel<uint16_t>, dim3((uint32_t)((chunks + 255) / 256)), dim3(256), 0, st,
                       (const uint16_t *)x, (v2i *)q, s, (uint32_t)chunks, G, s_stride_m, s_stride_g, eps);
     }
-    // Four chunks per lane where that still gives every compute unit two workgroups, else one: a small input is bound by
-    // the latency of its one load, and the arithmetic of four chunks in a row behind it only adds to that ([8, 14336]
-    // and [64, 4096]: 2.7 us a launch in a captured graph with four, 1.95 with one, where an empty kernel takes 1.8;
-    // [640, 4096]: 3.3 and 2.6; from [1024, 4096] on the two are level).
+    // Two chunks per lane on large inputs, else one: a small input is bound by the latency of its one load, and the arithmetic
+    // of more chunks in a row behind it only adds to that ([8, 14336] and [64, 4096]: 2.7 us a launch in a captured graph with
+    // four, 1.95 with one, where an empty kernel takes 1.8); a large one has requests enough in flight with two, and ends more
+    // evenly than with four or eight (us with one / two / four / eight: [640, 7168] 4.7 / 4.5 / 5.3 / 6.3, [1024, 7168] 6.3 / 5.8 /
+    // 6.7 / 7.0, [4096, 7168] 18.0 / 17.4 / 18.7 / 19.8, [4096, 18432] 40.6 / 37.6 / 39.5 / 43.4, [16384, 7168] 61.0 / 56.4 / 58.6 /
+    // 63.9; [333, 7168] 3.3 / 3.7 / 4.2 / 5.1, [640, 18432] and [2047, 7168] level).
     auto go = [&](auto unroll) {
         constexpr int U = decltype(unroll)::value;
         const auto kernel = row_major ? (f16 ? group_quant_kernel<U, true, true> : group_quant_kernel<U, true, false>)
@@ -247,6 +249,6 @@ extern "C" int mi355_group_quant_fp8(const void *x, int32_t x_dtype, void *q, fl
         return launch(kernel, dim3(blocks), dim3(256), 0, st, (const v4i *)x, (v2i *)q, s, (uint32_t)chunks, G, s_stride_m,
                       s_stride_g);
     };
-    if (chunks >= (int64_t)device_cus() * 2048) return go(std::integral_constant<int, 4>{});
+    if (chunks >= (int64_t)device_cus() * 2048) return go(std::integral_constant<int, 2>{});
     return go(std::integral_constant<int, 1>{});
 }

@@ -82,10 +82,11 @@ __device__ __forceinline__ v4i silu_mul_chunk(const v4i &g, const v4i &u) {
     return o;
 }
 
-// Four chunks per lane where that still gives every compute unit two workgroups, else one: a small launch is bound by the
-// latency of its loads and of the arithmetic behind them, not by the memory (silu_and_mul / with the quantizer, in a
-// captured graph: [4, 28672] 3.7 / 4.5 us with four, 2.3 / 2.5 with one; [512, 4096] 3.9 / 4.8 and 2.8 / 3.1; level from
-// [512, 28672] on).
+// Two chunks per lane on large launches, else one: a small one is bound by the latency of its loads and of the arithmetic behind
+// them, not by the memory (silu_and_mul / with the quantizer, in a captured graph: [4, 28672] 3.7 / 4.5 us with four, 2.3 / 2.5 with
+// one; [512, 4096] 3.9 / 4.8 and 2.8 / 3.1); a large one has requests enough in flight with two and ends more evenly than with four
+// (us with one / two / four: [333, 28672] 7.5 / 7.7 / 8.4, with the quantizer 8.2 / 7.7 / 9.3; [4096, 28672] 57.5 / 58.3 / 62.5 and
+// 62.8 / 53.7 / 59.9; [32768, 4096] 66.1 / 65.8 / 70.2 and 72.7 / 61.1 / 67.7).
 static bool unroll_pays(int64_t chunks) { return chunks >= (int64_t)device_cus() * 2048; }
 
 // Row/column of output chunk c (8 elements) when a row holds cpr chunks.
@@ -385,7 +386,7 @@ extern "C" int mi355_silu_and_mul(const void *in, void *out, int64_t M, int64_t 
                           (const uint16_t *)in, (uint16_t *)out, (uint32_t)chunks, cpr, 256u / cpr, 256u % cpr, in_stride_m,
                           out_stride_m);
         };
-        return unroll_pays(chunks) ? go(std::integral_constant<int, 4>{}) : go(std::integral_constant<int, 1>{});
+        return unroll_pays(chunks) ? go(std::integral_constant<int, 2>{}) : go(std::integral_constant<int, 1>{});
     } else {
         int64_t total = M * H;
         if ((total + 255) / 256 >= (int64_t)1 << 31) return MI355_EUNSUPPORTED;
@@ -440,7 +441,7 @@ extern "C" int mi355_silu_and_mul_group_quant_fp8(const void *in, void *q, float
                       (const uint16_t *)in, (v2i *)q, s, (uint32_t)chunks, cpr, 256u / cpr, 256u % cpr, in_stride_m,
                       s_stride_m, s_stride_g);
     };
-    return unroll_pays(chunks) ? go(std::integral_constant<int, 4>{}) : go(std::integral_constant<int, 1>{});
+    return unroll_pays(chunks) ? go(std::integral_constant<int, 2>{}) : go(std::integral_constant<int, 1>{});
 }
 
 extern "C" int mi355_moe_sum_reduce(const void *in, void *out, int64_t T, int32_t topk, int64_t H, void *stream) {
