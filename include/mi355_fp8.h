@@ -162,7 +162,8 @@ int32_t mi355_block_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, size_t ws_byt
 int32_t mi355_block_fp8_gemm_launched(int64_t M, int64_t N, int64_t K, size_t ws_bytes, int32_t cus);
 
 /* 1 where that AUTO call runs as tiles over M (the kernel of MI355_GEMM_ROWS_MTILED, in up to four rounds) instead of the kernel
- * above, 0 where not: at 209..4096 rows, N >= 640 and 1024 <= K <= 20480 it does wherever the tiles are estimated to be 3 % ahead.
+ * above, 0 where not: at 209..4096 rows (80..208 instead of MI355_GEMM_TILE128 only), N >= 640 and 1024 <= K <= 20480 it does
+ * wherever the tiles are estimated to be 3 % ahead.
  * K is never shared in them, so the result has the bits of MI355_GEMM_TILE256, and of the kernel above unless that shares K.
  * Launches nothing; no counterpart in the reference. */
 int32_t mi355_block_fp8_gemm_over_m(int64_t M, int64_t N, int64_t K, size_t ws_bytes, int32_t cus);

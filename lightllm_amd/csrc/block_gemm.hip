@@ -713,14 +713,14 @@ static double rowsm_ns(int64_t M, int64_t N, int64_t K, int64_t mt, int64_t wv, 
 
 static RowsMPlan rowsm_plan(int64_t M, int64_t N, int64_t K, int cus) {
     RowsMPlan best = rowsm_round_plan(M, N, cus);
-    if (M <= 208 || M > 4096 || N < 640 || cus < 8) return best;
+    if (M < 80 || M > 4096 || N < 640 || cus < 8) return best;
     double best_ns = best.mt ? 0.96 * rowsm_ns(M, N, K, best.mt, best.wv, cus) : 0.0;
     const int64_t blocks = (M + 15) / 16;
     for (int wv = 5; wv <= 8; ++wv) {
         const int64_t tn = (N + 32 * wv - 1) / (32 * wv);
         for (int64_t mt = wv == 7 ? 9 : 1; mt <= 13; ++mt) {
             const int64_t tm = (blocks + mt - 1) / mt;
-            if (tm * tn > 4 * (int64_t)cus || !rowsm_lds_ok(mt, wv, K)) continue;
+            if (tm < 2 || tm * tn > 4 * (int64_t)cus || !rowsm_lds_ok(mt, wv, K)) continue;  // (the kernel numbers two m tiles and more)
             const double ns = rowsm_ns(M, N, K, mt, wv, cus);
             if (best.mt == 0 || ns < best_ns) {
                 best = {(int)mt, wv, (int)tm, (int)tn};
@@ -950,15 +950,17 @@ static double other_ns(int64_t M, int64_t N, int64_t K, int variant, int cus) {
     return 0.0;
 }
 
-// Tiles over M instead of what the table names: above 208 rows where the estimates say 3 % less (the weight stream's K loop
+// Tiles over M instead of what the table names: from 80 rows on where the estimates say 3 % less (the weight stream's K loop
 // multiplies two thirds as fast as the 256x256 tile's, on tiles that leave little of the device idle and nothing to padding or
 // partial sums).  4400 of 7500 shapes, 1.13 times as fast over all of them, 30 more than 2 % slower (8 % at most); us, before / here:
 // 300 x 4096 x 4096 26.3 / 19.4, 340 x 6144 x 4096 32.0 / 21.4, 300 x 28672 x 4096 68.3 / 51.0, 380 x 27648 x 5120 85.9 / 68.7,
 // 1200 x 6144 x 4096 50.7 / 38.3, 1700 x 5120 x 13824 156 / 122, 1200 x 7168 x 18432 207 / 167, 2500 x 4096 x 4096 55.4 / 46.7.
-// The plan keeps the table's name, by which the kernels' sums are compared; from K = 8192 on the 256x128 tiles with K shared do run
+// From 80 to 208 rows instead of the 128x128 tiles only (a short K): 1.58 times as fast over 496 shapes, none slower (118 x 5744 x 1792
+// 19.6 / 9.1, 143 x 2032 x 1920 20.2 / 9.2).  The plan keeps the table's name, by which the kernels' sums are compared; from K = 8192 on the 256x128 tiles with K shared do run
 // under theirs (1.17 times behind there, 1.3 to 1.8 times on a shorter K).
 static bool rowsm_ahead(int64_t M, int64_t N, int64_t K, int variant, int cus) {
-    if (M <= 208 || M > 4096 || N < 640 || K < 1024 || K > 20480 || cus < 192) return false;
+    if (M < 80 || M > 4096 || N < 640 || K < 1024 || K > 20480 || cus < 192) return false;
+    if (M <= 208 && variant != MI355_GEMM_TILE128) return false;
     const RowsMPlan pl = rowsm_plan(M, N, K, cus);
     if (pl.mt == 0) return false;
     if (variant == MI355_GEMM_TILE256x128) return K < 8192;

@@ -340,14 +340,14 @@ def test_launched_kernel_query():
 
 
 def test_over_m_query():
-    """Tiles over M instead of the table's kernel: only above 208 rows, on either side of the lines as timed."""
+    """Tiles over M instead of the table's kernel: only from 80 rows on, on either side of the lines as timed."""
     from lightllm_amd import _lib
 
     lib = _lib.lib()
     for shape, want in [((300, 4096, 4096), 1), ((340, 6144, 4096), 1), ((1700, 5120, 13824), 1), ((2500, 4096, 4096), 1),
                         ((380, 24576, 1536), 1), ((512, 4096, 4096), 1), ((333, 27648, 5120), 1), ((4096, 36864, 7168), 0),
-                        ((1024, 7168, 18432), 0), ((640, 7168, 18432), 0), ((4096, 4096, 4096), 0), ((208, 4096, 4096), 0),
-                        ((5000, 4096, 4096), 0), ((300, 512, 4096), 0), ((300, 4096, 896), 0), ((300, 4096, 4096 + 64), 0)]:
+                        ((1024, 7168, 18432), 0), ((640, 7168, 18432), 0), ((4096, 4096, 4096), 0), ((208, 4096, 4096), 1),
+                        ((118, 5744, 1792), 1), ((79, 5744, 1792), 0), ((128, 24576, 1536), 0), ((5000, 4096, 4096), 0), ((300, 512, 4096), 0), ((300, 4096, 896), 0), ((300, 4096, 4096 + 64), 0)]:
         assert lib.mi355_block_fp8_gemm_over_m(*shape, 1 << 34, 256) == want, shape
     assert lib.mi355_block_fp8_gemm_over_m(300, 4096, 4096, 1 << 34, 64) == 0
     for m, n, k in _sweep_shapes(6, 2000):
@@ -355,7 +355,7 @@ def test_over_m_query():
             over = lib.mi355_block_fp8_gemm_over_m(m, n, k, ws_bytes, 256)
             if lib.mi355_block_fp8_gemm_launched(m, n, k, ws_bytes, 256) == 12:
                 assert over == 1
-            elif m <= 208 or m > 4096:
+            elif m < 80 or m > 4096:
                 assert over == 0, (m, n, k)
 
 

@@ -639,7 +639,8 @@ def test_rows_tiled_over_m_very_long_k(hip):
 # one to four rounds of tiles, every width of workgroup, one row or one weight row past a tile, the edges of the rule's ranges
 @pytest.mark.parametrize("M,N,K", [(209, 6144, 4096), (300, 4096, 4096), (340, 6145, 4096), (380, 24576, 1536), (1200, 6144, 4096),
                                    (2500, 4096, 4096), (4096, 640, 1024), (1700, 5120, 13824), (1300, 7169, 20480), (3209, 2112, 7168),
-                                   (1400, 9001, 2048), (300, 28672, 4096), (756, 5056, 6016)])
+                                   (1400, 9001, 2048), (300, 28672, 4096), (756, 5056, 6016), (80, 700, 1024),
+                                   (118, 5744, 1792), (143, 2033, 1920), (208, 3568, 1920)])
 def test_tiles_over_m_instead_of_the_tables_kernel(hip, M, N, K):
     """What AUTO runs there has the bits of the 256x256 tiles (K whole, in order), with row- and column-major activation scales."""
     print(f"gemm over M M={M} N={N} K={K}", flush=True)
