@@ -583,7 +583,7 @@ static bool rows128_ahead_of_stream(int64_t M, int64_t N, int64_t K, int cus) {
 // memory-side cache).  At 65..128 rows it beats the 128x128 tiles by 10 to 30 % (DeepSeek-V3 down, M = 128: 39.5 us
 // against 50.0; Llama-3 down: 27.9 against 30.3) unless K is short (q_b, K = 1536: 21.7 against 17.0).  At 17..64 rows it is
 // the faster one on the larger weights (rows128_ahead_of_stream), at 16 rows on a few kinds of them (below).
-static bool rows128_pays(int64_t M, int64_t N, int64_t K, int cus) {
+static bool rows128_pays(int64_t M, int64_t N, int64_t K, int cus, bool allow_streamk) {
     if (M > 384 || M < 16) return false;
     if (rows128_over_m(M, N, K, cus)) return true;
     if (M == 16) {
@@ -605,7 +605,7 @@ static bool rows128_pays(int64_t M, int64_t N, int64_t K, int cus) {
         const int64_t tiles = (N + 127) / 128;
         // from about 340 rows on the 256x256 tiles with a panel split of K overtake it on the large weights
         // (DeepSeek-V3 down, M = 352 / 384: 79.4 / 78.3 us against 82.9 / 87.5; Llama-3 down stays: 49.7 against 44.8)
-        if (M > 336 && N * K >= 100000000ll &&
+        if (M > 336 && N * K >= 100000000ll && allow_streamk &&
             stream_k_pays(((M + 255) / 256) * ((N + 255) / 256), K / kBlockK, cus, (M + 255) / 256))
             return false;
         // (with more than cus/4 tiles of 128 weight rows only up to 320 rows: N = 10240, K = 8192, M = 257 / 300:
@@ -633,7 +633,7 @@ static bool rows128_pays(int64_t M, int64_t N, int64_t K, int cus) {
         // from about 200 rows the panel split of the 256x256 tiles is level or ahead on the large weights, its time
         // flat in M (DeepSeek-V3 down, M = 208 / 240 / 256: 55.1 / 54.9 / 56.9 us against 58.4 / 60.4 / 63.3;
         // o_proj 53.1 / 52.8 / 58.1 against 54.9 / 57.5 / 57.6)
-        if (M > 200 && N * K >= 100000000ll && stream_k_pays((N + 255) / 256, K / kBlockK, cus, 1)) return false;
+        if (M > 200 && N * K >= 100000000ll && allow_streamk && stream_k_pays((N + 255) / 256, K / kBlockK, cus, 1)) return false;
         // and on small weights the 128x128 tiles with K shared (N = 4096, K = 4096, M = 224 / 256: 18.9 / 19.0 us
         // against 20.9 / 21.3; N = 7168, K = 2304, M = 256: 19.7 against 23.0)
         if (M > 192 && N * K < 20000000ll) return false;
@@ -851,11 +851,14 @@ static int64_t n_split_rows(int64_t M, int64_t N, int64_t K, int cus);
 //     (few 256x256 tiles or a short K)               128x128 tiles, K shared between workgroups when they are few
 //                                                    (M >= 768 and N <= 3072: 256x128 tiles with K shared)
 //   otherwise                                        256x256 ping-pong tiles
-static int pick_variant(int64_t M, int64_t N, int64_t K, int cus, bool allow_rows128 = true) {
+// Without room for the partial tiles of stream-K (allow_streamk) its shapes go to the rows below it: 128x128 tiles are 1.25 times
+// as fast as a few 256x256 ones there, level from about 80 of those on (2684 shapes of 129..6000 rows, K = 5120..29440; us, 256x256 /
+// 128x128: 175 x 6112 x 5888 65.0 / 49.2, 2831 x 176 x 8448 87.5 / 68.9; 507 x 14976 x 25216, 118 tiles, 8 % the other way).
+static int pick_variant(int64_t M, int64_t N, int64_t K, int cus, bool allow_rows128 = true, bool allow_streamk = true) {
     // up to 16 rows the per-unit stream also beats the stream with the activation block in LDS where both apply
     // (N = 18432, K = 7168, M = 16: 23.6 us against 27.5; N = 7168, K = 18432: 25.4 against 27.2)
     if (streamcu_pays(M, N, K, cus)) return MI355_GEMM_SKINNY_CU;
-    if (allow_rows128 && rows128_pays(M, N, K, cus)) return MI355_GEMM_ROWS128;
+    if (allow_rows128 && rows128_pays(M, N, K, cus, allow_streamk)) return MI355_GEMM_ROWS128;
     if (allow_rows128 && rowsm_pays(M, N, K, cus)) return MI355_GEMM_ROWS_MTILED;
     if (xshare_pays(M, N, K, cus)) return MI355_GEMM_SKINNY_XSHARE;
     if (M <= 64) return MI355_GEMM_SKINNY;
@@ -865,7 +868,8 @@ static int pick_variant(int64_t M, int64_t N, int64_t K, int cus, bool allow_row
     // one or two K steps: the 256x256 tile's first requests and its epilogue are most of its time (N = 7168,
     // K = 256, M = 4096: 21.3 us for the 128x128 tiles against 27.6)
     if (KB <= 2) return MI355_GEMM_TILE128;
-    if (M > 128 && stream_k_pays(t256, KB, cus, (M + 255) / 256)) return MI355_GEMM_TILE256_STREAMK;
+    const bool shares = M > 128 && stream_k_pays(t256, KB, cus, (M + 255) / 256);
+    if (shares && allow_streamk) return MI355_GEMM_TILE256_STREAMK;
     // 257..384 rows leave the second 256-row tile at most half full; where the 256x256 tiles need a second round
     // anyway the 128x128 ones are ahead (N = 36864, K = 7168, M = 257 / 384: 144 / 148 us against 161 / 165) -
     // unless the second round is small enough to run as a launch of its own (130 / 139 us then)
@@ -878,7 +882,7 @@ static int pick_variant(int64_t M, int64_t N, int64_t K, int cus, bool allow_row
         // ... and, from two 256-row tiles on, a wider N under a long K (N = 5120, K = 5120, M = 400 / 512: 35.4 /
         // 37.6 us against 44.7 / 45.1; N = 4096, K = 7168, M = 640: 54.6 against 60.3; on N = 1536 the 128x128 tiles
         // keep their lead, 21.8 against 25.2, and with K = 4096 too)
-        if (((M >= 768 && (N + 127) / 128 <= 24 && (N + 127) / 128 >= 12) || (M > 384 && KB >= 40 && (N + 127) / 128 >= 20)) &&
+        if (!shares && ((M >= 768 && (N + 127) / 128 <= 24 && (N + 127) / 128 >= 12) || (M > 384 && KB >= 40 && (N + 127) / 128 >= 20)) &&
             tile256x128_splits(M, N, K, cus) >= 2)
             return MI355_GEMM_TILE256x128;
         return MI355_GEMM_TILE128;
@@ -1015,21 +1019,18 @@ static size_t workspace_bytes_for(int64_t M, int64_t N, int64_t K, int32_t varia
 // The kernel an AUTO call launches (first) for a problem in the fast layout: the table's choice, or - where a limit
 // of that kernel is not met or its workspace is missing - the next kernel with fewer preconditions.  The chain ends
 // in tiles that take every fast layout and run unsplit without a workspace, so AUTO never fails for want of one.
-// The 256-row stream is checked first because the table's other choice for its shapes can be any of the kernels
-// checked after it.
+// Stream-K's workspace and the 256-row stream are looked at first because the table's other choice for their shapes can be any of
+// the kernels checked after them.
 static int resolve_auto(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int64_t as_m, int64_t as_k,
                         bool ws_usable, size_t ws_bytes, int cus) {
-    int variant = pick_variant(M, N, K, cus);
+    const bool streamk = ws_usable && ws_bytes >= stream_k_workspace(cus / 8 * 8);  // (every plan of it takes that much)
+    int variant = pick_variant(M, N, K, cus, true, streamk);
     if (variant == MI355_GEMM_ROWS_MTILED && !rowsm_limits_ok(rowsm_plan(M, N, K, cus), M, K, lda, as_m, as_k))
-        variant = pick_variant(M, N, K, cus, false);
+        variant = pick_variant(M, N, K, cus, false, streamk);
     if (variant == MI355_GEMM_ROWS128 &&
         (!rows128_limits_ok(M, N, K, lda, as_m, as_k, cus) ||
          (rows128_splits(M, N, K, cus) > 1 && (!ws_usable || ws_bytes < rows128_workspace(M, N, K, cus)))))
-        variant = pick_variant(M, N, K, cus, false);
-    // stream-K needs its partial-tile slots; without them the plain tile loop gives the same result
-    if (variant == MI355_GEMM_TILE256_STREAMK &&
-        (!ws_usable || ws_bytes < workspace_bytes_for(M, N, K, variant, cus)))
-        variant = MI355_GEMM_TILE256;
+        variant = pick_variant(M, N, K, cus, false, streamk);
     if (variant == MI355_GEMM_SKINNY_XSHARE &&
         (N * ldw >= (1ll << 32) || M * lda >= (1ll << 32) || M * as_m >= (1ll << 32) ||
          (N + XshareCfg::BN - 1) / XshareCfg::BN * 4 > MI355_WS_COUNTER_BYTES))

@@ -403,6 +403,21 @@ def test_auto_never_fails_for_want_of_a_workspace():
         assert lib.mi355_block_fp8_gemm_plan(m, n, k, 1 << 34, 0) == lib.mi355_block_fp8_gemm_variant(m, n, k)
 
 
+def test_no_stream_k_without_its_workspace():
+    """Where the table shares K between 256x256 tiles and the workspace of that is missing (none, or the fixed scratch), the
+    choice is the table's without stream-K: a few 256x256 tiles by themselves leave most of the device idle (us, 256x256 / here
+    without a workspace: 175 x 6112 x 5888 65.0 / 49.2, 2831 x 176 x 8448 87.5 / 68.9, 204 x 9600 x 7424 80.3 / 62.4)."""
+    from lightllm_amd import _lib
+
+    lib = _lib.lib()
+    T256, T128, ROWS = 1, 2, 10
+    for ws_bytes in (0, _lib.WS_COUNTER_BYTES + (8 << 20)):
+        for shape, want in [((175, 6112, 5888), T128), ((204, 9600, 7424), T128), ((2831, 176, 8448), T128), ((4966, 16, 7552), T128),
+                            ((1621, 528, 7296), T128), ((208, 10080, 7680), T128), ((3877, 240, 9472), T128), ((204, 31744, 5888), ROWS),
+                            ((2048, 4096, 14336), T256)]:
+            assert lib.mi355_block_fp8_gemm_plan(*shape, ws_bytes, 256) == want, (shape, ws_bytes)
+
+
 @pytest.mark.parametrize("cus", [8, 64, 128, 304])
 def test_shape_table_off_256_compute_units(cus):
     """The table's thresholds are all relative to the compute-unit count but were measured at 256.  On other counts
