@@ -214,9 +214,8 @@ __global__ __launch_bounds__(64 * WV) void block_fp8_gemm_rows128_kernel(const G
     const uint32_t wr0 = wdst + xr0, wr1 = wdst + xr1;
     const uint32_t sr8 = chunk_off + (uint32_t)(r16 >> 3) * 256u + (uint32_t)(r16 & 7) * 4u;
 
-    // ---- the W scales of the tile's n blocks go to LDS once, ahead of everything else (a register copy behind the first
-    // requests would wait for all of them to land)
-    {
+    // ---- the W scales of the tile's n blocks go to LDS once
+    auto issue_w_scales = [&]() {
         const int nb0 = n0 / kBlockN, last = (p.N + kBlockN - 1) / kBlockN - 1 - nb0, count = Cfg::NBLK * steps;
         const float *base = p.Ws + (int64_t)nb0 * p.ws_n + (int64_t)kb_begin * p.ws_k;
         const bool near = p.ws_n >= 0 && p.ws_k >= 0 && p.ws_n < (1 << 27) && p.ws_k < (1 << 27) / steps;  // 32-bit byte offsets
@@ -227,19 +226,23 @@ __global__ __launch_bounds__(64 * WV) void block_fp8_gemm_rows128_kernel(const G
                 else ((float *)(lds + Cfg::kWsOff))[i] = base[min(b, last) * p.ws_n + it * p.ws_k];
             }
         }
-    }
+    };
     // ---- first requests, in the order of the steady state: step j issues W(j+NSW), then X(j+NSX) (kWFirst: X(j+NSX), then
     // W(j+NSW+1)).  A scale chunk is requested by the step behind the one that requests its first X block, or earlier: it has to
-    // be older than the W rows that may be in flight when that block is waited for.
+    // be older than the W rows that may be in flight when that block is waited for.  The W scales stand behind what step 0
+    // multiplies and ahead of what may be in flight when step 0 is waited for (ahead of everything else they cost a short K 0.3 to
+    // 0.5 us: 30 x 52776 x 256 6.8 / 6.4 us, 76 x 58128 x 256 8.7 / 8.2, 20 x 52336 x 640 10.0 / 9.7).
     constexpr int kAhead = kWFirst ? 1 : 0;
 #pragma unroll
     for (int j = -3; j < 0; ++j) {
         const int wi = j + NSW, xi = j + NSX;
         if (wi >= 0 && wi < steps) issue_w(wi, wi);
+        if (wi == 0 && NSX > NSW) issue_w_scales();
         if (xi >= 0 && xi < steps) {
             issue_x(xi, xi);
             if (xi == 0 || (xi < NSX - 1 + kAhead && (turn(xi) & 7) == 0)) issue_scales(turn(xi) >> 3);
         }
+        if (wi == 0 && NSX == NSW) issue_w_scales();
     }
     const float *wsl = (const float *)(lds + Cfg::kWsOff) + ((n0 + wave * WNS) / kBlockN - n0 / kBlockN) * steps;
 
@@ -343,6 +346,7 @@ __global__ __launch_bounds__(64 * WV) void block_fp8_gemm_rows128_kernel(const G
     };
     // step 0 has landed (what follows it in the order of the first requests may be in flight)
     if (steps >= 3) wait_vmcnt<(NSX - 1) * NXW + (NSW - 1) * NWW>();
+    else if (steps == 2) wait_vmcnt<NXW + NWW>();
     else wait_vmcnt<0>();
     lds_barrier();
     static_for<TN>([&](auto k) { read_w(k, wf[0], lds); });
