@@ -65,6 +65,8 @@ struct Rows128Cfg {
     // ring slots of W and of X: three where they fit beside the scales of a long K
     static constexpr int NSW = MT <= 8 ? 3 : 2;
     static constexpr int NSX = XS ? XS : 3 * kXBytes + NSW * kWBytes + 2 * kChunkBytes <= 157 * 1024 ? 3 : 2;
+    // (the counts of requests in flight hold where an X slot is requested as far ahead as a W slot, or farther)
+    static_assert(NSX >= NSW, "");
     // X row blocks are read from LDS in groups of at most this many; one group's reads run beside another's products
     static constexpr int kGroup = TN == 1 ? 4 : MT == 7 || MT == 8 ? 4 : 3;
     static constexpr int NG = 2 * ((MT + 2 * kGroup - 1) / (2 * kGroup)), G = (MT + NG - 1) / NG;  // (even: two buffers in turn)
