@@ -822,6 +822,7 @@ static size_t tile256x128_workspace(int64_t M, int64_t N, int splits) {
 }
 
 static int64_t n_split_rows(int64_t M, int64_t N, int64_t K, int cus);
+static double other_ns(int64_t M, int64_t N, int64_t K, int variant, int cus);
 
 // The shape -> kernel table (measured on the DeepSeek-V3 and Llama-3 linears over M = 128..4096):
 //   129 <= M <= 384, K >= 2048, at most cus/2 tiles
@@ -846,7 +847,8 @@ static int64_t n_split_rows(int64_t M, int64_t N, int64_t K, int cus);
 //   M <= 64                                          weight streaming (M > 48 and N/128 about the unit count, or M > 32 in
 //                                                    more than five rounds: the kernel that shares the activation block
 //                                                    in the workgroup)
-//   few 256x256 tiles, long K                        stream-K (the plain loop would leave most units idle)
+//   few 256x256 tiles, long K                        stream-K (the plain loop would leave most units idle), from 513 rows on
+//                                                    where the 128x128 tiles are not estimated ahead
 //   128x128 tiles fit one round of two per unit and
 //     (few 256x256 tiles or a short K)               128x128 tiles, K shared between workgroups when they are few
 //                                                    (M >= 768 and N <= 3072: 256x128 tiles with K shared)
@@ -869,13 +871,20 @@ static int pick_variant(int64_t M, int64_t N, int64_t K, int cus, bool allow_row
     // K = 256, M = 4096: 21.3 us for the 128x128 tiles against 27.6)
     if (KB <= 2) return MI355_GEMM_TILE128;
     const bool shares = M > 128 && stream_k_pays(t256, KB, cus, (M + 255) / 256);
-    if (shares && allow_streamk) return MI355_GEMM_TILE256_STREAMK;
+    const bool small = t128 <= 2 * (int64_t)cus && (t256 < (int64_t)cus * 3 / 8 || KB <= 64);  // 128x128 tiles fit the device
+    // From three m tiles on a narrow N the 128x128 tiles, which share K in shorter runs, are ahead of the panel split (us, panel /
+    // 128x128: 517 x 611 x 12288 31.6 / 21.2, 1058 x 128 x 23168 31.5 / 18.3, 1392 x 528 x 10112 33.9 / 29.1).  The panel's estimate
+    // is low where the tiles are few; with 8 % on it 76 of 1535 shapes of 513 rows and more with up to 36 256x256 tiles run more
+    // than 2 % behind the faster of the two, 15 % at most (all of them on the panel split: 562, 1.8 times).
+    const bool tiles128 = shares && small && M > 512 &&
+                          1.08 * other_ns(M, N, K, MI355_GEMM_TILE256_STREAMK, cus) > other_ns(M, N, K, MI355_GEMM_TILE128, cus);
+    if (shares && allow_streamk && !tiles128) return MI355_GEMM_TILE256_STREAMK;
     // 257..384 rows leave the second 256-row tile at most half full; where the 256x256 tiles need a second round
     // anyway the 128x128 ones are ahead (N = 36864, K = 7168, M = 257 / 384: 144 / 148 us against 161 / 165) -
     // unless the second round is small enough to run as a launch of its own (130 / 139 us then)
     if (M > 256 && M <= 384 && t256 > cus && t128 <= 4 * (int64_t)cus && n_split_rows(M, N, K, cus) == 0)
         return MI355_GEMM_TILE128;
-    if (t128 <= 2 * (int64_t)cus && (t256 < (int64_t)cus * 3 / 8 || KB <= 64)) {
+    if (small) {
         // a narrow N under many rows: 256x128 tiles with K shared load half as much X per product as the 128x128
         // ones and still fill the device (q_a+kv_a, N = 2112, K = 7168, M = 768 / 1024 / 1536: 35.0 / 40.6 / 50.6 us
         // against 38.7 / 60.2 / 60.6; not under 12 n tiles: N = 256 / 512, M = 1024: 17.5 / 17.5 against 20.6 / 21.4)

@@ -418,6 +418,18 @@ def test_no_stream_k_without_its_workspace():
             assert lib.mi355_block_fp8_gemm_plan(*shape, ws_bytes, 256) == want, (shape, ws_bytes)
 
 
+def test_panel_split_on_a_narrow_n():
+    """From three m tiles on the panel split of K is taken only where it is ahead of the 128x128 tiles with K shared (us, panel /
+    128x128: 517 x 611 x 12288 31.6 / 21.2, 1058 x 128 x 23168 31.5 / 18.3, 1392 x 528 x 10112 33.9 / 29.1)."""
+    from lightllm_amd import _lib
+
+    lib = _lib.lib()
+    T128, STREAMK = 2, 8
+    for shape, want in [((517, 611, 12288), T128), ((1058, 128, 23168), T128), ((1392, 528, 10112), T128), ((787, 912, 7936), T128),
+                        ((1457, 224, 24448), T128), ((1772, 3760, 27392), STREAMK), ((640, 7168, 18432), STREAMK), ((1024, 2560, 14336), STREAMK)]:
+        assert lib.mi355_block_fp8_gemm_plan(*shape, 1 << 34, 256) == want, shape
+
+
 @pytest.mark.parametrize("cus", [8, 64, 128, 304])
 def test_shape_table_off_256_compute_units(cus):
     """The table's thresholds are all relative to the compute-unit count but were measured at 256.  On other counts
