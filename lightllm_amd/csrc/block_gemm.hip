@@ -965,19 +965,25 @@ static double other_ns(int64_t M, int64_t N, int64_t K, int variant, int cus) {
 
 // Tiles over M instead of what the table names: from 80 rows on where the estimates say 3 % less (the weight stream's K loop
 // multiplies two thirds as fast as the 256x256 tile's, on tiles that leave little of the device idle and nothing to padding or
-// partial sums).  4400 of 7500 shapes, 1.13 times as fast over all of them, 30 more than 2 % slower (8 % at most); us, before / here:
-// 300 x 4096 x 4096 26.3 / 19.4, 340 x 6144 x 4096 32.0 / 21.4, 300 x 28672 x 4096 68.3 / 51.0, 380 x 27648 x 5120 85.9 / 68.7,
-// 1200 x 6144 x 4096 50.7 / 38.3, 1700 x 5120 x 13824 156 / 122, 1200 x 7168 x 18432 207 / 167, 2500 x 4096 x 4096 55.4 / 46.7.
-// From 80 to 208 rows instead of the 128x128 tiles only (a short K): 1.58 times as fast over 496 shapes, none slower (118 x 5744 x 1792
-// 19.6 / 9.1, 143 x 2032 x 1920 20.2 / 9.2).  The plan keeps the table's name, by which the kernels' sums are compared; from K = 8192 on the 256x128 tiles with K shared do run
-// under theirs (1.17 times behind there, 1.3 to 1.8 times on a shorter K).
+// partial sums).  rowsm_ns was fitted to launches whose smaller weights the memory-side cache held; from HBM a K step of mt row blocks
+// takes about 100 / mt ns more (one row block 340 to 375 ns, two 380 to 460), and that decides against a kernel that shares K
+// (us, over M / 128x128: 566 x 640 x 6400 21.4 / 17.2, 250 x 2800 x 5504 23.8 / 19.2, 266 x 2112 x 7168 25.6 / 22.6).
+// Weights from HBM, random shapes and the ten model weights: 1535 shapes of 80..4096 rows run over M, 1.27 times as fast, 12 of them
+// more than 2 % slower (7 % at most; without the 100 / mt ns 212 more shapes, 126 of them more than 2 % slower, 28 % at most); us,
+// before / here: 300 x 4096 x 4096 26.3 / 19.1, 340 x 6144 x 4096 32.0 / 21.4, 300 x 28672 x 4096 65.0 / 47.8, 380 x 27648 x 5120
+// 85.9 / 68.7, 1200 x 6144 x 4096 50.7 / 38.3, 1700 x 5120 x 13824 156 / 122, 1200 x 7168 x 18432 207 / 167.
+// From 80 to 208 rows instead of the 128x128 tiles only (118 x 5744 x 1792 19.6 / 9.1, 143 x 2032 x 1920 20.2 / 9.2).  The plan keeps
+// the table's name, by which the kernels' sums are compared; from K = 8192 on the 256x128 tiles with K shared do run under theirs (1.17
+// times behind there, 1.3 to 1.8 times on a shorter K).
 static bool rowsm_ahead(int64_t M, int64_t N, int64_t K, int variant, int cus) {
     if (M < 80 || M > 4096 || N < 640 || K < 1024 || K > 20480 || cus < 192) return false;
     if (M <= 208 && variant != MI355_GEMM_TILE128) return false;
     const RowsMPlan pl = rowsm_plan(M, N, K, cus);
     if (pl.mt == 0) return false;
     if (variant == MI355_GEMM_TILE256x128) return K < 8192;
-    return rowsm_ns(M, N, K, pl.mt, pl.wv, cus) < 0.97 * other_ns(M, N, K, variant, cus);
+    const int64_t rounds = ((int64_t)pl.tiles_m * pl.tiles_n + cus - 1) / cus;
+    const double from_hbm = 100.0 * rounds * (K / kBlockK) / pl.mt;
+    return rowsm_ns(M, N, K, pl.mt, pl.wv, cus) + from_hbm < 0.97 * other_ns(M, N, K, variant, cus);
 }
 
 // Workspace of a launch plan on a device with `cus` compute units.

@@ -359,6 +359,17 @@ def test_over_m_query():
                 assert over == 0, (m, n, k)
 
 
+def test_over_m_query_where_k_is_shared():
+    """With the weights from HBM a step of few row blocks waits for its weight rows, so a kernel that shares K keeps these (us, over M
+    / here: 566 x 640 x 6400 21.4 / 17.2, 250 x 2800 x 5504 23.8 / 19.2, 266 x 2112 x 7168 25.6 / 22.6, 929 x 1408 x 9216 36.4 / 33.3)."""
+    from lightllm_amd import _lib
+
+    lib = _lib.lib()
+    for shape, want in [((566, 640, 6400), 0), ((250, 2800, 5504), 0), ((266, 2112, 7168), 0), ((140, 912, 6144), 0), ((929, 1408, 9216), 0),
+                        ((302, 4608, 7680), 0), ((300, 4096, 4096), 1), ((281, 3926, 2432), 1), ((184, 4464, 2560), 1)]:
+        assert lib.mi355_block_fp8_gemm_over_m(*shape, 1 << 34, 256) == want, shape
+
+
 _T256, _T128, _SKINNY, _GENERIC, _T256x128, _STREAMK, _XSHARE, _ROWS, _CU, _ROWSM = 1, 2, 3, 4, 5, 8, 9, 10, 11, 12
 
 
