@@ -822,7 +822,7 @@ static size_t tile256x128_workspace(int64_t M, int64_t N, int splits) {
 }
 
 static int64_t n_split_rows(int64_t M, int64_t N, int64_t K, int cus);
-static double other_ns(int64_t M, int64_t N, int64_t K, int variant, int cus);
+static double other_ns(int64_t M, int64_t N, int64_t K, int variant, size_t ws_bytes, int cus);
 
 // The shape -> kernel table (measured on the DeepSeek-V3 and Llama-3 linears over M = 128..4096):
 //   129 <= M <= 384, K >= 2048, at most cus/2 tiles
@@ -877,7 +877,7 @@ static int pick_variant(int64_t M, int64_t N, int64_t K, int cus, bool allow_row
     // is low where the tiles are few; with 8 % on it 76 of 1535 shapes of 513 rows and more with up to 36 256x256 tiles run more
     // than 2 % behind the faster of the two, 15 % at most (all of them on the panel split: 562, 1.8 times).
     const bool tiles128 = shares && small && M > 512 &&
-                          1.08 * other_ns(M, N, K, MI355_GEMM_TILE256_STREAMK, cus) > other_ns(M, N, K, MI355_GEMM_TILE128, cus);
+                          1.08 * other_ns(M, N, K, MI355_GEMM_TILE256_STREAMK, SIZE_MAX, cus) > other_ns(M, N, K, MI355_GEMM_TILE128, SIZE_MAX, cus);
     if (shares && allow_streamk && !tiles128) return MI355_GEMM_TILE256_STREAMK;
     // 257..384 rows leave the second 256-row tile at most half full; where the 256x256 tiles need a second round
     // anyway the 128x128 ones are ahead (N = 36864, K = 7168, M = 257 / 384: 144 / 148 us against 161 / 165) -
@@ -933,8 +933,9 @@ static int64_t n_split_rows(int64_t M, int64_t N, int64_t K, int cus) {
 }
 
 // What the table's other choices take above 208 rows, in ns: fits to the same shapes (256x256 tiles 2.8 % rms, 128x128 tiles 3.4,
-// panel split of K 5.0, weight stream of one m tile 4.7), 0 for what was not fitted.
-static double other_ns(int64_t M, int64_t N, int64_t K, int variant, int cus) {
+// panel split of K 5.0, weight stream of one m tile 4.7), 0 for what was not fitted.  `ws_bytes` of workspace: the 128x128 tiles run
+// K whole without room for their partial sums (the estimate is 6 % low there).
+static double other_ns(int64_t M, int64_t N, int64_t K, int variant, size_t ws_bytes, int cus) {
     const double kb = (double)(K / kBlockK), weights = 1e-6 * N * K, out = 1e-6 * M * N, c = cus;
     const int64_t KB = K / kBlockK, tm = (M + 255) / 256, tn = (N + 255) / 256, t = tm * tn;
     if (variant == MI355_GEMM_TILE256) {
@@ -945,7 +946,9 @@ static double other_ns(int64_t M, int64_t N, int64_t K, int variant, int cus) {
         return common + full * (8233.0 + 1012.0 * kb);
     }
     if (variant == MI355_GEMM_TILE128) {
-        const int64_t splits = tile128_splits(M, N, K, cus), w = ((M + 127) / 128) * ((N + 127) / 128) * splits;
+        int64_t splits = tile128_splits(M, N, K, cus);
+        if (ws_bytes < tile128_workspace(M, N, (int)splits)) splits = 1;
+        const int64_t w = ((M + 127) / 128) * ((N + 127) / 128) * splits;
         const double steps = (double)((KB + splits - 1) / splits), two = (double)((w + 2 * cus - 1) / (2 * cus));
         return 2938.0 + steps * (743.0 * two + 100.9 * ((w + cus - 1) / cus) + 164.9 * w / c) + 2938.0 * two + 81.0 * out + 32.5 * weights +
                (splits > 1 ? 2069.0 + 11.6 * w : 0.0);
@@ -975,15 +978,19 @@ static double other_ns(int64_t M, int64_t N, int64_t K, int variant, int cus) {
 // From 80 to 208 rows instead of the 128x128 tiles only (118 x 5744 x 1792 19.6 / 9.1, 143 x 2032 x 1920 20.2 / 9.2).  The plan keeps
 // the table's name, by which the kernels' sums are compared; from K = 8192 on the 256x128 tiles with K shared do run under theirs (1.17
 // times behind there, 1.3 to 1.8 times on a shorter K).
-static bool rowsm_ahead(int64_t M, int64_t N, int64_t K, int variant, int cus) {
+// `ws_bytes` (0: none that can be used): what the table's kernel shares K with.  Without it that runs K whole on too few tiles, and
+// the tiles over M are 1.5 to 3.4 times as fast (us, K whole / over M: 300 x 1024 x 18432 147 / 59, 768 x 2112 x 8192
+// 104 / 34; 812 shapes, bit-equal).
+static bool rowsm_ahead(int64_t M, int64_t N, int64_t K, int variant, size_t ws_bytes, int cus) {
     if (M < 80 || M > 4096 || N < 640 || K < 1024 || K > 20480 || cus < 192) return false;
     if (M <= 208 && variant != MI355_GEMM_TILE128) return false;
     const RowsMPlan pl = rowsm_plan(M, N, K, cus);
     if (pl.mt == 0) return false;
-    if (variant == MI355_GEMM_TILE256x128) return K < 8192;
+    if (variant == MI355_GEMM_TILE256x128)
+        return K < 8192 || ws_bytes < tile256x128_workspace(M, N, tile256x128_splits(M, N, K, cus));
     const int64_t rounds = ((int64_t)pl.tiles_m * pl.tiles_n + cus - 1) / cus;
     const double from_hbm = 100.0 * rounds * (K / kBlockK) / pl.mt;
-    return rowsm_ns(M, N, K, pl.mt, pl.wv, cus) + from_hbm < 0.97 * other_ns(M, N, K, variant, cus);
+    return rowsm_ns(M, N, K, pl.mt, pl.wv, cus) + from_hbm < 0.97 * other_ns(M, N, K, variant, ws_bytes, cus);
 }
 
 // Workspace of a launch plan on a device with `cus` compute units.
@@ -1095,7 +1102,7 @@ extern "C" int32_t mi355_block_fp8_gemm_over_m(int64_t M, int64_t N, int64_t K, 
     if (cus <= 0) cus = device_cus();
     const int variant = mi355_block_fp8_gemm_launched(M, N, K, ws_bytes, cus);
     if (variant == MI355_GEMM_ROWS_MTILED) return 1;
-    return rowsm_ahead(M, N, K, variant, cus) && rowsm_limits_ok(rowsm_plan(M, N, K, cus), M, K, K, K / kBlockK, 1) ? 1 : 0;
+    return rowsm_ahead(M, N, K, variant, ws_bytes, cus) && rowsm_limits_ok(rowsm_plan(M, N, K, cus), M, K, K, K / kBlockK, 1) ? 1 : 0;
 }
 
 extern "C" int32_t mi355_block_fp8_gemm_launched(int64_t M, int64_t N, int64_t K, size_t ws_bytes, int32_t cus) {
@@ -1142,7 +1149,7 @@ static int block_fp8_gemm_impl(const void *A, const void *B, const float *As, co
         variant = fast && blocks128 ? resolve_auto(M, N, K, lda, ldb_n, as_m, as_k, ws_usable, ws_bytes, cus)
                                     : MI355_GEMM_GENERIC;
         variant = launched_for(variant, M, N, K, lda, ldb_n, as_m, ws_usable, ws_bytes, cus);
-        if (rowsm_ahead(M, N, K, variant, cus) && rowsm_limits_ok(rowsm_plan(M, N, K, cus), M, K, lda, as_m, as_k))
+        if (rowsm_ahead(M, N, K, variant, ws_usable ? ws_bytes : 0, cus) && rowsm_limits_ok(rowsm_plan(M, N, K, cus), M, K, lda, as_m, as_k))
             variant = MI355_GEMM_ROWS_MTILED;
     }
     if (was_auto && variant == MI355_GEMM_TILE256) {

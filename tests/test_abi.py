@@ -370,6 +370,17 @@ def test_over_m_query_where_k_is_shared():
         assert lib.mi355_block_fp8_gemm_over_m(*shape, 1 << 34, 256) == want, shape
 
 
+def test_over_m_query_without_a_workspace():
+    """A kernel that shares K runs it whole where its partial sums have no room, and is compared as that (us, K whole / over M: 300 x
+    1024 x 18432 147 / 59, 768 x 2112 x 8192 104 / 34)."""
+    from lightllm_amd import _lib
+
+    lib = _lib.lib()
+    for shape in [(300, 1024, 18432), (202, 705, 18816), (768, 2112, 8192), (487, 2768, 11008)]:
+        over = [lib.mi355_block_fp8_gemm_over_m(*shape, ws_bytes, 256) for ws_bytes in (0, 65536, 65536 + (8 << 20), 1 << 26, 1 << 34)]
+        assert over == [1, 1, 1, 0, 0], (shape, over)
+
+
 _T256, _T128, _SKINNY, _GENERIC, _T256x128, _STREAMK, _XSHARE, _ROWS, _CU, _ROWSM = 1, 2, 3, 4, 5, 8, 9, 10, 11, 12
 
 

@@ -652,6 +652,21 @@ def test_tiles_over_m_instead_of_the_tables_kernel(hip, M, N, K):
     assert torch.equal(c, _run(xq, xs.t().contiguous().t(), wq, ws, None))
 
 
+# a kernel that shares K gives way without room for its partial sums: the 128x128 and 256x128 tiles' edges of the rule
+@pytest.mark.parametrize("M,N,K", [(300, 1024, 18432), (202, 705, 18816), (768, 2112, 8192), (124, 15460, 14592), (487, 2769, 11008)])
+def test_tiles_over_m_without_a_workspace(hip, M, N, K):
+    print(f"gemm over M, no workspace M={M} N={N} K={K}", flush=True)
+    if _lib_cus() == 256:
+        assert hip.mi355_block_fp8_gemm_over_m(M, N, K, 0, 0) == 1 and hip.mi355_block_fp8_gemm_over_m(M, N, K, 1 << 34, 0) == 0
+    xq, xs, wq, ws = _prep(M, N, K, seed=M + N)
+    c = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    rc = hip.mi355_block_fp8_gemm(xq.data_ptr(), wq.data_ptr(), xs.data_ptr(), ws.data_ptr(), c.data_ptr(), M, N, K, K, 1, K, N, xs.stride(0),
+                                  xs.stride(1), 1, ws.stride(0), 128, 128, None, 0, 0, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert rc == 0, hip.mi355_error_string(rc)
+    assert torch.equal(c.view(torch.int16), _run(xq, xs, wq, ws, "tile256").view(torch.int16))
+
+
 # 209..352 rows in two or three tiles of the activation-block stream, 385..960 rows on a wider N: the edges of both ranges, row counts
 # that leave the last tile one row, N that leaves the last column of tiles one weight row, the shortest and longest K
 @pytest.mark.parametrize("M,N,K,variant", [(209, 12288, 2048, "rows128"), (225, 12289, 1536, "rows128"), (352, 27648, 1536, "rows128"),
