@@ -704,8 +704,8 @@ static bool rowsm_lds_ok(int64_t mt, int64_t wv, int64_t K) {
 // 1024..18432, the nine most likely tiles of each; weights from HBM; 6 % rms).  A K step of a tile (its products; the X block,
 // which every wave reads; its W rows; two slots of W instead of three; more than six waves), what all tiles pull together, the
 // output and the weights; 2.9 us a round.  The tile of the least estimate is 0.8 % behind the fastest one on average.
-static double rowsm_ns(int64_t M, int64_t N, int64_t K, int64_t mt, int64_t wv, int cus) {
-    const int64_t tm = ((M + 15) / 16 + mt - 1) / mt, tn = (N + 32 * wv - 1) / (32 * wv), t = tm * tn;
+static double rowsm_ns(int64_t M, int64_t N, int64_t K, const RowsMPlan &pl, int cus) {
+    const int mt = pl.mt, wv = pl.wv, t = pl.tiles_m * pl.tiles_n;
     const double kb = (double)(K / kBlockK), rounds = (double)((t + cus - 1) / cus);
     const double step = 83.0 + 0.457 * mt * wv + 49.95 * mt + 18.96 * wv + (mt > 8 ? 59.7 : 0.0) + (wv > 6 ? 9.9 : 0.0) + (wv == 8 ? 23.6 : 0.0);
     return 792.0 + rounds * (2939.0 + kb * step) + 6.0 * kb * t / cus * (mt + 2 * wv) + M * N * 4.91e-4 + N * K * 7.95e-5;
@@ -714,16 +714,17 @@ static double rowsm_ns(int64_t M, int64_t N, int64_t K, int64_t mt, int64_t wv, 
 static RowsMPlan rowsm_plan(int64_t M, int64_t N, int64_t K, int cus) {
     RowsMPlan best = rowsm_round_plan(M, N, cus);
     if (M < 80 || M > 4096 || N < 640 || cus < 8) return best;
-    double best_ns = best.mt ? 0.96 * rowsm_ns(M, N, K, best.mt, best.wv, cus) : 0.0;
-    const int64_t blocks = (M + 15) / 16;
+    double best_ns = best.mt ? 0.96 * rowsm_ns(M, N, K, best, cus) : 0.0;
+    const int blocks = (int)((M + 15) / 16);
     for (int wv = 5; wv <= 8; ++wv) {
         const int64_t tn = (N + 32 * wv - 1) / (32 * wv);
-        for (int64_t mt = wv == 7 ? 9 : 1; mt <= 13; ++mt) {
-            const int64_t tm = (blocks + mt - 1) / mt;
-            if (tm < 2 || tm * tn > 4 * (int64_t)cus || !rowsm_lds_ok(mt, wv, K)) continue;  // (the kernel numbers two m tiles and more)
-            const double ns = rowsm_ns(M, N, K, mt, wv, cus);
+        if (2 * tn > 4 * (int64_t)cus) continue;  // (the kernel numbers two m tiles and more)
+        for (int mt = wv == 7 ? 9 : 1; mt <= 13; ++mt) {
+            const RowsMPlan pl = {mt, wv, (blocks + mt - 1) / mt, (int)tn};
+            if (pl.tiles_m < 2 || pl.tiles_m * pl.tiles_n > 4 * cus || !rowsm_lds_ok(mt, wv, K)) continue;
+            const double ns = rowsm_ns(M, N, K, pl, cus);
             if (best.mt == 0 || ns < best_ns) {
-                best = {(int)mt, wv, (int)tm, (int)tn};
+                best = pl;
                 best_ns = ns;
             }
         }
@@ -981,16 +982,19 @@ static double other_ns(int64_t M, int64_t N, int64_t K, int variant, size_t ws_b
 // `ws_bytes` (0: none that can be used): what the table's kernel shares K with.  Without it that runs K whole on too few tiles, and
 // the tiles over M are 1.5 to 3.4 times as fast (us, K whole / over M: 300 x 1024 x 18432 147 / 59, 768 x 2112 x 8192
 // 104 / 34; 812 shapes, bit-equal).
-static bool rowsm_ahead(int64_t M, int64_t N, int64_t K, int variant, size_t ws_bytes, int cus) {
-    if (M < 80 || M > 4096 || N < 640 || K < 1024 || K > 20480 || cus < 192) return false;
-    if (M <= 208 && variant != MI355_GEMM_TILE128) return false;
-    const RowsMPlan pl = rowsm_plan(M, N, K, cus);
-    if (pl.mt == 0) return false;
+static RowsMPlan rowsm_ahead(int64_t M, int64_t N, int64_t K, int variant, size_t ws_bytes, int cus) {
+    const RowsMPlan none = {0, 0, 0, 0};
+    if (M < 80 || M > 4096 || N < 640 || K < 1024 || K > 20480 || cus < 192) return none;
+    if (M <= 208 && variant != MI355_GEMM_TILE128) return none;
     if (variant == MI355_GEMM_TILE256x128)
-        return K < 8192 || ws_bytes < tile256x128_workspace(M, N, tile256x128_splits(M, N, K, cus));
-    const int64_t rounds = ((int64_t)pl.tiles_m * pl.tiles_n + cus - 1) / cus;
+        return K < 8192 || ws_bytes < tile256x128_workspace(M, N, tile256x128_splits(M, N, K, cus)) ? rowsm_plan(M, N, K, cus) : none;
+    const double other = other_ns(M, N, K, variant, ws_bytes, cus);
+    if (other == 0.0) return none;
+    const RowsMPlan pl = rowsm_plan(M, N, K, cus);
+    if (pl.mt == 0) return none;
+    const int rounds = (pl.tiles_m * pl.tiles_n + cus - 1) / cus;
     const double from_hbm = 100.0 * rounds * (K / kBlockK) / pl.mt;
-    return rowsm_ns(M, N, K, pl.mt, pl.wv, cus) + from_hbm < 0.97 * other_ns(M, N, K, variant, ws_bytes, cus);
+    return rowsm_ns(M, N, K, pl, cus) + from_hbm < 0.97 * other ? pl : none;
 }
 
 // Workspace of a launch plan on a device with `cus` compute units.
@@ -1044,11 +1048,14 @@ static size_t workspace_bytes_for(int64_t M, int64_t N, int64_t K, int32_t varia
 // Stream-K's workspace and the 256-row stream are looked at first because the table's other choice for their shapes can be any of
 // the kernels checked after them.
 static int resolve_auto(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int64_t as_m, int64_t as_k,
-                        bool ws_usable, size_t ws_bytes, int cus) {
+                        bool ws_usable, size_t ws_bytes, int cus, RowsMPlan *tiles = nullptr) {
     const bool streamk = ws_usable && ws_bytes >= stream_k_workspace(cus / 8 * 8);  // (every plan of it takes that much)
     int variant = pick_variant(M, N, K, cus, true, streamk);
-    if (variant == MI355_GEMM_ROWS_MTILED && !rowsm_limits_ok(rowsm_plan(M, N, K, cus), M, K, lda, as_m, as_k))
-        variant = pick_variant(M, N, K, cus, false, streamk);
+    if (variant == MI355_GEMM_ROWS_MTILED) {
+        const RowsMPlan pl = rowsm_plan(M, N, K, cus);
+        if (!rowsm_limits_ok(pl, M, K, lda, as_m, as_k)) variant = pick_variant(M, N, K, cus, false, streamk);
+        else if (tiles) *tiles = pl;
+    }
     if (variant == MI355_GEMM_ROWS128 &&
         (!rows128_limits_ok(M, N, K, lda, as_m, as_k, cus) ||
          (rows128_splits(M, N, K, cus) > 1 && (!ws_usable || ws_bytes < rows128_workspace(M, N, K, cus)))))
@@ -1083,6 +1090,20 @@ static int launched_for(int variant, int64_t M, int64_t N, int64_t K, int64_t ld
     return skinny_rows_check(M, N, K, lda, ldw, as_m, cus, ws_usable, ws_bytes) == MI355_OK ? MI355_GEMM_SKINNY_ROWS : variant;
 }
 
+// The kernel an AUTO call launches (first), `tiles` its tiles where that is ROWS_MTILED: the plan is made once a call.
+static int auto_launch(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int64_t as_m, int64_t as_k, bool ws_usable,
+                       size_t ws_bytes, int cus, RowsMPlan &tiles) {
+    tiles = {0, 0, 0, 0};
+    const int variant = launched_for(resolve_auto(M, N, K, lda, ldw, as_m, as_k, ws_usable, ws_bytes, cus, &tiles), M, N, K, lda, ldw, as_m,
+                                     ws_usable, ws_bytes, cus);
+    if (variant == MI355_GEMM_ROWS_MTILED) {
+        if (tiles.mt == 0) tiles = rowsm_plan(M, N, K, cus);
+        return variant;
+    }
+    tiles = rowsm_ahead(M, N, K, variant, ws_usable ? ws_bytes : 0, cus);
+    return rowsm_limits_ok(tiles, M, K, lda, as_m, as_k) ? MI355_GEMM_ROWS_MTILED : variant;
+}
+
 }  // namespace mi355
 
 using namespace mi355;
@@ -1100,9 +1121,9 @@ extern "C" int32_t mi355_block_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, si
 
 extern "C" int32_t mi355_block_fp8_gemm_over_m(int64_t M, int64_t N, int64_t K, size_t ws_bytes, int32_t cus) {
     if (cus <= 0) cus = device_cus();
-    const int variant = mi355_block_fp8_gemm_launched(M, N, K, ws_bytes, cus);
-    if (variant == MI355_GEMM_ROWS_MTILED) return 1;
-    return rowsm_ahead(M, N, K, variant, ws_bytes, cus) && rowsm_limits_ok(rowsm_plan(M, N, K, cus), M, K, K, K / kBlockK, 1) ? 1 : 0;
+    if (M <= 0 || N <= 0 || K <= 0 || K % kBlockK != 0) return 0;
+    RowsMPlan tiles;
+    return auto_launch(M, N, K, K, K, K / kBlockK, 1, ws_bytes > 0, ws_bytes, cus, tiles) == MI355_GEMM_ROWS_MTILED ? 1 : 0;
 }
 
 extern "C" int32_t mi355_block_fp8_gemm_launched(int64_t M, int64_t N, int64_t K, size_t ws_bytes, int32_t cus) {
@@ -1144,13 +1165,10 @@ static int block_fp8_gemm_impl(const void *A, const void *B, const float *As, co
                       256 * lda < (1ll << 32) && 256 * ldb_n < (1ll << 32) && 256 * as_m * 4 < (1ll << 32) &&
                       as_m >= 0 && as_k >= 0;
     const bool was_auto = variant == MI355_GEMM_AUTO;
+    RowsMPlan over_m = {0, 0, 0, 0};
     if (was_auto) {
         const bool ws_usable = ws && ((uintptr_t)ws & 15) == 0;
-        variant = fast && blocks128 ? resolve_auto(M, N, K, lda, ldb_n, as_m, as_k, ws_usable, ws_bytes, cus)
-                                    : MI355_GEMM_GENERIC;
-        variant = launched_for(variant, M, N, K, lda, ldb_n, as_m, ws_usable, ws_bytes, cus);
-        if (rowsm_ahead(M, N, K, variant, ws_usable ? ws_bytes : 0, cus) && rowsm_limits_ok(rowsm_plan(M, N, K, cus), M, K, lda, as_m, as_k))
-            variant = MI355_GEMM_ROWS_MTILED;
+        variant = fast && blocks128 ? auto_launch(M, N, K, lda, ldb_n, as_m, as_k, ws_usable, ws_bytes, cus, over_m) : MI355_GEMM_GENERIC;
     }
     if (was_auto && variant == MI355_GEMM_TILE256) {
         const int64_t n1 = n_split_rows(M, N, K, cus);
@@ -1270,7 +1288,7 @@ static int block_fp8_gemm_impl(const void *A, const void *B, const float *As, co
             }
         }
         case MI355_GEMM_ROWS_MTILED: {
-            const RowsMPlan mp = rowsm_plan(M, N, K, cus);
+            const RowsMPlan mp = was_auto ? over_m : rowsm_plan(M, N, K, cus);
             if (!was_auto && rowsm_round_plan(M, N, cus).mt == 0) return MI355_EUNSUPPORTED;  // by name: a single round
             if (!rowsm_limits_ok(mp, M, K, lda, as_m, as_k)) return MI355_EUNSUPPORTED;
             return launch_rowsm(a, mp, st);
