@@ -997,11 +997,22 @@ static RowsMPlan rowsm_ahead(int64_t M, int64_t N, int64_t K, int variant, size_
     return rowsm_ns(M, N, K, pl, cus) + from_hbm < 0.97 * other ? pl : none;
 }
 
+static int auto_launch(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldw, int64_t as_m, int64_t as_k, bool ws_usable,
+                       size_t ws_bytes, int cus, RowsMPlan &tiles);
+
+// Whether an AUTO call in packed layout runs as tiles over M with any workspace and without one.
+static bool over_m_without_workspace(int64_t M, int64_t N, int64_t K, int cus) {
+    RowsMPlan tiles;
+    return M >= 80 && M <= 4096 && auto_launch(M, N, K, K, K, K / kBlockK, 1, true, SIZE_MAX, cus, tiles) == MI355_GEMM_ROWS_MTILED &&
+           auto_launch(M, N, K, K, K, K / kBlockK, 1, false, 0, cus, tiles) == MI355_GEMM_ROWS_MTILED;
+}
+
 // Workspace of a launch plan on a device with `cus` compute units.
 static size_t workspace_bytes_for(int64_t M, int64_t N, int64_t K, int32_t variant, int cus) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     if (K % kBlockK != 0) return 0;
     if (variant == MI355_GEMM_AUTO) {
+        if (over_m_without_workspace(M, N, K, cus)) return 0;
         variant = pick_variant(M, N, K, cus);
         const int64_t n1 = variant == MI355_GEMM_TILE256 ? n_split_rows(M, N, K, cus) : 0;
         if (n1 > 0) {

@@ -381,6 +381,21 @@ def test_over_m_query_without_a_workspace():
         assert over == [1, 1, 1, 0, 0], (shape, over)
 
 
+def test_tiles_over_m_ask_for_no_workspace():
+    """An AUTO call that runs as tiles over M asks for none of the workspace of the kernel they stand in for (600 x 2560 x 8192: the
+    128 MiB of stream-K), and runs as that without it."""
+    from lightllm_amd import _lib
+
+    lib = _lib.lib()
+    for shape in [(600, 2560, 8192), (1024, 2112, 8192), (300, 4096, 4096), (2500, 4096, 4096), (118, 5744, 1792)]:
+        assert lib.mi355_block_fp8_gemm_workspace_bytes(*shape, 0) == 0, shape
+    for m, n, k in _sweep_shapes(7, 2000):
+        over = [lib.mi355_block_fp8_gemm_over_m(m, n, k, ws_bytes, 0) for ws_bytes in (0, 1 << 34)]
+        need = lib.mi355_block_fp8_gemm_workspace_bytes(m, n, k, 0)
+        assert need > 0 or not over[1] or over[0], (m, n, k)
+        assert lib.mi355_block_fp8_gemm_over_m(m, n, k, need, 0) == over[1], (m, n, k)
+
+
 _T256, _T128, _SKINNY, _GENERIC, _T256x128, _STREAMK, _XSHARE, _ROWS, _CU, _ROWSM = 1, 2, 3, 4, 5, 8, 9, 10, 11, 12
 
 
