@@ -970,10 +970,10 @@ static double other_ns(int64_t M, int64_t N, int64_t K, int variant, size_t ws_b
 // Tiles over M instead of what the table names: from 80 rows on where the estimates say 3 % less (the weight stream's K loop
 // multiplies two thirds as fast as the 256x256 tile's, on tiles that leave little of the device idle and nothing to padding or
 // partial sums).  rowsm_ns was fitted to launches whose smaller weights the memory-side cache held; from HBM a K step of mt row blocks
-// takes about 100 / mt ns more (one row block 340 to 375 ns, two 380 to 460), and that decides against a kernel that shares K
+// takes about 100 / mt ns more up to four of them (one row block 340 to 375 ns, two 380 to 460), and that decides against a kernel that shares K
 // (us, over M / 128x128: 566 x 640 x 6400 21.4 / 17.2, 250 x 2800 x 5504 23.8 / 19.2, 266 x 2112 x 7168 25.6 / 22.6).
-// Weights from HBM, random shapes and the ten model weights: 1535 shapes of 80..4096 rows run over M, 1.27 times as fast, 12 of them
-// more than 2 % slower (7 % at most; without the 100 / mt ns 212 more shapes, 126 of them more than 2 % slower, 28 % at most); us,
+// Weights from HBM, random shapes and the ten model weights: 1564 shapes of 80..4096 rows run over M, 1.27 times as fast, 12 of them
+// more than 2 % slower (7 % at most; without the 100 / mt ns 183 more shapes, 126 of them more than 2 % slower, 28 % at most); us,
 // before / here: 300 x 4096 x 4096 26.3 / 19.1, 340 x 6144 x 4096 32.0 / 21.4, 300 x 28672 x 4096 65.0 / 47.8, 380 x 27648 x 5120
 // 85.9 / 68.7, 1200 x 6144 x 4096 50.7 / 38.3, 1700 x 5120 x 13824 156 / 122, 1200 x 7168 x 18432 207 / 167.
 // From 80 to 208 rows instead of the 128x128 tiles only (118 x 5744 x 1792 19.6 / 9.1, 143 x 2032 x 1920 20.2 / 9.2).  The plan keeps
@@ -993,7 +993,7 @@ static RowsMPlan rowsm_ahead(int64_t M, int64_t N, int64_t K, int variant, size_
     const RowsMPlan pl = rowsm_plan(M, N, K, cus);
     if (pl.mt == 0) return none;
     const int rounds = (pl.tiles_m * pl.tiles_n + cus - 1) / cus;
-    const double from_hbm = 100.0 * rounds * (K / kBlockK) / pl.mt;
+    const double from_hbm = pl.mt <= 4 ? 100.0 * rounds * (K / kBlockK) / pl.mt : 0.0;
     return rowsm_ns(M, N, K, pl, cus) + from_hbm < 0.97 * other ? pl : none;
 }
 
