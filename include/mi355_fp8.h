@@ -149,12 +149,14 @@ int32_t mi355_block_fp8_gemm_variant(int64_t M, int64_t N, int64_t K);
 
 /* The kernel an MI355_GEMM_AUTO call launches (first) for a packed, 16-byte aligned problem when it is handed a
  * workspace of `ws_bytes` bytes (0 = none), on a device with `cus` compute units (<= 0: the current device): the
- * table's choice, or the kernel it falls back to where that choice's workspace is missing - the chain always ends in
+ * table's choice, or the kernel it falls back to where that choice's workspace is missing, unless tiles over M run instead
+ * (mi355_block_fp8_gemm_over_m) - the chain always ends in
  * a kernel that runs without one, so AUTO never returns MI355_EWORKSPACE.  Launches nothing.  No counterpart in the
  * reference; for tests of the table off the device it was measured on, and for callers that size workspaces. */
 int32_t mi355_block_fp8_gemm_plan(int64_t M, int64_t N, int64_t K, size_t ws_bytes, int32_t cus);
 
-/* The code of the kernel that the call of mi355_block_fp8_gemm_plan launches.  It differs from the plan's where the table's
+/* The code of the kernel that the call of mi355_block_fp8_gemm_plan launches unless mi355_block_fp8_gemm_over_m is 1 (many calls of
+ * 209..4096 rows): then tiles over M run instead of it.  It differs from the plan's where the table's
  * MI355_GEMM_ROWS128 covers more than one kernel: MI355_GEMM_SKINNY_ROWS at 65..128 rows, MI355_GEMM_ROWS_MTILED at 209..352.
  * Asked for by this code a launch is AUTO's, bit for bit, but for MI355_GEMM_ROWS128 from 65 rows on under K a multiple of 4096
  * (see there), the second launch that MI355_GEMM_TILE256 may be followed by and calls that run as tiles over M
@@ -163,12 +165,14 @@ int32_t mi355_block_fp8_gemm_launched(int64_t M, int64_t N, int64_t K, size_t ws
 
 /* 1 where that AUTO call runs as tiles over M (the kernel of MI355_GEMM_ROWS_MTILED, in up to four rounds) instead of the kernel
  * above, 0 where not: at 209..4096 rows (80..208 instead of MI355_GEMM_TILE128 only), N >= 640 and 1024 <= K <= 20480 it does
- * wherever the tiles are estimated to be 3 % ahead.
+ * wherever the tiles are estimated to be 3 % ahead of that kernel as it runs with `ws_bytes` of workspace; instead of
+ * MI355_GEMM_TILE256x128 always below K = 8192 and without the workspace of its shared K, never otherwise.
  * K is never shared in them, so the result has the bits of MI355_GEMM_TILE256, and of the kernel above unless that shares K.
  * Launches nothing; no counterpart in the reference. */
 int32_t mi355_block_fp8_gemm_over_m(int64_t M, int64_t N, int64_t K, size_t ws_bytes, int32_t cus);
 
-/* Bytes of workspace the launch plan of the CURRENT device needs for this shape and variant (0 = none). */
+/* Bytes of workspace the launch plan of the CURRENT device needs for this shape and variant (0 = none; MI355_GEMM_AUTO asks for none
+ * where it runs as tiles over M with or without one). */
 size_t mi355_block_fp8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int32_t variant);
 
 /* mi355_block_fp8_gemm for callers that cannot allocate device memory (code under HIP graph capture, tight serving

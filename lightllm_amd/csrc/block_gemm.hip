@@ -155,8 +155,9 @@ static bool stream_k_pays(int64_t tiles, int64_t KB, int cus, int64_t tiles_m) {
     // x 10240 36.9 / 38.4, 266 x 1232 x 12928 25.5 / 30.2, 597 x 1296 x 11136 30.8 / 34.7; 684 x 1696 x 10112 36.1 / 33.7)
     const bool few = tiles_m <= 2 ? tiles * 64 < 3 * (int64_t)cus || (tiles * 32 < 3 * (int64_t)cus && KB < 96)
                                   : tiles_m == 3 && tiles * 64 < 5 * (int64_t)cus && KB < 96;
-    // three m tiles under a short K or on a narrow N keep the 256x128 tiles, which share K the same way, whatever it costs
-    // (600 x 5120 x 6144 52 us against 42, 768 x 2112 x 8192 36.5 / 34.0)
+    // three m tiles under a short K or on a narrow N keep the name of the 256x128 tiles, which share K the same way and with which
+    // launches by name are compared, although the panel split is ahead (600 x 5120 x 6144 52 us against 42, 768 x 2112 x 8192 36.5 /
+    // 34.0); below K = 8192 AUTO runs them over M
     const bool kept = tiles_m == 3 && (KB <= 48 || (tiles <= 27 && KB <= 64));
     if (MI355_SK_PANEL && panel > 0 && KB >= 40 && tiles * panel * 8 >= (int64_t)cus * 3 && !few && !kept) return true;
     const int groups = stream_k_groups(tiles, KB, cus);
@@ -738,14 +739,16 @@ static bool rowsm_limits_ok(const RowsMPlan &pl, int64_t M, int64_t K, int64_t l
     return rowsm_lds_ok(pl.mt, pl.wv, K);
 }
 
-// Where it pays (forced against the table's previous choice over N = 1024..8192, K = 1536..14336, M = 400..4096,
+// Where the table names it (forced against the table's previous choice with the K loop before the pipelined one, over N =
+// 1024..8192, K = 1536..14336, M = 400..4096,
 // 256 units).  With K <= 5120 and at most 8 row blocks per tile (three ring slots) it is ahead on every N <= 5120:
 // 1.2 to 2.0 times with up to 4 row blocks (N = 4096, K = 4096, M = 512 / 1024 / 2048: 22.4 / 28.8 / 42.0 us against
 // 27.9 / 36.5 / 47.2; N = 2112, K = 2048, M = 1024: 1.95 times), 1.0 to 1.2 with 5..8; from N = 6144 on and with more
-// row blocks (two slots) the square tiles are level or ahead.  With K = 6144 .. 7168 the panel split of the 256x256
+// row blocks (two slots) the square tiles were level or ahead.  With K = 6144 .. 7168 the panel split of the 256x256
 // tiles shares K between idle units and takes most of the gain: 2..6 row blocks on N <= 3072 are still 1.04 to 1.3
 // times ahead (q_a+kv_a, N = 2112, K = 7168, M = 512 / 1024 / 2048: 1.11 / 1.12 / 1.04), a single block or a wider N
-// is behind.  From K = 8192 on the kernels that share K win everywhere.
+// was behind, and from K = 8192 on the kernels that share K.  With the K loop as it is now the tiles are ahead of those on many more
+// shapes; rowsm_ahead decides that by estimates, and this rule which of them have the name.
 // On a wider N, K <= 5120: up to 960 rows and N = 15360 with at most 8 row blocks (us, before / here: N = 6144, K = 4096, M = 450 /
 // 700 / 850 36.4 / 41.4 / 43.0 against 28.2 / 33.9 / 35.6; 8192 x 4096, M = 400 / 640 36.4 / 42.9 against 29.7 / 37.2; 10240
 // x 5120, M = 512 55.4 / 45.3; 12288 x 4096, M = 400 / 640 44.2 / 45.3 against 37.1 / 44.3).
@@ -933,7 +936,8 @@ static int64_t n_split_rows(int64_t M, int64_t N, int64_t K, int cus) {
     return n1 > 0 && n1 < N ? n1 : 0;
 }
 
-// What the table's other choices take above 208 rows, in ns: fits to the same shapes (256x256 tiles 2.8 % rms, 128x128 tiles 3.4,
+// What the table's other choices take above 208 rows (the 128x128 tiles from 80 on), in ns: fits to the same shapes (256x256
+// tiles 2.8 % rms, 128x128 tiles 3.4,
 // panel split of K 5.0, weight stream of one m tile 4.7), 0 for what was not fitted.  `ws_bytes` of workspace: the 128x128 tiles run
 // K whole without room for their partial sums (the estimate is 6 % low there).
 static double other_ns(int64_t M, int64_t N, int64_t K, int variant, size_t ws_bytes, int cus) {

@@ -1,4 +1,5 @@
-// Block-scaled FP8 GEMM for at most 384 activation rows on gfx950: a weight stream with the activation block in LDS.
+// Block-scaled FP8 GEMM on gfx950, a weight stream with the activation block in LDS: at most 384 activation rows as one block, or
+// tiled over M for up to 4096 rows and more.
 //
 // With so few rows of X every weight byte is used once (TN = 2) per launch, so the launch is a stream over W, and
 // the square tiles spend it badly: a 128x128 tile keeps 16 KiB of W per K step in flight and one round of such tiles
@@ -23,7 +24,7 @@
 //   7168 52.8 / 45.9, 960 x 6144 x 4096 40.5 / 32.8, 160 x 36864 x 7168 80.3 / 68.6, 384 x 4096 x 14336 51.4 / 45.2, 80 x
 //   28672 x 4096 32.4 / 29.4; level where the memory is the bound (48 x 36864 x 7168 52.3 / 52.7, 32 x 18432 x 7168 30.9).
 //   X scales come in [rows][8 steps] chunks by 4-byte requests (any scale layout); the W scales of the tile's
-//   128-wide n blocks are requested to LDS once.
+//   128-wide n blocks are requested to LDS once, behind the rows of the first step.
 //   A compute unit pulls 35 to 40 GB/s from HBM through this tile, so the launch wants a workgroup on every unit:
 //   when the tiles are too few for that the K range is shared between workgroups.  Their partial sums are
 //   16*MT x 128*TN floats each, too many for the last workgroup of a tile to add alone (one compute unit reads
@@ -35,7 +36,8 @@
 //   The same holds for 129..208 rows on a wide N, whose 128-row tiles need a second round and whose 256x256 tiles
 //   leave units idle: workgroups of 4..7 waves at TN = 1 (64..112 weight rows) or, on a wider N still, 5..8 waves at
 //   TN = 2 with up to 13 row blocks (160..256 weight rows), whichever makes one round.  Every wave reads the whole X
-//   block from LDS, so the time of such a launch grows with M and the square tiles take over from about 220 rows.
+//   block from LDS, so the time of such a launch grows with M: from 209 rows on the same tile runs over several m tiles (up to 13
+//   row blocks each, in one to four rounds), wherever that is estimated ahead of the square tiles and of a shared K.
 //
 //   (Half-width tiles of four waves on two slots, two workgroups to a unit, were tried for shapes whose 256-row
 //   tiles leave units idle and cannot share K usefully - N = 36864: 144 tiles on 256 units - and were slower: 85 us
