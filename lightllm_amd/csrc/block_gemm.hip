@@ -634,7 +634,11 @@ static bool rows128_pays(int64_t M, int64_t N, int64_t K, int cus, bool allow_st
         // from about 200 rows the panel split of the 256x256 tiles is level or ahead on the large weights, its time
         // flat in M (DeepSeek-V3 down, M = 208 / 240 / 256: 55.1 / 54.9 / 56.9 us against 58.4 / 60.4 / 63.3;
         // o_proj 53.1 / 52.8 / 58.1 against 54.9 / 57.5 / 57.6)
-        if (M > 200 && N * K >= 100000000ll && allow_streamk && stream_k_pays((N + 255) / 256, K / kBlockK, cus, 1)) return false;
+        // With fewer than eight runs of K (a wider N or a shorter K) it is behind: of 415 such shapes none is ahead by more than
+        // 4 %, 1.11 times behind in the middle (203 x 31072 x 5760 77.9 us, 67.9 here before the pipelined K loop, 211 x 9152 x
+        // 11520 61.3 / 44.9, 204 x 32336 x 6144 84.2 / 61.2).
+        const bool runs8 = (N + 255) / 256 * 8 <= cus && K >= 96 * kBlockK;
+        if (M > 200 && N * K >= 100000000ll && runs8 && allow_streamk && stream_k_pays((N + 255) / 256, K / kBlockK, cus, 1)) return false;
         // and on small weights the 128x128 tiles with K shared (N = 4096, K = 4096, M = 224 / 256: 18.9 / 19.0 us
         // against 20.9 / 21.3; N = 7168, K = 2304, M = 256: 19.7 against 23.0)
         if (M > 192 && N * K < 20000000ll) return false;
@@ -831,7 +835,7 @@ static double other_ns(int64_t M, int64_t N, int64_t K, int variant, size_t ws_b
 // The shape -> kernel table (measured on the DeepSeek-V3 and Llama-3 linears over M = 128..4096):
 //   129 <= M <= 384, K >= 2048, at most cus/2 tiles
 //     of 128 weight rows (cus if M <= 160; above
-//     256 rows only if N*K >= 2e7; 201..256 and
+//     256 rows only if N*K >= 2e7; 201..256 (eight runs) and
 //     337..384 rows on N*K >= 1e8 go to the panel
 //     split of stream-K instead)                     the weight stream with the activation block in LDS
 //   129 <= M <= 208 (192), 0.55 cus .. cus tiles of

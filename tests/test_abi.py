@@ -467,6 +467,18 @@ def test_panel_split_on_a_narrow_n():
         assert lib.mi355_block_fp8_gemm_plan(*shape, 1 << 34, 256) == want, shape
 
 
+def test_panel_split_at_201_to_256_rows():
+    """One m tile on a large weight: the panel split of K takes over from the activation-block stream only where it has eight runs
+    and more (us, panel / stream: 204 x 32336 x 6144 84.2 / 61.2, 211 x 9152 x 11520 61.3 / 44.9)."""
+    from lightllm_amd import _lib
+
+    lib = _lib.lib()
+    ROWS, STREAMK = 10, 8
+    for shape, want in [((203, 31072, 5760), ROWS), ((211, 9152, 11520), ROWS), ((204, 32336, 6144), ROWS), ((203, 16000, 7040), ROWS),
+                        ((240, 7168, 18432), STREAMK), ((256, 7168, 14336), STREAMK), ((200, 7168, 18432), ROWS)]:
+        assert lib.mi355_block_fp8_gemm_plan(*shape, 1 << 34, 256) == want, shape
+
+
 @pytest.mark.parametrize("cus", [8, 64, 128, 304])
 def test_shape_table_off_256_compute_units(cus):
     """The table's thresholds are all relative to the compute-unit count but were measured at 256.  On other counts
