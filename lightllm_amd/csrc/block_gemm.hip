@@ -151,10 +151,8 @@ static bool stream_k_pays(int64_t tiles, int64_t KB, int cus, int64_t tiles_m) {
     // 640 x 7168 x 18432 123 / 104, 640 x 4096 x 7168 57 / 40, 700 x 5120 x 13824 93 / 67, 1280 x 5120 x 8192 96 / 69,
     // 1772 x 3760 x 27392 281 / 177; 1024 x 7168 x 18432, one workgroup per tile, 164 / 135)
     const int panel = tiles % tiles_m == 0 ? sk_panel_splits((int)tiles_m, (int)(tiles / tiles_m), (int)KB, cus) : 0;
-    // (one to three m tiles on a narrow N: the 128-row tiles are ahead, 462 x 1840 x 9344 28.7 us against 32.4, 443 x 2608
-    // x 10240 36.9 / 38.4, 266 x 1232 x 12928 25.5 / 30.2, 597 x 1296 x 11136 30.8 / 34.7; 684 x 1696 x 10112 36.1 / 33.7)
-    const bool few = tiles_m <= 2 ? tiles * 64 < 3 * (int64_t)cus || (tiles * 32 < 3 * (int64_t)cus && KB < 96)
-                                  : tiles_m == 3 && tiles * 64 < 5 * (int64_t)cus && KB < 96;
+    // (one m tile on a narrow N: the 128-row tiles are ahead; more are compared in pick_variant)
+    const bool few = tiles_m == 1 && (tiles * 64 < 3 * (int64_t)cus || (tiles * 32 < 3 * (int64_t)cus && KB < 96));
     // three m tiles under a short K or on a narrow N keep the name of the 256x128 tiles, which share K the same way and with which
     // launches by name are compared, although the panel split is ahead (600 x 5120 x 6144 52 us against 42, 768 x 2112 x 8192 36.5 /
     // 34.0); below K = 8192 AUTO runs them over M
@@ -880,11 +878,12 @@ static int pick_variant(int64_t M, int64_t N, int64_t K, int cus, bool allow_row
     if (KB <= 2) return MI355_GEMM_TILE128;
     const bool shares = M > 128 && stream_k_pays(t256, KB, cus, (M + 255) / 256);
     const bool small = t128 <= 2 * (int64_t)cus && (t256 < (int64_t)cus * 3 / 8 || KB <= 64);  // 128x128 tiles fit the device
-    // From three m tiles on a narrow N the 128x128 tiles, which share K in shorter runs, are ahead of the panel split (us, panel /
-    // 128x128: 517 x 611 x 12288 31.6 / 21.2, 1058 x 128 x 23168 31.5 / 18.3, 1392 x 528 x 10112 33.9 / 29.1).  The panel's estimate
-    // is low where the tiles are few; with 8 % on it 76 of 1535 shapes of 513 rows and more with up to 36 256x256 tiles run more
-    // than 2 % behind the faster of the two, 15 % at most (all of them on the panel split: 562, 1.8 times).
-    const bool tiles128 = shares && small && M > 512 &&
+    // On a narrow N the 128x128 tiles, which share K in shorter runs, are ahead of the panel split (us, panel / 128x128: 517 x 611 x
+    // 12288 31.6 / 21.2, 1058 x 128 x 23168 31.5 / 18.3, 462 x 1840 x 9344 32.4 / 28.7; 403 x 1232 x 32128 40.1 / 51.5).  The panel's
+    // estimate is low where the tiles are few; with 8 % on it 76 of 1535 shapes of 513 rows and more with up to 36 256x256 tiles run
+    // more than 2 % behind the faster of the two, 15 % at most (all of them on the panel split: 562, 1.8 times).  Two m tiles are
+    // compared below three 32nds of the units, beyond which the panel split is ahead.
+    const bool tiles128 = shares && small && (M > 512 || (M > 256 && t256 * 32 < 3 * (int64_t)cus)) &&
                           1.08 * other_ns(M, N, K, MI355_GEMM_TILE256_STREAMK, SIZE_MAX, cus) > other_ns(M, N, K, MI355_GEMM_TILE128, SIZE_MAX, cus);
     if (shares && allow_streamk && !tiles128) return MI355_GEMM_TILE256_STREAMK;
     // 257..384 rows leave the second 256-row tile at most half full; where the 256x256 tiles need a second round

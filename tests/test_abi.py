@@ -376,7 +376,7 @@ def test_over_m_query_without_a_workspace():
     from lightllm_amd import _lib
 
     lib = _lib.lib()
-    for shape in [(300, 1024, 18432), (202, 705, 18816), (768, 2112, 8192), (487, 2768, 11008)]:
+    for shape in [(300, 1024, 18432), (202, 705, 18816), (768, 2112, 8192), (124, 15460, 14592)]:
         over = [lib.mi355_block_fp8_gemm_over_m(*shape, ws_bytes, 256) for ws_bytes in (0, 65536, 65536 + (8 << 20), 1 << 26, 1 << 34)]
         assert over == [1, 1, 1, 0, 0], (shape, over)
 
@@ -456,14 +456,15 @@ def test_no_stream_k_without_its_workspace():
 
 
 def test_panel_split_on_a_narrow_n():
-    """From three m tiles on the panel split of K is taken only where it is ahead of the 128x128 tiles with K shared (us, panel /
-    128x128: 517 x 611 x 12288 31.6 / 21.2, 1058 x 128 x 23168 31.5 / 18.3, 1392 x 528 x 10112 33.9 / 29.1)."""
+    """From 257 rows on the panel split of K is taken only where it is ahead of the 128x128 tiles with K shared (us, panel / 128x128:
+    517 x 611 x 12288 31.6 / 21.2, 1058 x 128 x 23168 31.5 / 18.3, 1392 x 528 x 10112 33.9 / 29.1, 403 x 1232 x 32128 40.1 / 51.5)."""
     from lightllm_amd import _lib
 
     lib = _lib.lib()
     T128, STREAMK = 2, 8
     for shape, want in [((517, 611, 12288), T128), ((1058, 128, 23168), T128), ((1392, 528, 10112), T128), ((787, 912, 7936), T128),
-                        ((1457, 224, 24448), T128), ((1772, 3760, 27392), STREAMK), ((640, 7168, 18432), STREAMK), ((1024, 2560, 14336), STREAMK)]:
+                        ((1457, 224, 24448), T128), ((1772, 3760, 27392), STREAMK), ((403, 1232, 32128), STREAMK), ((474, 1280, 28160), STREAMK),
+                        ((462, 1840, 9344), T128), ((640, 7168, 18432), STREAMK), ((1024, 2560, 14336), STREAMK)]:
         assert lib.mi355_block_fp8_gemm_plan(*shape, 1 << 34, 256) == want, shape
 
 
