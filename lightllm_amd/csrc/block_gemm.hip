@@ -853,8 +853,8 @@ static double other_ns(int64_t M, int64_t N, int64_t K, int variant, size_t ws_b
 //   M <= 64                                          weight streaming (M > 48 and N/128 about the unit count, or M > 32 in
 //                                                    more than five rounds: the kernel that shares the activation block
 //                                                    in the workgroup)
-//   few 256x256 tiles, long K                        stream-K (the plain loop would leave most units idle), from 513 rows on
-//                                                    where the 128x128 tiles are not estimated ahead
+//   few 256x256 tiles, long K                        stream-K (the plain loop would leave most units idle), from 513 rows on,
+//                                                    on few tiles from 257, where the 128x128 tiles are not estimated ahead
 //   128x128 tiles fit one round of two per unit and
 //     (few 256x256 tiles or a short K)               128x128 tiles, K shared between workgroups when they are few
 //                                                    (M >= 768 and N <= 3072: 256x128 tiles with K shared)
